@@ -32,26 +32,26 @@ WEIGHTS_SEED = 20    # of a model's weights: one checkpoint for all prompts
 def listed():
     return [
         # one key projection of a decode step: the smallest call, launch and latency
-        {"name": "k_proj, 1 row", "what": "linear", "rows": 1, "out": 1024, "in": 4096},
+        {"name": "k_proj 1 row", "what": "linear", "rows": 1, "out": 1024, "in": 4096},
         # what a decoder layer asks of the linears for one token
-        {"name": "layer, 1 row", "what": "row", "hidden": 4096, "kv": 1024, "ffn": 12288},
+        {"name": "layer 1 row", "what": "row", "hidden": 4096, "kv": 1024, "ffn": 12288},
         # a handful of sequences decoded together, or a draft of five tokens checked
-        {"name": "o_proj, 5 rows", "what": "linear", "rows": 5, "out": 4096, "in": 4096},
+        {"name": "o_proj 5 rows", "what": "linear", "rows": 5, "out": 4096, "in": 4096},
         # a larger batch, and rows that fill no tile
-        {"name": "down_proj, 57 rows", "what": "linear", "rows": 57, "out": 4096, "in": 12288},
+        {"name": "down_proj 57 rows", "what": "linear", "rows": 57, "out": 4096, "in": 12288},
         # the prompt length the benchmark is quoted on, at the fused gate and up call site
-        {"name": "gate_up, 322 rows", "what": "linear", "rows": 322, "out": 24576, "in": 4096},
+        {"name": "gate_up 322 rows", "what": "linear", "rows": 322, "out": 24576, "in": 4096},
         # a long prompt
-        {"name": "gate_proj, 2047 rows", "what": "linear", "rows": 2047, "out": 12288, "in": 4096},
+        {"name": "gate_proj 2047 rows", "what": "linear", "rows": 2047, "out": 12288, "in": 4096},
         # the forward pass around the layer at the 8B sizes (four of its layers): prompt, and an answer
-        {"name": "qwen3, prompt", "what": "prompt", "model": "qwen3", "width": 4096, "layers": 4, "tokens": 322},
-        {"name": "qwen3, answer", "what": "generate", "model": "qwen3", "width": 4096, "layers": 4, "tokens": 40, "new": 64},
+        {"name": "qwen3 prompt", "what": "prompt", "model": "qwen3", "width": 4096, "layers": 4, "tokens": 322},
+        {"name": "qwen3 answer", "what": "generate", "model": "qwen3", "width": 4096, "layers": 4, "tokens": 40, "new": 64},
         # the models with bfloat16 weights at the benchmark's 2k sizes: a long document, and an answer
-        {"name": "takosun, prompt", "what": "prompt", "model": "takosun", "width": 2048, "layers": 4, "tokens": 4095},
-        {"name": "takosun, answer", "what": "generate", "model": "takosun", "width": 2048, "layers": 4, "tokens": 33, "new": 64},
-        {"name": "dimesun, prompt", "what": "prompt", "model": "dimesun", "width": 2048, "layers": 2, "tokens": 2048},
+        {"name": "takosun prompt", "what": "prompt", "model": "takosun", "width": 2048, "layers": 4, "tokens": 4095},
+        {"name": "takosun answer", "what": "generate", "model": "takosun", "width": 2048, "layers": 4, "tokens": 33, "new": 64},
+        {"name": "dimesun prompt", "what": "prompt", "model": "dimesun", "width": 2048, "layers": 2, "tokens": 2048},
         # a caller that samples by itself: one call and one row of logits a token
-        {"name": "dimesun, steps", "what": "steps", "model": "dimesun", "width": 2048, "layers": 2, "tokens": 33, "new": 32},
+        {"name": "dimesun steps", "what": "steps", "model": "dimesun", "width": 2048, "layers": 2, "tokens": 33, "new": 32},
     ]
 
 
