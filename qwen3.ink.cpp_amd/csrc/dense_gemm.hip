@@ -1,43 +1,117 @@
 // C = A W^T on the matrix cores for weights in bfloat16 (v_mfma_f32_32x32x16_bf16) or float
 // (v_mfma_f32_32x32x2_f32: true 32-bit products and sums).
 //
-// A workgroup of four waves takes a BM x BN tile, a wave a quarter of it in 32 x 32 pieces.  K goes in steps of
-// 128 bytes per row; a step's rows are copied global -> LDS by direct 16-byte loads, two stages, the next step's
-// copies in flight while the current one is multiplied.  In LDS chunk c of row r sits at place c ^ (r & 7), so that
-// the 32 rows a wave reads at one chunk column spread over the banks.  A fragment is the same 16 bytes per lane for
-// both types: lane l holds row l & 31, chunk 2 kk + (l >> 5).
+// A workgroup takes a BM x BN tile, each of its waves an equal part of it in 32 x 32 pieces.  K goes in steps of 128 bytes
+// per row; a step's rows are copied global -> LDS by direct 16-byte loads into one of STAGES stages, later steps' copies in
+// flight while one is multiplied.  In LDS chunk c of row r sits at place c ^ (r & 7), so that the 32 rows a wave reads at one
+// chunk column spread over the banks.  A fragment is the same 16 bytes per lane for both types: lane l holds row l & 31,
+// chunk 2 kk + (l >> 5).
+//
+// What bounds it: bytes per product.  A 128 x 128 tile asks the L2 for 64 bytes a clock and CU at the matrix cores' full rate,
+// which is all the L2 gives, and reads LDS as fast as LDS goes; a 256 x 256 tile asks for half of the one and three quarters of
+// the other.  4095 x 12288 x 2048 in bfloat16 with the gated epilogue: 340 us with 128 x 128 tiles whose copies the compiler
+// waited for ahead of every step's first LDS read (see lds16), 210 us = 980 TFLOP/s with 256 x 256.  4095 x 2048 x 6144: 140 us and
+// 120 us, 2048 x 2048 x 2048: 47 us and 29 us.
 #include "dense_common.h"
 
 namespace a81w41 {
 namespace {
 
-__device__ __forceinline__ void mma(f32x16& acc, const uint4& a, const uint4& b, bf16*) {
+__device__ __forceinline__ void mma(f32x16& acc, const lds16& a, const lds16& b, bf16*) {
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&a), *reinterpret_cast<const bf16x8*>(&b), acc, 0, 0, 0);
 }
-__device__ __forceinline__ void mma(f32x16& acc, const uint4& a, const uint4& b, float*) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.x), __uint_as_float(b.x), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.y), __uint_as_float(b.y), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
+__device__ __forceinline__ void mma(f32x16& acc, const lds16& a, const lds16& b, float*) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[0]), __uint_as_float(b[0]), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[1]), __uint_as_float(b[1]), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[2]), __uint_as_float(b[2]), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[3]), __uint_as_float(b[3]), acc, 0, 0, 0);
 }
 
 struct NoHeads {};
 
-// X: HeadRows<T> with the epilogue kHeads, NoHeads with the others
-template <typename T, int BM, int BN, Epilogue EPI, typename X>
-__global__ __launch_bounds__(256, 2) void dense_gemm_kernel(GemmArgs g, X heads) {
-    constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 32, FN = WN / 32;
-    constexpr int LA = BM / 32, LB = BN / 32;  // direct copies per thread and stage
+// the value of the lane whose number differs in the lowest bit
+__device__ __forceinline__ float swap_neighbours(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
+}
+// At most `pending` of this wave's vector-memory operations are outstanding, and none of its LDS reads; then everybody's.
+template <int PENDING>
+__device__ __forceinline__ void wait_copies_and_meet() {
+    __builtin_amdgcn_s_waitcnt((PENDING & 15) | (PENDING >> 4) << 14 | 0x0070);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// Results of a wave's 32 x 32 pieces: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32.
+template <typename T, int FM, int FN, Epilogue EPI, typename X>
+__device__ __forceinline__ void store_pieces(const GemmArgs& g, const X& heads, const f32x16 (&acc)[FM][FN], int m0, int rows, int wm, int col0,
+                                             long long batch) {
+    const int lane = threadIdx.x & 63, l31 = lane & 31, half = lane >> 5;
+    [[maybe_unused]] int pos = 0;
+    if constexpr (EPI == Epilogue::kHeads) pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1);
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            const int col = col0 + j * 32 + l31, r0 = wm + i * 32 + 4 * half;
+            if constexpr (EPI == Epilogue::kGatedPair) {
+                // Lanes 16 .. 31 and 48 .. 63 hold the ups of the 16 lanes before them.  Of two rows v, v + 1 the gates of the
+                // second and the ups of the first trade places: every lane then has both of one row, and no unit is formed twice.
+                const int odd = (lane >> 4) & 1;
+                T* dst = static_cast<T*>(g.C) + (col >> 5) * 16 + (col & 15);
+#pragma unroll
+                for (int v = 0; v < 16; v += 2) {
+                    const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i][j][v]), __float_as_uint(acc[i][j][v + 1]), false, false);
+                    const float unit = gated_unit(g.unit, __uint_as_float(both[0]), __uint_as_float(both[1]));
+                    const int r = r0 + 8 * (v >> 2) + (v & 3) + odd;
+                    if (r < rows && col < g.N) dst[(size_t)(m0 + r) * g.ldc] = (T)unit;
+                }
+                continue;
+            }
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int r = r0 + 8 * (v >> 2) + (v & 3);
+                const size_t row = m0 + r;
+                if constexpr (EPI == Epilogue::kHeads) {
+                    const float other = swap_neighbours(acc[i][j][v]);
+                    if (r < rows && col < g.N) store_head_column(heads, pos, (int)row, col, acc[i][j][v], other);
+                } else if (r < rows && col < g.N) {
+                    if constexpr (EPI == Epilogue::kFloat) {
+                        (static_cast<float*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = acc[i][j][v];
+                    } else {
+                        float f = acc[i][j][v];
+                        if constexpr (EPI == Epilogue::kHeadGate) f *= sigmoid(g.head_gate[row * g.ld_gate + batch]);
+                        (static_cast<T*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = (T)f;
+                    }
+                }
+            }
+        }
+}
+
+// Rows of tiles that are walked together: an XCD's workgroups then share these rows and a few column panels in its L2.
+constexpr int kBandRows = 2048;
+
+// X: HeadRows<T> with the epilogue kHeads, NoHeads with the others.  STAGES: how many steps LDS holds; all but one are under way.
+// PIPE: a step's operands are read one 16-byte column ahead of their products; without it the other workgroup of the CU
+// fills the wait.
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PIPE, Epilogue EPI, typename X>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(GemmArgs g, X heads) {
+    constexpr int kThreads = 64 * WAVES_M * WAVES_N;
+    constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 32, FN = WN / 32;
+    constexpr int LA = BM * 8 / kThreads, LB = BN * 8 / kThreads;  // direct copies per thread and stage
     constexpr int kStage = (BM + BN) * 128;
-    __shared__ __attribute__((aligned(128))) uint8_t lds[2 * kStage];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    static_assert(STAGES >= 2 && (STAGES - 2) * (LA + LB) < 64, "copies a wait can leave outstanding");
+    __shared__ __attribute__((aligned(128))) uint8_t lds[STAGES * kStage];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l31 = lane & 31, half = lane >> 5;
-    // Tiles in the order (column panel, row tile), dealt to the XCDs in contiguous runs: a panel's weights then come
-    // into one L2.
+    // Tiles dealt to the XCDs in contiguous runs, in bands of kBandRows rows and inside one column panel after the other; a
+    // grouped product's in the order (column panel, row tile): a panel's weights come into one L2.
     const int n_nt = (g.N + BN - 1) / BN, n_mt = gridDim.x / n_nt;
     const int q = gridDim.x >> 3, r8 = gridDim.x & 7, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
     const int t = xcd < r8 ? xcd * (q + 1) + idx : r8 * (q + 1) + (xcd - r8) * q + idx;
-    const int mt = t % n_mt, nt = t / n_mt;
+    const int band = g.tiles ? n_mt : kBandRows / BM, first = t / (band * n_nt) * band;
+    const int high = min(band, n_mt - first), at = t - first * n_nt;
+    const int mt = first + at % high, nt = at / high;
     int m0 = mt * BM, rows = g.M - m0;
     long long batch = blockIdx.y;
     if (g.tiles) {
@@ -53,22 +127,22 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(GemmArgs g, X heads)
     const uint8_t *a_src[LA], *b_src[LB];
 #pragma unroll
     for (int i = 0; i < LA; i++) {
-        const int c = i * 256 + tid, r = c >> 3;
+        const int c = i * kThreads + tid, r = c >> 3;
         int row = m0 + min(r, rows - 1);
         if (g.a_rows) row = g.a_rows[row];
         a_src[i] = A + (size_t)row * g.lda * sizeof(T) + (((c & 7) ^ (r & 7)) << 4);
     }
 #pragma unroll
     for (int i = 0; i < LB; i++) {
-        const int c = i * 256 + tid, r = c >> 3;
+        const int c = i * kThreads + tid, r = c >> 3;
         b_src[i] = W + (size_t)min(n0 + r, g.N - 1) * g.ldw * sizeof(T) + (((c & 7) ^ (r & 7)) << 4);
     }
     auto copy_step = [&](int step, int stage) {
         uint8_t* base = lds + stage * kStage + wave * 1024;
 #pragma unroll
-        for (int i = 0; i < LA; i++) copy16_to_lds(a_src[i] + (size_t)step * 128, base + i * 4096);
+        for (int i = 0; i < LA; i++) copy16_to_lds(a_src[i] + (size_t)step * 128, base + i * kThreads * 16);
 #pragma unroll
-        for (int i = 0; i < LB; i++) copy16_to_lds(b_src[i] + (size_t)step * 128, base + BM * 128 + i * 4096);
+        for (int i = 0; i < LB; i++) copy16_to_lds(b_src[i] + (size_t)step * 128, base + BM * 128 + i * kThreads * 16);
     };
     f32x16 acc[FM][FN];
 #pragma unroll
@@ -77,81 +151,72 @@ __global__ __launch_bounds__(256, 2) void dense_gemm_kernel(GemmArgs g, X heads)
         for (int j = 0; j < FN; j++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-    const int wm = (wave & 1) * WM, wn = (wave >> 1) * WN;
+    const int wm = (wave % WAVES_M) * WM, wn = (wave / WAVES_M) * WN;
     const int n_steps = g.K * (int)sizeof(T) / 128;
-    copy_step(0, 0);
+    for (int step = 0; step < STAGES - 1 && step < n_steps; step++) copy_step(step, step);
+    int stage = 0;
     for (int step = 0; step < n_steps; step++) {
-        // this wave's copies of the step are in LDS, then everybody's; and nobody still reads the other stage
-        __builtin_amdgcn_s_waitcnt(0x0070);
-        __syncthreads();
-        if (step + 1 < n_steps) copy_step(step + 1, (step + 1) & 1);
-        const uint8_t* sa = lds + (step & 1) * kStage;
+        // the copies of the step are in LDS, later ones may be under way; and nobody still reads the stage before it
+        if (step + STAGES - 2 < n_steps)
+            wait_copies_and_meet<(STAGES - 2) * (LA + LB)>();
+        else
+            wait_copies_and_meet<0>();
+        if (step + STAGES - 1 < n_steps) copy_step(step + STAGES - 1, stage ? stage - 1 : STAGES - 1);
+        const uint8_t* sa = lds + stage * kStage;
         const uint8_t* sb = sa + BM * 128;
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-            uint4 a[FM], b[FN];
+        stage = stage + 1 < STAGES ? stage + 1 : 0;
+        lds16 a[2][FM], b[2][FN];
+        auto read = [&](int kk) {
 #pragma unroll
             for (int i = 0; i < FM; i++) {
                 const int r = wm + i * 32 + l31;
-                a[i] = *reinterpret_cast<const uint4*>(sa + r * 128 + (((2 * kk + half) ^ (r & 7)) << 4));
+                a[kk & 1][i] = *reinterpret_cast<const lds16*>(sa + r * 128 + (((2 * kk + half) ^ (r & 7)) << 4));
             }
 #pragma unroll
             for (int j = 0; j < FN; j++) {
                 const int r = wn + j * 32 + l31;
-                b[j] = *reinterpret_cast<const uint4*>(sb + r * 128 + (((2 * kk + half) ^ (r & 7)) << 4));
+                b[kk & 1][j] = *reinterpret_cast<const lds16*>(sb + r * 128 + (((2 * kk + half) ^ (r & 7)) << 4));
             }
+        };
+        if constexpr (PIPE) read(0);
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            if constexpr (PIPE) __builtin_amdgcn_sched_barrier(0);
+            if (!PIPE) read(kk);
+            if (PIPE && kk < 3) read(kk + 1);
+            if constexpr (PIPE) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < FM; i++)
 #pragma unroll
-                for (int j = 0; j < FN; j++) mma(acc[i][j], a[i], b[j], static_cast<T*>(nullptr));
+                for (int j = 0; j < FN; j++) mma(acc[i][j], a[kk & 1][i], b[kk & 1][j], static_cast<T*>(nullptr));
         }
     }
-    [[maybe_unused]] int pos = 0;
-    if constexpr (EPI == Epilogue::kHeads) pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1);
-    // register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32 of a piece
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const int col = n0 + wn + j * 32 + l31;
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int r = wm + i * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
-                const size_t row = m0 + r;
-                if constexpr (EPI == Epilogue::kGatedPair) {
-                    const float up = __shfl_xor(acc[i][j][v], 16, 64);
-                    if (r < rows && col < g.N && !(lane & 16))
-                        static_cast<T*>(g.C)[row * g.ldc + (col >> 5) * 16 + (col & 15)] = (T)gated_unit(g.unit, acc[i][j][v], up);
-                } else if constexpr (EPI == Epilogue::kHeads) {
-                    const float other = __shfl_xor(acc[i][j][v], 1, 64);
-                    if (r < rows && col < g.N) store_head_column(heads, pos, (int)row, col, acc[i][j][v], other);
-                } else if (r < rows && col < g.N) {
-                    if constexpr (EPI == Epilogue::kFloat) {
-                        (static_cast<float*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = acc[i][j][v];
-                    } else {
-                        float f = acc[i][j][v];
-                        if constexpr (EPI == Epilogue::kHeadGate) f *= sigmoid(g.head_gate[row * g.ld_gate + batch]);
-                        (static_cast<T*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = (T)f;
-                    }
-                }
-            }
-        }
+    store_pieces<T, FM, FN, EPI>(g, heads, acc, m0, rows, wm, n0 + wn, batch);
 }
 
-template <typename T, int BM, int BN, Epilogue EPI, typename X>
+// 256 x 256 tiles, one workgroup per CU, or 128 x 128, two per CU.  At K = 2048 a round of 256 large tiles takes 65 us whether
+// it is full or not, small tiles 44 us per 512 of them.
+bool large_tiles_preferred(long long large, long long small) { return (large + 255) / 256 * 750 <= small; }
+
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PIPE, Epilogue EPI, typename X>
 hipError_t launch_kernel(const GemmArgs& g, const X& heads, hipStream_t s) {
     const int n_mt = g.tiles ? g.max_tiles : (g.M + BM - 1) / BM, n_nt = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((dense_gemm_kernel<T, BM, BN, EPI, X>), dim3(n_mt * n_nt, g.batches), dim3(256), 0, s, g, heads);
+    hipLaunchKernelGGL((dense_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, STAGES, PIPE, EPI, X>), dim3(n_mt * n_nt, g.batches),
+                       dim3(64 * WAVES_M * WAVES_N), 0, s, g, heads);
     return hipGetLastError();
 }
 
 template <typename T, Epilogue EPI, typename X>
 hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
-    // large tiles where they still give every CU work; a grouped product's row tiles are kGroupTileRows high
-    const long long big = (long long)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.batches;
-    if (!g.tiles && g.M > 64 && big >= 192) return launch_kernel<T, 128, 128, EPI>(g, heads, s);
-    if (g.tiles && g.N >= 1024) return launch_kernel<T, kGroupTileRows, 128, EPI>(g, heads, s);
-    return launch_kernel<T, 64, 64, EPI>(g, heads, s);
+    auto tiles = [&](int size) { return (long long)((g.M + size - 1) / size) * ((g.N + size - 1) / size) * g.batches; };
+    // A product of 192 to 256 tiles of 128 x 128 has one for a CU: it takes twice the waves and four stages in LDS (2048^3: 29 us
+    // against 36 us with two).  Fewer give too few CUs work.  A grouped product's row tiles are kGroupTileRows high.
+    if constexpr (sizeof(T) == 2)
+        if (!g.tiles && large_tiles_preferred(tiles(256), tiles(128))) return launch_kernel<T, 256, 256, 2, 4, 2, true, EPI>(g, heads, s);
+    if (!g.tiles && g.M > 64 && tiles(128) > 256) return launch_kernel<T, 128, 128, 2, 2, 2, false, EPI>(g, heads, s);
+    if (!g.tiles && g.M > 64 && tiles(128) >= 192) return launch_kernel<T, 128, 128, 2, 4, 4, true, EPI>(g, heads, s);
+    if (g.tiles && g.N >= 1024) return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, false, EPI>(g, heads, s);
+    return launch_kernel<T, 64, 64, 2, 2, 4, false, EPI>(g, heads, s);
 }
 
 }  // namespace

@@ -1,0 +1,50 @@
+"""The tile sizes of the dense product: each chosen by size, all with the same bits for a row whatever the rows around it."""
+import numpy as np
+import pytest
+
+from tests import dimesun_fixture as dx
+from tests import takosun_fixture as tx
+
+pytestmark = pytest.mark.gpu
+
+
+# 256 x 256 tiles; 128 x 128 two per CU; 128 x 128 alone on a CU with four stages, from fewer steps than stages on
+@pytest.mark.parametrize("M,N,K", [(2047, 6136, 64), (1793, 6400, 192), (2300, 2050, 128), (2045, 2000, 64), (2045, 1990, 192),
+                                   (1921, 2048, 320)])
+def test_rows_of_a_product(pkg, M, N, K):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = torch.randn(N, K, device="cuda", generator=g).bfloat16()
+    got = pkg.ops.dense_gemm(a, w, K)
+    want = a.double() @ w.double().t()
+    # K exact products of size about 1, K sums rounded to 24 bits
+    assert (got.double() - want).abs().max().item() <= K * 2.0 ** -24 * 4 * K ** 0.5
+    for r in (0, 31, 64, M - 1):   # a single row runs on 64 x 64 tiles
+        assert torch.equal(pkg.ops.dense_gemm(a[r:r + 1], w, K)[0], got[r]), r
+
+
+def _same_in_portions(pkg, cfg, n, cuts):
+    """One pass over n tokens on large tiles, and the same in portions on small ones, attention by the kernel that goes row by row."""
+    ids = np.random.default_rng(5).integers(0, cfg["vocab"], n).astype(np.int32)
+    want = list(range(0, n, 97)) + [n - 1]
+    model = pkg.Model.random(cfg, n, "bfloat16", seed=3)
+    model.set_option("attention", 1)
+    whole = model.forward(ids, want)
+    model.reset()
+    parts, at = [], 0
+    while at < n:
+        m = min(cuts, n - at)
+        parts.append(model.forward(ids[at:at + m], [w - at for w in want if at <= w < at + m]))
+        at += m
+    assert np.isfinite(whole).all() and np.array_equal(whole, np.concatenate(parts))
+
+
+def test_gated_pairs_on_large_tiles(pkg):
+    cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.dense(6100))])
+    _same_in_portions(pkg, cfg, 2100, 64)
+
+
+def test_head_columns_on_large_tiles(pkg):
+    cfg = dx.config(64, 64, [dx.attention(32, 8, 128, 128, 70, 0.09, rot_dims=64, mlp=None)], (0, 1, 1))
+    _same_in_portions(pkg, cfg, 2100, 60)
