@@ -4,6 +4,7 @@
 //   rows      the queries of a group of heads look at the rows of their key/value head, [value | key] (grouped attention);
 //   expanded  keys and values of every head were formed beforehand: a key is [own part | part shared by all heads],
 //             values come transposed ([value column][key]).
+// The first, and the second for few rows, are here, the others in attend_prompt.hip.
 //
 // A wave owns 16 (or 2 x 16) query rows.  It forms the scores transposed, S^T = K Q^T (v_mfma_f32_16x16x32_bf16 with
 // the keys as rows), so that lane l holds scores of query l % 16 only: keys 16 t + 4 (l / 16) + i.  These registers
@@ -28,14 +29,12 @@ constexpr float kLowest = -1e30f;
 // key part, 0 otherwise).  KT keys per tile, NBUF tiles in LDS.
 // COLS (few rows): all four waves take the same query rows; each scores its 16 keys of a tile, the scores meet in LDS,
 // and each sums its quarter of the value columns.
-template <int DK, int DV, int KEY0, int WAVES, int QS, int KT, int NBUF, bool EXPANDED, bool COLS>
+template <int DK, int DV, int KEY0, int WAVES, int QS, int KT, int NBUF, bool COLS>
 __global__ __launch_bounds__(64 * WAVES, 1) void attend_kernel(AttendArgs<bf16> a) {
     constexpr int CK = DK / 8;                    // 16-byte chunks of a key row
-    constexpr int kKeyBytes = KT * DK * 2, kValueBytes = EXPANDED ? DV * KT * 2 : 0;
-    constexpr int CV = KT / 8;                    // chunks of a value row (transposed)
-    constexpr int kBuf = kKeyBytes + kValueBytes;
+    constexpr int kBuf = KT * DK * 2;
     constexpr int KS = (DK - KEY0) / 32, VF = DV / 16 / (COLS ? WAVES : 1), kRows = 16 * QS * (COLS ? 1 : WAVES);
-    static_assert(DK % 64 == 0 && KEY0 % 32 == 0 && DV % (COLS ? 16 * WAVES : 16) == 0 && KT % 32 == 0 && (!EXPANDED || CV == 8), "tile sizes");
+    static_assert(DK % 64 == 0 && KEY0 % 32 == 0 && DV % (COLS ? 16 * WAVES : 16) == 0 && KT % 32 == 0, "tile sizes");
     constexpr int kScoreRow = 16 * QS + 4;  // floats of a key's scores in LDS: lane groups fall into different banks
     static_assert(!COLS || KT == 16 * WAVES, "a wave scores 16 keys of a tile");
     __shared__ __attribute__((aligned(128))) uint8_t lds[NBUF * kBuf];
@@ -57,8 +56,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attend_kernel(AttendArgs<bf16> 
         key_begin = min(max(begin, key_begin), key_end);
     }
     const bf16* k_own = a.k_own + z * a.k_own_head;
-    const bf16* v_t = EXPANDED ? a.v_t + (size_t)z * a.dv * a.ld_v : nullptr;
-    const int own_chunks = a.k_own_width >> 3, all_chunks = own_chunks + (EXPANDED ? a.k_shared_width >> 3 : 0);
+    const int own_chunks = a.k_own_width >> 3;
     auto copy_tile = [&](int key0, int buf) {
         uint8_t* base = lds + buf * kBuf;
         for (int n = wave; n < KT * CK / 64; n += WAVES) {
@@ -72,15 +70,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attend_kernel(AttendArgs<bf16> 
                     src += a.v_width + (c - KEY0 / 8) * 8;
             } else if (c < own_chunks)
                 src += c * 8;
-            else if (EXPANDED && c < all_chunks)
-                src = a.k_shared + key * a.ld_k_shared + (c - own_chunks) * 8;
             copy16_to_lds(src, base + n * 1024);
         }
-        if constexpr (EXPANDED)
-            for (int n = wave; n < DV * CV / 64; n += WAVES) {
-                const int q = n * 64 + lane, r = q >> 3, c = (q & 7) ^ (r & 7);
-                copy16_to_lds(v_t + (size_t)min(r, a.dv - 1) * a.ld_v + key0 + c * 8, base + kKeyBytes + n * 1024);
-            }
     };
     // query operands
     bf16x8 qf[QS][KS];
@@ -96,7 +87,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attend_kernel(AttendArgs<bf16> 
         for (int k = 0; k < KS; k++) {
             uint4 u = make_uint4(0, 0, 0, 0);
             const int c = k * 4 + g;
-            if (c < all_chunks) u = *reinterpret_cast<const uint4*>(src + c * 8);
+            if (c < own_chunks) u = *reinterpret_cast<const uint4*>(src + c * 8);
             qf[s][k] = *reinterpret_cast<const bf16x8*>(&u);
         }
     }
@@ -114,12 +105,10 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attend_kernel(AttendArgs<bf16> 
     // i names four columns of key 4 g + i / 4 and receives its own column of the four keys.  The exclusive or of the chunk
     // places touches the low three bits of 2 f + ..., so four offsets serve all f.
     int value_at[4];
-    if constexpr (!EXPANDED) {
 #pragma unroll
-        for (int f = 0; f < 4; f++) {
-            const int r = 4 * g + (l15 >> 2);
-            value_at[f] = r * (DK * 2) + (((2 * (f0 + f) + ((l15 >> 1) & 1)) ^ (r & 7)) << 4) + (l15 & 1) * 8;
-        }
+    for (int f = 0; f < 4; f++) {
+        const int r = 4 * g + (l15 >> 2);
+        value_at[f] = r * (DK * 2) + (((2 * (f0 + f) + ((l15 >> 1) & 1)) ^ (r & 7)) << 4) + (l15 & 1) * 8;
     }
     const float scale = a.scale * kLog2e;
     const int n_tiles = (key_end - key_begin + KT - 1) / KT;
@@ -134,7 +123,6 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attend_kernel(AttendArgs<bf16> 
         __syncthreads();
         if (NBUF > 1 && tile + 1 < n_tiles) copy_tile(key0 + KT, (tile + 1) % NBUF);
         const uint8_t* kb = lds + (tile % NBUF) * kBuf;
-        const uint8_t* vb = kb + kKeyBytes;
         f32x4 sc[QS][KT / 16];
         auto score = [&](int t) {
 #pragma unroll
@@ -200,22 +188,11 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attend_kernel(AttendArgs<bf16> 
         for (int u = 0; u < KT / 32; u++)
 #pragma unroll
             for (int f = 0; f < VF; f++) {
-                bf16x8 vf;
-                if constexpr (EXPANDED) {
-                    const int r = (f0 + f) * 16 + l15;
-                    const uint8_t* row = vb + r * (KT * 2);
-                    const int c0 = u * 4 + (g >> 1);
-                    uint2 lo = *reinterpret_cast<const uint2*>(row + ((c0 ^ (r & 7)) << 4) + (g & 1) * 8);
-                    uint2 hi = *reinterpret_cast<const uint2*>(row + (((c0 + 2) ^ (r & 7)) << 4) + (g & 1) * 8);
-                    const uint4 w = make_uint4(lo.x, lo.y, hi.x, hi.y);
-                    vf = *reinterpret_cast<const bf16x8*>(&w);
-                } else {
-                    const uint8_t* at = kb + value_at[f & 3] + (f >> 2) * 128 + u * 32 * (DK * 2);
-                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at));
-                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 16 * (DK * 2)));
-                    const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                    vf = *reinterpret_cast<const bf16x8*>(&both);
-                }
+                const uint8_t* at = kb + value_at[f & 3] + (f >> 2) * 128 + u * 32 * (DK * 2);
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at));
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 16 * (DK * 2)));
+                const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                const bf16x8 vf = *reinterpret_cast<const bf16x8*>(&both);
 #pragma unroll
                 for (int s = 0; s < QS; s++) acc[s][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[s][u], acc[s][f], 0, 0, 0);
             }
@@ -278,27 +255,22 @@ __global__ __launch_bounds__(256) void merge_shares_kernel(AttendArgs<bf16> a, i
 }
 static_assert(kAttendMaxSplits <= 64, "the merge reads one share per lane");
 
-template <int DK, int DV, int KEY0, int WAVES, int QS, int KT, int NBUF, bool EXPANDED, bool COLS>
+template <int DK, int DV, int KEY0, int WAVES, int QS, int KT, int NBUF, bool COLS>
 hipError_t launch_kernel(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
     constexpr int rows = 16 * QS * (COLS ? 1 : WAVES);
-    hipLaunchKernelGGL((attend_kernel<DK, DV, KEY0, WAVES, QS, KT, NBUF, EXPANDED, COLS>), dim3((a.rows + rows - 1) / rows, heads, a.splits),
+    hipLaunchKernelGGL((attend_kernel<DK, DV, KEY0, WAVES, QS, KT, NBUF, COLS>), dim3((a.rows + rows - 1) / rows, heads, a.splits),
                        dim3(64 * WAVES), 0, s, a);
     return hipGetLastError();
 }
 template <int DK, int DV>
 hipError_t launch_shared(const AttendArgs<bf16>& a, hipStream_t s) {
-    return a.rows <= kAttendFewRows ? launch_kernel<DK, DV, 0, 4, 1, 64, 2, false, true>(a, 1, s)
-                                    : launch_kernel<DK, DV, 0, 4, 1, 32, 1, false, false>(a, 1, s);
+    return a.rows <= kAttendFewRows ? launch_kernel<DK, DV, 0, 4, 1, 64, 2, true>(a, 1, s)
+                                    : launch_kernel<DK, DV, 0, 4, 1, 32, 1, false>(a, 1, s);
 }
-// key and value columns: D at most each
-template <int D, int QS>
+// key and value columns: D at most each; few rows
+template <int D>
 hipError_t launch_rows(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
-    return a.rows <= kAttendFewRows ? launch_kernel<2 * D, D, D, 4, 1, 64, 2, false, true>(a, heads, s)
-                                    : launch_kernel<2 * D, D, D, 4, QS, 64, 2, false, false>(a, heads, s);
-}
-template <int DK, int DV>
-hipError_t launch_expanded(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
-    return launch_kernel<DK, DV, 0, 4, 2, 64, 2, true, false>(a, heads, s);
+    return launch_kernel<2 * D, D, D, 4, 1, 64, 2, true>(a, heads, s);
 }
 
 }  // namespace
@@ -315,17 +287,11 @@ hipError_t launch_attend_shared(const AttendArgs<bf16>& a, hipStream_t s) {
 }
 
 hipError_t launch_attend_rows(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
+    if (a.rows > kAttendFewRows) return launch_attend_rows_prompt(a, heads, s);
     const int widest = a.k_own_width > a.v_width ? a.k_own_width : a.v_width;
-    if (widest <= 64) return launch_rows<64, 2>(a, heads, s);
-    if (widest <= 128) return launch_rows<128, 2>(a, heads, s);
-    return launch_rows<256, 1>(a, heads, s);
-}
-
-hipError_t launch_attend_expanded(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
-    const int dk = a.k_own_width + a.k_shared_width;
-    if (dk <= 128 && a.dv <= 64) return launch_expanded<128, 64>(a, heads, s);
-    if (dk <= 192 && a.dv <= 128) return launch_expanded<192, 128>(a, heads, s);
-    return launch_expanded<320, 256>(a, heads, s);
+    if (widest <= 64) return launch_rows<64>(a, heads, s);
+    if (widest <= 128) return launch_rows<128>(a, heads, s);
+    return launch_rows<256>(a, heads, s);
 }
 
 hipError_t launch_merge_shares(const AttendArgs<bf16>& a, int heads, hipStream_t s) {

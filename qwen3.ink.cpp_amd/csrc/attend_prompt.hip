@@ -1,0 +1,325 @@
+// Causal attention of a prompt's many rows on the matrix cores, bfloat16, in two of attend_mfma.hip's forms:
+//   rows      the queries of a group of heads look at the rows of their key/value head, [value | key];
+//   expanded  a key is [own part | part shared by all heads], values come transposed ([value column][key]).
+//
+// A workgroup of KG x QW waves takes 32 QW query rows.  A wave owns 32 of them; KG waves share them, each with every KG-th tile of 64
+// keys, and meet at the end: a workgroup of two groups keeps two waves on every SIMD while its rows, and with them the
+// rows past the diagonal, stay few.  Scores are formed transposed, S^T = K Q^T (v_mfma_f32_32x32x16_bf16 with the keys
+// as rows), so that a lane holds scores of query l % 32 only.  Row r of a 32-key product is key r with bits 2 and 3
+// exchanged: register v of lane half h is then key 16 (v / 8) + 8 h + v % 8, and eight registers are, as they stand, the
+// B operand of a 16-key step of O^T = V^T P^T whose A operand is eight neighbouring keys.  Running maximum and sum are
+// one value per lane.  Scores, softmax and sums are fp32; the maximum follows every larger score, so that the heaviest
+// weight, 1, is exact in 16 bits (left behind by up to 2^8 it is not: 14 % more error for 8 % less time).
+//
+// A tile is copied global -> LDS by direct 16-byte loads, the next one while this one is worked on.  Key rows: chunk c of key k
+// at place c ^ (k % 4 + k / 8 % 2 * 4), so that eight rows r read at once fall on eight places; transposed values:
+// chunk c of column d at place c ^ d % 8.
+//
+// What bounds it: matrix ops and softmax of a SIMD's two waves, one after the other; then LDS, which gives an operand of 1 KiB
+// for every matrix op.  4095 rows of 16 heads, 192 + 128 columns: 117 us = 730 TFLOP/s, against 537 us with 16 x 16 matrix ops,
+// heads' rows dealt out one head after the other and one workgroup of four waves on a CU; 2048 rows in chunks of 1024, 16 heads
+// on 4 of 128 + 128 columns: 29 us against 71 us.
+#include "dense_common.h"
+
+namespace a81w41 {
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+typedef __attribute__((ext_vector_type(8))) short s16x8;
+typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLowest = -1e30f;
+constexpr int kTile = 64;      // keys
+
+__device__ __forceinline__ int place_of_key(int k) { return (k & 3) | (k >> 1 & 4); }
+// the larger, or the sum, of this lane's value and that of the other lane half
+__device__ __forceinline__ float other_half(float v) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(threadIdx.x & 32 ? both[0] : both[1]);
+}
+
+// DK: columns of a tile row; the scores take those from KEY0 on (rows form: the key part, 0 otherwise).  DV: value columns.
+template <int DK, int DV, int KEY0, int KG, int QW, bool EXPANDED>
+__global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kernel(AttendArgs<bf16> a) {
+    constexpr int CK = DK / 8, KS = (DK - KEY0) / 16, VF = DV / 32, kRows = 32 * QW;
+    constexpr int kKeyBytes = kTile * DK * 2, kBuf = kKeyBytes + (EXPANDED ? DV * kTile * 2 : 0);
+    constexpr int NK = kTile * CK / 64 / QW, NV = EXPANDED ? DV * 8 / 64 / QW : 0;  // copies of a wave and tile
+    static_assert(DK % 64 == 0 && DV % 32 == 0 && KEY0 % 64 == 0 && kTile * CK % (64 * QW) == 0 && DV * 8 % (64 * QW) == 0, "tile sizes");
+    static_assert(KG == 1 || 64 * 4 * (16 * VF + 2) * QW <= 2 * KG * kBuf, "the groups meet in LDS");
+    __shared__ __attribute__((aligned(128))) uint8_t lds[2 * KG * kBuf];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l31 = lane & 31, half = lane >> 5;
+    const int qw = wave % QW, kg = wave / QW;
+    // heads next to each other, the longest rows first: what is left over for a CU that is done is short
+    const int z = blockIdx.x, row0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * kRows;
+    const int pos = min(max(a.pos_dev[0], 0), a.max_seq - 1);
+    auto last_key = [&](int row) { return min(pos + row / a.rows_per_token, a.max_seq - 1); };
+    auto chunk_begin = [&](int key) { return a.chunk ? key - key % a.chunk : 0; };
+    const int wg_keys = last_key(min(row0 + kRows, a.rows) - 1) + 1;  // keys any row of the workgroup sees
+    int key_begin = chunk_begin(last_key(row0)), key_end = wg_keys;
+    if (a.splits > 1) {
+        const int from = chunk_begin(pos), all = last_key(a.rows - 1) + 1 - from;
+        const int share = ((all + a.splits - 1) / a.splits + kTile - 1) / kTile * kTile, begin = from + (int)blockIdx.z * share;
+        key_end = min(begin + share, wg_keys);
+        key_begin = min(max(begin, key_begin), key_end);
+    }
+    const int n_tiles = (key_end - key_begin + kTile - 1) / kTile, n_turns = (n_tiles + KG - 1) / KG;
+    const int own_chunks = a.k_own_width >> 3, all_chunks = own_chunks + (EXPANDED ? a.k_shared_width >> 3 : 0);
+
+    // This lane's 16 bytes of every copy, at the group's first tile; a turn moves them on by KG tiles.
+    const uint8_t* key_src[NK];
+    int key_step[NK];
+    const bf16* value_src[NV ? NV : 1];
+    uint8_t* const my_lds = lds + kg * 2 * kBuf;
+    auto key_place = [&](int n, int key, int* step) -> const uint8_t* {  // source of copy n if its row is that key
+        const int q = (n * QW + qw) * 64 + lane, r = q / CK, c = (q % CK) ^ place_of_key(r);
+        const bf16* src = a.k_own + z * a.k_own_head + (size_t)key * a.ld_k_own;
+        int ld = a.ld_k_own;
+        if constexpr (KEY0 > 0) {
+            if (c < KEY0 / 8)
+                src += c < (a.v_width >> 3) ? c * 8 : 0;
+            else if (c - KEY0 / 8 < own_chunks)
+                src += a.v_width + (c - KEY0 / 8) * 8;
+        } else if (c < own_chunks) {
+            src += c * 8;
+        } else if (EXPANDED && c < all_chunks) {
+            src = a.k_shared + (size_t)key * a.ld_k_shared + (c - own_chunks) * 8;
+            ld = a.ld_k_shared;
+        }
+        *step = ld * 2 * (KG * kTile);
+        return reinterpret_cast<const uint8_t*>(src);
+    };
+    auto row_of_copy = [&](int n) { return ((n * QW + qw) * 64 + lane) / CK; };
+#pragma unroll
+    for (int n = 0; n < NK; n++) key_src[n] = key_place(n, key_begin + kg * kTile + row_of_copy(n), &key_step[n]);
+    if constexpr (EXPANDED) {
+#pragma unroll
+        for (int n = 0; n < NV; n++) {
+            const int q = (n * QW + qw) * 64 + lane, r = q >> 3, c = (q & 7) ^ (r & 7);
+            value_src[n] = a.v_t + ((size_t)z * a.dv + min(r, a.dv - 1)) * a.ld_v + key_begin + kg * kTile + c * 8;
+        }
+    }
+    auto copy_tile = [&](int tile, int buf) {
+        uint8_t* base = my_lds + buf * kBuf + qw * 1024;
+        const int key0 = key_begin + tile * kTile;
+        if (key0 + kTile <= wg_keys) {
+#pragma unroll
+            for (int n = 0; n < NK; n++) {
+                copy16_to_lds(key_src[n], base + n * QW * 1024);
+                key_src[n] += key_step[n];
+            }
+        } else {  // the last rows stand in for those past the end
+#pragma unroll
+            for (int n = 0; n < NK; n++) {
+                int step;
+                copy16_to_lds(key_place(n, min(key0 + row_of_copy(n), wg_keys - 1), &step), base + n * QW * 1024);
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NV; n++) {
+            copy16_to_lds(value_src[n], base + kKeyBytes + n * QW * 1024);
+            value_src[n] += KG * kTile;
+        }
+    };
+
+    // Query operands; a negative scale is their sign, so that the largest score is the largest product.
+    const int wave_row0 = row0 + qw * 32, my_row = min(wave_row0 + l31, a.rows - 1), my_token = my_row / a.rows_per_token;
+    const int limit = last_key(my_row), first = chunk_begin(limit);
+    const int lowest_limit = last_key(min(wave_row0, a.rows - 1)), highest_limit = last_key(min(wave_row0 + 31, a.rows - 1));
+    const int highest_first = chunk_begin(highest_limit);
+    const float scale = fmaxf(fabsf(a.scale), 1e-30f) * kLog2e;  // a score of minus infinity times it stays that
+    bf16x8 qf[KS];
+    {
+        const bf16* src = a.q + z * a.q_head + (size_t)my_token * a.q_token + (my_row - my_token * a.rows_per_token) * a.ld_q;
+        const unsigned sign = a.scale < 0.f ? 0x80008000u : 0u;
+#pragma unroll
+        for (int k = 0; k < KS; k++) {
+            const int c = 2 * k + half;
+            uint4 u = make_uint4(0, 0, 0, 0);
+            if (c < all_chunks) u = *reinterpret_cast<const uint4*>(src + c * 8);
+            u = make_uint4(u.x ^ sign, u.y ^ sign, u.z ^ sign, u.w ^ sign);
+            qf[k] = *reinterpret_cast<const bf16x8*>(&u);
+        }
+    }
+    f32x16 acc[VF];
+#pragma unroll
+    for (int f = 0; f < VF; f++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[f][v] = 0.f;
+    const bool sink = a.sink && kg == 0 && (a.splits == 1 || blockIdx.z == 0);  // one lane half of one group of one share counts it
+    float mx = sink ? 0.f : kLowest, sum = sink && half == 0 ? 1.f : 0.f;
+
+    const int key_row = (l31 & 0x13) | (l31 & 4) << 1 | (l31 & 8) >> 1;  // bits 2 and 3 exchanged
+    const int key_at = key_row * (DK * 2), key_swap = place_of_key(key_row);
+    // Values that are columns of the key rows come by transposing reads (ds_read_b64_tr_b16): in a group of 16 lanes lane i
+    // names four columns of key i / 4 and receives its own column of the four keys.
+    int value_at[2];
+    if constexpr (!EXPANDED) {
+#pragma unroll
+        for (int f = 0; f < 2; f++) {
+            const int i = lane & 15, k = 8 * half + (i >> 2), c = 4 * f + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+            value_at[f] = k * (DK * 2) + ((c ^ place_of_key(k)) << 4) + (i & 1) * 8;
+        }
+    }
+
+    if (kg < n_tiles) copy_tile(kg, 0);
+    for (int turn = 0; turn < n_turns; turn++) {
+        const int tile = turn * KG + kg, key0 = key_begin + tile * kTile;
+        // the tile is in LDS, everybody's copies of it; and nobody still reads the other buffer
+        __builtin_amdgcn_s_waitcnt(0x0070);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (tile + KG < n_tiles) copy_tile(tile + KG, (turn + 1) & 1);
+        if (tile >= n_tiles || key0 > highest_limit) continue;
+        const uint8_t* kb = my_lds + (turn & 1) * kBuf;
+        const uint8_t* vb = kb + kKeyBytes;
+        f32x16 sc[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) sc[t][v] = 0.f;
+#pragma unroll
+            for (int k = 0; k < KS; k++) {
+                const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kb + key_at + t * 32 * (DK * 2) + (((KEY0 / 8 + 2 * k + half) ^ key_swap) << 4));
+                sc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[k], sc[t], 0, 0, 0);
+            }
+        }
+        if (key0 + kTile - 1 > lowest_limit || key0 < highest_first || key0 + kTile > key_end) {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const int key = key0 + 32 * t + 16 * (v >> 3) + 8 * half + (v & 7);
+                    if (key > limit || key < first || key >= key_end) sc[t][v] = -__builtin_inff();
+                }
+        }
+        float top = sc[0][0];
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) top = fmaxf(top, sc[t][v]);
+        top = fmaxf(top, other_half(top)) * scale;
+        if (__any(top > mx)) {
+            const float m = fmaxf(mx, top), keep = __builtin_amdgcn_exp2f(mx - m);
+            mx = m;
+            sum *= keep;
+#pragma unroll
+            for (int f = 0; f < VF; f++) acc[f] *= keep;
+        }
+        bf16x8 pf[4];
+        float add[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const float p = __builtin_amdgcn_exp2f(fmaf(sc[t][v], scale, -mx));
+                add[v & 3] += p;
+                pf[2 * t + (v >> 3)][v & 7] = (bf16)p;
+            }
+        sum += (add[0] + add[1]) + (add[2] + add[3]);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int f = 0; f < VF; f++) {
+                bf16x8 vf;
+                if constexpr (EXPANDED) {
+                    vf = *reinterpret_cast<const bf16x8*>(vb + (f * 32 + l31) * (kTile * 2) + (((2 * u + half) ^ (l31 & 7)) << 4));
+                } else {
+                    const uint8_t* at = kb + value_at[f & 1] + (f >> 1) * 128 + u * 16 * (DK * 2);
+                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at));
+                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 4 * (DK * 2)));
+                    const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                    vf = *reinterpret_cast<const bf16x8*>(&both);
+                }
+                acc[f] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[u], acc[f], 0, 0, 0);
+            }
+    }
+
+    sum += other_half(sum);
+    if constexpr (KG > 1) {  // the second group hands its share of the keys over; value column of register (f, v) at (f 16 + v)
+        static_assert(KG == 2, "two groups meet");
+        float* part = reinterpret_cast<float*>(lds) + (size_t)qw * (16 * VF + 2) * 64 + lane;
+        __syncthreads();
+        if (kg == 1) {
+            part[0] = mx, part[64] = sum;
+#pragma unroll
+            for (int f = 0; f < VF; f++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) part[(2 + f * 16 + v) * 64] = acc[f][v];
+        }
+        __syncthreads();
+        if (kg == 1) return;
+        const float other = part[0], m = fmaxf(mx, other), mine = __builtin_amdgcn_exp2f(mx - m), theirs = __builtin_amdgcn_exp2f(other - m);
+        sum = sum * mine + part[64] * theirs;
+        mx = m;
+#pragma unroll
+        for (int f = 0; f < VF; f++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[f][v] = acc[f][v] * mine + part[(2 + f * 16 + v) * 64] * theirs;
+    }
+    // register (f, v) holds value column 32 f + 8 (v / 4) + 4 half + v % 4 of query l % 32
+    const int r = wave_row0 + l31;
+    if (r >= a.rows) return;
+    if (a.splits > 1) {
+        const size_t at = ((size_t)blockIdx.z * gridDim.x + z) * a.rows + r;
+        if (half == 0) {
+            a.part_stats[2 * at] = mx;
+            a.part_stats[2 * at + 1] = sum;
+        }
+        float* dst = a.part + at * a.ld_part;
+#pragma unroll
+        for (int f = 0; f < VF; f++)
+#pragma unroll
+            for (int v = 0; v < 16; v += 4) {
+                const int d = 32 * f + 2 * v + 4 * half;
+                if (d < a.ld_part) *reinterpret_cast<f32x4*>(dst + d) = f32x4{acc[f][v], acc[f][v + 1], acc[f][v + 2], acc[f][v + 3]};
+            }
+        return;
+    }
+    float inv = 1.0f / sum;
+    if (a.head_gate) inv *= sigmoid(a.head_gate[(size_t)r * a.ld_gate + z]);
+    bf16* dst = a.out + z * a.out_head + (size_t)my_token * a.out_token + (r - my_token * a.rows_per_token) * a.ld_out;
+    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+    const bool whole = ((a.dv | a.ld_out | a.out_token) & 3) == 0 && (a.out_head & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 7) == 0;
+#pragma unroll
+    for (int f = 0; f < VF; f++)
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            const int d = 32 * f + 2 * v + 4 * half;
+            if (whole) {
+                if (d < a.dv)
+                    *reinterpret_cast<bf16x4*>(dst + d) =
+                        bf16x4{(bf16)(acc[f][v] * inv), (bf16)(acc[f][v + 1] * inv), (bf16)(acc[f][v + 2] * inv), (bf16)(acc[f][v + 3] * inv)};
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (d + i < a.dv) dst[d + i] = (bf16)(acc[f][v + i] * inv);
+            }
+        }
+}
+
+template <int DK, int DV, int KEY0, int KG, int QW, bool EXPANDED>
+hipError_t launch_kernel(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
+    hipLaunchKernelGGL((attend_prompt_kernel<DK, DV, KEY0, KG, QW, EXPANDED>), dim3(heads, (a.rows + 32 * QW - 1) / (32 * QW), a.splits),
+                       dim3(64 * KG * QW), 0, s, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+// Heads of more than 128 columns leave LDS and registers for one group only.
+hipError_t launch_attend_rows_prompt(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
+    const int widest = a.k_own_width > a.v_width ? a.k_own_width : a.v_width;
+    if (widest <= 64) return launch_kernel<128, 64, 64, 2, 4, false>(a, heads, s);
+    if (widest <= 128) return launch_kernel<256, 128, 128, 2, 4, false>(a, heads, s);
+    return launch_kernel<512, 256, 256, 1, 4, false>(a, heads, s);
+}
+
+hipError_t launch_attend_expanded(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
+    const int dk = a.k_own_width + a.k_shared_width;
+    if (dk <= 128 && a.dv <= 64) return launch_kernel<128, 64, 0, 2, 4, true>(a, heads, s);
+    if (dk <= 192 && a.dv <= 128) return launch_kernel<192, 128, 0, 2, 4, true>(a, heads, s);
+    return launch_kernel<320, 256, 0, 1, 4, true>(a, heads, s);
+}
+
+}  // namespace a81w41

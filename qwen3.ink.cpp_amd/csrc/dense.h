@@ -151,7 +151,7 @@ template <typename T>
 hipError_t launch_rotate_queries(const float* q, int ld_q, const LatentRows& in, const LatentShape& sh, int M, T* nope, int ld_nope,
                                  T* rot_out, int ld_rot, hipStream_t s);
 
-// ---- attention (attend_vector.hip, attend_mfma.hip) ------------------------------------------
+// ---- attention (attend_vector.hip, attend_mfma.hip, attend_prompt.hip) ------------------------------------------
 // Query row r of head z belongs to token r / rows_per_token of the pass: q + z q_head + token q_token + (r %
 // rows_per_token) ld_q; `out` is laid out likewise.  It sees the keys 0 .. pos + token, with chunk > 0 those from the first
 // position of its own chunk of that many positions on.  sink: a further key of score 0 without a value.
@@ -159,7 +159,8 @@ hipError_t launch_rotate_queries(const float* q, int ld_q, const LatentRows& in,
 // [splits][heads][rows][ld_part] with part_stats [splits][heads][rows][2] (maximum in powers of two, sum), for
 // launch_merge_shares.
 constexpr int kAttendMaxSplits = 64;
-constexpr int kAttendFewRows = 64;  // up to here a workgroup takes 16 query rows, above 64 or more
+constexpr int kAttendFewRows = 64;  // up to here a workgroup takes 16 query rows, above 64 (shared form) or kAttendPromptRows
+constexpr int kAttendPromptRows = 128;
 template <typename T>
 struct AttendArgs {
     const T* q = nullptr;
@@ -200,6 +201,7 @@ bool attend_rows_fits(int key, int value);  // stored widths
 bool attend_expanded_fits(int own, int shared, int dv);
 hipError_t launch_attend_shared(const AttendArgs<bf16>& a, hipStream_t s);
 hipError_t launch_attend_rows(const AttendArgs<bf16>& a, int heads, hipStream_t s);
+hipError_t launch_attend_rows_prompt(const AttendArgs<bf16>& a, int heads, hipStream_t s);  // what it does for many rows
 hipError_t launch_attend_expanded(const AttendArgs<bf16>& a, int heads, hipStream_t s);
 hipError_t launch_merge_shares(const AttendArgs<bf16>& a, int heads, hipStream_t s);
 

@@ -48,3 +48,30 @@ def test_gated_pairs_on_large_tiles(pkg):
 def test_head_columns_on_large_tiles(pkg):
     cfg = dx.config(64, 64, [dx.attention(32, 8, 128, 128, 70, 0.09, rot_dims=64, mlp=None)], (0, 1, 1))
     _same_in_portions(pkg, cfg, 2100, 60)
+
+
+# ---- attention over a prompt ------------------------------------------------------------------
+# Many turns of both key groups, ends inside a tile of 64 keys, of 128 rows and of a share; a scale below zero and of zero;
+# value widths and output strides that are no multiple of four.
+@pytest.mark.parametrize("M,pos,chunk,splits", [(97, 0, 0, 1), (700, 5, 0, 1), (641, 64, 0, 3), (520, 130, 192, 1), (333, 3, 500, 2)])
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128), (128, 125), (104, 61), (256, 254)])
+@pytest.mark.parametrize("scale", [0.09, -0.11, 0.0])
+def test_attention_over_a_prompt(pkg, M, pos, chunk, splits, dim, vdim, scale):
+    import torch
+    heads, kv_heads, seq = 6, 2, pos + M + 9
+    g = torch.Generator(device="cuda").manual_seed(M + dim)
+    value = (vdim + 7) // 8 * 8
+    q = torch.randn(M, heads, dim, device="cuda", generator=g).bfloat16()
+    rows = torch.randn(seq, kv_heads * (dim + value), device="cuda", generator=g).bfloat16()
+    rows[pos + M:] *= 1e4
+    got = pkg.ops.grouped_attention(q, rows, pos, kv_heads, dim, vdim, scale, chunk, False, 1, splits).double()
+    t, s = torch.arange(pos, pos + M, device="cuda")[:, None], torch.arange(seq, device="cuda")[None]
+    sees = (s <= t) & (s // chunk == t // chunk) if chunk else s <= t
+    parts = rows.double().view(seq, kv_heads, dim + value)
+    for h in range(heads):
+        part = parts[:, h // 3]
+        p = (q[:, h].double() @ part[:, value:].t() * scale).masked_fill(~sees, -1e300).softmax(1)
+        want = p @ part[:, :vdim]
+        # weights and the result are rounded to 8 significant bits: off by at most 2^-8 of each term and of the sum
+        bound = 2.0 ** -8 * (p @ part[:, :vdim].abs() + want.abs()) + 1e-5
+        assert ((got[:, h] - want).abs() <= bound).all(), (h, ((got[:, h] - want).abs() / bound).max().item())
