@@ -4,7 +4,7 @@
 //   rows      the queries of a group of heads look at the rows of their key/value head, [value | key] (grouped attention);
 //   expanded  keys and values of every head were formed beforehand: a key is [own part | part shared by all heads],
 //             values come transposed ([value column][key]).
-// The first, and the second for few rows, are here, the others in attend_prompt.hip.
+// The first, and the second up to kAttendShortRows rows, are here, the others in attend_prompt.hip.
 //
 // A wave owns 16 (or 2 x 16) query rows.  It forms the scores transposed, S^T = K Q^T (v_mfma_f32_16x16x32_bf16 with
 // the keys as rows), so that lane l holds scores of query l % 16 only: keys 16 t + 4 (l / 16) + i.  These registers
@@ -267,10 +267,11 @@ hipError_t launch_shared(const AttendArgs<bf16>& a, hipStream_t s) {
     return a.rows <= kAttendFewRows ? launch_kernel<DK, DV, 0, 4, 1, 64, 2, true>(a, 1, s)
                                     : launch_kernel<DK, DV, 0, 4, 1, 32, 1, false>(a, 1, s);
 }
-// key and value columns: D at most each; few rows
-template <int D>
+// key and value columns: D at most each; up to kAttendShortRows rows
+template <int D, int QS>
 hipError_t launch_rows(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
-    return launch_kernel<2 * D, D, D, 4, 1, 64, 2, true>(a, heads, s);
+    return a.rows <= kAttendFewRows ? launch_kernel<2 * D, D, D, 4, 1, 64, 2, true>(a, heads, s)
+                                    : launch_kernel<2 * D, D, D, 4, QS, 64, 2, false>(a, heads, s);
 }
 
 }  // namespace
@@ -287,11 +288,11 @@ hipError_t launch_attend_shared(const AttendArgs<bf16>& a, hipStream_t s) {
 }
 
 hipError_t launch_attend_rows(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
-    if (a.rows > kAttendFewRows) return launch_attend_rows_prompt(a, heads, s);
+    if (a.rows > kAttendShortRows) return launch_attend_rows_prompt(a, heads, s);
     const int widest = a.k_own_width > a.v_width ? a.k_own_width : a.v_width;
-    if (widest <= 64) return launch_rows<64>(a, heads, s);
-    if (widest <= 128) return launch_rows<128>(a, heads, s);
-    return launch_rows<256>(a, heads, s);
+    if (widest <= 64) return launch_rows<64, 2>(a, heads, s);
+    if (widest <= 128) return launch_rows<128, 2>(a, heads, s);
+    return launch_rows<256, 1>(a, heads, s);
 }
 
 hipError_t launch_merge_shares(const AttendArgs<bf16>& a, int heads, hipStream_t s) {

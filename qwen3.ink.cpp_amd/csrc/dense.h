@@ -159,8 +159,11 @@ hipError_t launch_rotate_queries(const float* q, int ld_q, const LatentRows& in,
 // [splits][heads][rows][ld_part] with part_stats [splits][heads][rows][2] (maximum in powers of two, sum), for
 // launch_merge_shares.
 constexpr int kAttendMaxSplits = 64;
-constexpr int kAttendFewRows = 64;  // up to here a workgroup takes 16 query rows, above 64 (shared form) or kAttendPromptRows
-constexpr int kAttendPromptRows = 128;
+constexpr int kAttendFewRows = 64;  // up to here a workgroup takes 16 query rows, above 64 or more
+// The rows form takes 64 or 128 rows a workgroup up to kAttendShortRows, kAttendPromptRows above.  At 132 rows the two kernels take 15
+// and 11 us, both next to what a launch takes, at 400 and 512 rows 11 and 10 us; short prompts keep the order of their sums, which a
+// router behind them may feel.
+constexpr int kAttendShortRows = 512, kAttendPromptRows = 128;
 template <typename T>
 struct AttendArgs {
     const T* q = nullptr;

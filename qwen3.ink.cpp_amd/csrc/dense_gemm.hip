@@ -12,6 +12,8 @@
 // the other.  4095 x 12288 x 2048 in bfloat16 with the gated epilogue: 340 us with 128 x 128 tiles whose copies the compiler
 // waited for ahead of every step's first LDS read (see lds16), 210 us = 980 TFLOP/s with 256 x 256.  4095 x 2048 x 6144: 140 us and
 // 120 us, 2048 x 2048 x 2048: 47 us and 29 us.
+#include <type_traits>
+
 #include "dense_common.h"
 
 namespace a81w41 {
@@ -33,59 +35,58 @@ struct NoHeads {};
 __device__ __forceinline__ float swap_neighbours(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
 }
-// At most `pending` of this wave's vector-memory operations are outstanding, and none of its LDS reads; then everybody's.
+// At most PENDING of this wave's vector-memory operations are outstanding, and none of its LDS reads.
 template <int PENDING>
-__device__ __forceinline__ void wait_copies_and_meet() {
+__device__ __forceinline__ void wait_copies() {
     __builtin_amdgcn_s_waitcnt((PENDING & 15) | (PENDING >> 4) << 14 | 0x0070);
     asm volatile("" ::: "memory");
+}
+// The same of every wave of the workgroup.
+template <int PENDING>
+__device__ __forceinline__ void wait_copies_and_meet() {
+    wait_copies<PENDING>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
 
-// Results of a wave's 32 x 32 pieces: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32.
-template <typename T, int FM, int FN, Epilogue EPI, typename X>
-__device__ __forceinline__ void store_pieces(const GemmArgs& g, const X& heads, const f32x16 (&acc)[FM][FN], int m0, int rows, int wm, int col0,
-                                             long long batch) {
-    const int lane = threadIdx.x & 63, l31 = lane & 31, half = lane >> 5;
+// NV registers of a 32 x 32 product: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4 from row0 on, column l % 32 from
+// col0 on; rows from `rows` on are not stored.
+template <typename T, Epilogue EPI, int NV, typename V, typename X>
+__device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, const V& x, int m0, int rows, int row0, int col0, long long batch) {
+    const int lane = threadIdx.x & 63, col = col0 + (lane & 31), r0 = row0 + 4 * (lane >> 5);
+    if constexpr (EPI == Epilogue::kGatedPair) {
+        // Lanes 16 .. 31 and 48 .. 63 hold the ups of the 16 lanes before them.  Of two rows v, v + 1 the gates of the second and the
+        // ups of the first trade places: every lane then has both of one row, and no unit is formed twice.
+        const int odd = (lane >> 4) & 1;
+        T* dst = static_cast<T*>(g.C) + (col >> 5) * 16 + (col & 15);
+#pragma unroll
+        for (int v = 0; v < NV; v += 2) {
+            const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[v]), __float_as_uint(x[v + 1]), false, false);
+            const float unit = gated_unit(g.unit, __uint_as_float(both[0]), __uint_as_float(both[1]));
+            const int r = r0 + 8 * (v >> 2) + (v & 3) + odd;
+            if (r < rows && col < g.N) dst[(size_t)(m0 + r) * g.ldc] = (T)unit;
+        }
+        return;
+    }
     [[maybe_unused]] int pos = 0;
     if constexpr (EPI == Epilogue::kHeads) pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1);
 #pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const int col = col0 + j * 32 + l31, r0 = wm + i * 32 + 4 * half;
-            if constexpr (EPI == Epilogue::kGatedPair) {
-                // Lanes 16 .. 31 and 48 .. 63 hold the ups of the 16 lanes before them.  Of two rows v, v + 1 the gates of the
-                // second and the ups of the first trade places: every lane then has both of one row, and no unit is formed twice.
-                const int odd = (lane >> 4) & 1;
-                T* dst = static_cast<T*>(g.C) + (col >> 5) * 16 + (col & 15);
-#pragma unroll
-                for (int v = 0; v < 16; v += 2) {
-                    const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i][j][v]), __float_as_uint(acc[i][j][v + 1]), false, false);
-                    const float unit = gated_unit(g.unit, __uint_as_float(both[0]), __uint_as_float(both[1]));
-                    const int r = r0 + 8 * (v >> 2) + (v & 3) + odd;
-                    if (r < rows && col < g.N) dst[(size_t)(m0 + r) * g.ldc] = (T)unit;
-                }
-                continue;
-            }
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int r = r0 + 8 * (v >> 2) + (v & 3);
-                const size_t row = m0 + r;
-                if constexpr (EPI == Epilogue::kHeads) {
-                    const float other = swap_neighbours(acc[i][j][v]);
-                    if (r < rows && col < g.N) store_head_column(heads, pos, (int)row, col, acc[i][j][v], other);
-                } else if (r < rows && col < g.N) {
-                    if constexpr (EPI == Epilogue::kFloat) {
-                        (static_cast<float*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = acc[i][j][v];
-                    } else {
-                        float f = acc[i][j][v];
-                        if constexpr (EPI == Epilogue::kHeadGate) f *= sigmoid(g.head_gate[row * g.ld_gate + batch]);
-                        (static_cast<T*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = (T)f;
-                    }
-                }
+    for (int v = 0; v < NV; v++) {
+        const int r = r0 + 8 * (v >> 2) + (v & 3);
+        const size_t row = m0 + r;
+        if constexpr (EPI == Epilogue::kHeads) {
+            const float other = swap_neighbours(x[v]);
+            if (r < rows && col < g.N) store_head_column(heads, pos, (int)row, col, x[v], other);
+        } else if (r < rows && col < g.N) {
+            if constexpr (EPI == Epilogue::kFloat) {
+                (static_cast<float*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = x[v];
+            } else {
+                float f = x[v];
+                if constexpr (EPI == Epilogue::kHeadGate) f *= sigmoid(g.head_gate[row * g.ld_gate + batch]);
+                (static_cast<T*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = (T)f;
             }
         }
+    }
 }
 
 // Rows of tiles that are walked together: an XCD's workgroups then share these rows and a few column panels in its L2.
@@ -191,7 +192,106 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(G
                 for (int j = 0; j < FN; j++) mma(acc[i][j], a[kk & 1][i], b[kk & 1][j], static_cast<T*>(nullptr));
         }
     }
-    store_pieces<T, FM, FN, EPI>(g, heads, acc, m0, rows, wm, n0 + wn, batch);
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) store_piece<T, EPI, 16>(g, heads, acc[i][j], m0, rows, wm + i * 32, n0 + wn + j * 32, batch);
+}
+
+// Few rows, so few tiles that a CU has one at most: what counts is that the weights are under way and that a step is short.  64
+// rows and 32 columns a workgroup of six waves: two multiply 32 rows each, reading a step's operands beside the products of the step
+// before, two copy A nine steps ahead, two copy W 19 steps ahead.  A wave that copies and multiplies takes 0.3 us a step
+// however much is under way, these 0.13 us (a trip to memory of 2.4 us in 19 steps, one to the L2 of 0.9 us in nine).  The sums go
+// in the order of the other kernels.  33 rows, 784 x 2048: 21 us with 64 x 64 tiles and one step's copies waited for at once, 7.7 us
+// here; 2048 x 6144: 81 us and 19 us.  Cutting K between waves is no faster (7.5 and 20 us) and sums in another order.
+template <typename T, Epilogue EPI, typename X>
+__global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X heads) {
+    constexpr int SA = 10, SW = 20, kStageA = 64 * 128, kStageW = 32 * 128;
+    __shared__ __attribute__((aligned(128))) uint8_t lds[SA * kStageA + SW * kStageW];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l31 = lane & 31, half = lane >> 5;
+    // row tiles of a column panel next to each other on one XCD
+    const int n_mt = (g.M + 63) / 64;
+    const int q = gridDim.x >> 3, r8 = gridDim.x & 7, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+    const int t = xcd < r8 ? xcd * (q + 1) + idx : r8 * (q + 1) + (xcd - r8) * q + idx;
+    const int m0 = t % n_mt * 64, n0 = t / n_mt * 32, rows = g.M - m0, n_steps = g.K * (int)sizeof(T) / 128;
+    const long long batch = blockIdx.y;
+    const int copy_row = (wave & 1) * (wave < 4 ? 32 : 16) + (lane >> 3), swapped = ((lane & 7) ^ (lane >> 3)) << 4;  // of the wave's first copy
+    uint8_t* const lds_w = lds + SA * kStageA;
+    if (wave >= 2) {  // COPIES a step and wave, 8 rows each, into a ring of S stages
+        auto run = [&](auto copies, auto stages, const uint8_t* (&src)[4], uint8_t* ring, int stage_bytes) {
+            constexpr int COPIES = decltype(copies)::value, S = decltype(stages)::value;
+            uint8_t* to = ring + (wave & 1) * COPIES * 1024;
+            auto copy_step = [&](int slot) {
+#pragma unroll
+                for (int i = 0; i < COPIES; i++) {
+                    copy16_to_lds(src[i], to + slot * stage_bytes + i * 1024);
+                    src[i] += 128;
+                }
+            };
+            for (int step = 0; step < S - 1 && step < n_steps; step++) copy_step(step);
+            int slot = S - 1;
+            for (int step = 0; step < n_steps; step++) {
+                if (step + S - 2 < n_steps)
+                    wait_copies_and_meet<(S - 2) * COPIES>();
+                else
+                    wait_copies_and_meet<0>();
+                if (step + S - 1 < n_steps) copy_step(slot);
+                slot = slot + 1 < S ? slot + 1 : 0;
+            }
+        };
+        const uint8_t* src[4];
+        if (wave < 4) {
+            const uint8_t* A = reinterpret_cast<const uint8_t*>(static_cast<const T*>(g.A) + batch * g.a_step);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                int row = m0 + min(copy_row + 8 * i, rows - 1);
+                if (g.a_rows) row = g.a_rows[row];
+                src[i] = A + (size_t)row * g.lda * sizeof(T) + swapped;
+            }
+            run(std::integral_constant<int, 4>{}, std::integral_constant<int, SA>{}, src, lds, kStageA);
+        } else {
+            const uint8_t* W = reinterpret_cast<const uint8_t*>(static_cast<const T*>(g.W) + batch * g.w_step);
+#pragma unroll
+            for (int i = 0; i < 2; i++) src[i] = W + (size_t)min(n0 + copy_row + 8 * i, g.N - 1) * g.ldw * sizeof(T) + swapped;
+            run(std::integral_constant<int, 2>{}, std::integral_constant<int, SW>{}, src, lds_w, kStageW);
+        }
+        return;
+    }
+    f32x16 acc;
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = 0.f;
+    lds16 a[2][4], w[2][4];
+    int slot_a = 0, slot_w = 0;
+    auto read = [&](lds16 (&x)[4], lds16 (&y)[4]) {
+        const uint8_t *pa = lds + slot_a * kStageA + wave * 4096 + l31 * 128, *pw = lds_w + slot_w * kStageW + l31 * 128;
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) {
+            const int at = ((2 * kk + half) ^ (l31 & 7)) << 4;
+            x[kk] = *reinterpret_cast<const lds16*>(pa + at);
+            y[kk] = *reinterpret_cast<const lds16*>(pw + at);
+        }
+        slot_a = slot_a + 1 < SA ? slot_a + 1 : 0;
+        slot_w = slot_w + 1 < SW ? slot_w + 1 : 0;
+    };
+    auto multiply = [&](const lds16 (&x)[4], const lds16 (&y)[4]) {
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++) mma(acc, x[kk], y[kk], static_cast<T*>(nullptr));
+    };
+    // meet: the step is in LDS; its reads then run beside the products of the step before
+    wait_copies_and_meet<0>();
+    read(a[0], w[0]);
+    for (int step = 1; step < n_steps; step += 2) {
+        wait_copies_and_meet<0>();
+        read(a[1], w[1]);
+        multiply(a[0], w[0]);
+        if (step + 1 < n_steps) {
+            wait_copies_and_meet<0>();
+            read(a[0], w[0]);
+        }
+        multiply(a[1], w[1]);
+    }
+    if (n_steps & 1) multiply(a[0], w[0]);
+    store_piece<T, EPI, 16>(g, heads, acc, m0, rows, wave * 32, n0, batch);
 }
 
 // 256 x 256 tiles, one workgroup per CU, or 128 x 128, two per CU.  At K = 2048 a round of 256 large tiles takes 65 us whether
@@ -207,6 +307,12 @@ hipError_t launch_kernel(const GemmArgs& g, const X& heads, hipStream_t s) {
 }
 
 template <typename T, Epilogue EPI, typename X>
+hipError_t launch_few(const GemmArgs& g, const X& heads, hipStream_t s) {
+    hipLaunchKernelGGL((dense_gemm_few_kernel<T, EPI, X>), dim3((g.M + 63) / 64 * ((g.N + 31) / 32), g.batches), dim3(384), 0, s, g, heads);
+    return hipGetLastError();
+}
+
+template <typename T, Epilogue EPI, typename X>
 hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
     auto tiles = [&](int size) { return (long long)((g.M + size - 1) / size) * ((g.N + size - 1) / size) * g.batches; };
     // A product of 192 to 256 tiles of 128 x 128 has one for a CU: it takes twice the waves and four stages in LDS (2048^3: 29 us
@@ -216,6 +322,11 @@ hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
     if (!g.tiles && g.M > 64 && tiles(128) > 256) return launch_kernel<T, 128, 128, 2, 2, 2, false, EPI>(g, heads, s);
     if (!g.tiles && g.M > 64 && tiles(128) >= 192) return launch_kernel<T, 128, 128, 2, 4, 4, true, EPI>(g, heads, s);
     if (g.tiles && g.N >= 1024) return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, false, EPI>(g, heads, s);
+    // So few tiles of 64 x 32 that no CU gets a second one (us, against 64 x 64 tiles with four stages): 33 rows, 784 x 2048 7.7 /
+    // 12.5, 2048 x 6144 19 / 31; 256 rows, 2048 x 2048 10.2 / 13.5; with a second one 300 rows, 2048 x 2048 17.2 / 13.8, and 33
+    // rows, 12288 x 2048 20 / 16.
+    const long long few = (long long)((g.N + 31) / 32) * ((g.M + 63) / 64) * g.batches;
+    if (!g.tiles && few <= 256) return launch_few<T, EPI>(g, heads, s);
     return launch_kernel<T, 64, 64, 2, 2, 4, false, EPI>(g, heads, s);
 }
 

@@ -417,11 +417,12 @@ AttendArgs<T> DimesunModel<T>::attend_args(const AttentionConfig& c, const RunCa
     a.out_head = (long long)R * c.vdim, a.out_token = ld_attn_, a.ld_out = c.vdim;
     a.part = part_, a.part_stats = part_stats_, a.ld_part = (c.vdim + 3) / 4 * 4;
     a.scale = c.scale, a.chunk = c.chunk, a.sink = true, a.pos_dev = pos, a.max_seq = max_seq();
-    // enough workgroups for the chip, at least two tiles of 64 keys for each of a prompt, one otherwise
+    // enough workgroups for the chip, at least one tile of 64 keys for each, or two of a long prompt's
     const int keys = std::min(plan_ctx, c.chunk + M - 1);
-    const bool few = a.rows <= kAttendFewRows;
-    const int groups = c.kv_heads * (few ? (a.rows + 15) / 16 : (a.rows + kAttendPromptRows - 1) / kAttendPromptRows);
-    const int shares = few ? std::min((keys + 63) / 64, 512 / groups) : std::min((keys + 127) / 128, 256 / groups);
+    const bool prompt = a.rows > kAttendShortRows;
+    const int group_rows = prompt ? kAttendPromptRows : a.rows <= kAttendFewRows ? 16 : 64;
+    const int groups = c.kv_heads * ((a.rows + group_rows - 1) / group_rows);
+    const int shares = prompt ? std::min((keys + 127) / 128, 256 / groups) : std::min((keys + 63) / 64, 512 / groups);
     a.splits = opt_split_ ? opt_split_ : std::min(kAttendMaxSplits, std::max(1, shares));
     a.splits = std::max<int>(1, std::min<size_t>(a.splits, part_rows_ / ((size_t)c.heads * M)));
     return a;
