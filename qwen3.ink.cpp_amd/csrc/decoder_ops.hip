@@ -4,6 +4,8 @@
 // Every index that depends on device data is clamped into its array.
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
+
 #include "decoder_session.h"
 
 namespace a81w41 {
@@ -99,6 +101,21 @@ __global__ __launch_bounds__(1024) void argmax_token_kernel(const float* __restr
     }
 }
 
+// What the host left in pinned memory, read over the bus: a launch in the stream's order, where a copy would make the host wait twice.
+__global__ __launch_bounds__(256) void take_tokens_kernel(const int* host_ids, int n, int* __restrict__ ids, const int* host_want, int n_want,
+                                                        int* __restrict__ want) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n)
+        ids[i] = host_ids[i];
+    else if (i - n < n_want)
+        want[i - n] = host_want[i - n];
+}
+__global__ __launch_bounds__(256) void give_floats_kernel(const float* __restrict__ x, float* host, size_t n) {
+    for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) host[i] = x[i];
+}
+__global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ p, size_t n) {
+    for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) p[i] = 0;
+}
 __global__ void advance_kernel(int* __restrict__ pos_dev, int by) {
     if (threadIdx.x == 0 && blockIdx.x == 0) pos_dev[0] += by;
 }
@@ -126,6 +143,19 @@ hipError_t launch_embed_rows(const int* ids, const void* table, TableType type, 
 hipError_t launch_argmax_token(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev,
                                hipStream_t s) {
     hipLaunchKernelGGL(argmax_token_kernel, dim3(1), dim3(1024), 0, s, logits, n, next_id, history, history_len, step_dev);
+    return hipGetLastError();
+}
+hipError_t launch_take_tokens(const int* host_ids, int n, int* ids, const int* host_want, int n_want, int* want, hipStream_t s) {
+    hipLaunchKernelGGL(take_tokens_kernel, dim3((n + n_want + 255) / 256), dim3(256), 0, s, host_ids, n, ids, host_want, n_want, want);
+    return hipGetLastError();
+}
+hipError_t launch_give_floats(const float* x, float* host, size_t n, hipStream_t s) {
+    hipLaunchKernelGGL(give_floats_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 256)), dim3(256), 0, s, x, host, n);
+    return hipGetLastError();
+}
+hipError_t launch_zero_words(void* p, size_t words, hipStream_t s) {
+    hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)std::min<size_t>((words + 255) / 256, 1024)), dim3(256), 0, s,
+                       static_cast<unsigned*>(p), words);
     return hipGetLastError();
 }
 hipError_t launch_advance(int* pos_dev, int by, hipStream_t s) {

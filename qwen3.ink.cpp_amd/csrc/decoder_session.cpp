@@ -14,6 +14,10 @@
 
 namespace a81w41 {
 
+namespace {
+constexpr size_t kStagedFloats = 1 << 18;  // logits that go out through pinned memory; more of them, or a longer row, by a copy
+}
+
 CachePlanes::~CachePlanes() {
     for (void* p : planes_) (void)hipFree(p);
 }
@@ -35,8 +39,8 @@ int CachePlanes::add_state(size_t bytes, void** state) {
     return 0;
 }
 
-int CachePlanes::clear_states() {
-    for (const auto& st : states_) A81W41_HIP_TRY(hipMemset(st.first, 0, st.second));
+int CachePlanes::clear_states(hipStream_t s) {
+    for (const auto& st : states_) A81W41_HIP_TRY(launch_zero_words(st.first, st.second / 4, s));
     return 0;
 }
 
@@ -54,6 +58,9 @@ int DecoderSession::init_session(int max_seq, int vocab, int max_rows) {
     A81W41_HIP_TRY(hipMemset(pos, 0, sizeof(int)));
     A81W41_HIP_TRY(hipMemset(step, 0, sizeof(int)));
     A81W41_TRY(reserve_logits(1));
+    staged_floats_ = std::max<size_t>(vocab, kStagedFloats);
+    A81W41_HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&staged_ids_), 2 * (size_t)max_rows * sizeof(int), hipHostMallocDefault));
+    A81W41_HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&staged_logits_), staged_floats_ * sizeof(float), hipHostMallocDefault));
     A81W41_HIP_TRY(hipStreamCreate(&stream));
     return 0;
 }
@@ -62,6 +69,8 @@ DecoderSession::~DecoderSession() {
     if (stream) (void)hipStreamSynchronize(stream);
     void* bufs[] = {ids, want_dev, pos, step, history, logits};
     for (void* b : bufs) (void)hipFree(b);
+    if (staged_ids_) (void)hipHostFree(staged_ids_);
+    if (staged_logits_) (void)hipHostFree(staged_logits_);
     if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -77,18 +86,18 @@ int DecoderSession::reserve_logits(int rows) {
 }
 
 int DecoderSession::reset() {
-    A81W41_HIP_TRY(hipStreamSynchronize(stream));
-    A81W41_HIP_TRY(hipMemset(pos, 0, sizeof(int)));
-    A81W41_HIP_TRY(hipMemset(step, 0, sizeof(int)));
-    A81W41_TRY(cache.clear_states());
+    A81W41_HIP_TRY(launch_zero_words(pos, 1, stream));
+    A81W41_HIP_TRY(launch_zero_words(step, 1, stream));
+    A81W41_TRY(cache.clear_states(stream));
     host_pos = 0;
     return 0;
 }
 
-// The ids and wanted rows of a pass of at most max_rows_ tokens.
+// The ids and wanted rows of a pass of at most max_rows_ tokens.  No earlier upload may still be waiting in the stream.
 int DecoderSession::upload(const int* token_ids, int n, const int* want, int n_want) {
-    A81W41_HIP_TRY(hipMemcpy(ids, token_ids, (size_t)n * sizeof(int), hipMemcpyHostToDevice));
-    if (n_want) A81W41_HIP_TRY(hipMemcpy(want_dev, want, (size_t)n_want * sizeof(int), hipMemcpyHostToDevice));
+    std::copy_n(token_ids, n, staged_ids_);
+    std::copy_n(want, n_want, staged_ids_ + max_rows_);
+    A81W41_HIP_TRY(launch_take_tokens(staged_ids_, n, ids, staged_ids_ + max_rows_, n_want, want_dev, stream));
     return 0;
 }
 
@@ -111,11 +120,16 @@ int DecoderSession::forward(const int* token_ids, int n, const int* want, int n_
         plan_ctx = host_pos + m;
         A81W41_TRY(upload(token_ids + at, m, local.data(), nw));
         A81W41_TRY(enqueue_pass(m, local.data(), nw, stream));
+        const size_t out = logits_host ? (size_t)nw * vocab_ : 0;
+        const bool staged = out && out <= staged_floats_;
+        if (staged) A81W41_HIP_TRY(launch_give_floats(logits, staged_logits_, out, stream));
         A81W41_HIP_TRY(hipStreamSynchronize(stream));
         host_pos += m;
         A81W41_TRY(check_passes());
-        if (logits_host && nw)
-            A81W41_HIP_TRY(hipMemcpy(logits_host + (size_t)w0 * vocab_, logits, (size_t)nw * vocab_ * sizeof(float), hipMemcpyDeviceToHost));
+        if (staged)
+            std::copy_n(staged_logits_, out, logits_host + (size_t)w0 * vocab_);
+        else if (out)
+            A81W41_HIP_TRY(hipMemcpy(logits_host + (size_t)w0 * vocab_, logits, out * sizeof(float), hipMemcpyDeviceToHost));
         w0 += nw;
     }
     return 0;
@@ -145,13 +159,16 @@ int DecoderSession::generate_greedy(const int* prompt, int n_prompt, int n_new, 
     const hipEvent_t e0 = own.ev[0], e1 = own.ev[1], e2 = own.ev[2], e3 = own.ev[3];
     const int last_row = (n_prompt - 1) % max_rows_;  // of the prompt's last portion
     A81W41_TRY(upload(prompt, std::min(n_prompt, max_rows_), &last_row, 1));
-    A81W41_HIP_TRY(hipMemset(step, 0, sizeof(int)));
+    A81W41_HIP_TRY(launch_zero_words(step, 1, s));
     A81W41_HIP_TRY(hipEventRecord(e0, s));
     const int last_ctx = host_pos + n_prompt + n_new - 1;  // also what the decode steps captured below will reach
     for (int at = 0; at < n_prompt; at += max_rows_) {
         const int m = std::min(max_rows_, n_prompt - at);
         plan_ctx = m == 1 ? last_ctx : host_pos + at + m;
-        if (at) A81W41_TRY(upload(prompt + at, m, nullptr, 0));
+        if (at) {
+            A81W41_HIP_TRY(hipStreamSynchronize(s));
+            A81W41_TRY(upload(prompt + at, m, nullptr, 0));
+        }
         A81W41_TRY(enqueue_pass(m, &last_row, at + m == n_prompt ? 1 : 0, s));
     }
     // first new token: argmax of the prompt's logits; it becomes the next pass's input id

@@ -40,6 +40,10 @@ hipError_t launch_embed_rows(const int* ids, const void* table, TableType type, 
 hipError_t launch_argmax_token(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev,
                                hipStream_t s);
 hipError_t launch_advance(int* pos_dev, int by, hipStream_t s);
+// ids[0 .. n) and want[0 .. n_want) from pinned host memory; n floats into pinned host memory; words of zeros.
+hipError_t launch_take_tokens(const int* host_ids, int n, int* ids, const int* host_want, int n_want, int* want, hipStream_t s);
+hipError_t launch_give_floats(const float* x, float* host, size_t n, hipStream_t s);
+hipError_t launch_zero_words(void* p, size_t words, hipStream_t s);
 
 // What a sequence holds on the device, zero when allocated, freed with the object: cache planes of max_seq rows, which a new
 // sequence overwrites, and recurrent states, which go back to zero when the sequence is given back.
@@ -51,7 +55,7 @@ class CachePlanes {
     ~CachePlanes();
     int add(size_t bytes, void** plane);
     int add_state(size_t bytes, void** state);
-    int clear_states();
+    int clear_states(hipStream_t s);  // enqueues only; states are whole words
     size_t bytes() const { return bytes_; }
 
    private:
@@ -64,7 +68,7 @@ class DecoderSession {
    public:
     virtual ~DecoderSession();
 
-    int reset();
+    int reset();  // enqueues only
     // n new tokens on top of the cached context; logits of the rows want[0..n_want) (rising places among the n tokens) go
     // to logits_host [n_want][vocab] (may be null).  Cut into passes of at most max_rows tokens.  Synchronises.
     int forward(const int* token_ids, int n, const int* want, int n_want, float* logits_host);
@@ -106,6 +110,10 @@ class DecoderSession {
     int reserve_logits(int rows);
     int upload(const int* token_ids, int n, const int* want, int n_want);
     int max_seq_ = 0, vocab_ = 0, max_rows_ = 0;
+    // pinned: ids and wanted rows of a pass, read by an enqueued kernel until the stream is next waited for; logits on their way out
+    int* staged_ids_ = nullptr;
+    float* staged_logits_ = nullptr;
+    size_t staged_floats_ = 0;
 };
 
 }  // namespace a81w41

@@ -75,3 +75,15 @@ def test_attention_over_a_prompt(pkg, M, pos, chunk, splits, dim, vdim, scale):
         # weights and the result are rounded to 8 significant bits: off by at most 2^-8 of each term and of the sum
         bound = 2.0 ** -8 * (p @ part[:, :vdim].abs() + want.abs()) + 1e-5
         assert ((got[:, h] - want).abs() <= bound).all(), (h, ((got[:, h] - want).abs() / bound).max().item())
+
+
+def test_logits_that_do_not_fit_the_staging(pkg):
+    """Nine rows of 32768 logits are copied, eight and fewer go out through pinned memory."""
+    cfg = tx.config(32768, 64, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.dense(64))])
+    ids = np.arange(5, 35, dtype=np.int32)
+    model = pkg.Model.random(cfg, 64, "bfloat16", seed=3)
+    nine = model.forward(ids, range(3, 30, 3))
+    model.reset()
+    eight = model.forward(ids, range(3, 27, 3))
+    model.reset()
+    assert nine.shape == (9, 32768) and np.array_equal(nine[:8], eight) and np.array_equal(nine[8], model.forward(ids[:28])[0])
