@@ -106,19 +106,19 @@ __device__ __forceinline__ void group_inverse_rms(F x, int width, int groups, fl
 }
 
 // A row whose norm groups are whole float4s, dealt to a workgroup so that a group's threads are neighbours and a thread
-// holds at most kParts float4s, all of one group: the row stays in registers between its norms.
-template <int THREADS>
+// holds at most PARTS float4s, all of one group: the row stays in registers between its norms.
+template <int THREADS, int PARTS = 4>
 class RowParts {
    public:
-    static constexpr int kParts = 4;
-    __device__ __forceinline__ RowParts(int width, int groups) : groups_(groups), size_(width / groups) {
+    static constexpr int kParts = PARTS;
+    __host__ __device__ __forceinline__ RowParts(int width, int groups, int thread) : groups_(groups), size_(width / groups) {
         int per = 1;
         while (per < groups && per < THREADS) per <<= 1;
         log_tpg_ = 31 - __builtin_clz((unsigned)(THREADS / per));
-        group_ = threadIdx.x >> log_tpg_;
-        at_ = threadIdx.x & ((1 << log_tpg_) - 1);
+        group_ = thread >> log_tpg_;
+        at_ = thread & ((1 << log_tpg_) - 1);
     }
-    __device__ __forceinline__ bool fits() const {
+    __host__ __device__ __forceinline__ bool fits() const {
         return groups_ <= THREADS && (size_ & 3) == 0 && (size_ >> 2) <= (kParts << log_tpg_);
     }
     // first element of this thread's k-th float4, -1 if it has none

@@ -140,11 +140,12 @@ __device__ __forceinline__ void copy_row(float* xs, const float* src, int n, int
 }
 
 // The residual step and the norm of RowStep into xs; workgroup 0 of the launch also writes the stream.  Rows whose parts
-// are whole float4s and fit four of them per thread are requested at once by load() and stay in registers (a part's
+// are whole float4s and fit PARTS of them per thread are requested at once by load() and stay in registers (a part's
 // threads are neighbours); other rows are read when they are needed.
+template <int PARTS>
 class StepRow {
    public:
-    __device__ __forceinline__ explicit StepRow(const RowStep& p) : p_(p), parts_(p.width, p.norm_h.groups), fast_(parts_.fits()) {}
+    __device__ __forceinline__ explicit StepRow(const RowStep& p) : p_(p), parts_(p.width, p.norm_h.groups, threadIdx.x), fast_(parts_.fits()) {}
     __device__ __forceinline__ void load() {
         if (!fast_) return;
 #pragma unroll
@@ -188,7 +189,7 @@ class StepRow {
     }
 
    private:
-    static constexpr int kParts = RowParts<kThreads>::kParts;
+    static constexpr int kParts = PARTS;
     __device__ void slow(float* xs, int padded, float* inv, float* red) const {
         const RowStep& p = p_;
         const int t = threadIdx.x, W = p.width;
@@ -218,7 +219,7 @@ class StepRow {
         __syncthreads();
     }
     const RowStep& p_;
-    RowParts<kThreads> parts_;
+    RowParts<kThreads, PARTS> parts_;
     bool fast_;
     float4 x_[kParts], y_[kParts], wy_[kParts], before_[kParts], wh_[kParts];
 };
@@ -235,11 +236,11 @@ struct HeadsEmit {
 };
 
 // emit gets W[n] . row, in pairs of n
-template <typename T, typename Emit>
+template <typename T, int PARTS, typename Emit>
 __global__ __launch_bounds__(kThreads) void gemv_step_kernel(RowStep p, const T* __restrict__ w, int ld, int N, Emit emit) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     float *xs = smem, *red = xs + ld, *inv = red + kThreads / 64;
-    StepRow row(p);
+    StepRow<PARTS> row(p);
     row.load();
     const int chunks = ld * (int)sizeof(T) / 16, pairs = (N + 1) / 2;
     const Deal d = deal_rows<T>(chunks, gridDim.x);
@@ -443,7 +444,7 @@ __device__ __forceinline__ void choose_experts(const ExpertRows& e, float* z, in
 }
 
 // act = unit(gate, up) for the token's experts (blockIdx.y < top) and the dense or shared feed-forward (the last).
-template <typename T>
+template <typename T, int PARTS>
 __global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(RowStep p, const float* __restrict__ h, ExpertRows e,
                                                                const T* __restrict__ experts, const T* __restrict__ dense, int ld,
                                                                float* __restrict__ act) {
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(RowStep p, const
     __shared__ float best[kMaxTop];
     float *xs = smem, *red = xs + ld, *inv = red + kThreads / 64;
     const int slot = blockIdx.y;
-    StepRow row(p);
+    StepRow<PARTS> row(p);
     if (!h) row.load();
     if (e.logits) choose_experts(e, red, ids, best);  // the places of red and inv are free until the row is formed
     const T* w = slot < e.top ? experts + (size_t)(e.logits ? ids[slot] : expert_of(e, slot)) * e.pair_rows * ld : dense;
@@ -543,7 +544,7 @@ __global__ __launch_bounds__(kThreads) void gemv_ff_down_kernel(ExpertRows e, co
 class MixerPrologue {
    public:
     __device__ __forceinline__ explicit MixerPrologue(const MixerRow& m)
-        : m_(m), parts_(m.width, m.norm ? m.heads : 1), quads_(m.shares.part && m.vdim % 4 == 0), normed_(m.norm && parts_.fits()) {}
+        : m_(m), parts_(m.width, m.norm ? m.heads : 1, threadIdx.x), quads_(m.shares.part && m.vdim % 4 == 0), normed_(m.norm && parts_.fits()) {}
     __device__ __forceinline__ void load() {
         const int t = threadIdx.x;
         if (quads_) {
@@ -743,19 +744,30 @@ size_t step_lds(int ld, const RowStep& p) {
     return (ld + kThreads / 64 + groups) * sizeof(float);
 }
 
+// A row that fits two float4s a thread (2048 elements in 8 groups, say) leaves registers for four workgroups on a CU, one that needs
+// four for three.  32768 x 2048 (a head, 1024 workgroups): 32.7 us with three, 27.2 us = 4.9 TB/s with four; 6192 x 2048: 12.1 and
+// 9.5 us.  Forcing the larger form into registers for four spills and is slower (gate and up 14.4 -> 19.6 us).
+bool fits_two_parts(const RowStep& p) { return RowParts<kThreads, 2>(p.width, p.norm_h.groups, 0).fits(); }
+
+template <typename T, typename Emit>
+hipError_t launch_step(const RowStep& p, const T* w, int ld, int N, const Emit& emit, hipStream_t s) {
+    const dim3 grid(workgroups<T>(N, ld, kMaxGrid)), threads(kThreads);
+    if (fits_two_parts(p))
+        hipLaunchKernelGGL((gemv_step_kernel<T, 2, Emit>), grid, threads, step_lds(ld, p), s, p, w, ld, N, emit);
+    else
+        hipLaunchKernelGGL((gemv_step_kernel<T, 4, Emit>), grid, threads, step_lds(ld, p), s, p, w, ld, N, emit);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 template <typename T>
 hipError_t launch_gemv_step(const RowStep& p, const T* w, int ld, int N, float* C, hipStream_t s) {
-    hipLaunchKernelGGL((gemv_step_kernel<T, PlainEmit>), dim3(workgroups<T>(N, ld, kMaxGrid)), dim3(kThreads), step_lds(ld, p), s, p, w, ld,
-                       N, PlainEmit{C, N, 1.f});
-    return hipGetLastError();
+    return launch_step(p, w, ld, N, PlainEmit{C, N, 1.f}, s);
 }
 template <typename T>
 hipError_t launch_gemv_step_heads(const RowStep& p, const T* w, int ld, int N, const HeadRows<T>& heads, hipStream_t s) {
-    hipLaunchKernelGGL((gemv_step_kernel<T, HeadsEmit<T>>), dim3(workgroups<T>(N, ld, kMaxGrid)), dim3(kThreads), step_lds(ld, p), s, p, w,
-                       ld, N, HeadsEmit<T>{heads, N});
-    return hipGetLastError();
+    return launch_step(p, w, ld, N, HeadsEmit<T>{heads, N}, s);
 }
 template <typename T>
 hipError_t launch_gemv_plain(const float* x, int K, const T* w, int ld, int N, float* C, hipStream_t s) {
@@ -794,8 +806,12 @@ hipError_t launch_gemv_gate_up(const RowStep& p, const float* h, const ExpertRow
     const size_t router = e.logits ? (ld + e.experts) * sizeof(float) : 0, lds = step_lds(ld, p);
     // behind a router a workgroup first has to learn its expert: two rounds of rows for each of the 512 that fit the chip at once
     const int limit = e.logits && slots < 16 ? 512 / slots : e.logits ? 32 : kMaxGrid;
-    hipLaunchKernelGGL(gemv_gate_up_kernel<T>, dim3(workgroups<T>(2 * most, ld, limit), slots), dim3(kThreads), lds > router ? lds : router, s,
-                       p, h, e, experts, dense, ld, act);
+    const dim3 grid(workgroups<T>(2 * most, ld, limit), slots), threads(kThreads);
+    const size_t bytes = lds > router ? lds : router;
+    if (h || fits_two_parts(p))  // with the row already normed there are no parts
+        hipLaunchKernelGGL((gemv_gate_up_kernel<T, 2>), grid, threads, bytes, s, p, h, e, experts, dense, ld, act);
+    else
+        hipLaunchKernelGGL((gemv_gate_up_kernel<T, 4>), grid, threads, bytes, s, p, h, e, experts, dense, ld, act);
     return hipGetLastError();
 }
 template <typename T>

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kThreads) void residual_norm_kernel(const float* x,
                                                                 int width, const float* __restrict__ add) {
     constexpr int P = RowParts<kThreads>::kParts;
     __shared__ float red[kThreads / 64];
-    const RowParts<kThreads> parts(width, norm_h.groups);
+    const RowParts<kThreads> parts(width, norm_h.groups, threadIdx.x);
     const size_t m = blockIdx.x, base = m * width;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 r[P], v[P];

@@ -87,3 +87,17 @@ def test_logits_that_do_not_fit_the_staging(pkg):
     eight = model.forward(ids, range(3, 27, 3))
     model.reset()
     assert nine.shape == (9, 32768) and np.array_equal(nine[:8], eight) and np.array_equal(nine[8], model.forward(ids[:28])[0])
+
+
+# a residual row in two float4s a thread at most, in three or four, and past what a thread holds
+@pytest.mark.parametrize("width", [2048, 2052, 4096, 4100])
+def test_one_token_rows(pkg, width):
+    cfg = tx.config(50, width, 1, [tx.layer(tx.mixer(1, 8, 8, 8, 16, 24, 0.4), tx.dense(40)),
+                                   tx.layer(tx.mixer(1, 8, 8, 8, 16, 24, 0.4, kv_from=0), tx.moe(2, 1, 16, shared=24))])
+    model = pkg.Model.random(cfg, 8, "float32", seed=3)
+    got = [model.forward([t]) for t in (7, 7, 49, 3)]
+    model.reset()
+    model.set_option("unfused", 1)
+    for i, t in enumerate((7, 7, 49, 3)):   # the same sums in 32 bits in another order, two layers deep
+        want = model.forward([t])
+        assert np.linalg.norm(got[i] - want) <= 3e-5 * np.linalg.norm(want), i
