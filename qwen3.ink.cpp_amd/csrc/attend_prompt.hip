@@ -11,9 +11,9 @@
 // one value per lane.  Scores, softmax and sums are fp32; the maximum follows every larger score, so that the heaviest
 // weight, 1, is exact in 16 bits (left behind by up to 2^8 it is not: 14 % more error for 8 % less time).
 //
-// A tile is copied global -> LDS by direct 16-byte loads, the next one while this one is worked on.  Key rows: chunk c of key k
-// at place c ^ (k % 4 + k / 8 % 2 * 4), so that eight rows r read at once fall on eight places; transposed values:
-// chunk c of column d at place c ^ d % 8.
+// A tile is copied global -> LDS by direct 16-byte loads, the next one while this one is worked on.  Chunk c of key k sits at place
+// c ^ k % 16, or, where rows are an odd number of 128 bytes, c ^ k / 2 % 8; chunk c of a transposed value column d at c ^ d / 2 % 8:
+// sixteen rows read at one chunk column cover the 256 bytes of all banks.
 //
 // What bounds it: matrix ops and softmax of a SIMD's two waves, one after the other; then LDS, which gives an operand of 1 KiB
 // for every matrix op.  4095 rows of 16 heads, 192 + 128 columns: 117 us = 730 TFLOP/s, against 537 us with 16 x 16 matrix ops,
@@ -31,7 +31,10 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLowest = -1e30f;
 constexpr int kTile = 64;      // keys
 
-__device__ __forceinline__ int place_of_key(int k) { return (k & 3) | (k >> 1 & 4); }
+template <int DK>
+__device__ __forceinline__ int place_of_key(int k) {
+    return DK % 128 ? (k >> 1) & 7 : k & 15;
+}
 // the larger, or the sum, of this lane's value and that of the other lane half
 __device__ __forceinline__ float other_half(float v) {
     const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -71,7 +74,7 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
     const bf16* value_src[NV ? NV : 1];
     uint8_t* const my_lds = lds + kg * 2 * kBuf;
     auto key_place = [&](int n, int key, int* step) -> const uint8_t* {  // source of copy n if its row is that key
-        const int q = (n * QW + qw) * 64 + lane, r = q / CK, c = (q % CK) ^ place_of_key(r);
+        const int q = (n * QW + qw) * 64 + lane, r = q / CK, c = (q % CK) ^ place_of_key<DK>(r);
         const bf16* src = a.k_own + z * a.k_own_head + (size_t)key * a.ld_k_own;
         int ld = a.ld_k_own;
         if constexpr (KEY0 > 0) {
@@ -94,7 +97,7 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
     if constexpr (EXPANDED) {
 #pragma unroll
         for (int n = 0; n < NV; n++) {
-            const int q = (n * QW + qw) * 64 + lane, r = q >> 3, c = (q & 7) ^ (r & 7);
+            const int q = (n * QW + qw) * 64 + lane, r = q >> 3, c = (q & 7) ^ ((r >> 1) & 7);
             value_src[n] = a.v_t + ((size_t)z * a.dv + min(r, a.dv - 1)) * a.ld_v + key_begin + kg * kTile + c * 8;
         }
     }
@@ -149,16 +152,19 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
     float mx = sink ? 0.f : kLowest, sum = sink && half == 0 ? 1.f : 0.f;
 
     const int key_row = (l31 & 0x13) | (l31 & 4) << 1 | (l31 & 8) >> 1;  // bits 2 and 3 exchanged
-    const int key_at = key_row * (DK * 2), key_swap = place_of_key(key_row);
+    const int key_at = key_row * (DK * 2), key_swap = place_of_key<DK>(key_row);
     // Values that are columns of the key rows come by transposing reads (ds_read_b64_tr_b16): in a group of 16 lanes lane i
     // names four columns of key i / 4 and receives its own column of the four keys.
-    int value_at[2];
+    constexpr int VA = VF < 4 ? VF : 4;
+    int value_at[VA][2];  // by f % 4, and for the first and the second four keys
     if constexpr (!EXPANDED) {
 #pragma unroll
-        for (int f = 0; f < 2; f++) {
-            const int i = lane & 15, k = 8 * half + (i >> 2), c = 4 * f + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
-            value_at[f] = k * (DK * 2) + ((c ^ place_of_key(k)) << 4) + (i & 1) * 8;
-        }
+        for (int f = 0; f < VA; f++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int i = lane & 15, k = 8 * half + 4 * j + (i >> 2), c = 4 * f + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+                value_at[f][j] = k * (DK * 2) + ((c ^ place_of_key<DK>(k)) << 4) + (i & 1) * 8;
+            }
     }
 
     if (kg < n_tiles) copy_tile(kg, 0);
@@ -223,11 +229,11 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
             for (int f = 0; f < VF; f++) {
                 bf16x8 vf;
                 if constexpr (EXPANDED) {
-                    vf = *reinterpret_cast<const bf16x8*>(vb + (f * 32 + l31) * (kTile * 2) + (((2 * u + half) ^ (l31 & 7)) << 4));
+                    vf = *reinterpret_cast<const bf16x8*>(vb + (f * 32 + l31) * (kTile * 2) + (((2 * u + half) ^ ((l31 >> 1) & 7)) << 4));
                 } else {
-                    const uint8_t* at = kb + value_at[f & 1] + (f >> 1) * 128 + u * 16 * (DK * 2);
-                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at));
-                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + 4 * (DK * 2)));
+                    const uint8_t* at = kb + (f >> 2) * 256 + u * 16 * (DK * 2);
+                    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + value_at[f & 3][0]));
+                    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + value_at[f & 3][1]));
                     const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
                     vf = *reinterpret_cast<const bf16x8*>(&both);
                 }

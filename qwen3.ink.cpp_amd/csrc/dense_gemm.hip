@@ -3,8 +3,7 @@
 //
 // A workgroup takes a BM x BN tile, each of its waves an equal part of it in 32 x 32 pieces.  K goes in steps of 128 bytes
 // per row; a step's rows are copied global -> LDS by direct 16-byte loads into one of STAGES stages, later steps' copies in
-// flight while one is multiplied.  In LDS chunk c of row r sits at place c ^ (r & 7), so that the 32 rows a wave reads at one
-// chunk column spread over the banks.  A fragment is the same 16 bytes per lane for both types: lane l holds row l & 31,
+// flight while one is multiplied.  A fragment is the same 16 bytes per lane for both types: lane l holds row l & 31,
 // chunk 2 kk + (l >> 5).
 //
 // What bounds it: bytes per product.  A 128 x 128 tile asks the L2 for 64 bytes a clock and CU at the matrix cores' full rate,
@@ -30,6 +29,9 @@ __device__ __forceinline__ void mma(f32x16& acc, const lds16& a, const lds16& b,
 }
 
 struct NoHeads {};
+
+// Chunk c of row r sits at place c ^ this: sixteen rows read at one chunk column then cover the 256 bytes of all banks.
+__device__ __forceinline__ int place_of_row(int r) { return (r >> 1) & 7; }
 
 // the value of the lane whose number differs in the lowest bit
 __device__ __forceinline__ float swap_neighbours(float v) {
@@ -131,12 +133,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(G
         const int c = i * kThreads + tid, r = c >> 3;
         int row = m0 + min(r, rows - 1);
         if (g.a_rows) row = g.a_rows[row];
-        a_src[i] = A + (size_t)row * g.lda * sizeof(T) + (((c & 7) ^ (r & 7)) << 4);
+        a_src[i] = A + (size_t)row * g.lda * sizeof(T) + (((c & 7) ^ place_of_row(r)) << 4);
     }
 #pragma unroll
     for (int i = 0; i < LB; i++) {
         const int c = i * kThreads + tid, r = c >> 3;
-        b_src[i] = W + (size_t)min(n0 + r, g.N - 1) * g.ldw * sizeof(T) + (((c & 7) ^ (r & 7)) << 4);
+        b_src[i] = W + (size_t)min(n0 + r, g.N - 1) * g.ldw * sizeof(T) + (((c & 7) ^ place_of_row(r)) << 4);
     }
     auto copy_step = [&](int step, int stage) {
         uint8_t* base = lds + stage * kStage + wave * 1024;
@@ -171,12 +173,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(G
 #pragma unroll
             for (int i = 0; i < FM; i++) {
                 const int r = wm + i * 32 + l31;
-                a[kk & 1][i] = *reinterpret_cast<const lds16*>(sa + r * 128 + (((2 * kk + half) ^ (r & 7)) << 4));
+                a[kk & 1][i] = *reinterpret_cast<const lds16*>(sa + r * 128 + (((2 * kk + half) ^ place_of_row(r)) << 4));
             }
 #pragma unroll
             for (int j = 0; j < FN; j++) {
                 const int r = wn + j * 32 + l31;
-                b[kk & 1][j] = *reinterpret_cast<const lds16*>(sb + r * 128 + (((2 * kk + half) ^ (r & 7)) << 4));
+                b[kk & 1][j] = *reinterpret_cast<const lds16*>(sb + r * 128 + (((2 * kk + half) ^ place_of_row(r)) << 4));
             }
         };
         if constexpr (PIPE) read(0);
@@ -215,7 +217,8 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
     const int t = xcd < r8 ? xcd * (q + 1) + idx : r8 * (q + 1) + (xcd - r8) * q + idx;
     const int m0 = t % n_mt * 64, n0 = t / n_mt * 32, rows = g.M - m0, n_steps = g.K * (int)sizeof(T) / 128;
     const long long batch = blockIdx.y;
-    const int copy_row = (wave & 1) * (wave < 4 ? 32 : 16) + (lane >> 3), swapped = ((lane & 7) ^ (lane >> 3)) << 4;  // of the wave's first copy
+    const int copy_row = (wave & 1) * (wave < 4 ? 32 : 16) + (lane >> 3);  // of the wave's first copy
+    auto swapped = [&](int i) { return ((lane & 7) ^ place_of_row(copy_row + 8 * i)) << 4; };
     uint8_t* const lds_w = lds + SA * kStageA;
     if (wave >= 2) {  // COPIES a step and wave, 8 rows each, into a ring of S stages
         auto run = [&](auto copies, auto stages, const uint8_t* (&src)[4], uint8_t* ring, int stage_bytes) {
@@ -246,13 +249,13 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
             for (int i = 0; i < 4; i++) {
                 int row = m0 + min(copy_row + 8 * i, rows - 1);
                 if (g.a_rows) row = g.a_rows[row];
-                src[i] = A + (size_t)row * g.lda * sizeof(T) + swapped;
+                src[i] = A + (size_t)row * g.lda * sizeof(T) + swapped(i);
             }
             run(std::integral_constant<int, 4>{}, std::integral_constant<int, SA>{}, src, lds, kStageA);
         } else {
             const uint8_t* W = reinterpret_cast<const uint8_t*>(static_cast<const T*>(g.W) + batch * g.w_step);
 #pragma unroll
-            for (int i = 0; i < 2; i++) src[i] = W + (size_t)min(n0 + copy_row + 8 * i, g.N - 1) * g.ldw * sizeof(T) + swapped;
+            for (int i = 0; i < 2; i++) src[i] = W + (size_t)min(n0 + copy_row + 8 * i, g.N - 1) * g.ldw * sizeof(T) + swapped(i);
             run(std::integral_constant<int, 2>{}, std::integral_constant<int, SW>{}, src, lds_w, kStageW);
         }
         return;
@@ -266,7 +269,7 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
         const uint8_t *pa = lds + slot_a * kStageA + wave * 4096 + l31 * 128, *pw = lds_w + slot_w * kStageW + l31 * 128;
 #pragma unroll
         for (int kk = 0; kk < 4; kk++) {
-            const int at = ((2 * kk + half) ^ (l31 & 7)) << 4;
+            const int at = ((2 * kk + half) ^ place_of_row(l31)) << 4;
             x[kk] = *reinterpret_cast<const lds16*>(pa + at);
             y[kk] = *reinterpret_cast<const lds16*>(pw + at);
         }
