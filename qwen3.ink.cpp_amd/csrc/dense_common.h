@@ -36,32 +36,47 @@ __device__ __forceinline__ int expert_rank(const float* z, int n, int e) {
     return rank;
 }
 
-// One column of a HeadRows product for row m: `own` is its value, `other` that of its pair's other column.
+// Where one column of a HeadRows product goes.
 template <typename T>
-__device__ __forceinline__ void store_head_column(const HeadRows<T>& p, int pos, int m, int col, float own, float other) {
-    const int nq = p.heads * p.dim, nk = p.kv_heads * p.dim, nv = p.kv_heads * p.vdim;
-    if (col >= nq + nk + nv) {
-        p.rest[(size_t)m * p.ld_rest + col - nq - nk - nv] = own;
-        return;
+class HeadColumn {
+   public:
+    __device__ __forceinline__ HeadColumn(const HeadRows<T>& p, int col) : p_(p) {
+        const int nq = p.heads * p.dim, nk = p.kv_heads * p.dim, nv = p.kv_heads * p.vdim;
+        rest_ = col >= nq + nk + nv;
+        cached_ = col >= nq;
+        if (rest_) {
+            at_ = col - nq - nk - nv;
+        } else if (col >= nq + nk) {
+            const int c = col - nq - nk, h = c / p.vdim;
+            at_ = h * (p.vdim + p.dim) + (c - h * p.vdim);
+        } else {
+            const int c = cached_ ? col - nq : col, h = c / p.dim, d = c - h * p.dim;
+            at_ = cached_ ? h * (p.vdim + p.dim) + p.vdim + d : c;
+            if ((d >> 1) < p.rot_pairs) pair_ = d >> 1, second_ = d & 1;
+        }
     }
-    const int at = min(pos + m, p.max_seq - 1);
-    if (col >= nq + nk) {
-        const int c = col - nq - nk, h = c / p.vdim;
-        p.cache[(size_t)at * p.ld_cache + h * (p.vdim + p.dim) + (c - h * p.vdim)] = (T)own;
-        return;
+    // of row m, the token at position pos + m
+    __device__ __forceinline__ void angle(int m, int pos, float& cs, float& sn) const {
+        if (pair_ < 0) return;
+        const size_t i = (size_t)min(pos + m, p_.max_seq - 1) * p_.rot_pairs + pair_;
+        cs = p_.cos_t[i], sn = p_.sin_t[i];
     }
-    const bool key = col >= nq;
-    const int c = key ? col - nq : col, h = c / p.dim, d = c - h * p.dim;
-    if ((d >> 1) < p.rot_pairs) {
-        const size_t i = (size_t)at * p.rot_pairs + (d >> 1);
-        const float cs = p.cos_t[i], sn = p.sin_t[i];
-        own = (d & 1) ? own * cs + other * sn : own * cs - other * sn;
+    // `own` is the column's value in row m, `other` that of its pair's other column
+    __device__ __forceinline__ void store(int m, int pos, float own, float other, float cs, float sn) const {
+        if (pair_ >= 0) own = second_ ? own * cs + other * sn : own * cs - other * sn;
+        if (rest_)
+            p_.rest[(size_t)m * p_.ld_rest + at_] = own;
+        else if (cached_)
+            p_.cache[(size_t)min(pos + m, p_.max_seq - 1) * p_.ld_cache + at_] = (T)own;
+        else
+            p_.q[(size_t)m * (p_.heads * p_.dim) + at_] = (T)own;
     }
-    if (key)
-        p.cache[(size_t)at * p.ld_cache + h * (p.vdim + p.dim) + p.vdim + d] = (T)own;
-    else
-        p.q[(size_t)m * nq + c] = (T)own;
-}
+
+   private:
+    const HeadRows<T>& p_;
+    int at_, pair_ = -1;
+    bool rest_, cached_, second_ = false;
+};
 
 // One direct copy global -> LDS of 16 bytes per lane: lane l's bytes land at lds_base + 16 l (lds_base uniform).
 __device__ __forceinline__ void copy16_to_lds(const void* global_src, void* lds_base) {

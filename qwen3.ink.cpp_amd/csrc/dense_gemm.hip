@@ -70,16 +70,26 @@ __device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, c
         }
         return;
     }
-    [[maybe_unused]] int pos = 0;
-    if constexpr (EPI == Epilogue::kHeads) pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1);
+    if constexpr (EPI == Epilogue::kHeads) {
+        // the column's place once, then the rows' angles all at a time
+        const HeadColumn<T> to(heads, min(col, g.N - 1));
+        const int pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1);
+        float cs[NV], sn[NV];
+#pragma unroll
+        for (int v = 0; v < NV; v++) to.angle(min(m0 + r0 + 8 * (v >> 2) + (v & 3), g.M - 1), pos, cs[v], sn[v]);
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+            const int r = r0 + 8 * (v >> 2) + (v & 3);
+            const float other = swap_neighbours(x[v]);
+            if (r < rows && col < g.N) to.store(m0 + r, pos, x[v], other, cs[v], sn[v]);
+        }
+        return;
+    }
 #pragma unroll
     for (int v = 0; v < NV; v++) {
         const int r = r0 + 8 * (v >> 2) + (v & 3);
         const size_t row = m0 + r;
-        if constexpr (EPI == Epilogue::kHeads) {
-            const float other = swap_neighbours(x[v]);
-            if (r < rows && col < g.N) store_head_column(heads, pos, (int)row, col, x[v], other);
-        } else if (r < rows && col < g.N) {
+        if (r < rows && col < g.N) {
             if constexpr (EPI == Epilogue::kFloat) {
                 (static_cast<float*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = x[v];
             } else {

@@ -230,8 +230,14 @@ struct HeadsEmit {
     int N;
     __device__ void operator()(int n, float s0, float s1) const {
         const int pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1);
-        store_head_column(heads, pos, 0, 2 * n, s0, s1);
-        if (2 * n + 1 < N) store_head_column(heads, pos, 0, 2 * n + 1, s1, s0);
+        store(2 * n, pos, s0, s1);
+        if (2 * n + 1 < N) store(2 * n + 1, pos, s1, s0);
+    }
+    __device__ void store(int col, int pos, float own, float other) const {
+        const HeadColumn<T> to(heads, col);
+        float cs = 1.f, sn = 0.f;
+        to.angle(0, pos, cs, sn);
+        to.store(0, pos, own, other, cs, sn);
     }
 };
 
