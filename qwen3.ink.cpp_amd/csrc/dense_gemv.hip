@@ -814,7 +814,9 @@ hipError_t launch_gemv_gate_up(const RowStep& p, const float* h, const ExpertRow
     const int limit = e.logits && slots < 16 ? 512 / slots : e.logits ? 32 : kMaxGrid;
     const dim3 grid(workgroups<T>(2 * most, ld, limit), slots), threads(kThreads);
     const size_t bytes = lds > router ? lds : router;
-    if (h || fits_two_parts(p))  // with the row already normed there are no parts
+    // with the row already normed there are no parts and its length alone decides: Dimesun with rows of 4096, a token, 0.762 ms
+    // with the smaller form and 0.756 ms with the larger
+    if (h ? ld <= 2 * 4 * kThreads : fits_two_parts(p))
         hipLaunchKernelGGL((gemv_gate_up_kernel<T, 2>), grid, threads, bytes, s, p, h, e, experts, dense, ld, act);
     else
         hipLaunchKernelGGL((gemv_gate_up_kernel<T, 4>), grid, threads, bytes, s, p, h, e, experts, dense, ld, act);
