@@ -16,9 +16,9 @@
 // sixteen rows read at one chunk column cover the 256 bytes of all banks.
 //
 // What bounds it: matrix ops and softmax of a SIMD's two waves, one after the other; then LDS, which gives an operand of 1 KiB
-// for every matrix op.  4095 rows of 16 heads, 192 + 128 columns: 117 us = 730 TFLOP/s, against 537 us with 16 x 16 matrix ops,
+// for every matrix op.  4095 rows of 16 heads, 192 + 128 columns: 120 us = 712 TFLOP/s, against 537 us with 16 x 16 matrix ops,
 // heads' rows dealt out one head after the other and one workgroup of four waves on a CU; 2048 rows in chunks of 1024, 16 heads
-// on 4 of 128 + 128 columns: 29 us against 71 us.
+// on 4 of 128 + 128 columns: 31 us against 71 us.
 #include "dense_common.h"
 
 namespace a81w41 {
