@@ -129,7 +129,7 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
     const int limit = last_key(my_row), first = chunk_begin(limit);
     const int lowest_limit = last_key(min(wave_row0, a.rows - 1)), highest_limit = last_key(min(wave_row0 + 31, a.rows - 1));
     const int highest_first = chunk_begin(highest_limit);
-    const float scale = fmaxf(fabsf(a.scale), 1e-30f) * kLog2e;  // a score of minus infinity times it stays that
+    const float scale = fabsf(a.scale) * kLog2e;
     bf16x8 qf[KS];
     {
         const bf16* src = a.q + z * a.q_head + (size_t)my_token * a.q_token + (my_row - my_token * a.rows_per_token) * a.ld_q;
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[f][v] = 0.f;
     const bool sink = a.sink && kg == 0 && (a.splits == 1 || blockIdx.z == 0);  // one lane half of one group of one share counts it
-    float mx = sink ? 0.f : kLowest, sum = sink && half == 0 ? 1.f : 0.f;
+    float mx = sink || scale == 0.f ? 0.f : kLowest, sum = sink && half == 0 ? 1.f : 0.f;
 
     const int key_row = (l31 & 0x13) | (l31 & 4) << 1 | (l31 & 8) >> 1;  // bits 2 and 3 exchanged
     const int key_at = key_row * (DK * 2), key_swap = place_of_key<DK>(key_row);
@@ -218,7 +218,9 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
         for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                const float p = __builtin_amdgcn_exp2f(fmaf(sc[t][v], scale, -mx));
+                // a modifier of the exponential's instruction: a weight that is no number (of a score that is none, or of a masked one
+                // under a scale of zero) becomes 0
+                const float p = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(fmaf(sc[t][v], scale, -mx)), 0.f, 1.f);
                 add[v & 3] += p;
                 pf[2 * t + (v >> 3)][v & 7] = (bf16)p;
             }

@@ -77,6 +77,72 @@ def test_attention_over_a_prompt(pkg, M, pos, chunk, splits, dim, vdim, scale):
         assert ((got[:, h] - want).abs() <= bound).all(), (h, ((got[:, h] - want).abs() / bound).max().item())
 
 
+def _weights_of(scores, sees, sink):
+    """Softmax over the keys that are seen, in 64 bits; a score that is no number takes its key away."""
+    import torch
+    s = torch.where(sees & ~scores.isnan(), scores, -float("inf"))
+    if sink:
+        s = torch.cat([s, torch.zeros_like(s[:, :1])], 1)
+    return s.softmax(1)[:, :sees.shape[1]]
+
+
+def _assert_attended(got, p, v, gate=1.0):
+    want = p @ v * gate
+    bad = want.isnan()
+    assert (got.isnan() == bad).all()
+    bound = 2.0 ** -8 * ((p @ v.abs()) * gate + want.abs()) + 1e-5
+    assert ((got - want).abs() <= bound)[~bad].all(), ((got - want).abs() / bound)[~bad].max().item()
+
+
+# Keys that give no number, minus infinity and, late in the sequence, infinity, as the first key of all and among others; by the kernel
+# of short prompts (150 tokens of three heads on one) and that of long ones.
+@pytest.mark.parametrize("M,splits", [(150, 1), (700, 1), (700, 3)])
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("scale", [0.09, 0.0])
+@pytest.mark.parametrize("sink", [False, True])
+def test_keys_without_a_score(pkg, M, splits, dim, scale, sink):
+    import torch
+    heads, kv_heads = 6, 2
+    g = torch.Generator(device="cuda").manual_seed(M + dim)
+    q = torch.randn(M, heads, dim, device="cuda", generator=g).bfloat16()
+    q[..., 11] = q[..., 11].abs() + 0.5
+    rows = torch.randn(M, kv_heads * 2 * dim, device="cuda", generator=g).bfloat16()
+    rows[0, dim + 5] = rows[77, dim] = rows[64, 3 * dim + 9] = float("nan")
+    rows[40, dim + 11] = rows[130, 3 * dim + 11] = -float("inf")
+    rows[M - 40, dim + 11] = float("inf")
+    got = pkg.ops.grouped_attention(q, rows, 0, kv_heads, dim, dim, scale, 0, sink, 1, splits).double()
+    sees = torch.ones(M, M, dtype=torch.bool, device="cuda").tril()
+    parts = rows.double().view(M, kv_heads, 2 * dim)
+    for h in range(heads):
+        part = parts[:, h // 3]
+        scores = (q[:, h, None].double() * part[None, :, dim:]).sum(2) * scale
+        _assert_attended(got[:, h], _weights_of(scores, sees, sink), part[:, :dim])
+
+
+@pytest.mark.parametrize("dim,rot,vdim", [(64, 32, 64), (128, 64, 128), (256, 64, 256)])
+@pytest.mark.parametrize("scale", [0.09, 0.0])
+def test_formed_keys_without_a_score(pkg, dim, rot, vdim, scale):
+    import torch
+    M, heads = 300, 3
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    q = torch.randn(M, heads, dim + rot, device="cuda", generator=g).bfloat16()
+    q[..., 11] = q[..., 11].abs() + 0.5
+    k = torch.randn(M, heads * dim, device="cuda", generator=g).bfloat16()
+    k_rot = torch.randn(M, rot, device="cuda", generator=g).bfloat16()
+    v = torch.randn(heads * vdim, (M + 63) // 64 * 64, device="cuda", generator=g).bfloat16()
+    gates = torch.randn(M, heads, device="cuda", generator=g)
+    k[0, 5] = k[77, 2 * dim + 1] = k_rot[64, 2] = float("nan")
+    k[40, 11] = -float("inf")
+    k[M - 40, dim + 11] = float("inf")
+    got = pkg.ops.formed_attention(q, k, k_rot, v, gates, 0, vdim, scale).double().view(M, heads, vdim)
+    sees = torch.ones(M, M, dtype=torch.bool, device="cuda").tril()
+    for h in range(heads):
+        keys = torch.cat([k[:, h * dim:(h + 1) * dim], k_rot], 1).double()
+        scores = (q[:, h, None].double() * keys[None]).sum(2) * scale
+        p = _weights_of(scores, sees, False)
+        _assert_attended(got[:, h], p, v[h * vdim:(h + 1) * vdim, :M].double().t(), gates[:, h:h + 1].double().sigmoid())
+
+
 def test_logits_that_do_not_fit_the_staging(pkg):
     """Nine rows of 32768 logits are copied, eight and fewer go out through pinned memory."""
     cfg = tx.config(32768, 64, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.dense(64))])
