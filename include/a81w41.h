@@ -380,7 +380,7 @@ enum {
     A81W41_QWEN3_BUF_ACT = 6, A81W41_QWEN3_BUF_LOGITS = 7
 };
 int a81w41_qwen3_read_buffer(a81w41_qwen3 *model, int which, float *host_out, size_t count);
-/* Forget the cached context (position 0). */
+/* Forget the cached context (position 0).  Only enqueues; an error on the device shows in the next call that synchronises. */
 int a81w41_qwen3_reset(a81w41_qwen3 *model);
 /* Qwen3ForCausalLM::forward: n_tokens new token ids (host) on top of the cached context;
  * logits of the last token ([vocab] fp32) are copied to logits_host if it is not NULL.

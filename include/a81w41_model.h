@@ -30,7 +30,8 @@ int a81w41_model_vocab(const a81w41_model *model);
 int a81w41_model_max_seq(const a81w41_model *model);
 int a81w41_model_position(const a81w41_model *model); /* tokens in the cache */
 
-/* Give back what the sequence holds in the cache: the next token is at position 0. */
+/* Give back what the sequence holds in the cache: the next token is at position 0.  Only enqueues the clearing, ahead of
+ * whatever the model does next; an error on the device shows in the next call that synchronises. */
 int a81w41_model_reset(a81w41_model *model);
 /* n_tokens new tokens (host) on top of the cached ones.  logits_host [n_want][vocab] receives the logits at the
  * places want[0..n_want) among them, which must rise; n_want may be 0.  Synchronises. */

@@ -93,8 +93,16 @@ int DecoderSession::reset() {
     return 0;
 }
 
-// The ids and wanted rows of a pass of at most max_rows_ tokens.  No earlier upload may still be waiting in the stream.
+int DecoderSession::drain() {
+    A81W41_HIP_TRY(hipStreamSynchronize(stream));
+    upload_waits_ = false;
+    return 0;
+}
+
+// The ids and wanted rows of a pass of at most max_rows_ tokens.
 int DecoderSession::upload(const int* token_ids, int n, const int* want, int n_want) {
+    if (upload_waits_) A81W41_TRY(drain());  // of an earlier portion, or of a pass that failed on its way
+    upload_waits_ = true;
     std::copy_n(token_ids, n, staged_ids_);
     std::copy_n(want, n_want, staged_ids_ + max_rows_);
     A81W41_HIP_TRY(launch_take_tokens(staged_ids_, n, ids, staged_ids_ + max_rows_, n_want, want_dev, stream));
@@ -123,7 +131,7 @@ int DecoderSession::forward(const int* token_ids, int n, const int* want, int n_
         const size_t out = logits_host ? (size_t)nw * vocab_ : 0;
         const bool staged = out && out <= staged_floats_;
         if (staged) A81W41_HIP_TRY(launch_give_floats(logits, staged_logits_, out, stream));
-        A81W41_HIP_TRY(hipStreamSynchronize(stream));
+        A81W41_TRY(drain());
         host_pos += m;
         A81W41_TRY(check_passes());
         if (staged)
@@ -165,16 +173,13 @@ int DecoderSession::generate_greedy(const int* prompt, int n_prompt, int n_new, 
     for (int at = 0; at < n_prompt; at += max_rows_) {
         const int m = std::min(max_rows_, n_prompt - at);
         plan_ctx = m == 1 ? last_ctx : host_pos + at + m;
-        if (at) {
-            A81W41_HIP_TRY(hipStreamSynchronize(s));
-            A81W41_TRY(upload(prompt + at, m, nullptr, 0));
-        }
+        if (at) A81W41_TRY(upload(prompt + at, m, nullptr, 0));
         A81W41_TRY(enqueue_pass(m, &last_row, at + m == n_prompt ? 1 : 0, s));
     }
     // first new token: argmax of the prompt's logits; it becomes the next pass's input id
     A81W41_HIP_TRY(launch_argmax_token(logits, vocab_, ids, history, history_len, step, s));
     A81W41_HIP_TRY(hipEventRecord(e1, s));
-    A81W41_HIP_TRY(hipStreamSynchronize(s));
+    A81W41_TRY(drain());
     host_pos += n_prompt;
 
     const int n_steps = n_new - 1;

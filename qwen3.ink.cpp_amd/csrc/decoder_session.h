@@ -109,8 +109,11 @@ class DecoderSession {
    private:
     int reserve_logits(int rows);
     int upload(const int* token_ids, int n, const int* want, int n_want);
+    int drain();  // waits for the stream
     int max_seq_ = 0, vocab_ = 0, max_rows_ = 0;
-    // pinned: ids and wanted rows of a pass, read by an enqueued kernel until the stream is next waited for; logits on their way out
+    // pinned: ids and wanted rows of a pass, read by an enqueued kernel until the stream is next drained (upload_waits_ until then);
+    // logits on their way out
+    bool upload_waits_ = false;
     int* staged_ids_ = nullptr;
     float* staged_logits_ = nullptr;
     size_t staged_floats_ = 0;
