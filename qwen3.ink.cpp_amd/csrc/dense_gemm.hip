@@ -340,6 +340,11 @@ hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
     // rows, 12288 x 2048 20 / 16.
     const long long few = (long long)((g.N + 31) / 32) * ((g.M + 63) / 64) * g.batches;
     if (!g.tiles && few <= 256) return launch_few<T, EPI>(g, heads, s);
+    // 64 x 64 tiles with four stages fit a CU twice, with two stages five times: more tiles than 512 would go in rounds.  bfloat16,
+    // us with four / two: 1030 rows, 544 tiles, 2048 x 1024 15.9 / 12.2, 2048 x 6144 63 / 50; 1000 grouped tiles, 512 x 512 14.7 /
+    // 11.6; in one round, 400 rows, 448 tiles, 4096 x 4096 27.5 / 34.  float, 1030 rows, 2048 x 1024: 60.5 / 56.9.
+    const long long tiles64 = (long long)(g.tiles ? g.max_tiles : (g.M + 63) / 64) * ((g.N + 63) / 64) * g.batches;
+    if (tiles64 > 512) return launch_kernel<T, 64, 64, 2, 2, 2, false, EPI>(g, heads, s);
     return launch_kernel<T, 64, 64, 2, 2, 4, false, EPI>(g, heads, s);
 }
 

@@ -8,9 +8,10 @@ from tests import takosun_fixture as tx
 pytestmark = pytest.mark.gpu
 
 
-# 256 x 256 tiles; 128 x 128 two per CU; 128 x 128 alone on a CU with four stages, from fewer steps than stages on
+# 256 x 256 tiles; 128 x 128 two per CU; 128 x 128 alone on a CU with four stages, from fewer steps than stages on; 64 x 64, more of
+# them than fit two on every CU
 @pytest.mark.parametrize("M,N,K", [(2047, 6136, 64), (1793, 6400, 192), (2300, 2050, 128), (2045, 2000, 64), (2045, 1990, 192),
-                                   (1921, 2048, 320)])
+                                   (1921, 2048, 320), (1025, 1990, 64), (1030, 2048, 192), (700, 3070, 320)])
 def test_rows_of_a_product(pkg, M, N, K):
     import torch
     g = torch.Generator(device="cuda").manual_seed(M)
@@ -42,6 +43,11 @@ def _same_in_portions(pkg, cfg, n, cuts):
 
 def test_gated_pairs_on_large_tiles(pkg):
     cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.dense(6100))])
+    _same_in_portions(pkg, cfg, 2100, 100)
+
+
+def test_experts_on_many_small_tiles(pkg):
+    cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.moe(8, 2, 250))])
     _same_in_portions(pkg, cfg, 2100, 100)
 
 
