@@ -308,8 +308,14 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
 }
 
 // 256 x 256 tiles, one workgroup per CU, or 128 x 128, two per CU.  At K = 2048 a round of 256 large tiles takes 65 us whether
-// it is full or not, small tiles 44 us per 512 of them.
-bool large_tiles_preferred(long long large, long long small) { return (large + 255) / 256 * 750 <= small; }
+// it is full or not, small tiles 44 us per 512 of them; small ones overlap a round's end with the next one's start, so that large ones
+// have to be fuller where there are several rounds.  us with small / large, 768 small tiles a round: one round, 2047 rows, 6144 x 512
+// 26.0 / 24.1, x 2048 61.2 / 60.0; two, 1030 rows, 32768 x 512 61.3 / 64.6, 3000 rows, 8192 x 2048 111 / 117; with 864 a round,
+// 1030 rows, 24576 x 2048 123.8 / 122.0.
+bool large_tiles_preferred(long long large, long long small) {
+    const long long rounds = (large + 255) / 256;
+    return rounds * (rounds > 1 ? 800 : 750) <= small;
+}
 
 template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PIPE, Epilogue EPI, typename X>
 hipError_t launch_kernel(const GemmArgs& g, const X& heads, hipStream_t s) {
