@@ -814,9 +814,10 @@ hipError_t launch_gemv_gate_up(const RowStep& p, const float* h, const ExpertRow
     const int limit = e.logits && slots < 16 ? 512 / slots : e.logits ? 32 : kMaxGrid;
     const dim3 grid(workgroups<T>(2 * most, ld, limit), slots), threads(kThreads);
     const size_t bytes = lds > router ? lds : router;
-    // with the row already normed there are no parts and its length alone decides: Dimesun with rows of 4096, a token, 0.762 ms
-    // with the smaller form and 0.756 ms with the larger
-    if (h ? ld <= 2 * 4 * kThreads : fits_two_parts(p))
+    // A row that is already normed is held in no parts: the workgroups that stream behind a router are two a CU, and the larger form
+    // has the registers they want.  Dimesun, a token: rows of 4096 416 us with the smaller form and 413 with the larger, 2048 both 197,
+    // 1536 167.0 and 166.3, 1024 133.5 and 133.1.
+    if (!h && fits_two_parts(p))
         hipLaunchKernelGGL((gemv_gate_up_kernel<T, 2>), grid, threads, bytes, s, p, h, e, experts, dense, ld, act);
     else
         hipLaunchKernelGGL((gemv_gate_up_kernel<T, 4>), grid, threads, bytes, s, p, h, e, experts, dense, ld, act);
