@@ -25,6 +25,38 @@ def test_rows_of_a_product(pkg, M, N, K):
         assert torch.equal(pkg.ops.dense_gemm(a[M - m:], w, K), got[M - m:]), m
 
 
+# The float forms of 128 x 128, two per CU, one per CU and 64 x 64.
+@pytest.mark.parametrize("M,N,K", [(2300, 2050, 32), (2047, 4100, 96), (2045, 1990, 160), (1025, 1990, 64)])
+def test_rows_of_a_float_product(pkg, M, N, K):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, w = torch.randn(M, K, device="cuda", generator=g), torch.randn(N, K, device="cuda", generator=g)
+    got = pkg.ops.dense_gemm(a, w, K)
+    # K products and K sums of size about 1, each rounded to 24 bits
+    assert (got.double() - a.double() @ w.double().t()).abs().max().item() <= 2 * K * 2.0 ** -24 * 4 * K ** 0.5
+    for m in (33, 100):
+        assert torch.equal(pkg.ops.dense_gemm(a[M - m:], w, K), got[M - m:]), m
+
+
+# Steps of 128 bytes of K around the ring lengths of the kernel for few rows, 10 stages of rows and 20 of weights, and past them; one and
+# two row tiles, ragged columns.  The same rows among many more go through 64 x 64 and 128 x 128 tiles.
+@pytest.mark.parametrize("steps", [9, 10, 11, 19, 20, 21, 22, 97])
+@pytest.mark.parametrize("M,N", [(33, 784), (65, 1990)])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_few_rows_around_the_ring(pkg, steps, M, N, dtype):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(steps)
+    bf16 = dtype == "bfloat16"
+    K = steps * (64 if bf16 else 32)
+    a = torch.randn(2047, K, device="cuda", generator=g).to(getattr(torch, dtype))
+    w = torch.randn(N, K, device="cuda", generator=g).to(getattr(torch, dtype))
+    got = pkg.ops.dense_gemm(a[:M], w, K)
+    # K products (exact in bfloat16) and K sums, rounded to 24 bits
+    bound = (1 if bf16 else 2) * K * 2.0 ** -24 * 4 * K ** 0.5
+    assert (got.double() - a[:M].double() @ w.double().t()).abs().max().item() <= bound
+    assert torch.equal(pkg.ops.dense_gemm(a, w, K)[:M], got)
+
+
 def _same_in_portions(pkg, cfg, n, cuts):
     """One pass over n tokens on large tiles, and the same in portions on small ones, attention by the kernel that goes row by row."""
     ids = np.random.default_rng(5).integers(0, cfg["vocab"], n).astype(np.int32)
@@ -58,7 +90,7 @@ def test_head_columns_on_large_tiles(pkg):
 
 # ---- attention over a prompt ------------------------------------------------------------------
 # Many turns of both key groups, ends inside a tile of 64 keys, of 128 rows and of a share; a scale below zero and of zero;
-# value widths and output strides that are no multiple of four.
+# value widths and output strides that are no multiple of four.  97 tokens of three heads go to the kernel of short prompts.
 @pytest.mark.parametrize("M,pos,chunk,splits", [(97, 0, 0, 1), (700, 5, 0, 1), (641, 64, 0, 3), (520, 130, 192, 1), (333, 3, 500, 2)])
 @pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128), (128, 125), (104, 61), (256, 254)])
 @pytest.mark.parametrize("scale", [0.09, -0.11, 0.0])
@@ -81,6 +113,44 @@ def test_attention_over_a_prompt(pkg, M, pos, chunk, splits, dim, vdim, scale):
         # weights and the result are rounded to 8 significant bits: off by at most 2^-8 of each term and of the sum
         bound = 2.0 ** -8 * (p @ part[:, :vdim].abs() + want.abs()) + 1e-5
         assert ((got[:, h] - want).abs() <= bound).all(), (h, ((got[:, h] - want).abs() / bound).max().item())
+
+
+# A sink as the models have it, in all the shares there can be (most of them empty) and in one; more than 512 rows of a key head.
+@pytest.mark.parametrize("M,pos,chunk,splits", [(700, 5, 0, 1), (200, 0, 0, 64), (641, 64, 192, 5)])
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 128), (256, 254)])
+def test_attention_over_a_prompt_with_a_sink(pkg, M, pos, chunk, splits, dim, vdim):
+    import torch
+    heads, kv_heads, seq = 6, 2, pos + M
+    g = torch.Generator(device="cuda").manual_seed(M + dim)
+    value = (vdim + 7) // 8 * 8
+    q = torch.randn(M, heads, dim, device="cuda", generator=g).bfloat16()
+    rows = torch.randn(seq, kv_heads * (dim + value), device="cuda", generator=g).bfloat16()
+    got = pkg.ops.grouped_attention(q, rows, pos, kv_heads, dim, vdim, 0.09, chunk, True, 1, splits).double()
+    t, s = torch.arange(pos, pos + M, device="cuda")[:, None], torch.arange(seq, device="cuda")[None]
+    sees = (s <= t) & (s // chunk == t // chunk) if chunk else s <= t
+    parts = rows.double().view(seq, kv_heads, dim + value)
+    for h in range(heads):
+        part = parts[:, h // 3]
+        _assert_attended(got[:, h], _weights_of(q[:, h].double() @ part[:, value:].t() * 0.09, sees, True), part[:, :vdim])
+
+
+@pytest.mark.parametrize("M,pos", [(1100, 0), (515, 333)])
+@pytest.mark.parametrize("dim,rot,vdim", [(64, 32, 64), (128, 64, 128), (192, 64, 256)])
+def test_formed_attention_over_a_prompt(pkg, M, pos, dim, rot, vdim):
+    import torch
+    heads, seq = 3, pos + M
+    g = torch.Generator(device="cuda").manual_seed(M + dim)
+    q = torch.randn(M, heads, dim + rot, device="cuda", generator=g).bfloat16()
+    k = torch.randn(seq, heads * dim, device="cuda", generator=g).bfloat16()
+    k_rot = torch.randn(seq, rot, device="cuda", generator=g).bfloat16()
+    v = torch.randn(heads * vdim, (seq + 63) // 64 * 64, device="cuda", generator=g).bfloat16()
+    gates = torch.randn(M, heads, device="cuda", generator=g)
+    got = pkg.ops.formed_attention(q, k, k_rot, v, gates, pos, vdim, 0.07).double().view(M, heads, vdim)
+    sees = torch.arange(seq, device="cuda")[None] <= torch.arange(pos, seq, device="cuda")[:, None]
+    for h in range(heads):
+        keys = torch.cat([k[:, h * dim:(h + 1) * dim], k_rot], 1).double()
+        p = _weights_of(q[:, h].double() @ keys.t() * 0.07, sees, False)
+        _assert_attended(got[:, h], p, v[h * vdim:(h + 1) * vdim, :seq].double().t(), gates[:, h:h + 1].double().sigmoid())
 
 
 def _weights_of(scores, sees, sink):
