@@ -212,19 +212,35 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
 #pragma unroll
             for (int f = 0; f < VF; f++) acc[f] *= keep;
         }
-        bf16x8 pf[4];
-        float add[4] = {0.f, 0.f, 0.f, 0.f};
+        auto weights_sum = [&]() {
+            float add[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) add[v & 3] += sc[t][v];
+            return (add[0] + add[1]) + (add[2] + add[3]);
+        };
 #pragma unroll
         for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                // a modifier of the exponential's instruction: a weight that is no number (of a score that is none, or of a masked one
-                // under a scale of zero) becomes 0
-                const float p = __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(fmaf(sc[t][v], scale, -mx)), 0.f, 1.f);
-                add[v & 3] += p;
-                pf[2 * t + (v >> 3)][v & 7] = (bf16)p;
-            }
-        sum += (add[0] + add[1]) + (add[2] + add[3]);
+            for (int v = 0; v < 16; v++) sc[t][v] = __builtin_amdgcn_exp2f(fmaf(sc[t][v], scale, -mx));
+        float add = weights_sum();
+        // A weight that is no number, of a score that is none or of a masked one under a scale of zero, is 0.  Its sum tells, so that the
+        // other tiles go without a comparison for every weight: 1 to 2 % of the time, against 1 to 5 % with all of them (a clamp to 0 .. 1
+        // in the exponential's instruction is free but moves the last bits of sums).
+        if (__builtin_expect(__any(add != add), 0)) {
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) sc[t][v] = fmaxf(sc[t][v], 0.f);
+            add = weights_sum();
+        }
+        sum += add;
+        bf16x8 pf[4];
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) pf[2 * t + (v >> 3)][v & 7] = (bf16)sc[t][v];
 #pragma unroll
         for (int u = 0; u < 4; u++)
 #pragma unroll
