@@ -216,8 +216,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void attend_kernel(AttendArgs<bf16> 
             for (int f = 0; f < VF; f++)
                 if ((f0 + f) * 16 + 4 * g < a.ld_part) *reinterpret_cast<f32x4*>(dst + (f0 + f) * 16 + 4 * g) = acc[s][f];
         } else {
-            float inv = 1.0f / all;
-            if (a.head_gate) inv *= sigmoid(a.head_gate[(size_t)r * a.ld_gate + z]);
+            const float inv = 1.0f / all;
             const int token = r / a.rows_per_token;
             bf16* dst = a.out + z * a.out_head + (size_t)token * a.out_token + (r - token * a.rows_per_token) * a.ld_out;
 #pragma unroll

@@ -11,9 +11,10 @@
 // one value per lane.  Scores, softmax and sums are fp32; the maximum follows every larger score, so that the heaviest
 // weight, 1, is exact in 16 bits (left behind by up to 2^8 it is not: 14 % more error for 8 % less time).
 //
-// A tile is copied global -> LDS by direct 16-byte loads, the next one while this one is worked on.  Chunk c of key k sits at place
-// c ^ k % 16, or, where rows are an odd number of 128 bytes, c ^ k / 2 % 8; chunk c of a transposed value column d at c ^ d / 2 % 8:
-// sixteen rows read at one chunk column cover the 256 bytes of all banks.
+// A tile is copied global -> LDS by direct 16-byte loads, the next one while this one is worked on; in the rows form only while its
+// scores and weights are formed, as the compiler waits for every copy under way ahead of the first transposing read of values.
+// Chunk c of key k sits at place c ^ k % 16, or, where rows are an odd number of 128 bytes, c ^ k / 2 % 8; chunk c of a transposed
+// value column d at c ^ d / 2 % 8: sixteen rows read at one chunk column cover the 256 bytes of all banks.
 //
 // What bounds it: matrix ops and softmax of a SIMD's two waves, one after the other; then LDS, which gives an operand of 1 KiB
 // for every matrix op.  4095 rows of 16 heads, 192 + 128 columns: 120 us = 712 TFLOP/s, against 537 us with 16 x 16 matrix ops,
@@ -35,7 +36,7 @@ template <int DK>
 __device__ __forceinline__ int place_of_key(int k) {
     return DK % 128 ? (k >> 1) & 7 : k & 15;
 }
-// the larger, or the sum, of this lane's value and that of the other lane half
+// the value of the lane 32 away
 __device__ __forceinline__ float other_half(float v) {
     const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(threadIdx.x & 32 ? both[0] : both[1]);
@@ -331,19 +332,24 @@ hipError_t launch_kernel(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
 
 }  // namespace
 
-// Heads of more than 128 columns leave LDS and registers for one group only.
+constexpr int kQW = kAttendPromptRows / 32;
+
+// Heads of more than 128 columns leave LDS and registers for one group only.  us against the 16 x 16 kernel that took these rows before:
+// 8 heads on 2, 256 + 256 columns, 330 rows 29.1 / 29.7, 2000 rows 121 / 128.
 hipError_t launch_attend_rows_prompt(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
     const int widest = a.k_own_width > a.v_width ? a.k_own_width : a.v_width;
-    if (widest <= 64) return launch_kernel<128, 64, 64, 2, 4, false>(a, heads, s);
-    if (widest <= 128) return launch_kernel<256, 128, 128, 2, 4, false>(a, heads, s);
-    return launch_kernel<512, 256, 256, 1, 4, false>(a, heads, s);
+    if (widest <= 64) return launch_kernel<128, 64, 64, 2, kQW, false>(a, heads, s);
+    if (widest <= 128) return launch_kernel<256, 128, 128, 2, kQW, false>(a, heads, s);
+    return launch_kernel<512, 256, 256, 1, kQW, false>(a, heads, s);
 }
 
+// The widest form takes all 512 registers and spills 50 of them, addresses of copies, whose reloads wait for the copies before.  It is
+// the faster one all the same (us, against 16 x 16): 8 heads, 192 + 64 and 256 columns, 330 rows 36 / 51, 2000 rows 159 / 212.
 hipError_t launch_attend_expanded(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
     const int dk = a.k_own_width + a.k_shared_width;
-    if (dk <= 128 && a.dv <= 64) return launch_kernel<128, 64, 0, 2, 4, true>(a, heads, s);
-    if (dk <= 192 && a.dv <= 128) return launch_kernel<192, 128, 0, 2, 4, true>(a, heads, s);
-    return launch_kernel<320, 256, 0, 1, 4, true>(a, heads, s);
+    if (dk <= 128 && a.dv <= 64) return launch_kernel<128, 64, 0, 2, kQW, true>(a, heads, s);
+    if (dk <= 192 && a.dv <= 128) return launch_kernel<192, 128, 0, 2, kQW, true>(a, heads, s);
+    return launch_kernel<320, 256, 0, 1, kQW, true>(a, heads, s);
 }
 
 }  // namespace a81w41

@@ -160,9 +160,9 @@ hipError_t launch_rotate_queries(const float* q, int ld_q, const LatentRows& in,
 // launch_merge_shares.
 constexpr int kAttendMaxSplits = 64;
 constexpr int kAttendFewRows = 64;  // up to here a workgroup takes 16 query rows, above 64 or more
-// The rows form takes 64 or 128 rows a workgroup up to kAttendShortRows, kAttendPromptRows above.  At 132 rows the two kernels take 15
-// and 11 us, both next to what a launch takes, at 400 and 512 rows 11 and 10 us; short prompts keep the order of their sums, which a
-// router behind them may feel.
+// Up to kAttendShortRows rows of a key head the rows form goes to attend_mfma.hip's kernel, above to attend_prompt.hip's with
+// kAttendPromptRows rows a workgroup.  The line is not where the second becomes the faster one: it takes 11 us against 15 at 132 rows
+// and 10 against 11 at 400 and 512.  Short prompts keep the order of their sums instead, on which a router behind them may depend.
 constexpr int kAttendShortRows = 512, kAttendPromptRows = 128;
 template <typename T>
 struct AttendArgs {

@@ -8,10 +8,9 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((address_space(3))) void* dense_lds_ptr;
-// What a kernel reads out of LDS while direct copies into other parts of it are under way is read as vectors of these types: ahead
-// of a read through HIP's uint4 or uint2 the compiler waits for every copy (s_waitcnt vmcnt(0)).
+// What a kernel reads out of LDS while direct copies into other parts of it are under way is read as vectors of this type: ahead
+// of a read through HIP's uint4 the compiler waits for every copy (s_waitcnt vmcnt(0)).
 typedef __attribute__((ext_vector_type(4))) unsigned lds16;
-typedef __attribute__((ext_vector_type(2))) unsigned lds8;
 
 __device__ __forceinline__ float dense_wave_sum(float v, int width = 64) {
     for (int off = width >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

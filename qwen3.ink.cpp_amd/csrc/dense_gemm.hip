@@ -9,8 +9,8 @@
 // What bounds it: bytes per product.  A 128 x 128 tile asks the L2 for 64 bytes a clock and CU at the matrix cores' full rate,
 // which is all the L2 gives, and reads LDS as fast as LDS goes; a 256 x 256 tile asks for half of the one and three quarters of
 // the other.  4095 x 12288 x 2048 in bfloat16 with the gated epilogue: 340 us with 128 x 128 tiles whose copies the compiler
-// waited for ahead of every step's first LDS read (see lds16), 210 us = 980 TFLOP/s with 256 x 256.  4095 x 2048 x 6144: 140 us and
-// 120 us, 2048 x 2048 x 2048: 47 us and 29 us.
+// waited for ahead of every step's first LDS read (see lds16), 215 us = 960 TFLOP/s with 256 x 256.  4095 x 2048 x 6144: 146 us and
+// 115 us, 2048 x 2048 x 2048: 46 us and 27 us.
 #include <type_traits>
 
 #include "dense_common.h"
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(G
 // rows and 32 columns a workgroup of six waves: two multiply 32 rows each, reading a step's operands beside the products of the step
 // before, two copy A nine steps ahead, two copy W 19 steps ahead.  A wave that copies and multiplies takes 0.3 us a step
 // however much is under way, these 0.13 us (a trip to memory of 2.4 us in 19 steps, one to the L2 of 0.9 us in nine).  The sums go
-// in the order of the other kernels.  33 rows, 784 x 2048: 21 us with 64 x 64 tiles and one step's copies waited for at once, 7.7 us
+// in the order of the other kernels.  33 rows, 784 x 2048: 28 us with 64 x 64 tiles and one step's copies waited for at once, 8.8 us
 // here; 2048 x 6144: 81 us and 19 us.  Cutting K between waves is no faster (7.5 and 20 us) and sums in another order.
 template <typename T, Epilogue EPI, typename X>
 __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X heads) {
