@@ -308,13 +308,13 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
 }
 
 // 256 x 256 tiles, one workgroup per CU, or 128 x 128, two per CU.  At K = 2048 a round of 256 large tiles takes 65 us whether
-// it is full or not, small tiles 44 us per 512 of them; small ones overlap a round's end with the next one's start, so that large ones
-// have to be fuller where there are several rounds.  us with small / large, 768 small tiles a round: one round, 2047 rows, 6144 x 512
-// 26.0 / 24.1, x 2048 61.2 / 60.0; two, 1030 rows, 32768 x 512 61.3 / 64.6, 3000 rows, 8192 x 2048 111 / 117; with 864 a round,
-// 1030 rows, 24576 x 2048 123.8 / 122.0.
-bool large_tiles_preferred(long long large, long long small) {
+// it is full or not, small tiles 44 us per 512 of them.  Over several rounds small ones overlap the end of one with the start of the
+// next, which counts where rounds are short: with exactly 768 of them a round, us with small / large, 2047 rows, 12288 x 1024 66 / 69,
+// x 2048 117 / 120, x 4096 227 / 224; 3000 rows, 8192 x 512 40.8 / 43.2, x 2048 118 / 122, x 6144 331 / 329.  With a few more they
+// begin one more round (2048 rows, 12320 x 2048, 776 a round, 131 / 125); one round, 2047 rows, 6144 x 1024 39.8 / 36.4.
+bool large_tiles_preferred(long long large, long long small, int K) {
     const long long rounds = (large + 255) / 256;
-    return rounds * (rounds > 1 ? 800 : 750) <= small;
+    return rounds * (rounds > 1 && K <= 2048 ? 769 : 750) <= small;
 }
 
 template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PIPE, Epilogue EPI, typename X>
@@ -337,7 +337,7 @@ hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
     // A product of 192 to 256 tiles of 128 x 128 has one for a CU: it takes twice the waves and four stages in LDS (2048^3: 29 us
     // against 36 us with two).  Fewer give too few CUs work.  A grouped product's row tiles are kGroupTileRows high.
     if constexpr (sizeof(T) == 2)
-        if (!g.tiles && large_tiles_preferred(tiles(256), tiles(128))) return launch_kernel<T, 256, 256, 2, 4, 2, true, EPI>(g, heads, s);
+        if (!g.tiles && large_tiles_preferred(tiles(256), tiles(128), g.K)) return launch_kernel<T, 256, 256, 2, 4, 2, true, EPI>(g, heads, s);
     if (!g.tiles && g.M > 64 && tiles(128) > 256) return launch_kernel<T, 128, 128, 2, 2, 2, false, EPI>(g, heads, s);
     if (!g.tiles && g.M > 64 && tiles(128) >= 192) return launch_kernel<T, 128, 128, 2, 4, 4, true, EPI>(g, heads, s);
     if (g.tiles && g.N >= 1024) return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, false, EPI>(g, heads, s);
