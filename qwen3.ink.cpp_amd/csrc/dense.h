@@ -289,6 +289,11 @@ struct LatentShares {
 template <typename T>
 hipError_t launch_gemv_values(const float* o_lat, int ld_o, const LatentShares& shares, const LatentShape& sh, const T* uv, int ld,
                               const float* gates, float* attn, hipStream_t s);
+// Attention over a short context and that product in one launch (latent_token.hip), bfloat16: attn [heads][vdim] of a token, q_lat
+// [heads][ld_cache] against the rows of `cache`.
+bool latent_token_fits(const LatentShape& sh);
+hipError_t launch_latent_token(const bf16* q_lat, const LatentRows& in, const LatentShape& sh, const bf16* cache, const bf16* uv, int ld_uv,
+                               const float* gates, float* attn, hipStream_t s);
 // The feed-forwards a token uses: `top` of `experts` by table (0: none), and one every token uses (dense_ff 0: none).
 struct ExpertRows {
     const int *ids = nullptr, *table = nullptr;

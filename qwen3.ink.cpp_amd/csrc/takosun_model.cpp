@@ -88,6 +88,10 @@ Config read_config(const Json& j) {
     return c;
 }
 
+// Context up to which a token's attention and value product are one launch, whose workgroups each read all keys: us a token of four
+// layers, one launch / two, 16 heads, 256 keys 265.6 / 293.0, 512 280.0 / 293.8, 768 294.5 / 294.1; 8 heads, 512 203 / 212, 768 217 / 213.
+constexpr int kLatentTokenKeys = 512;
+
 }  // namespace
 
 template <typename T>
@@ -159,6 +163,7 @@ class TakosunModel final : public DenseModel<T> {
     int attend_formed(const Layer& L, const LatentShape& sh, int M, const float* gates, hipStream_t s);
     AttendArgs<T> shared_attend(const Layer& L, const LatentShape& sh, int M) const;
     int enqueue_one_token(int n_want, hipStream_t s);
+    int attend_one_token(const Layer& L, const LatentShape& sh, const LatentRows& in, const float* gates, hipStream_t s);
     int feed_forward_one_token(const Layer& L, const LayerConfig& lc, const RowStep& step, hipStream_t s);
     LatentRows latent_rows(const Layer& L) const;
     int feed_forward(const Layer& L, const LayerConfig& lc, int M, hipStream_t s, SublayerOut* out);
@@ -479,8 +484,37 @@ int TakosunModel<T>::feed_forward_one_token(const Layer& L, const LayerConfig& l
     return 0;
 }
 
-// The pass for one token: the row work between two products runs inside the product that consumes it, eight launches a
-// layer.  The sum over the earlier states of the mean over depth is
+// One token's attention: its queries are in q_, its gated values go to attn_row_.
+template <typename T>
+int TakosunModel<T>::attend_one_token(const Layer& L, const LatentShape& sh, const LatentRows& in, const float* gates, hipStream_t s) {
+    A81W41_HIP_TRY(launch_gemv_absorb<T>(q_, in, sh, L.uk_t.data, L.uk_t.ld, q_lat_, s));
+    if constexpr (kMatrixAttention) {
+        if (!opt_attention_ && !opt_split_ && plan_ctx <= kLatentTokenKeys && latent_token_fits(sh)) {
+            A81W41_HIP_TRY(launch_latent_token(q_lat_, in, sh, L.cache, L.uv.data, L.uv.ld, gates, attn_row_, s));
+            return 0;
+        }
+    }
+    const int ld_rank = pad_k<T>(sh.rank);
+    LatentShares shares;
+    if constexpr (kMatrixAttention) {
+        if (opt_attention_ != 1 && attend_shared_fits(sh.rank + sh.rot, sh.rank)) {
+            AttendArgs<T> a = shared_attend(L, sh, 1);
+            a.splits = std::max(a.splits, 2);  // shares stay fp32; the product with W_uv merges them
+            A81W41_HIP_TRY(launch_attend_shared(a, s));
+            shares = LatentShares{a.part, a.part_stats, a.splits, a.ld_part};
+        }
+    }
+    if (!shares.part) {
+        AttendArgs<T> a = shared_attend(L, sh, 1);
+        a.ld_out = ld_rank, a.out_token = sh.heads * ld_rank;
+        A81W41_HIP_TRY((launch_attend_vector<T, float>(a, 1, o_lat_row_, s)));
+    }
+    A81W41_HIP_TRY(launch_gemv_values<T>(o_lat_row_, ld_rank, shares, sh, L.uv.data, L.uv.ld, gates, attn_row_, s));
+    return 0;
+}
+
+// The pass for one token: the row work between two products runs inside the product that consumes it, seven launches a
+// layer (eight behind a long context).  The sum over the earlier states of the mean over depth is
 // formed beside the query product, so that the next layer's first product adds only the newest state.
 template <typename T>
 int TakosunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
@@ -500,24 +534,7 @@ int TakosunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
         depth.states = states_, depth.state_step = state_step(), depth.coef = L.dwa, depth.n = i + 1;
         const LatentRows in = latent_rows(L);
         A81W41_HIP_TRY(launch_gemv_query<T>(in, sh, L.uq.data, L.uq.ld, q_, own ? L.cache : nullptr, depth, W, before_, s));
-        A81W41_HIP_TRY(launch_gemv_absorb<T>(q_, in, sh, L.uk_t.data, L.uk_t.ld, q_lat_, s));
-        const int ld_rank = pad_k<T>(sh.rank);
-        LatentShares shares;
-        if constexpr (kMatrixAttention) {
-            if (opt_attention_ != 1 && attend_shared_fits(sh.rank + sh.rot, sh.rank)) {
-                AttendArgs<T> a = shared_attend(L, sh, 1);
-                a.splits = std::max(a.splits, 2);  // shares stay fp32; the product with W_uv merges them
-                A81W41_HIP_TRY(launch_attend_shared(a, s));
-                shares = LatentShares{a.part, a.part_stats, a.splits, a.ld_part};
-            }
-        }
-        if (!shares.part) {
-            AttendArgs<T> a = shared_attend(L, sh, 1);
-            a.ld_out = ld_rank, a.out_token = sh.heads * ld_rank;
-            A81W41_HIP_TRY((launch_attend_vector<T, float>(a, 1, o_lat_row_, s)));
-        }
-        A81W41_HIP_TRY(launch_gemv_values<T>(o_lat_row_, ld_rank, shares, sh, L.uv.data, L.uv.ld, down_ + sh.q_rank + (own ? sh.rank + sh.rot : 0),
-                                             attn_row_, s));
+        A81W41_TRY(attend_one_token(L, sh, in, down_ + sh.q_rank + (own ? sh.rank + sh.rot : 0), s));
         A81W41_HIP_TRY(launch_gemv_plain<T>(attn_row_, sh.heads * sh.vdim, L.o.data, L.o.ld, W, y_, s));
         step = RowStep{};
         step.width = W, step.x = x, step.y = y_, step.norm_y = norm(L.norm1b);
