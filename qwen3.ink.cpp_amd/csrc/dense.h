@@ -48,11 +48,15 @@ struct HeadRows {
     float* rest = nullptr;
     int ld_rest = 0;
 };
-// A row tile of a grouped product: rows [row0, row0 + rows) belong to one expert.
+// A grouped product's rows come sorted by expert, its row tiles in the same order.  What a tile's workgroup has to know: the expert, the
+// number of the expert's first tile, and the expert's rows [row0, row0 + rows).
 struct GroupTile {
-    int expert, row0, rows;
+    int expert, first, row0, rows;
 };
-constexpr int kGroupTileRows = 64;
+// How high the tiles are, for `rows` rows in all.  us of gate and up / down with 64 / 128 rows a tile, width 2048, units of 1024:
+// 256 rows for an expert on average 130.8 / 69.8 and 121.4 / 67.1, 128 rows 84.9 / 46.5 and 82.0 / 44.8, 75 rows 69.5 / 35.5 and 86.3 / 43.5.
+constexpr int kGroupTileRows = 64, kGroupTileManyRows = 128;
+inline int group_tile_rows(long long rows, int experts) { return rows >= 128LL * experts ? kGroupTileManyRows : kGroupTileRows; }
 struct GemmArgs {
     const void* A = nullptr;  // [M][lda], or gathered: row r of the product is row a_rows[r] of A
     const void* W = nullptr;  // [N][ldw]
@@ -66,10 +70,13 @@ struct GemmArgs {
     const float* head_gate = nullptr;
     int ld_gate = 0;
     GatedUnit unit;
-    // grouped: tile t of *n_tiles (at most max_tiles) runs its rows against expert e's weights W + e w_step
+    // grouped: tile t of *n_tiles (at most max_tiles, tile_rows high) runs its rows against expert e's weights W + e w_step
     const GroupTile* tiles = nullptr;
     const int* n_tiles = nullptr;
-    int max_tiles = 0;
+    int max_tiles = 0, tile_rows = 0;
+    void group(const GroupTile* list, const int* n, int experts) {  // M is the number of all rows
+        tiles = list, n_tiles = n, tile_rows = group_tile_rows(M, experts), max_tiles = M / tile_rows + (experts < M ? experts : M);
+    }
 };
 template <typename T>
 hipError_t launch_dense_gemm(const GemmArgs& g, Epilogue epi, hipStream_t s);
@@ -113,8 +120,8 @@ hipError_t launch_residual_norm(const float* x, const SublayerOut& y, const Grou
 
 // ---- experts (dense_rows.hip) ----------------------------------------------------------------
 // Token m uses the experts table[ids[m]][0..top), or table[m][0..top) without ids (entries of one row are distinct).  Rows
-// sorted by expert: src_rows[r] = token of row r, slot_rows[m * top + k] = row of slot k; tiles of at most kGroupTileRows
-// rows, their number in *n_tiles.
+// sorted by expert: src_rows[r] = token of row r, slot_rows[m * top + k] = row of slot k; tiles of
+// group_tile_rows, their number in *n_tiles.
 hipError_t launch_expert_rows(const int* ids, const int* table, int vocab, int top, int experts, int M, int* src_rows,
                               int* slot_rows, GroupTile* tiles, int* n_tiles, hipStream_t s);
 // The `top` largest of logits[m][0..experts) + bias (the lower number first among equals): chosen [M][top], largest first,

@@ -9,8 +9,8 @@
 // What bounds it: bytes per product.  A 128 x 128 tile asks the L2 for 64 bytes a clock and CU at the matrix cores' full rate,
 // which is all the L2 gives, and reads LDS as fast as LDS goes; a 256 x 256 tile asks for half of the one and three quarters of
 // the other.  4095 x 12288 x 2048 in bfloat16 with the gated epilogue: 340 us with 128 x 128 tiles whose copies the compiler
-// waited for ahead of every step's first LDS read (see lds16), 215 us = 960 TFLOP/s with 256 x 256.  4095 x 2048 x 6144: 146 us and
-// 115 us, 2048 x 2048 x 2048: 46 us and 27 us.
+// waited for ahead of every step's first LDS read (see lds16), 190 us = 1.08 PFLOP/s with 256 x 256.  4095 x 2048 x 6144: 146 us and
+// 106 us, 2048 x 2048 x 2048: 46 us and 25 us.
 #include <type_traits>
 
 #include "dense_common.h"
@@ -27,6 +27,14 @@ __device__ __forceinline__ void mma(f32x16& acc, const lds16& a, const lds16& b,
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[2]), __uint_as_float(b[2]), acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[3]), __uint_as_float(b[3]), acc, 0, 0, 0);
 }
+
+// A unit that is rounded to bfloat16 next: the hardware's exponential and reciprocal, a unit of 24 bits off at most in what they return.
+// Of 36 us that the epilogue of 4095 x 12288 x 2048 took, 10 were the library's exponential and division.
+__device__ __forceinline__ float unit_of(const GatedUnit& p, float gate, float up, bf16*) {
+    const float g = fminf(gate, p.limit), u = fminf(fmaxf(up, -p.limit), p.limit);
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * p.slope * g)) * (u + p.shift);
+}
+__device__ __forceinline__ float unit_of(const GatedUnit& p, float gate, float up, float*) { return gated_unit(p, gate, up); }
 
 struct NoHeads {};
 
@@ -64,7 +72,7 @@ __device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, c
 #pragma unroll
         for (int v = 0; v < NV; v += 2) {
             const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[v]), __float_as_uint(x[v + 1]), false, false);
-            const float unit = gated_unit(g.unit, __uint_as_float(both[0]), __uint_as_float(both[1]));
+            const float unit = unit_of(g.unit, __uint_as_float(both[0]), __uint_as_float(both[1]), static_cast<T*>(nullptr));
             const int r = r0 + 8 * (v >> 2) + (v & 3) + odd;
             if (r < rows && col < g.N) dst[(size_t)(m0 + r) * g.ldc] = (T)unit;
         }
@@ -105,34 +113,43 @@ __device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, c
 constexpr int kBandRows = 2048;
 
 // X: HeadRows<T> with the epilogue kHeads, NoHeads with the others.  STAGES: how many steps LDS holds; all but one are under way.
-// PIPE: a step's operands are read one 16-byte column ahead of their products; without it the other workgroup of the CU
-// fills the wait.
+// PIPE: a step's operands are read one 16-byte column ahead of their products, also into the next step: the waves meet before a step's
+// last products, whose operands are in registers by then, so that its stage is free for new copies and the next step's first
+// reads run beside those products.  4095 x 12288 x 2048, gated: 200.6 us with the meeting between two steps, 189.5 so (with the unit
+// below).  Without PIPE the other workgroup of the CU fills the wait.
 template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PIPE, Epilogue EPI, typename X>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(GemmArgs g, X heads) {
     constexpr int kThreads = 64 * WAVES_M * WAVES_N;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 32, FN = WN / 32;
     constexpr int LA = BM * 8 / kThreads, LB = BN * 8 / kThreads;  // direct copies per thread and stage
     constexpr int kStage = (BM + BN) * 128;
-    static_assert(STAGES >= 2 && (STAGES - 2) * (LA + LB) < 64, "copies a wait can leave outstanding");
+    static_assert(STAGES >= 2 && (STAGES - 1) * (LA + LB) < 64, "copies a wait can leave outstanding");
     __shared__ __attribute__((aligned(128))) uint8_t lds[STAGES * kStage];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l31 = lane & 31, half = lane >> 5;
-    // Tiles dealt to the XCDs in contiguous runs, in bands of kBandRows rows and inside one column panel after the other; a
-    // grouped product's in the order (column panel, row tile): a panel's weights come into one L2.
-    const int n_nt = (g.N + BN - 1) / BN, n_mt = gridDim.x / n_nt;
-    const int q = gridDim.x >> 3, r8 = gridDim.x & 7, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int t = xcd < r8 ? xcd * (q + 1) + idx : r8 * (q + 1) + (xcd - r8) * q + idx;
-    const int band = g.tiles ? n_mt : kBandRows / BM, first = t / (band * n_nt) * band;
-    const int high = min(band, n_mt - first), at = t - first * n_nt;
-    const int mt = first + at % high, nt = at / high;
-    int m0 = mt * BM, rows = g.M - m0;
+    // Tiles dealt to the XCDs in contiguous runs, in bands of kBandRows rows and inside one column panel after the other.  A grouped
+    // product's go expert by expert, column panel by column panel: an XCD then reads the rows of a few experts once and their weights
+    // once.  With the rows of all experts for one panel after the other (8192 rows of 4 KB, 32 experts, 16 panels) the rows were read from
+    // behind the L2 again for every panel, 512 MB beside 268 MB of weights: 133.6 us, so 127.4.
+    const int n_nt = (g.N + BN - 1) / BN, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+    const int all = g.tiles ? *g.n_tiles * n_nt : gridDim.x, q = all >> 3, r8 = all & 7;
+    if (idx >= q + (xcd < r8 ? 1 : 0)) return;
+    const int t = xcd * q + min(xcd, r8) + idx;
+    int m0, rows, nt;
     long long batch = blockIdx.y;
     if (g.tiles) {
-        if (mt >= *g.n_tiles) return;
-        const GroupTile gt = g.tiles[mt];
-        m0 = gt.row0;
-        rows = gt.rows;
+        const GroupTile gt = g.tiles[t / n_nt];
+        const int count = (gt.rows + BM - 1) / BM, at = t - gt.first * n_nt, skip = at % count * BM;
+        nt = at / count;
+        m0 = gt.row0 + skip;
+        rows = gt.rows - skip;
         batch = gt.expert;
+    } else {
+        const int n_mt = all / n_nt, band = kBandRows / BM, first = t / (band * n_nt) * band;
+        const int high = min(band, n_mt - first), at = t - first * n_nt;
+        m0 = (first + at % high) * BM;
+        nt = at / high;
+        rows = g.M - m0;
     }
     const int n0 = nt * BN;
     const uint8_t* A = reinterpret_cast<const uint8_t*>(static_cast<const T*>(g.A) + (g.tiles ? 0 : batch * g.a_step));
@@ -166,42 +183,74 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(G
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
     const int wm = (wave % WAVES_M) * WM, wn = (wave / WAVES_M) * WN;
     const int n_steps = g.K * (int)sizeof(T) / 128;
-    for (int step = 0; step < STAGES - 1 && step < n_steps; step++) copy_step(step, step);
-    int stage = 0;
-    for (int step = 0; step < n_steps; step++) {
-        // the copies of the step are in LDS, later ones may be under way; and nobody still reads the stage before it
-        if (step + STAGES - 2 < n_steps)
-            wait_copies_and_meet<(STAGES - 2) * (LA + LB)>();
+    lds16 a[2][FM], b[2][FN];
+    auto read = [&](int kk, const uint8_t* sa) {
+        const uint8_t* sb = sa + BM * 128;
+#pragma unroll
+        for (int i = 0; i < FM; i++) {
+            const int r = wm + i * 32 + l31;
+            a[kk & 1][i] = *reinterpret_cast<const lds16*>(sa + r * 128 + (((2 * kk + half) ^ place_of_row(r)) << 4));
+        }
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            const int r = wn + j * 32 + l31;
+            b[kk & 1][j] = *reinterpret_cast<const lds16*>(sb + r * 128 + (((2 * kk + half) ^ place_of_row(r)) << 4));
+        }
+    };
+    auto multiply = [&](int kk) {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) mma(acc[i][j], a[kk & 1][i], b[kk & 1][j], static_cast<T*>(nullptr));
+    };
+    if constexpr (PIPE) {
+        for (int step = 0; step < STAGES && step < n_steps; step++) copy_step(step, step);
+        if (n_steps >= STAGES)
+            wait_copies_and_meet<(STAGES - 1) * (LA + LB)>();
         else
             wait_copies_and_meet<0>();
-        if (step + STAGES - 1 < n_steps) copy_step(step + STAGES - 1, stage ? stage - 1 : STAGES - 1);
-        const uint8_t* sa = lds + stage * kStage;
-        const uint8_t* sb = sa + BM * 128;
-        stage = stage + 1 < STAGES ? stage + 1 : 0;
-        lds16 a[2][FM], b[2][FN];
-        auto read = [&](int kk) {
+        read(0, lds);
+        int stage = 0;
+        for (int step = 0; step < n_steps; step++) {
+            const uint8_t* sa = lds + stage * kStage;
+            const int next = stage + 1 < STAGES ? stage + 1 : 0;
 #pragma unroll
-            for (int i = 0; i < FM; i++) {
-                const int r = wm + i * 32 + l31;
-                a[kk & 1][i] = *reinterpret_cast<const lds16*>(sa + r * 128 + (((2 * kk + half) ^ place_of_row(r)) << 4));
+            for (int kk = 0; kk < 3; kk++) {
+                __builtin_amdgcn_sched_barrier(0);
+                read(kk + 1, sa);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(kk);
             }
-#pragma unroll
-            for (int j = 0; j < FN; j++) {
-                const int r = wn + j * 32 + l31;
-                b[kk & 1][j] = *reinterpret_cast<const lds16*>(sb + r * 128 + (((2 * kk + half) ^ place_of_row(r)) << 4));
+            __builtin_amdgcn_sched_barrier(0);
+            if (step + 1 < n_steps) {
+                if (step + STAGES <= n_steps)
+                    wait_copies_and_meet<(STAGES - 2) * (LA + LB)>();
+                else
+                    wait_copies_and_meet<0>();
+                if (step + STAGES < n_steps) copy_step(step + STAGES, stage);
+                read(0, lds + next * kStage);
+                __builtin_amdgcn_sched_barrier(0);
             }
-        };
-        if constexpr (PIPE) read(0);
+            multiply(3);
+            stage = next;
+        }
+    } else {
+        for (int step = 0; step < STAGES - 1 && step < n_steps; step++) copy_step(step, step);
+        int stage = 0;
+        for (int step = 0; step < n_steps; step++) {
+            // the copies of the step are in LDS, later ones may be under way; and nobody still reads the stage before it
+            if (step + STAGES - 2 < n_steps)
+                wait_copies_and_meet<(STAGES - 2) * (LA + LB)>();
+            else
+                wait_copies_and_meet<0>();
+            if (step + STAGES - 1 < n_steps) copy_step(step + STAGES - 1, stage ? stage - 1 : STAGES - 1);
+            const uint8_t* sa = lds + stage * kStage;
+            stage = stage + 1 < STAGES ? stage + 1 : 0;
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-            if constexpr (PIPE) __builtin_amdgcn_sched_barrier(0);
-            if (!PIPE) read(kk);
-            if (PIPE && kk < 3) read(kk + 1);
-            if constexpr (PIPE) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int j = 0; j < FN; j++) mma(acc[i][j], a[kk & 1][i], b[kk & 1][j], static_cast<T*>(nullptr));
+            for (int kk = 0; kk < 4; kk++) {
+                read(kk, sa);
+                multiply(kk);
+            }
         }
     }
 #pragma unroll
@@ -224,7 +273,7 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
     // row tiles of a column panel next to each other on one XCD
     const int n_mt = (g.M + 63) / 64;
     const int q = gridDim.x >> 3, r8 = gridDim.x & 7, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
-    const int t = xcd < r8 ? xcd * (q + 1) + idx : r8 * (q + 1) + (xcd - r8) * q + idx;
+    const int t = xcd * q + min(xcd, r8) + idx;
     const int m0 = t % n_mt * 64, n0 = t / n_mt * 32, rows = g.M - m0, n_steps = g.K * (int)sizeof(T) / 128;
     const long long batch = blockIdx.y;
     const int copy_row = (wave & 1) * (wave < 4 ? 32 : 16) + (lane >> 3);  // of the wave's first copy
@@ -331,26 +380,61 @@ hipError_t launch_few(const GemmArgs& g, const X& heads, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Grouped products: the row tiles' height is that of the list.
+template <typename T, Epilogue EPI, typename X>
+hipError_t launch_grouped(const GemmArgs& g, const X& heads, hipStream_t s) {
+    auto panels = [&](int width) { return (long long)((g.N + width - 1) / width); };
+    if (g.tile_rows == kGroupTileManyRows) {
+        // One 128 x 256 tile on a CU where its rounds of 256 come out seven tenths full or more, half of the experts' last tiles being
+        // there, otherwise two 128 x 128.  us, the second / the first: 2048 tokens of 4 experts out of 32, 2048 x 2048 gated 124.9 /
+        // 121.4, 1536 x 1536 66.1 / 63.5; 0.63 of two rounds full, 1024 x 1024 39.5 / 41.5.
+        const int whole = g.M / kGroupTileManyRows;
+        const long long tiles = (whole + g.max_tiles) / 2 * panels(256), rounds = (tiles + 255) / 256;
+        if (10 * tiles >= 7 * 256 * rounds) return launch_kernel<T, kGroupTileManyRows, 256, 2, 4, 3, true, EPI>(g, heads, s);
+        return launch_kernel<T, kGroupTileManyRows, 128, 2, 2, 2, true, EPI>(g, heads, s);
+    }
+    // 64 x 128 tiles with two stages fit a CU three times, with three stages twice and have more of the weights under way, which counts where
+    // there are few rounds.  us with two / three: 600 tokens of 4 out of 32, 2048 x 2048 gated 80.5 / 69.5, 64 tokens 64.3 / 63.2, 16
+    // tokens, 1024 x 1024 15.7 / 12.1; 2048 tokens, 1024 x 1024 36.4 / 38.0.
+    if (g.N >= 1024) {
+        if (g.max_tiles * panels(128) <= 1200) return launch_kernel<T, kGroupTileRows, 128, 2, 4, 3, true, EPI>(g, heads, s);
+        return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, true, EPI>(g, heads, s);
+    }
+    // see launch_by_size: 1000 tiles, 512 x 512 14.7 us with four stages, 11.6 with two
+    if (g.max_tiles * panels(64) > 512) return launch_kernel<T, kGroupTileRows, 64, 2, 2, 2, false, EPI>(g, heads, s);
+    return launch_kernel<T, kGroupTileRows, 64, 2, 2, 4, false, EPI>(g, heads, s);
+}
+
 template <typename T, Epilogue EPI, typename X>
 hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
-    auto tiles = [&](int size) { return (long long)((g.M + size - 1) / size) * ((g.N + size - 1) / size) * g.batches; };
-    // A product of 192 to 256 tiles of 128 x 128 has one for a CU: it takes twice the waves and four stages in LDS (2048^3: 29 us
-    // against 36 us with two).  Fewer give too few CUs work.  A grouped product's row tiles are kGroupTileRows high.
+    if constexpr (EPI == Epilogue::kGatedPair || EPI == Epilogue::kFloat)
+        if (g.tiles) return launch_grouped<T, EPI>(g, heads, s);
+    auto tiles = [&](int rows, int cols) { return (long long)((g.M + rows - 1) / rows) * ((g.N + cols - 1) / cols) * g.batches; };
+    // One round of a tile for each CU, three quarters full or more; a tile has the larger one's stages and waves, so that its rows and
+    // weights are under way early.
+    auto one_round = [&](int rows, int cols) { return g.M > 64 && tiles(rows, cols) >= 192 && tiles(rows, cols) <= 256; };
     if constexpr (sizeof(T) == 2)
-        if (!g.tiles && large_tiles_preferred(tiles(256), tiles(128), g.K)) return launch_kernel<T, 256, 256, 2, 4, 2, true, EPI>(g, heads, s);
-    if (!g.tiles && g.M > 64 && tiles(128) > 256) return launch_kernel<T, 128, 128, 2, 2, 2, false, EPI>(g, heads, s);
-    if (!g.tiles && g.M > 64 && tiles(128) >= 192) return launch_kernel<T, 128, 128, 2, 4, 4, true, EPI>(g, heads, s);
-    if (g.tiles && g.N >= 1024) return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, false, EPI>(g, heads, s);
+        if (large_tiles_preferred(tiles(256, 256), tiles(128, 128), g.K)) return launch_kernel<T, 256, 256, 2, 4, 2, true, EPI>(g, heads, s);
+    // us, so / with 128 x 128 tiles: 4095 rows, 2048 x 2048 39.6 / 41.1, 2048 x 6144 106 / 109; 2048 rows, 3104 x 2048 36.3 / 40.4
+    if (one_round(128, 256)) return launch_kernel<T, 128, 256, 2, 4, 3, true, EPI>(g, heads, s);
+    // 2048^3: 24.8 us with twice the waves and four stages, 33 us as two a CU
+    if (one_round(128, 128)) return launch_kernel<T, 128, 128, 2, 4, 4, true, EPI>(g, heads, s);
+    if (g.M > 64 && tiles(128, 128) > 256) {
+        // 300 rows, 12288 x 2048 26.7 / 36.8
+        if (one_round(64, 256)) return launch_kernel<T, 64, 256, 2, 4, 3, true, EPI>(g, heads, s);
+        return launch_kernel<T, 128, 128, 2, 2, 2, false, EPI>(g, heads, s);
+    }
+    // us, so / with 64 x 64 tiles: 1024 rows, 2048 x 2048 15.2 / 16.0, x 6144 45.1 / 49.2; 600 rows, 3072 x 1536 12.2 / 13.4; 180 rows, 9216
+    // x 1536 14.6 / 16.3
+    if (one_round(64, 128)) return launch_kernel<T, 64, 128, 2, 4, 3, true, EPI>(g, heads, s);
     // So few tiles of 64 x 32 that no CU gets a second one (us, against 64 x 64 tiles with four stages): 33 rows, 784 x 2048 7.7 /
     // 12.5, 2048 x 6144 19 / 31; 256 rows, 2048 x 2048 10.2 / 13.5; with a second one 300 rows, 2048 x 2048 17.2 / 13.8, and 33
     // rows, 12288 x 2048 20 / 16.
-    const long long few = (long long)((g.N + 31) / 32) * ((g.M + 63) / 64) * g.batches;
-    if (!g.tiles && few <= 256) return launch_few<T, EPI>(g, heads, s);
+    if (tiles(64, 32) <= 256) return launch_few<T, EPI>(g, heads, s);
     // 64 x 64 tiles with four stages fit a CU twice, with two stages five times: more tiles than 512 would go in rounds.  bfloat16,
-    // us with four / two: 1030 rows, 544 tiles, 2048 x 1024 15.9 / 12.2, 2048 x 6144 63 / 50; 1000 grouped tiles, 512 x 512 14.7 /
-    // 11.6; in one round, 400 rows, 448 tiles, 4096 x 4096 27.5 / 34.  float, 1030 rows, 2048 x 1024: 60.5 / 56.9.
-    const long long tiles64 = (long long)(g.tiles ? g.max_tiles : (g.M + 63) / 64) * ((g.N + 63) / 64) * g.batches;
-    if (tiles64 > 512) return launch_kernel<T, 64, 64, 2, 2, 2, false, EPI>(g, heads, s);
+    // us with four / two: 1030 rows, 544 tiles, 2048 x 1024 15.9 / 12.2, 2048 x 6144 63 / 50; in one round, 400 rows, 448 tiles, 4096 x
+    // 4096 27.5 / 34.  float, 1030 rows, 2048 x 1024: 60.5 / 56.9.
+    if (tiles(64, 64) > 512) return launch_kernel<T, 64, 64, 2, 2, 2, false, EPI>(g, heads, s);
     return launch_kernel<T, 64, 64, 2, 2, 4, false, EPI>(g, heads, s);
 }
 

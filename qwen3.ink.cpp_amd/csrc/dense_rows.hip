@@ -210,7 +210,7 @@ static_assert(kMaxTop <= 64, "one weight per lane");
 __global__ __launch_bounds__(1024) void expert_rows_kernel(const int* __restrict__ ids, const int* __restrict__ table, int vocab,
                                                          int top, int experts, int M, int* __restrict__ src_rows,
                                                          int* __restrict__ slot_rows, GroupTile* __restrict__ tiles,
-                                                         int* __restrict__ n_tiles) {
+                                                         int* __restrict__ n_tiles, int tile_rows) {
     extern __shared__ int cnt[];  // [experts] counts, [experts] first rows, [experts] first tiles, [16]
     int *first = cnt + experts, *tile0 = first + experts, *tmp = tile0 + experts;
     const int t = threadIdx.x, total = M * top;
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(1024) void expert_rows_kernel(const int* __restrict
     __syncthreads();
     for (int e = t; e < experts; e += 1024) {
         first[e] = cnt[e];
-        tile0[e] = (cnt[e] + kGroupTileRows - 1) / kGroupTileRows;
+        tile0[e] = (cnt[e] + tile_rows - 1) / tile_rows;
     }
     __syncthreads();
     block_exclusive_scan(first, experts, tmp);
@@ -244,8 +244,7 @@ __global__ __launch_bounds__(1024) void expert_rows_kernel(const int* __restrict
     if (t == 0) *n_tiles = all_tiles;
     for (int e = t; e < experts; e += 1024) {
         const int n = cnt[e];
-        for (int k = 0; k * kGroupTileRows < n; k++)
-            tiles[tile0[e] + k] = GroupTile{e, first[e] + k * kGroupTileRows, min(kGroupTileRows, n - k * kGroupTileRows)};
+        for (int k = 0; k * tile_rows < n; k++) tiles[tile0[e] + k] = GroupTile{e, tile0[e], first[e], n};
     }
     __syncthreads();
     // where a token's row lands among its expert's rows does not matter: a row's result does not depend on its place
@@ -300,7 +299,7 @@ hipError_t launch_expert_rows(const int* ids, const int* table, int vocab, int t
                               int* slot_rows, GroupTile* tiles, int* n_tiles, hipStream_t s) {
     const size_t lds = (3 * (size_t)experts + 16) * sizeof(int);
     hipLaunchKernelGGL(expert_rows_kernel, dim3(1), dim3(1024), lds, s, ids, table, vocab, top, experts, M, src_rows, slot_rows,
-                       tiles, n_tiles);
+                       tiles, n_tiles, group_tile_rows((long long)M * top, experts));
     return hipGetLastError();
 }
 

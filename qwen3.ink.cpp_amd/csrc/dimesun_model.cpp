@@ -481,7 +481,7 @@ int DimesunModel<T>::routed_experts(const Layer& L, const LayerConfig& lc, int M
     GemmArgs g = product(h_, ld_h_, L.experts.gate_up, act_, ld, M * f.top);
     g.N = cols, g.w_step = (long long)cols * L.experts.gate_up.ld, g.a_rows = src_rows_;
     g.unit = GatedUnit{f.limit, 1.702f, 1.f};
-    g.tiles = tiles_, g.n_tiles = n_tiles_, g.max_tiles = M * f.top / kGroupTileRows + std::min(f.experts, M * f.top);
+    g.group(tiles_, n_tiles_, f.experts);
     A81W41_HIP_TRY(launch_dense_gemm<T>(g, Epilogue::kGatedPair, s));
     g.A = act_, g.lda = ld, g.a_rows = nullptr, g.W = L.experts.down.data, g.ldw = g.K = L.experts.down.ld;
     g.N = W, g.w_step = (long long)W * L.experts.down.ld, g.C = y2_, g.ldc = W;

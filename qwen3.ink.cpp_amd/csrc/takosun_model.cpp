@@ -458,7 +458,7 @@ int TakosunModel<T>::feed_forward(const Layer& L, const LayerConfig& lc, int M, 
     const int ld = pad_k<T>(f.ff), cols = pair_columns(f.ff);
     GemmArgs g = product(h_, ld_h_, L.ff.gate_up, act_, ld, M * f.top);
     g.N = cols, g.w_step = (long long)cols * L.ff.gate_up.ld, g.a_rows = src_rows_;
-    g.tiles = tiles_, g.n_tiles = n_tiles_, g.max_tiles = M * f.top / kGroupTileRows + std::min(f.experts, M * f.top);
+    g.group(tiles_, n_tiles_, f.experts);
     A81W41_HIP_TRY(launch_dense_gemm<T>(g, Epilogue::kGatedPair, s));
     g.A = act_, g.lda = ld, g.a_rows = nullptr, g.W = L.ff.down.data, g.ldw = g.K = L.ff.down.ld;
     g.N = W, g.w_step = (long long)W * L.ff.down.ld, g.C = y2_, g.ldc = W;

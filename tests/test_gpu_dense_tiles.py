@@ -243,3 +243,44 @@ def test_one_token_rows(pkg, width):
     for i, t in enumerate((7, 7, 49, 3)):   # the same sums in 32 bits in another order, two layers deep
         want = model.forward([t])
         assert np.linalg.norm(got[i] - want) <= 3e-5 * np.linalg.norm(want), i
+
+
+# One round of 128 x 256 tiles, of 64 x 256 and of 64 x 128, three stages each: fewer steps than stages, as many, more; ragged rows and columns
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 448])
+@pytest.mark.parametrize("M,N", [(2045, 3100), (300, 12280), (1000, 2000)])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_one_round_of_tiles(pkg, M, N, K, dtype):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(K)
+    bf16 = dtype == "bfloat16"
+    K = K if bf16 else K // 2
+    a = torch.randn(M, K, device="cuda", generator=g).to(getattr(torch, dtype))
+    w = torch.randn(N, K, device="cuda", generator=g).to(getattr(torch, dtype))
+    got = pkg.ops.dense_gemm(a, w, K)
+    # K products (exact in bfloat16) and K sums, rounded to 24 bits
+    bound = (1 if bf16 else 2) * K * 2.0 ** -24 * 4 * K ** 0.5
+    assert (got.double() - a.double() @ w.double().t()).abs().max().item() <= bound
+    assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
+
+
+# Experts' rows in tiles of 128 (one pass) and of 64 (portions): 128 x 256 and 128 x 128 tiles, 64 x 128 with two and three stages, 64 x 64;
+# experts with few rows or none, tables of few ids against many
+@pytest.mark.parametrize("n,experts,top,ff,width", [(2100, 8, 2, 600, 1088), (1100, 4, 1, 2048, 64), (700, 5, 3, 96, 2048), (1400, 16, 2, 520, 320)])
+def test_experts_in_tiles_of_two_heights(pkg, n, experts, top, ff, width):
+    cfg = tx.config(40, width, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.moe(experts, top, ff, shared=40))])
+    _same_in_portions(pkg, cfg, n, 100)
+
+
+# a gated unit at the limits of its gate: the hardware's exponential and reciprocal against the library's in the 32-bit mode
+def test_gated_units_of_large_gates(pkg, tmp_path):
+    from oracle import takosun_forward as tf
+    cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.dense(96))])
+    w = tf.random_weights(cfg, 12)
+    w["l0.mlp.gate"] = tf.round_bf16(w["l0.mlp.gate"] * 150)   # gates of some hundreds, both signs
+    tx.write_model(str(tmp_path), cfg, w)
+    ids = np.arange(40) % 64
+    want = tf.TakosunOracle(cfg, w).forward(ids)
+    for dtype, tol in (("float32", 3e-5), ("bfloat16", 0.06)):
+        got = pkg.Model.load(str(tmp_path), 64, dtype).forward(ids, range(40))
+        err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+        assert err.max() <= tol, (dtype, err.max())
