@@ -552,3 +552,19 @@ def test_9_to_32_rows_on_wide_layers_stage_their_rows_per_super_block(pkg, ora, 
         assert row_err(got.cpu().numpy(), want) <= 5e-6, M
         assert torch.equal(got, pkg.ops.gemm_fp32(dev(torch, ba), dev(torch, bw), M, N, K)), M
         assert torch.equal(got, layer.forward(dev(torch, x))), M
+
+
+def test_current_stream_and_output_rows(pkg):
+    import torch
+
+    class Rows(torch.Tensor):
+        pass
+
+    side = torch.cuda.Stream()
+    assert pkg.ops._stream() == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert pkg.ops._stream() == side.cuda_stream
+    x = torch.zeros(2, 3, 64, device="cuda", requires_grad=True)
+    for rows in (x, x.as_subclass(Rows), x.detach().half()):   # always a plain float tensor that asks for no gradient
+        out = pkg.ops._float_rows(rows, 24)
+        assert type(out) is torch.Tensor and out.dtype is torch.float32 and out.shape == (2, 3, 24) and out.is_cuda and not out.requires_grad
