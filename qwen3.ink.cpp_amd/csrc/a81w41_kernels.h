@@ -114,6 +114,7 @@ struct GemmScratch {
     float* partials = nullptr;
     unsigned* arrivals = nullptr;
     int max_partials = 0;
+    bool any_split = false;  // there for every call (a context's), so that a call may split K that would not have needed one
 };
 hipError_t gemm_scratch_create(GemmScratch* out);  // 64 MiB + counters on the current device
 void gemm_scratch_destroy(GemmScratch* ws);

@@ -424,6 +424,7 @@ int a81w41_context_create(int max_rows, int max_cols, a81w41_context** out) {
     ctx->max_elems = (int64_t)max_rows * max_cols;
     ctx->act_bytes = (size_t)(ctx->max_elems / 64) * a81w41::kABlock32;
     HIP_TRY(a81w41::gemm_scratch_create(&ctx->gemm_scratch));
+    ctx->gemm_scratch.any_split = true;
     // A6 holds 2 B per value, rows padded to a multiple of 32 (calls that use it have more than 32 rows)
     ctx->a6_bytes = 4 * (size_t)ctx->max_elems;
     hipError_t e = hipMalloc(&ctx->act_scratch, ctx->act_bytes);

@@ -116,6 +116,49 @@ __device__ __forceinline__ uint32_t b_slot_byte(int gl, int k, int jj) {
     return Geom::kStageB + (24 * gl + (k + 2 * (gl & 3)) % 24) * 16 + 4 * (jj & 3);
 }
 
+// The wave's copies of a stage of the tile at (m_base, n_base).
+__device__ __forceinline__ TileDma tile_copies(const uint8_t* A, const uint8_t* B, int M, int nb_n, int nb_k, int m_base, int n_base,
+                                               int wave, int lane) {
+    // Copy q = i*4 + wave of a stage moves chunks 64q..64q+63: copies 0..4 are activation rows (5 chunks per
+    // row), 5..7 weight blocks.  Rows past M alias the last row and column groups past N the last group;
+    // neither is ever stored.
+    TileDma dma;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int q = i * 4 + wave;
+        const int c = q * 64 + lane;
+        dma.lds_off[i] = q * 1024;
+        if (q < 5) {
+            const int row = c / 5, piece = c - row * 5;
+            const int m_rel = min(m_base + row, M - 1) - m_base;
+            dma.base[i] = A + (size_t)m_base * nb_k * kABlock32;
+            dma.step[i] = kABlock32;
+            dma.voff[i] = (uint32_t)m_rel * nb_k * kABlock32 + 16 * piece;
+        } else {
+            const int s = c - 320;
+            const int gl = s / 24, pos = s - gl * 24;
+            const int k = (pos - 2 * (gl & 3) + 24) % 24;  // slot pos of block gl holds chunk k
+            const int g_rel = min((n_base >> 3) + gl, nb_n - 1) - (n_base >> 3);
+            dma.base[i] = B + (size_t)(n_base >> 3) * nb_k * kWBlock32;
+            dma.step[i] = kWBlock32;
+            dma.voff[i] = (uint32_t)g_rel * nb_k * kWBlock32 + 16 * k;
+        }
+    }
+    return dma;
+}
+
+// Where a lane of the wave at (row0, col0) of the tile reads its operands.
+__device__ __forceinline__ TileRead tile_places(int row0, int col0, int r, int kh) {
+    TileRead rd;
+    rd.a = (row0 + r) * kABlock32;
+    const int col = col0 + r, gl = col >> 3, jj = col & 7;
+    rd.dW = b_slot_byte(gl, 2 * kh + (jj >> 2), jj);
+    rd.mW = b_slot_byte(gl, 4 + 2 * kh + (jj >> 2), jj);
+#pragma unroll
+    for (int t = 0; t < 4; t++) rd.w[t] = b_slot_byte(gl, 8 + 2 * (4 * kh + t) + (jj >> 2), jj);
+    return rd;
+}
+
 // This wave's two direct-to-LDS copies of a stage for super-block sb.
 __device__ __forceinline__ void tile_issue(const TileDma& d, uint8_t* lds, int buf, int sb, int lane) {
 #pragma unroll
@@ -230,16 +273,7 @@ __device__ __forceinline__ void tile_kernel_body(const uint8_t* __restrict__ A, 
     const int nb_n = N >> 3;
     const int row0 = (wave >> 1) * 32, col0 = (wave & 1) * 32;
 
-    TileRead rd;
-    {
-        rd.a = (row0 + r) * kABlock32;
-        const int col = col0 + r, gl = col >> 3, jj = col & 7;
-        rd.dW = b_slot_byte(gl, 2 * kh + (jj >> 2), jj);
-        rd.mW = b_slot_byte(gl, 4 + 2 * kh + (jj >> 2), jj);
-#pragma unroll
-        for (int t = 0; t < 4; t++) rd.w[t] = b_slot_byte(gl, 8 + 2 * (4 * kh + t) + (jj >> 2), jj);
-    }
-
+    const TileRead rd = tile_places(row0, col0, r, kh);
     for (int item = blockIdx.x; item < sc.items; item += gridDim.x) {
         int tau, k0, n_sb, part = -1;  // part >= 0: index of this item's partial tile
         if (item < sc.whole) {
@@ -258,31 +292,7 @@ __device__ __forceinline__ void tile_kernel_body(const uint8_t* __restrict__ A, 
         tile_xy(tau, sc.tiles_m, sc.tiles_n, sc.band, tx, ty);
         const int m_base = ty * kTileM, n_base = tx * kTileN;
 
-        // Copy q = i*4 + wave of a stage moves chunks 64q..64q+63: copies 0..4 are activation rows (5 chunks per
-        // row), 5..7 weight blocks.  Rows past M alias the last row and column groups past N the last group;
-        // neither is ever stored.
-        TileDma dma;
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int q = i * 4 + wave;
-            const int c = q * 64 + lane;
-            dma.lds_off[i] = q * 1024;
-            if (q < 5) {
-                const int row = c / 5, piece = c - row * 5;
-                const int m_rel = min(m_base + row, M - 1) - m_base;
-                dma.base[i] = A + (size_t)m_base * nb_k * kABlock32;
-                dma.step[i] = kABlock32;
-                dma.voff[i] = (uint32_t)m_rel * nb_k * kABlock32 + 16 * piece;
-            } else {
-                const int s = c - 320;
-                const int gl = s / 24, pos = s - gl * 24;
-                const int k = (pos - 2 * (gl & 3) + 24) % 24;  // slot pos of block gl holds chunk k
-                const int g_rel = min((n_base >> 3) + gl, nb_n - 1) - (n_base >> 3);
-                dma.base[i] = B + (size_t)(n_base >> 3) * nb_k * kWBlock32;
-                dma.step[i] = kWBlock32;
-                dma.voff[i] = (uint32_t)g_rel * nb_k * kWBlock32 + 16 * k;
-            }
-        }
+        const TileDma dma = tile_copies(A, B, M, nb_n, nb_k, m_base, n_base, wave, lane);
 
         v16f acc = {0};
         const bool wave_live = m_base + row0 < M;  // else: rows all past M
@@ -391,6 +401,111 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4,
     __shared__ unsigned s_arrived;
     const Schedule sc = {tiles_m, tiles_n, whole, r, c, chunk, whole + r * c, band};
     tile_kernel_body(A, B, C, M, N, nb_k, sc, partials, arrivals, lds, s_arrived);
+}
+
+// Few tiles: a workgroup of TEAMS times four waves takes one tile, or one of `c` parts of its K range, each team of four
+// waves an equal share of the super-blocks with a ring of its own, and their sums meet in LDS.  One such workgroup of four teams
+// fills a CU like four workgroups of the kernel above, two of two teams likewise; the four would have to be parts of a tile's K range
+// that meet in memory (16 KB each, a counter, and a trip back for the last to arrive), and a K range of less than 16
+// super-blocks a part was not cut at all, which left one wave on a SIMD.  57 rows, 4096
+// x 12288: 27.1 us with four parts of four waves, 21.6 us with four of sixteen; 120 rows, 2504 x 1408: 11.9 us with four waves a tile,
+// 10.0 with eight; see plan_teams.
+template <int TEAMS>
+__global__ __launch_bounds__(kTileThreads * TEAMS) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_a81w41_team_kernel(
+    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int nb_k, int tiles_m, int tiles_n, int c, int band,
+    float* __restrict__ C, float* __restrict__ partials, unsigned* __restrict__ arrivals) {
+    constexpr int kRing = Geom::kRing, kOwn = 16 / TEAMS;  // sums of a lane that its team finishes
+    extern __shared__ __align__(16) uint8_t all_lds[];     // TEAMS rings
+    __shared__ unsigned s_arrived;
+    const int lane = threadIdx.x & 63, tid = threadIdx.x & (kTileThreads - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), team = __builtin_amdgcn_readfirstlane(threadIdx.x / kTileThreads);
+    uint8_t* lds = all_lds + team * Geom::kLdsBytes;
+    const int r = lane & 31, kh = lane >> 5, row0 = (wave >> 1) * 32, col0 = (wave & 1) * 32;
+    const int T = tiles_m * tiles_n, ch = blockIdx.x / T, tau = blockIdx.x - ch * T;
+    int tx, ty;
+    tile_xy(tau, tiles_m, tiles_n, band, tx, ty);
+    const int m_base = ty * Geom::kTileM, n_base = tx * Geom::kTileN;
+    const int from = nb_k * ch / c, all = nb_k * (ch + 1) / c - from;
+    const int begin = all * team / TEAMS, n_sb = all * (team + 1) / TEAMS - begin, n_steps = (all + TEAMS - 1) / TEAMS;
+    const int k0 = from + begin;
+    const TileRead rd = tile_places(row0, col0, r, kh);
+    const TileDma dma = tile_copies(A, B, M, N >> 3, nb_k, m_base, n_base, wave, lane);
+    const bool wave_live = m_base + row0 < M;
+    v16f acc = {0};
+    // as in the kernel above; a team past its share copies its last super-block again (or, without any, the range's first)
+    auto sb = [&](int u) { return max(min(k0 + min(u, n_sb - 1), nb_k - 1), 0); };
+#pragma unroll
+    for (int st = 0; st < kRing - 1; st++) tile_issue(dma, lds, st, sb(st), lane);
+    for (int t = 0; t < n_steps; t += kRing) {
+#pragma unroll
+        for (int p = 0; p < kRing; p++) {
+            const int u = t + p;
+            __builtin_amdgcn_sched_barrier(0);
+            wait_vmcnt<(kRing - 2) * Geom::kCopies>();
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            tile_issue(dma, lds, (p + kRing - 1) % kRing, sb(u + kRing - 1), lane);
+            if (wave_live && u < n_sb) {
+                TileOps o;
+                TileProd F;
+                tile_read(o, lds, p, rd, kh);
+                tile_mfma(o, F, acc);
+                tile_epilogue(F, acc);
+            }
+        }
+    }
+    wait_vmcnt<0>();
+    __syncthreads();  // the rings can be reused
+    float* sums = reinterpret_cast<float*>(all_lds);
+#pragma unroll
+    for (int v = 0; v < 16; v++) sums[(team * 16 + v) * kTileThreads + tid] = acc[v];
+    __syncthreads();
+    float own[kOwn];
+#pragma unroll
+    for (int v = 0; v < kOwn; v++) {
+        own[v] = 0.f;
+#pragma unroll
+        for (int k = 0; k < TEAMS; k++) own[v] += sums[(k * 16 + team * kOwn + v) * kTileThreads + tid];
+    }
+    const int n = n_base + col0 + r;
+    auto store = [&]() {
+        if (!wave_live || n >= N) return;
+#pragma unroll
+        for (int v = 0; v < kOwn; v++) {
+            const int a = team * kOwn + v, m = m_base + row0 + 8 * (a >> 2) + 4 * kh + (a & 3);
+            if (m < M) C[(size_t)m * N + n] = own[v];
+        }
+    };
+    if (c == 1) return store();
+    // parts of a K range meet as in the kernel above; thread tid of team k holds the 8-byte elements kOwn/2 k .. of its lane
+    unsigned long long* mine = reinterpret_cast<unsigned long long*>(partials) + (size_t)(tau * c + ch) * (kPartialWords / 2) + tid;
+#pragma unroll
+    for (int v = 0; v < kOwn / 2; v++) {
+        const unsigned long long bits = ((unsigned long long)__float_as_uint(own[2 * v + 1]) << 32) | __float_as_uint(own[2 * v]);
+        __hip_atomic_store(mine + (team * (kOwn / 2) + v) * kTileThreads, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    wait_vmcnt<0>();
+    __syncthreads();
+    if (threadIdx.x == 0) s_arrived = atomicAdd(&arrivals[tau], 1u);
+    __syncthreads();
+    if (s_arrived != (unsigned)(c - 1)) return;
+    unsigned long long bits[4][kOwn / 2];  // c is at most 4
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int v = 0; v < kOwn / 2; v++) {
+            unsigned long long* at = reinterpret_cast<unsigned long long*>(partials) + (size_t)(tau * c + min(k, c - 1)) * (kPartialWords / 2) + tid;
+            bits[k][v] = __hip_atomic_load(at + (team * (kOwn / 2) + v) * kTileThreads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+    for (int v = 0; v < kOwn; v++) {
+        own[v] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (k < c) own[v] += __uint_as_float((unsigned)(bits[k][v >> 1] >> (v & 1) * 32));
+    }
+    store();
+    if (threadIdx.x == 0) __hip_atomic_store(&arrivals[tau], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---- scratch of the K-split path --------------------------------------------------------------
@@ -504,6 +619,50 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     return sc.r * c <= max_partials;
 }
 
+// Teams of waves of a launch, 0: the kernel without; c: how many parts a tile's K range is cut into, which meet in the scratch.
+struct TeamPlan {
+    int teams = 0, c = 1;
+};
+// `sc` is the schedule that the kernel without teams would have; may_split: the caller has a scratch also where that one needs none.
+//
+// A CU takes 0.36 us for a super-block of a tile with four waves, 0.24 with eight and 0.235 with sixteen; a launch has 4.5 us
+// besides, and parts that meet in memory 2.5 (two) to 3.3 us (four).  us without teams / so, for T tiles of K values:
+//   T <= CUs, K <= 2048, two teams: 40 tiles, K = 1408 11.9 / 10.0; 144, K = 1536 12.9 / 10.7; 32, K = 512 7.3 / 5.8
+//   a quarter of the CUs, four parts of four teams: 64, K = 12288 27.1 / 21.6; 64, K = 4096 14.2 / 12.7; 48, K = 4608 20.0 / 13.6; at K = 2048 the
+//     schedule's own four parts 11.0 / 11.3
+//   half of the CUs, two parts of four teams: 128, K = 4096 16.6 / 16.2; 96, K = 4608 20.3 / 17.9; K = 3072, the schedule's own four 14.5 / 15.2
+//   T <= CUs, four teams: 256, K = 4096 23.6 / 21.3, K = 3072 19.9 / 17.7; 192, K = 4608 24.9 / 23.0; the schedule's own four, 192, K = 4096
+//     19.4 / 20.4, 250, K = 12288 51 / 55
+//   up to two tiles a CU, two teams where the schedule cuts K: 432, K = 1536 18.0 / 16.7; 448, K = 2048 21.9 / 20.8; 288, K = 1536 15.5 / 16.4,
+//     448, K = 704, which it does not cut, 10.6 / 11.6
+// K that is no multiple of 512 the schedule did not cut: 40 rows, 2504 x 3712 25.6 / 11.8, 90 rows 25.9 / 14.6, 180 rows 26.0 / 15.8.
+TeamPlan plan_teams(const Schedule& sc, int nb_k, int cus, bool may_split) {
+    const int T = sc.tiles_m * sc.tiles_n, mode = tuning_env_int("A81W41_GEMM_TEAMS");  // tuning builds: 9 = never, else how many
+    const bool own_four = sc.c == 4;
+    if (sc.c > 1) may_split = true;
+    if (mode == 9) return {};
+    if (mode == 2 || mode == 4) return {mode, 1};
+    if (T > cus) return T <= 2 * cus && 16 * T >= 27 * cus && nb_k <= 40 && sc.c > 1 ? TeamPlan{2, 1} : TeamPlan{};
+    if (nb_k <= 32) return own_four && nb_k > 24 && 2 * T <= cus ? TeamPlan{} : TeamPlan{2, 1};
+    if (4 * T <= cus) return {4, may_split ? 4 : 1};
+    if (2 * T <= cus) return own_four && nb_k < 64 ? TeamPlan{} : TeamPlan{4, may_split ? 2 : 1};
+    return own_four && nb_k >= 64 && (nb_k >= 96 || 8 * T <= 7 * cus) ? TeamPlan{} : TeamPlan{4, 1};
+}
+
+template <int TEAMS>
+hipError_t launch_teams(const void* A, const void* B, float* C, int M, int N, int nb_k, const Schedule& sc, int c, const GemmScratch& ws, hipStream_t s) {
+    const int lds = TEAMS * Geom::kLdsBytes;
+    if (lds > 64 * 1024) {  // asked per call: per device, no shared flag
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_a81w41_team_kernel<TEAMS>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(gemm_a81w41_team_kernel<TEAMS>, dim3(sc.tiles_m * sc.tiles_n * c), dim3(TEAMS * kTileThreads), lds, s,
+                       static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(B), M, N, nb_k, sc.tiles_m, sc.tiles_n, c, sc.band, C,
+                       ws.partials, ws.arrivals);
+    return hipGetLastError();
+}
+
 hipError_t launch_tiles(const void* A, const void* B, float* C, int M, int N, int K, const GemmScratch& ws, hipStream_t s) {
     DeviceInfo* d = nullptr;
     {
@@ -513,8 +672,12 @@ hipError_t launch_tiles(const void* A, const void* B, float* C, int M, int N, in
     }
     Schedule sc;
     int grid = 0;
-    if (!make_schedule(M, N, K, d->slots, d->cus, ws.max_partials, sc, grid)) return hipErrorInvalidValue;
+    const bool fits = make_schedule(M, N, K, d->slots, d->cus, ws.max_partials, sc, grid);
     const int nb_k = K / 64;
+    const TeamPlan teams = plan_teams(sc, nb_k, d->cus, ws.any_split);
+    if (teams.teams ? teams.c > 1 && sc.tiles_m * sc.tiles_n * teams.c > ws.max_partials : !fits) return hipErrorInvalidValue;
+    if (teams.teams == 4) return launch_teams<4>(A, B, C, M, N, nb_k, sc, teams.c, ws, s);
+    if (teams.teams == 2) return launch_teams<2>(A, B, C, M, N, nb_k, sc, 1, ws, s);
     hipLaunchKernelGGL(gemm_a81w41_tile64_kernel, dim3(grid), dim3(kTileThreads), Geom::kLdsBytes, s,
                        static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(B), M, N, nb_k, sc.tiles_m, sc.tiles_n, sc.whole,
                        sc.r, sc.c, sc.chunk, sc.band, C, ws.partials, ws.arrivals);
@@ -671,6 +834,8 @@ int gemm_partial_tiles(int M, int N, int K) {
     Schedule sc;
     int grid = 0;
     make_schedule(M, N, K, d->slots, d->cus, kMaxPartials, sc, grid);
+    const TeamPlan teams = plan_teams(sc, K / 64, d->cus, false);
+    if (teams.teams) return teams.c > 1 ? sc.tiles_m * sc.tiles_n * teams.c : 0;
     return sc.r * sc.c;
 }
 

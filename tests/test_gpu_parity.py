@@ -568,3 +568,27 @@ def test_current_stream_and_output_rows(pkg):
     for rows in (x, x.as_subclass(Rows), x.detach().half()):   # always a plain float tensor that asks for no gradient
         out = pkg.ops._float_rows(rows, 24)
         assert type(out) is torch.Tensor and out.dtype is torch.float32 and out.shape == (2, 3, 24) and out.is_cuda and not out.requires_grad
+
+
+# Teams of four waves on one tile: two teams, four; a tile's K range whole, in two and in four parts (a layer's scratch; without it whole);
+# fewer super-blocks than teams, counts that no team divides, ragged rows and columns; between one and two tiles a CU.
+@pytest.mark.parametrize("M,N,K", [(40, 64, 64), (33, 72, 192), (64, 1000, 1408), (130, 136, 2048), (65, 520, 2112), (57, 4096, 2496),
+                                   (90, 4104, 2496), (180, 4096, 2496), (200, 4096, 2560), (40, 2504, 4096), (250, 4096, 4096), (190, 9216, 512)])
+def test_teams_of_waves_on_a_tile(pkg, ora, synth, torch, M, N, K):
+    w4, scale, offset = synth.weight_files(N, K, seed=M)
+    layer = pkg.Linear.from_arrays(w4, scale, offset, N=N, K=K)
+    layer.set_kernel("int8")
+    b16, b32 = (ora.repack(w4, scale, offset, K, N, fp32=f) for f in (False, True))
+    x = synth.activations(M, K, seed=N, outliers=True)
+    xd = dev(torch, x)
+    got = layer.forward(xd)
+    a = pkg.ops.quantize(xd, True)
+    alone = pkg.ops.gemm_fp32(a, dev(torch, b32), M, N, K)
+    rows = sorted({0, 31, 32, 63, M // 2, M - 1} & set(range(M)))
+    want = np.concatenate([ora.linear_forward(np.concatenate([x[m:m + 1]] * 2), b16, b32, N)[:1] for m in rows])
+    # fp32 sums of K / 32 terms in another order: 2^-24 of the row each, with room for their cancellation
+    for y in (got, alone):
+        assert row_err(y.cpu().numpy()[rows], want) < K / 32 * 2.0 ** -24 * 4 + 2e-6
+    # the last of several parts to arrive adds them in order, whoever it is
+    for _ in range(5):
+        assert torch.equal(layer.forward(xd), got)
