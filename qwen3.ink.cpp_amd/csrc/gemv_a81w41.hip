@@ -97,7 +97,8 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_a81w41_fp16_kernel(const voi
     };
 
     // Activation prologue.  All global loads of a chunk are issued before the first
-    // is consumed, so the prologue costs about one memory round trip, not one per element.
+    // is consumed, so the prologue costs about one memory round trip, not one per element.  A slice that is there is loaded
+    // without a branch, by threads past the row's end its last element, which they drop.
     constexpr int kChunk = 4;
     if (!kFromBlob) {
         const float4* x4 = reinterpret_cast<const float4*>(A_or_x);
@@ -106,16 +107,14 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_a81w41_fp16_kernel(const voi
             float4 v[kChunk];
 #pragma unroll
             for (int u = 0; u < kChunk; u++) {
-                const int i = base + u * kThreads + tid;
-                v[u] = (i < n_vec) ? x4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+                if (base + u * kThreads < n_vec) v[u] = x4[min(base + u * kThreads + tid, n_vec - 1)];
             }
             float4 up[PRO == kProSiluMul ? kChunk : 1];  // kProSiluMul: x4 is the gate half of a [2K] row, the up half follows it
             float4 g[kAddNorm ? kChunk : 1], rr[kAddNorm ? kChunk : 1];  // norm weights and residual, requested with the row
             if (PRO == kProSiluMul) {
 #pragma unroll
                 for (int u = 0; u < kChunk; u++) {
-                    const int i = base + u * kThreads + tid;
-                    up[PRO == kProSiluMul ? u : 0] = (i < n_vec) ? x4[n_vec + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (base + u * kThreads < n_vec) up[PRO == kProSiluMul ? u : 0] = x4[n_vec + min(base + u * kThreads + tid, n_vec - 1)];
                 }
             }
             if (kAddNorm) {
@@ -123,9 +122,10 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_a81w41_fp16_kernel(const voi
                 const float4* w4 = reinterpret_cast<const float4*>(pro.norm_w);
 #pragma unroll
                 for (int u = 0; u < kChunk; u++) {
-                    const int i = base + u * kThreads + tid;
-                    g[kAddNorm ? u : 0] = (i < n_vec) ? w4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-                    rr[kAddNorm ? u : 0] = (i < n_vec && r4 != nullptr) ? r4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (base + u * kThreads >= n_vec) break;
+                    const int i = min(base + u * kThreads + tid, n_vec - 1);
+                    g[kAddNorm ? u : 0] = w4[i];
+                    if (r4 != nullptr) rr[kAddNorm ? u : 0] = r4[i];
                 }
             }
             if (base == 0) request_first_weights();
@@ -215,8 +215,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemv_a81w41_fp16_kernel(const voi
             uint2 v[kChunk];
 #pragma unroll
             for (int u = 0; u < kChunk; u++) {
-                const int i = base + u * kThreads + tid;
-                v[u] = (i < n_w) ? A64[i] : make_uint2(0, 0);
+                if (base + u * kThreads < n_w) v[u] = A64[min(base + u * kThreads + tid, n_w - 1)];
             }
             if (base == 0) request_first_weights();
 #pragma unroll
