@@ -100,14 +100,24 @@ int DecoderSession::drain() {
 }
 
 // The ids and wanted rows of a pass of at most max_rows_ tokens.
-int DecoderSession::upload(const int* token_ids, int n, const int* want, int n_want) {
+int DecoderSession::upload(const int* token_ids, int n, const int* want, int n_want, const TokenRow* row) {
     if (upload_waits_) A81W41_TRY(drain());  // of an earlier portion, or of a pass that failed on its way
     upload_waits_ = true;
     std::copy_n(token_ids, n, staged_ids_);
     std::copy_n(want, n_want, staged_ids_ + max_rows_);
-    A81W41_HIP_TRY(launch_take_tokens(staged_ids_, n, ids, staged_ids_ + max_rows_, n_want, want_dev, stream));
+    if (row)  // a single token
+        A81W41_HIP_TRY(launch_take_token(staged_ids_, ids, want_dev, *row, stream));
+    else
+        A81W41_HIP_TRY(launch_take_tokens(staged_ids_, n, ids, staged_ids_ + max_rows_, n_want, want_dev, stream));
     return 0;
 }
+
+// What the launches around a pass do of it, while this object lives.
+struct DecoderSession::Ends {
+    DecoderSession* s;
+    Ends(DecoderSession* session, bool row, bool advance) : s(session) { s->row_given = row, s->advance_given = advance; }
+    ~Ends() { s->row_given = s->advance_given = false; }
+};
 
 int DecoderSession::forward(const int* token_ids, int n, const int* want, int n_want, float* logits_host) {
     if (!token_ids || n_want < 0 || (n_want && !want)) return failf(A81W41_ERR_INVALID_ARG, "null argument");
@@ -126,11 +136,13 @@ int DecoderSession::forward(const int* token_ids, int n, const int* want, int n_
         const int nw = (int)local.size();
         A81W41_TRY(reserve_logits(std::max(nw, 1)));
         plan_ctx = host_pos + m;
-        A81W41_TRY(upload(token_ids + at, m, local.data(), nw));
-        A81W41_TRY(enqueue_pass(m, local.data(), nw, stream));
         const size_t out = logits_host ? (size_t)nw * vocab_ : 0;
         const bool staged = out && out <= staged_floats_;
-        if (staged) A81W41_HIP_TRY(launch_give_floats(logits, staged_logits_, out, stream));
+        TokenRow row;
+        const Ends ends(this, m == 1 && token_row(&row), staged);
+        A81W41_TRY(upload(token_ids + at, m, local.data(), nw, row_given ? &row : nullptr));
+        A81W41_TRY(enqueue_pass(m, local.data(), nw, stream));
+        if (staged) A81W41_HIP_TRY(launch_give_floats(logits, staged_logits_, out, pos, m, stream));
         A81W41_TRY(drain());
         host_pos += m;
         A81W41_TRY(check_passes());
@@ -168,16 +180,21 @@ int DecoderSession::generate_greedy(const int* prompt, int n_prompt, int n_new, 
     const int last_row = (n_prompt - 1) % max_rows_;  // of the prompt's last portion
     A81W41_TRY(upload(prompt, std::min(n_prompt, max_rows_), &last_row, 1));
     A81W41_HIP_TRY(launch_zero_words(step, 1, s));
+    TokenRow row;  // of a decode step's token, formed behind the step before
+    const bool rows = token_row(&row);
+    if (!rows) row = TokenRow{};
     A81W41_HIP_TRY(hipEventRecord(e0, s));
     const int last_ctx = host_pos + n_prompt + n_new - 1;  // also what the decode steps captured below will reach
     for (int at = 0; at < n_prompt; at += max_rows_) {
         const int m = std::min(max_rows_, n_prompt - at);
         plan_ctx = m == 1 ? last_ctx : host_pos + at + m;
         if (at) A81W41_TRY(upload(prompt + at, m, nullptr, 0));
-        A81W41_TRY(enqueue_pass(m, &last_row, at + m == n_prompt ? 1 : 0, s));
+        const bool last = at + m == n_prompt;
+        const Ends ends(this, false, last);
+        A81W41_TRY(enqueue_pass(m, &last_row, last ? 1 : 0, s));
+        // first new token: argmax of the prompt's logits; it becomes the next pass's input id
+        if (last) A81W41_HIP_TRY(launch_next_token(logits, vocab_, ids, history, history_len, step, pos, m, row, s));
     }
-    // first new token: argmax of the prompt's logits; it becomes the next pass's input id
-    A81W41_HIP_TRY(launch_argmax_token(logits, vocab_, ids, history, history_len, step, s));
     A81W41_HIP_TRY(hipEventRecord(e1, s));
     A81W41_TRY(drain());
     host_pos += n_prompt;
@@ -187,10 +204,15 @@ int DecoderSession::generate_greedy(const int* prompt, int n_prompt, int n_new, 
         plan_ctx = last_ctx;
         const int row0 = 0;
         // one decode step = a pass over the single id in ids[0] + argmax; captured once, replayed
+        auto step_once = [&]() -> int {
+            const Ends ends(this, rows, true);
+            A81W41_TRY(enqueue_pass(1, &row0, 1, s));
+            A81W41_HIP_TRY(launch_next_token(logits, vocab_, ids, history, history_len, step, pos, 1, row, s));
+            return 0;
+        };
         bool captured = false;
         if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) {
-            int st = enqueue_pass(1, &row0, 1, s);
-            if (st == 0 && launch_argmax_token(logits, vocab_, ids, history, history_len, step, s) != hipSuccess) st = 1;
+            int st = step_once();
             const hipError_t ee = hipStreamEndCapture(s, &own.graph);
             if (st == 0 && ee == hipSuccess && own.graph && hipGraphInstantiate(&own.exec, own.graph, nullptr, nullptr, 0) == hipSuccess)
                 captured = true;
@@ -201,8 +223,7 @@ int DecoderSession::generate_greedy(const int* prompt, int n_prompt, int n_new, 
             if (captured) {
                 A81W41_HIP_TRY(hipGraphLaunch(own.exec, s));
             } else {
-                A81W41_TRY(enqueue_pass(1, &row0, 1, s));
-                A81W41_HIP_TRY(launch_argmax_token(logits, vocab_, ids, history, history_len, step, s));
+                A81W41_TRY(step_once());
             }
         }
         A81W41_HIP_TRY(hipEventRecord(e2, s));

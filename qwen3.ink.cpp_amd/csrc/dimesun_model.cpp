@@ -139,7 +139,7 @@ Config read_config(const Json& j) {
 template <typename T>
 class DimesunModel final : public DenseModel<T> {
     using Base = DenseModel<T>;
-    using Base::cache, Base::ids, Base::logits, Base::max_seq, Base::plan_ctx, Base::pos, Base::stream, Base::want_dev;
+    using Base::cache, Base::ids, Base::logits, Base::max_seq, Base::plan_ctx, Base::pos, Base::stream, Base::want_dev, Base::row_given, Base::advance_given;
     using Base::allocate_array, Base::finish, Base::init_session, Base::kMatrixAttention, Base::kTable, Base::load_feed_forward,
         Base::load_matrix, Base::load_rotation, Base::load_vector, Base::product, Base::put_matrix, Base::upload_array;
     using Staging = typename Base::Staging;
@@ -184,6 +184,10 @@ class DimesunModel final : public DenseModel<T> {
 
    protected:
     int enqueue_pass(int M, const int* want, int n_want, hipStream_t s) override;
+    bool token_row(TokenRow* row) const override {
+        *row = TokenRow{embed_.data, kTable, embed_.ld, x_, cfg_.width, cfg_.vocab};
+        return one_token_fits_ && !opt_unfused_;
+    }
 
    private:
     struct Layer {
@@ -524,7 +528,7 @@ int DimesunModel<T>::mixer_one_token(const Layer& L, const LayerConfig& lc, cons
 template <typename T>
 int DimesunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
     const int W = cfg_.width;
-    A81W41_HIP_TRY(launch_embed_rows(ids, embed_.data, kTable, embed_.ld, x_, 1, W, cfg_.vocab, s));
+    if (!row_given) A81W41_HIP_TRY(launch_embed_rows(ids, embed_.data, kTable, embed_.ld, x_, 1, W, cfg_.vocab, s));
     RowStep step;  // what the next product's prologue does
     step.width = W, step.x = x_, step.norm_h = norm(layers_[cfg_.runs[0].layer].norm1);
     for (int i = 0; i < n_runs(); i++) {
@@ -547,7 +551,7 @@ int DimesunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
     }
     step.x_out = row_x_[n_runs() & 1];  // the state may be asked for even where no logits are
     A81W41_HIP_TRY(launch_gemv_step<T>(step, embed_.data, embed_.ld, n_want ? embed_.rows : 1, logits, s));
-    A81W41_HIP_TRY(launch_advance(pos, 1, s));
+    if (!advance_given) A81W41_HIP_TRY(launch_advance(pos, 1, s));
     return 0;
 }
 
@@ -579,7 +583,7 @@ int DimesunModel<T>::enqueue_pass(int M, const int* want, int n_want, hipStream_
         if (M > 1) g.a_rows = want_dev;
         A81W41_HIP_TRY(launch_dense_gemm<T>(g, Epilogue::kFloat, s));
     }
-    A81W41_HIP_TRY(launch_advance(pos, M, s));
+    if (!advance_given) A81W41_HIP_TRY(launch_advance(pos, M, s));
     return 0;
 }
 

@@ -62,6 +62,8 @@ struct a81w41_qwen3 : a81w41_model {
    protected:
     int ready() const override;
     int enqueue_pass(int M, const int* want, int n_want, hipStream_t s) override;
+    int one_token_pass(hipStream_t s);
+    bool token_row(a81w41::TokenRow* row) const override;
     int check_passes() override;
 };
 
@@ -102,7 +104,6 @@ int a81w41_qwen3::ready() const {
 }
 
 namespace {
-int enqueue_pass_one_token(a81w41_qwen3* m, hipStream_t s);
 bool one_token_pass_usable(const a81w41_qwen3* m);
 bool prefill_fusion_usable(const a81w41_qwen3* m);
 
@@ -112,7 +113,7 @@ bool prefill_fusion_usable(const a81w41_qwen3* m);
 // m->logits and advances the device position by M.  Enqueues only.
 int a81w41_qwen3::enqueue_pass(int M, const int* want, int n_want, hipStream_t s) {
     a81w41_qwen3* m = this;
-    if (M == 1 && one_token_pass_usable(m)) return enqueue_pass_one_token(m, s);
+    if (M == 1 && one_token_pass_usable(m)) return one_token_pass(s);
     const a81w41_qwen3_config& c = m->cfg;
     const int qkv_dim = m->qkv_dim(), q_dim = c.n_q_heads * kHeadDim;
     const float scale = m->attn_scale;  // scaling.bin, QwenAttention.cc:44-46
@@ -175,7 +176,7 @@ int a81w41_qwen3::enqueue_pass(int M, const int* want, int n_want, hipStream_t s
     // lm_head on the wanted tokens only: in generation the last one (QwenForCausalLM.cc:43-46)
     for (int i = 0; i < n_want; i++)
         Q_TRY(a81w41_linear_forward(m->lm_head, m->h + (size_t)want[i] * c.hidden, 1, m->logits + (size_t)i * c.vocab, s));
-    Q_HIP(a81w41::launch_advance(m->pos, M, s));
+    if (!advance_given) Q_HIP(a81w41::launch_advance(m->pos, M, s));
     return 0;
 }
 
@@ -202,7 +203,15 @@ int attention_step(a81w41_qwen3* m, LayerWeights& L, float* out, void* q_out, in
     return 0;
 }
 
-int enqueue_pass_one_token(a81w41_qwen3* m, hipStream_t s) {
+}  // namespace
+
+bool a81w41_qwen3::token_row(a81w41::TokenRow* row) const {
+    *row = a81w41::TokenRow{embedding, a81w41::TableType::kFp16, cfg.hidden, o, cfg.hidden, cfg.vocab};
+    return one_token_pass_usable(this);
+}
+
+int a81w41_qwen3::one_token_pass(hipStream_t s) {
+    a81w41_qwen3* m = this;
     const a81w41_qwen3_config& c = m->cfg;
     const int qkv_dim = m->qkv_dim();
     const float scale = m->attn_scale;
@@ -221,7 +230,8 @@ int enqueue_pass_one_token(a81w41_qwen3* m, hipStream_t s) {
     if (splits > fit) splits = fit;
     if (env_split > 0) splits = env_split;
     splits = splits < 1 ? 1 : (splits > a81w41::kAttentionMaxSplits ? a81w41::kAttentionMaxSplits : splits);
-    Q_HIP(a81w41::launch_embed_rows(m->ids, m->embedding, a81w41::TableType::kFp16, c.hidden, m->o, 1, c.hidden, c.vocab, s));  // pending = the embedding
+    if (!row_given)  // pending = the embedding
+        Q_HIP(a81w41::launch_embed_rows(m->ids, m->embedding, a81w41::TableType::kFp16, c.hidden, m->o, 1, c.hidden, c.vocab, s));
     // The linears and the attention of the pass are one dependent chain (QwenDecoderLayer.cc:39-105).  As links of
     // an overlapping chain each of them starts while its predecessor runs and requests its first weight blocks
     // (or cache rows) before it waits for it; same kernels' arithmetic, same bits.
@@ -325,9 +335,11 @@ int enqueue_pass_one_token(a81w41_qwen3* m, hipStream_t s) {
         Q_HIP(a81w41::launch_gemv_add_norm(m->o, pf, scratch, a81w41_linear_weight_fp16_dev(m->lm_head), m->logits, c.vocab,
                                            c.hidden, s));
     }
-    Q_HIP(a81w41::launch_advance(m->pos, 1, s));
+    if (!advance_given) Q_HIP(a81w41::launch_advance(m->pos, 1, s));
     return 0;
 }
+
+namespace {
 
 bool prefill_fusion_usable(const a81w41_qwen3* m) {
     if (m->opt_unfused) return false;

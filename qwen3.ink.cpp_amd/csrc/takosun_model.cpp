@@ -97,7 +97,7 @@ constexpr int kLatentTokenKeys = 512;
 template <typename T>
 class TakosunModel final : public DenseModel<T> {
     using Base = DenseModel<T>;
-    using Base::cache, Base::ids, Base::logits, Base::max_seq, Base::plan_ctx, Base::pos, Base::stream, Base::want_dev;
+    using Base::cache, Base::ids, Base::logits, Base::max_seq, Base::plan_ctx, Base::pos, Base::stream, Base::want_dev, Base::row_given, Base::advance_given;
     using Base::allocate_array, Base::finish, Base::init_session, Base::kMatrixAttention, Base::kTable, Base::load_feed_forward,
         Base::load_matrix, Base::load_rotation, Base::load_vector, Base::product, Base::put_matrix, Base::upload_array;
     using Staging = typename Base::Staging;
@@ -135,6 +135,10 @@ class TakosunModel final : public DenseModel<T> {
 
    protected:
     int enqueue_pass(int M, const int* want, int n_want, hipStream_t s) override;
+    bool token_row(TokenRow* row) const override {
+        *row = TokenRow{embed_.data, kTable, embed_.ld, states_, cfg_.width, cfg_.vocab};
+        return one_token_fits_ && !opt_unfused_;
+    }
 
    private:
     using FeedForward = GatedWeights<T>;
@@ -519,8 +523,7 @@ int TakosunModel<T>::attend_one_token(const Layer& L, const LatentShape& sh, con
 template <typename T>
 int TakosunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
     const int W = cfg_.width, n = n_layers();
-    A81W41_HIP_TRY(launch_embed_rows(ids, embed_.data, kTable, embed_.ld, states_, 1, W,
-                                     cfg_.vocab, s));
+    if (!row_given) A81W41_HIP_TRY(launch_embed_rows(ids, embed_.data, kTable, embed_.ld, states_, 1, W, cfg_.vocab, s));
     RowStep step;  // what the next product's prologue does
     step.x = states_, step.width = W, step.norm_h = norm(layers_[0].norm1);
     for (int i = 0; i < n; i++) {
@@ -548,7 +551,7 @@ int TakosunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
         step.norm_h = norm(i + 1 < n ? layers_[i + 1].norm1 : final_norm_);
     }
     if (n_want) A81W41_HIP_TRY(launch_gemv_step<T>(step, head_.data, head_.ld, head_.rows, logits, s));
-    A81W41_HIP_TRY(launch_advance(pos, 1, s));
+    if (!advance_given) A81W41_HIP_TRY(launch_advance(pos, 1, s));
     return 0;
 }
 
@@ -585,7 +588,7 @@ int TakosunModel<T>::enqueue_pass(int M, const int* want, int n_want, hipStream_
         if (M > 1) g.a_rows = want_dev;
         A81W41_HIP_TRY(launch_dense_gemm<T>(g, Epilogue::kFloat, s));
     }
-    A81W41_HIP_TRY(launch_advance(pos, M, s));
+    if (!advance_given) A81W41_HIP_TRY(launch_advance(pos, M, s));
     return 0;
 }
 

@@ -88,3 +88,24 @@ def test_two_models_side_by_side(pkg, tmp_path):
         want = oracle.forward(ids)
         err = np.linalg.norm(np.concatenate(got[k]) - want, axis=1) / np.linalg.norm(want, axis=1)
         assert err.max() <= 3e-5
+
+
+# The kernel between two tokens: vocabularies around its float4s and its 32768 logits a round, the lower of two equal logits, table
+# rows of eight values at a time and one at a time
+@pytest.mark.parametrize("vocab,width", [(2, 64), (6, 64), (4098, 62), (32772, 64), (70001, 62)])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_generation_takes_the_first_maximum(pkg, tmp_path, vocab, width, dtype):
+    from tests import takosun_fixture as tx
+    cfg = tx.config(vocab, width, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.4), tx.dense(32))])
+    w = tf.random_weights(cfg, vocab)
+    half = vocab // 2
+    w["head"][half:2 * half] = w["head"][:half]   # every logit twice
+    tx.write_model(str(tmp_path), cfg, w)
+    model = pkg.Model.load(str(tmp_path), 40, dtype)
+    got, _, _ = model.generate_greedy([1, 0, 1], 12)
+    model.reset()
+    logits = model.forward([1, 0, 1])[0]
+    for token in got.tolist():
+        assert token == int(logits.argmax())
+        logits = model.forward([token])[0]
+    assert model.position == 3 + 12
