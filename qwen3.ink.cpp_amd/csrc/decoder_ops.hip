@@ -149,7 +149,7 @@ __global__ __launch_bounds__(256) void take_token_kernel(const int* host_id, int
 }
 // Behind a pass's logits the position is free to advance.
 __global__ __launch_bounds__(256) void give_floats_kernel(const float* __restrict__ x, float* host, size_t n, int* __restrict__ pos_dev, int by) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) pos_dev[0] += by;
+    if (by && blockIdx.x == 0 && threadIdx.x == 0) pos_dev[0] += by;
     for (size_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) host[i] = x[i];
 }
 __global__ __launch_bounds__(256) void zero_words_kernel(unsigned* __restrict__ p, size_t n) {
@@ -179,12 +179,15 @@ hipError_t launch_embed_rows(const int* ids, const void* table, TableType type, 
     }
     return hipGetLastError();
 }
-hipError_t launch_next_token(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev, int* pos_dev, int by,
+static hipError_t next_token(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev, int* pos_dev, int by,
                              const TokenRow& row, hipStream_t s) {
     hipLaunchKernelGGL(next_token_kernel, dim3(1), dim3(1024), 0, s, logits, n, next_id, history, history_len, step_dev, pos_dev, by, row);
     return hipGetLastError();
 }
-hipError_t launch_take_token(const int* host_id, int* ids, int* want, const TokenRow& row, hipStream_t s) {
+hipError_t launch_argmax_token(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev, hipStream_t s) {
+    return next_token(logits, n, next_id, history, history_len, step_dev, nullptr, 0, TokenRow{}, s);
+}
+static hipError_t take_token(const int* host_id, int* ids, int* want, const TokenRow& row, hipStream_t s) {
     hipLaunchKernelGGL(take_token_kernel, dim3(1), dim3(256), 0, s, host_id, ids, want, row);
     return hipGetLastError();
 }
@@ -192,9 +195,14 @@ hipError_t launch_take_tokens(const int* host_ids, int n, int* ids, const int* h
     hipLaunchKernelGGL(take_tokens_kernel, dim3((n + n_want + 255) / 256), dim3(256), 0, s, host_ids, n, ids, host_want, n_want, want);
     return hipGetLastError();
 }
-hipError_t launch_give_floats(const float* x, float* host, size_t n, int* pos_dev, int by, hipStream_t s) {
+static hipError_t give_floats(const float* x, float* host, size_t n, int* pos_dev, int by, hipStream_t s) {
     hipLaunchKernelGGL(give_floats_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 256)), dim3(256), 0, s, x, host, n, pos_dev, by);
     return hipGetLastError();
+}
+hipError_t launch_give_floats(const float* x, float* host, size_t n, hipStream_t s) { return give_floats(x, host, n, nullptr, 0, s); }
+const JoinedLaunches* all_joined_launches() {
+    static const JoinedLaunches table = {take_token, next_token, give_floats};
+    return &table;
 }
 hipError_t launch_zero_words(void* p, size_t words, hipStream_t s) {
     hipLaunchKernelGGL(zero_words_kernel, dim3((unsigned)std::min<size_t>((words + 255) / 256, 1024)), dim3(256), 0, s,

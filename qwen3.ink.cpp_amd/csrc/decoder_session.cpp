@@ -106,9 +106,18 @@ int DecoderSession::upload(const int* token_ids, int n, const int* want, int n_w
     std::copy_n(token_ids, n, staged_ids_);
     std::copy_n(want, n_want, staged_ids_ + max_rows_);
     if (row)  // a single token
-        A81W41_HIP_TRY(launch_take_token(staged_ids_, ids, want_dev, *row, stream));
+        A81W41_HIP_TRY(joined_launches()->take_token(staged_ids_, ids, want_dev, *row, stream));
     else
         A81W41_HIP_TRY(launch_take_tokens(staged_ids_, n, ids, staged_ids_ + max_rows_, n_want, want_dev, stream));
+    return 0;
+}
+
+// Behind a pass over `by` tokens: its first maximum is the next pass's input id.
+int DecoderSession::next_token(const JoinedLaunches* joined, int by, const TokenRow& row) {
+    if (joined)
+        A81W41_HIP_TRY(joined->next_token(logits, vocab_, ids, history, history_len, step, pos, by, row, stream));
+    else
+        A81W41_HIP_TRY(launch_argmax_token(logits, vocab_, ids, history, history_len, step, stream));
     return 0;
 }
 
@@ -129,6 +138,7 @@ int DecoderSession::forward(const int* token_ids, int n, const int* want, int n_
             return failf(A81W41_ERR_INVALID_ARG, "the wanted places must rise and lie among the tokens");
     std::vector<int> local;
     int w0 = 0;
+    const JoinedLaunches* const joined = joined_launches();
     for (int at = 0; at < n; at += max_rows_) {
         const int m = std::min(max_rows_, n - at);
         local.clear();
@@ -139,10 +149,13 @@ int DecoderSession::forward(const int* token_ids, int n, const int* want, int n_
         const size_t out = logits_host ? (size_t)nw * vocab_ : 0;
         const bool staged = out && out <= staged_floats_;
         TokenRow row;
-        const Ends ends(this, m == 1 && token_row(&row), staged);
+        const Ends ends(this, joined && m == 1 && token_row(&row), joined && staged);
         A81W41_TRY(upload(token_ids + at, m, local.data(), nw, row_given ? &row : nullptr));
         A81W41_TRY(enqueue_pass(m, local.data(), nw, stream));
-        if (staged) A81W41_HIP_TRY(launch_give_floats(logits, staged_logits_, out, pos, m, stream));
+        if (advance_given)
+            A81W41_HIP_TRY(joined->give_floats(logits, staged_logits_, out, pos, m, stream));
+        else if (staged)
+            A81W41_HIP_TRY(launch_give_floats(logits, staged_logits_, out, stream));
         A81W41_TRY(drain());
         host_pos += m;
         A81W41_TRY(check_passes());
@@ -181,7 +194,8 @@ int DecoderSession::generate_greedy(const int* prompt, int n_prompt, int n_new, 
     A81W41_TRY(upload(prompt, std::min(n_prompt, max_rows_), &last_row, 1));
     A81W41_HIP_TRY(launch_zero_words(step, 1, s));
     TokenRow row;  // of a decode step's token, formed behind the step before
-    const bool rows = token_row(&row);
+    const JoinedLaunches* const joined = joined_launches();
+    const bool rows = joined && token_row(&row);
     if (!rows) row = TokenRow{};
     A81W41_HIP_TRY(hipEventRecord(e0, s));
     const int last_ctx = host_pos + n_prompt + n_new - 1;  // also what the decode steps captured below will reach
@@ -190,10 +204,9 @@ int DecoderSession::generate_greedy(const int* prompt, int n_prompt, int n_new, 
         plan_ctx = m == 1 ? last_ctx : host_pos + at + m;
         if (at) A81W41_TRY(upload(prompt + at, m, nullptr, 0));
         const bool last = at + m == n_prompt;
-        const Ends ends(this, false, last);
+        const Ends ends(this, false, joined && last);
         A81W41_TRY(enqueue_pass(m, &last_row, last ? 1 : 0, s));
-        // first new token: argmax of the prompt's logits; it becomes the next pass's input id
-        if (last) A81W41_HIP_TRY(launch_next_token(logits, vocab_, ids, history, history_len, step, pos, m, row, s));
+        if (last) A81W41_TRY(next_token(joined, m, row));  // first new token
     }
     A81W41_HIP_TRY(hipEventRecord(e1, s));
     A81W41_TRY(drain());
@@ -205,10 +218,9 @@ int DecoderSession::generate_greedy(const int* prompt, int n_prompt, int n_new, 
         const int row0 = 0;
         // one decode step = a pass over the single id in ids[0] + argmax; captured once, replayed
         auto step_once = [&]() -> int {
-            const Ends ends(this, rows, true);
+            const Ends ends(this, rows, joined != nullptr);
             A81W41_TRY(enqueue_pass(1, &row0, 1, s));
-            A81W41_HIP_TRY(launch_next_token(logits, vocab_, ids, history, history_len, step, pos, 1, row, s));
-            return 0;
+            return next_token(joined, 1, row);
         };
         bool captured = false;
         if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) {

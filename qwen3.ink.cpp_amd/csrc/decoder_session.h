@@ -45,15 +45,24 @@ struct TokenRow {
     float* out = nullptr;
     int hidden = 0, vocab = 0;
 };
-// First maximum of the logits to next_id and history; the step counter advances by one, the position by `by`; row: see above.
-hipError_t launch_next_token(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev, int* pos_dev, int by,
-                             const TokenRow& row, hipStream_t s);
-hipError_t launch_take_token(const int* host_id, int* ids, int* want, const TokenRow& row, hipStream_t s);  // one token with its row
+// First maximum of the logits to next_id and history; the step counter advances by one.
+hipError_t launch_argmax_token(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev, hipStream_t s);
 hipError_t launch_advance(int* pos_dev, int by, hipStream_t s);
-// ids[0 .. n) and want[0 .. n_want) from pinned host memory; n floats into pinned host memory, the position by `by`; words of zeros.
+// ids[0 .. n) and want[0 .. n_want) from pinned host memory; n floats into pinned host memory; words of zeros.
 hipError_t launch_take_tokens(const int* host_ids, int n, int* ids, const int* host_want, int n_want, int* want, hipStream_t s);
-hipError_t launch_give_floats(const float* x, float* host, size_t n, int* pos_dev, int by, hipStream_t s);
+hipError_t launch_give_floats(const float* x, float* host, size_t n, hipStream_t s);
 hipError_t launch_zero_words(void* p, size_t words, hipStream_t s);
+// The launches around a pass with parts of the pass in them, for a model that leaves those parts to its session.
+struct JoinedLaunches {
+    // one token and its row
+    hipError_t (*take_token)(const int* host_id, int* ids, int* want, const TokenRow& row, hipStream_t s);
+    // launch_argmax_token, the position by `by`, the row of the token found
+    hipError_t (*next_token)(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev, int* pos_dev, int by,
+                             const TokenRow& row, hipStream_t s);
+    // launch_give_floats, the position by `by`
+    hipError_t (*give_floats)(const float* x, float* host, size_t n, int* pos_dev, int by, hipStream_t s);
+};
+const JoinedLaunches* all_joined_launches();
 
 // What a sequence holds on the device, zero when allocated, freed with the object: cache planes of max_seq rows, which a new
 // sequence overwrites, and recurrent states, which go back to zero when the sequence is given back.
@@ -103,9 +112,12 @@ class DecoderSession {
     // position advances by M.  want_dev holds the wanted rows on the device (a pass over one token may not read it: it can
     // be part of a captured graph).  Enqueues only.
     virtual int enqueue_pass(int M, const int* want, int n_want, hipStream_t s) = 0;
-    // Where the next one-token pass takes its embedding row from if row_given says that it is there already; false: nowhere.
+    // Null: a pass always takes its rows and advances the position by itself.
+    virtual const JoinedLaunches* joined_launches() const { return nullptr; }
+    // With joined launches: where the next one-token pass has its embedding row if row_given says that it is there already;
+    // false: nowhere.
     virtual bool token_row(TokenRow*) const { return false; }
-    // Set around enqueue_pass by the loop: the embedding row is in place; somebody else advances the position.
+    // Set around enqueue_pass by the loop: the embedding row is in place; a joined launch behind the pass advances the position.
     bool row_given = false, advance_given = false;
     // After a synchronisation: whether the passes so far really worked.
     virtual int check_passes() { return 0; }
@@ -124,6 +136,7 @@ class DecoderSession {
     struct Ends;
     int reserve_logits(int rows);
     int upload(const int* token_ids, int n, const int* want, int n_want, const TokenRow* row = nullptr);
+    int next_token(const JoinedLaunches* joined, int by, const TokenRow& row);
     int drain();  // waits for the stream
     int max_seq_ = 0, vocab_ = 0, max_rows_ = 0;
     // pinned: ids and wanted rows of a pass, read by an enqueued kernel until the stream is next drained (upload_waits_ until then);

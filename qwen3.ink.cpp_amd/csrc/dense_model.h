@@ -50,6 +50,7 @@ class DenseModel : public a81w41_model {
     static constexpr TableType kTable = sizeof(T) == 2 ? TableType::kBf16 : TableType::kFp32;
 
     int ready() const override { return 0; }  // creation loads everything or fails
+    const JoinedLaunches* joined_launches() const override { return all_joined_launches(); }
 
     template <typename E>
     int allocate_array(size_t n, E** out, bool weight = false) {

@@ -63,6 +63,7 @@ struct a81w41_qwen3 : a81w41_model {
     int ready() const override;
     int enqueue_pass(int M, const int* want, int n_want, hipStream_t s) override;
     int one_token_pass(hipStream_t s);
+    const a81w41::JoinedLaunches* joined_launches() const override { return a81w41::all_joined_launches(); }
     bool token_row(a81w41::TokenRow* row) const override;
     int check_passes() override;
 };
