@@ -26,6 +26,7 @@ enum class Epilogue {
     kGatedPair,  // columns come as 16 gates, then their 16 ups, and so on: C (T) has N / 2 columns, the unit of gate and up
     kHeadGate,   // C (T) times the sigmoid of head_gate[row][batch]
     kHeads,      // queries, keys and values: rotated and stored as HeadRows says
+    kQueries,    // queries of latent attention, as LatentQueries says
 };
 // g = min(gate, limit), u = clamp(up, +-limit): g sigmoid(slope g) (u + shift).  As it stands: silu(gate) up.
 struct GatedUnit {
@@ -47,6 +48,17 @@ struct HeadRows {
     int max_seq = 0;
     float* rest = nullptr;
     int ld_rest = 0;
+};
+// Columns of heads, each [dim | one zero if dim is odd | rot]: the first to nope, head h of row m at (m heads + h) ld_nope, the last
+// to rotated, at (m heads + h) ld_rot, turned in neighbouring pairs by the angles of the token at *pos_dev + m.
+template <typename T>
+struct LatentQueries {
+    int heads = 0, dim = 0, rot = 0;
+    T *nope = nullptr, *rotated = nullptr;
+    int ld_nope = 0, ld_rot = 0;
+    const float *cos_t = nullptr, *sin_t = nullptr;  // [max_seq][rot / 2]
+    const int* pos_dev = nullptr;
+    int max_seq = 0;
 };
 // A grouped product's rows come sorted by expert, its row tiles in the same order.  What a tile's workgroup has to know: the expert, the
 // number of the expert's first tile, and the expert's rows [row0, row0 + rows).
@@ -82,6 +94,8 @@ template <typename T>
 hipError_t launch_dense_gemm(const GemmArgs& g, Epilogue epi, hipStream_t s);
 template <typename T>
 hipError_t launch_dense_gemm_heads(const GemmArgs& g, const HeadRows<T>& heads, hipStream_t s);  // g.C is not used
+template <typename T>
+hipError_t launch_dense_gemm_queries(const GemmArgs& g, const LatentQueries<T>& q, hipStream_t s);  // nor here
 
 // ---- rows (dense_rows.hip) ------------------------------------------------------------------
 // Norm in groups: the row is cut into `groups` parts, each divided by sqrt(mean of its squares + eps); times w.
@@ -131,11 +145,15 @@ hipError_t launch_router(const float* logits, int ld, const float* bias, int exp
 constexpr int kMaxRouted = 2048, kMaxTop = 64;  // experts of a router, and of a token
 
 // ---- latent attention (latent_attention.hip) ------------------------------------------------
-// Sizes of one mixer.  A cache row is [latent (rank) | rotated shared key part (rot)], zero up to ld_cache.
+// Sizes of one mixer.  A cache row is [latent (rank) | rotated shared key part (rot)], zero up to ld_cache.  Components of a rotated
+// part that turn together are neighbours there, by the order of the weights' rows, which queries and keys share.
 struct LatentShape {
     int heads = 0, dim = 0, rot = 0, vdim = 0, rank = 0, q_rank = 0;
     int ld_cache = 0;
     float scale = 0.f;
+    // a head's query [dim | rot] starts its rotated part at an even column
+    __host__ __device__ int turned_at() const { return dim + (dim & 1); }
+    __host__ __device__ int query_width() const { return turned_at() + rot; }
 };
 // The fused down-projection row is [query latent (q_rank) | latent (rank) | rotated part (rot) | head gates (heads)],
 // without the middle two where the layer reads another layer's cache.
@@ -152,11 +170,6 @@ struct LatentRows {
 // rows pos .. pos + M - 1.
 template <typename T>
 hipError_t launch_latent_rows(const LatentRows& in, const LatentShape& sh, int M, T* q_latent, int ld_q, T* cache, hipStream_t s);
-// q [M][ld_q] head by head [dim | rot]: the unrotated parts to nope (head h of token m at (m heads + h) ld_nope), the
-// rotated parts to rot_out (at (m heads + h) ld_rot).
-template <typename T>
-hipError_t launch_rotate_queries(const float* q, int ld_q, const LatentRows& in, const LatentShape& sh, int M, T* nope, int ld_nope,
-                                 T* rot_out, int ld_rot, hipStream_t s);
 
 // ---- attention (attend_vector.hip, attend_mfma.hip, attend_prompt.hip) ------------------------------------------
 // Query row r of head z belongs to token r / rows_per_token of the pass: q + z q_head + token q_token + (r %

@@ -35,47 +35,58 @@ __device__ __forceinline__ int expert_rank(const float* z, int n, int e) {
     return rank;
 }
 
-// Where one column of a HeadRows product goes.
-template <typename T>
-class HeadColumn {
-   public:
-    __device__ __forceinline__ HeadColumn(const HeadRows<T>& p, int col) : p_(p) {
-        const int nq = p.heads * p.dim, nk = p.kv_heads * p.dim, nv = p.kv_heads * p.vdim;
-        rest_ = col >= nq + nk + nv;
-        cached_ = col >= nq;
-        if (rest_) {
-            at_ = col - nq - nk - nv;
-        } else if (col >= nq + nk) {
-            const int c = col - nq - nk, h = c / p.vdim;
-            at_ = h * (p.vdim + p.dim) + (c - h * p.vdim);
-        } else {
-            const int c = cached_ ? col - nq : col, h = c / p.dim, d = c - h * p.dim;
-            at_ = cached_ ? h * (p.vdim + p.dim) + p.vdim + d : c;
-            if ((d >> 1) < p.rot_pairs) pair_ = d >> 1, second_ = d & 1;
-        }
-    }
-    // of row m, the token at position pos + m
-    __device__ __forceinline__ void angle(int m, int pos, float& cs, float& sn) const {
-        if (pair_ < 0) return;
-        const size_t i = (size_t)min(pos + m, p_.max_seq - 1) * p_.rot_pairs + pair_;
-        cs = p_.cos_t[i], sn = p_.sin_t[i];
-    }
-    // `own` is the column's value in row m, `other` that of its pair's other column
-    __device__ __forceinline__ void store(int m, int pos, float own, float other, float cs, float sn) const {
-        if (pair_ >= 0) own = second_ ? own * cs + other * sn : own * cs - other * sn;
-        if (rest_)
-            p_.rest[(size_t)m * p_.ld_rest + at_] = own;
-        else if (cached_)
-            p_.cache[(size_t)min(pos + m, p_.max_seq - 1) * p_.ld_cache + at_] = (T)own;
-        else
-            p_.q[(size_t)m * (p_.heads * p_.dim) + at_] = (T)own;
-    }
-
-   private:
-    const HeadRows<T>& p_;
-    int at_, pair_ = -1;
-    bool rest_, cached_, second_ = false;
+// Where one column of a HeadRows or LatentQueries product goes, from row m on: element d of the column at dst + d step (bytes), the
+// first `rows` rows, float instead of the element type for what is not a head's.  Columns with a pair turn with their neighbour.
+struct ColumnPlace {
+    uint8_t* dst;
+    int step, rows = 0x7fffffff, pair = -1;
+    bool as_float = false, second = false;
 };
+template <typename T>
+__device__ __forceinline__ ColumnPlace column_place(const HeadRows<T>& p, int col, int m, int pos) {
+    const int nq = p.heads * p.dim, nk = p.kv_heads * p.dim, nv = p.kv_heads * p.vdim;
+    ColumnPlace to;
+    int at;
+    if (col >= nq + nk + nv) {
+        to.as_float = true, to.step = p.ld_rest * (int)sizeof(float);
+        to.dst = reinterpret_cast<uint8_t*>(p.rest + (size_t)m * p.ld_rest + (col - nq - nk - nv));
+        return to;
+    }
+    const bool cached = col >= nq;
+    if (col >= nq + nk) {
+        const int c = col - nq - nk, h = c / p.vdim;
+        at = h * (p.vdim + p.dim) + (c - h * p.vdim);
+    } else {
+        const int c = cached ? col - nq : col, h = c / p.dim, d = c - h * p.dim;
+        at = cached ? h * (p.vdim + p.dim) + p.vdim + d : c;
+        if ((d >> 1) < p.rot_pairs) to.pair = d >> 1, to.second = d & 1;
+    }
+    const int width = cached ? p.ld_cache : nq;
+    to.step = width * (int)sizeof(T);
+    to.dst = reinterpret_cast<uint8_t*>((cached ? p.cache : p.q) + (size_t)(cached ? pos + m : m) * width + at);
+    if (cached) to.rows = p.max_seq - pos - m;
+    return to;
+}
+template <typename T>
+__device__ __forceinline__ ColumnPlace column_place(const LatentQueries<T>& p, int col, int m, int) {
+    const int at = p.dim + (p.dim & 1), width = at + p.rot, h = col / width, c = col - h * width;
+    ColumnPlace to;
+    const bool turned = c >= at;
+    if (turned) to.pair = (c - at) >> 1, to.second = (c - at) & 1;
+    const int ld = turned ? p.ld_rot : p.ld_nope;
+    to.step = p.heads * ld * (int)sizeof(T);
+    to.dst = reinterpret_cast<uint8_t*>((turned ? p.rotated : p.nope) + ((size_t)m * p.heads + h) * ld + (turned ? c - at : c));
+    if (!turned && c >= p.dim) to.rows = 0;
+    return to;
+}
+template <typename T>
+__device__ __forceinline__ int turned_pairs(const HeadRows<T>& p) {
+    return p.rot_pairs;
+}
+template <typename T>
+__device__ __forceinline__ int turned_pairs(const LatentQueries<T>& p) {
+    return p.rot >> 1;
+}
 
 // One direct copy global -> LDS of 16 bytes per lane: lane l's bytes land at lds_base + 16 l (lds_base uniform).
 __device__ __forceinline__ void copy16_to_lds(const void* global_src, void* lds_base) {

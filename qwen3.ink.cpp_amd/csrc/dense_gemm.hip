@@ -78,18 +78,39 @@ __device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, c
         }
         return;
     }
-    if constexpr (EPI == Epilogue::kHeads) {
-        // the column's place once, then the rows' angles all at a time
-        const HeadColumn<T> to(heads, min(col, g.N - 1));
+    if constexpr (EPI == Epilogue::kHeads || EPI == Epilogue::kQueries) {
+        // The column's place once, then, where the piece has columns that turn, the rows' angles all at a time; a piece without skips
+        // them, and rows follow by adding.  2048 x 3104 x 2048 with kHeads, 64 of 128 columns of a head turning: 51.5 us with an address
+        // for every element, 45.7 so.  4095 x 3072 x 768 with kQueries, 64 of 192: 38.7 us; in 32 bits first and turned by a launch of
+        // its own 32.6 + 21.5 us, with an address for every element no less than that.
         const int pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1);
+        const ColumnPlace to = column_place(heads, min(col, g.N - 1), m0 + r0, pos);
+        const bool turns = __any(to.pair >= 0);
         float cs[NV], sn[NV];
+        if (turns) {
+            const int pairs = turned_pairs(heads), own = max(to.pair, 0);
 #pragma unroll
-        for (int v = 0; v < NV; v++) to.angle(min(m0 + r0 + 8 * (v >> 2) + (v & 3), g.M - 1), pos, cs[v], sn[v]);
+            for (int v = 0; v < NV; v++) {
+                const unsigned i = __umul24(min(pos + m0 + r0 + 8 * (v >> 2) + (v & 3), heads.max_seq - 1), pairs) + own;
+                cs[v] = heads.cos_t[i], sn[v] = heads.sin_t[i];
+            }
+        }
+        uint8_t* dst = to.dst;
+        const int high = col < g.N ? min(rows - r0, to.rows) : 0;
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-            const int r = r0 + 8 * (v >> 2) + (v & 3);
-            const float other = swap_neighbours(x[v]);
-            if (r < rows && col < g.N) to.store(m0 + r, pos, x[v], other, cs[v], sn[v]);
+            if (v) dst += (v & 3) ? to.step : 5 * to.step;
+            float y = x[v];
+            if (turns) {
+                const float other = swap_neighbours(y), turned = to.second ? y * cs[v] + other * sn[v] : y * cs[v] - other * sn[v];
+                y = to.pair >= 0 ? turned : y;
+            }
+            if (8 * (v >> 2) + (v & 3) < high) {
+                if (to.as_float)
+                    *reinterpret_cast<float*>(dst) = y;
+                else
+                    *reinterpret_cast<T*>(dst) = (T)y;
+            }
         }
         return;
     }
@@ -112,7 +133,7 @@ __device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, c
 // Rows of tiles that are walked together: an XCD's workgroups then share these rows and a few column panels in its L2.
 constexpr int kBandRows = 2048;
 
-// X: HeadRows<T> with the epilogue kHeads, NoHeads with the others.  STAGES: how many steps LDS holds; all but one are under way.
+// X: HeadRows<T> with the epilogue kHeads, LatentQueries<T> with kQueries, NoHeads with the others.  STAGES: how many steps LDS holds; all but one are under way.
 // PIPE: a step's operands are read one 16-byte column ahead of their products, also into the next step: the waves meet before a step's
 // last products, whose operands are in registers by then, so that its stage is free for new copies and the next step's first
 // reads run beside those products.  4095 x 12288 x 2048, gated: 200.6 us with the meeting between two steps, 189.5 so (with the unit
@@ -447,7 +468,8 @@ hipError_t launch_dense_gemm(const GemmArgs& g, Epilogue epi, hipStream_t s) {
         case Epilogue::kElement: return launch_by_size<T, Epilogue::kElement>(g, NoHeads{}, s);
         case Epilogue::kGatedPair: return launch_by_size<T, Epilogue::kGatedPair>(g, NoHeads{}, s);
         case Epilogue::kHeadGate: return launch_by_size<T, Epilogue::kHeadGate>(g, NoHeads{}, s);
-        case Epilogue::kHeads: break;  // has a launcher of its own
+        case Epilogue::kHeads:
+        case Epilogue::kQueries: break;  // have launchers of their own
     }
     return hipErrorInvalidValue;
 }
@@ -455,9 +477,14 @@ template <typename T>
 hipError_t launch_dense_gemm_heads(const GemmArgs& g, const HeadRows<T>& heads, hipStream_t s) {
     return launch_by_size<T, Epilogue::kHeads>(g, heads, s);
 }
-#define INSTANTIATE(T)                                                              \
-    template hipError_t launch_dense_gemm<T>(const GemmArgs&, Epilogue, hipStream_t); \
-    template hipError_t launch_dense_gemm_heads<T>(const GemmArgs&, const HeadRows<T>&, hipStream_t);
+template <typename T>
+hipError_t launch_dense_gemm_queries(const GemmArgs& g, const LatentQueries<T>& q, hipStream_t s) {
+    return launch_by_size<T, Epilogue::kQueries>(g, q, s);
+}
+#define INSTANTIATE(T)                                                                                \
+    template hipError_t launch_dense_gemm<T>(const GemmArgs&, Epilogue, hipStream_t);                   \
+    template hipError_t launch_dense_gemm_heads<T>(const GemmArgs&, const HeadRows<T>&, hipStream_t); \
+    template hipError_t launch_dense_gemm_queries<T>(const GemmArgs&, const LatentQueries<T>&, hipStream_t);
 INSTANTIATE(bf16)
 INSTANTIATE(float)
 

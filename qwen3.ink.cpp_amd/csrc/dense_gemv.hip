@@ -246,7 +246,7 @@ struct HeadsEmit {
         store(2 * n, pos, s0, s1);
         if (2 * n + 1 < N) store(2 * n + 1, pos, s1, s0);
     }
-    // One column of one row, branch by branch; HeadColumn, which finds a place for many rows first, is slower here (rows of 4096, 772
+    // One column of one row, branch by branch; a place for many rows, as the products of more rows form it, is slower here (rows of 4096, 772
     // workgroups: 18.1 us, so 17.8).
     __device__ void store(int col, int pos, float own, float other) const {
         const HeadRows<T>& p = heads;
@@ -326,8 +326,8 @@ __global__ __launch_bounds__(kThreads) void gemv_query_kernel(LatentRows in, Lat
             const float* k = c + sh.rank;
             for (int i = t; i < half; i += kThreads) {
                 const float cs = in.cos_t[(size_t)p * half + i], sn = in.sin_t[(size_t)p * half + i];
-                dst[sh.rank + i] = (T)(k[i] * cs - k[i + half] * sn);
-                dst[sh.rank + half + i] = (T)(k[i + half] * cs + k[i] * sn);
+                dst[sh.rank + 2 * i] = (T)(k[2 * i] * cs - k[2 * i + 1] * sn);
+                dst[sh.rank + 2 * i + 1] = (T)(k[2 * i + 1] * cs + k[2 * i] * sn);
             }
         } else {
             const int i = extra * kThreads + t;
@@ -365,15 +365,15 @@ __global__ __launch_bounds__(kThreads) void gemv_absorb_kernel(const float* __re
                                                               const T* __restrict__ uk_t, int ld, T* __restrict__ q_lat) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     const int h = blockIdx.y, half = sh.rot >> 1;
-    const float* src = q + (size_t)h * (sh.dim + sh.rot);
+    const float *src = q + (size_t)h * sh.query_width(), *turned = src + sh.turned_at();
     T* dst = q_lat + (size_t)h * sh.ld_cache;
     if (blockIdx.x == 0) {
         const int p = min(max(in.pos_dev[0], 0), in.max_seq - 1);
         for (int j = threadIdx.x; j < half; j += kThreads) {
-            const float u = src[sh.dim + j], v = src[sh.dim + half + j];
+            const float u = turned[2 * j], v = turned[2 * j + 1];
             const float cs = in.cos_t[(size_t)p * half + j], sn = in.sin_t[(size_t)p * half + j];
-            dst[sh.rank + j] = (T)(u * cs - v * sn);
-            dst[sh.rank + half + j] = (T)(v * cs + u * sn);
+            dst[sh.rank + 2 * j] = (T)(u * cs - v * sn);
+            dst[sh.rank + 2 * j + 1] = (T)(v * cs + u * sn);
         }
     }
     const int N = sh.rank, chunks = ld * (int)sizeof(T) / 16, pairs = (N + 1) / 2;
@@ -816,7 +816,7 @@ hipError_t launch_gemv_plain(const float* x, int K, const T* w, int ld, int N, f
 template <typename T>
 hipError_t launch_gemv_query(const LatentRows& in, const LatentShape& sh, const T* w, int ld, float* q, T* cache, const DepthAverage& depth,
                              int width, float* before, hipStream_t s) {
-    const int N = sh.heads * (sh.dim + sh.rot), main_groups = workgroups<T>(N, ld, kMaxGrid);
+    const int N = sh.heads * sh.query_width(), main_groups = workgroups<T>(N, ld, kMaxGrid);
     const int extra = (cache ? 1 : 0) + (width + kThreads - 1) / kThreads;
     hipLaunchKernelGGL(gemv_query_kernel<T>, dim3(main_groups + extra), dim3(kThreads), (ld + kThreads / 64 + 1) * sizeof(float), s, in, sh,
                        w, ld, N, q, cache, depth, width, before, main_groups);

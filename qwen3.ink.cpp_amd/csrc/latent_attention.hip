@@ -28,32 +28,8 @@ __global__ __launch_bounds__(kThreads) void latent_rows_kernel(LatentRows in, La
     const float* k = c + sh.rank;
     for (int i = t; i < half; i += kThreads) {
         const float cs = in.cos_t[(size_t)p * half + i], sn = in.sin_t[(size_t)p * half + i];
-        dst[sh.rank + i] = (T)(k[i] * cs - k[i + half] * sn);
-        dst[sh.rank + half + i] = (T)(k[i + half] * cs + k[i] * sn);
-    }
-}
-
-// One workgroup per token.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void rotate_queries_kernel(const float* __restrict__ q, int ld_q, LatentRows in, LatentShape sh,
-                                                                 T* __restrict__ nope, int ld_nope, T* __restrict__ rot_out,
-                                                                 int ld_rot) {
-    const int m = blockIdx.x, t = threadIdx.x, half = sh.rot >> 1, per = sh.dim + half;
-    const int p = min(max(in.pos_dev[0] + m, 0), in.max_seq - 1);
-    const float* row = q + (size_t)m * ld_q;
-    for (int i = t; i < sh.heads * per; i += kThreads) {
-        const int h = i / per, d = i % per;
-        const float* src = row + h * (sh.dim + sh.rot);
-        const size_t o = (size_t)m * sh.heads + h;
-        if (d < sh.dim) {
-            nope[o * ld_nope + d] = (T)src[d];
-        } else {
-            const int j = d - sh.dim;
-            const float u = src[sh.dim + j], v = src[sh.dim + half + j];
-            const float cs = in.cos_t[(size_t)p * half + j], sn = in.sin_t[(size_t)p * half + j];
-            rot_out[o * ld_rot + j] = (T)(u * cs - v * sn);
-            rot_out[o * ld_rot + half + j] = (T)(v * cs + u * sn);
-        }
+        dst[sh.rank + 2 * i] = (T)(k[2 * i] * cs - k[2 * i + 1] * sn);
+        dst[sh.rank + 2 * i + 1] = (T)(k[2 * i + 1] * cs + k[2 * i] * sn);
     }
 }
 
@@ -65,18 +41,7 @@ hipError_t launch_latent_rows(const LatentRows& in, const LatentShape& sh, int M
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_rotate_queries(const float* q, int ld_q, const LatentRows& in, const LatentShape& sh, int M, T* nope, int ld_nope,
-                                 T* rot_out, int ld_rot, hipStream_t s) {
-    hipLaunchKernelGGL(rotate_queries_kernel<T>, dim3(M), dim3(kThreads), 0, s, q, ld_q, in, sh, nope, ld_nope, rot_out, ld_rot);
-    return hipGetLastError();
-}
-
-#define INSTANTIATE(T)                                                                                                           \
-    template hipError_t launch_latent_rows<T>(const LatentRows&, const LatentShape&, int, T*, int, T*, hipStream_t);               \
-    template hipError_t launch_rotate_queries<T>(const float*, int, const LatentRows&, const LatentShape&, int, T*, int, T*, int, \
-                                                 hipStream_t);
-INSTANTIATE(bf16)
-INSTANTIATE(float)
+template hipError_t launch_latent_rows<bf16>(const LatentRows&, const LatentShape&, int, bf16*, int, bf16*, hipStream_t);
+template hipError_t launch_latent_rows<float>(const LatentRows&, const LatentShape&, int, float*, int, float*, hipStream_t);
 
 }  // namespace a81w41

@@ -160,9 +160,12 @@ class TakosunModel final : public DenseModel<T> {
     long long state_step() const { return (long long)rows_ * cfg_.width; }
     GroupNorm norm(const float* w) const { return GroupNorm{w, cfg_.groups, cfg_.eps}; }
 
+    // The checkpoint's rotation turns component i with i + rot / 2; here the two are neighbours.
+    static int neighbours(int i, int rot) { return i < rot / 2 ? 2 * i : 2 * (i - rot / 2) + 1; }
     int load_weights(int max_seq, TensorSource& src);
     int allocate(int max_seq);
     int attention(const Layer& L, const LayerConfig& lc, int M, hipStream_t s);
+    int form_queries(const Layer& L, const LatentShape& sh, int M, T* nope, int ld_nope, T* rotated, int ld_rot, hipStream_t s);
     int attend_latent(const Layer& L, const LatentShape& sh, int M, hipStream_t s);
     int attend_formed(const Layer& L, const LatentShape& sh, int M, const float* gates, hipStream_t s);
     AttendArgs<T> shared_attend(const Layer& L, const LatentShape& sh, int M) const;
@@ -216,7 +219,10 @@ int TakosunModel<T>::load_weights(int max_seq, TensorSource& src) {
         Staging down(sh.q_rank + kv + sh.heads, width);
         A81W41_TRY(put_matrix(src, mix + "dq", sh.q_rank, width, down, 0));
         if (own) {
-            A81W41_TRY(put_matrix(src, mix + "dkv", kv, width, down, sh.q_rank));
+            std::vector<float> dkv;
+            A81W41_TRY(src.matrix(mix + "dkv", kv, width, dkv));
+            for (int r = 0; r < kv; r++)
+                down.put(sh.q_rank + (r < sh.rank ? r : sh.rank + neighbours(r - sh.rank, sh.rot)), dkv.data() + (size_t)r * width);
             A81W41_TRY(load_vector(src, mix + "dkv.norm", sh.rank, &L.kv_norm));
             void* plane = nullptr;
             A81W41_TRY(cache.add((size_t)max_seq * sh.ld_cache * sizeof(T), &plane));
@@ -227,7 +233,17 @@ int TakosunModel<T>::load_weights(int max_seq, TensorSource& src) {
         A81W41_TRY(put_matrix(src, mix + "g", sh.heads, width, down, sh.q_rank + kv));
         A81W41_TRY(finish(down, &L.down));
         A81W41_TRY(load_rotation(sh.rot, lc.rot_base, max_seq, &L.cos_t, &L.sin_t));
-        A81W41_TRY(load_matrix(src, mix + "uq", sh.heads * (sh.dim + sh.rot), sh.q_rank, &L.uq));
+        {   // queries head by head, the rotated part from an even column on
+            const int stored = sh.dim + sh.rot;
+            std::vector<float> uq;
+            A81W41_TRY(src.matrix(mix + "uq", sh.heads * stored, sh.q_rank, uq));
+            Staging st(sh.heads * sh.query_width(), sh.q_rank);
+            for (int r = 0; r < sh.heads * stored; r++) {
+                const int h = r / stored, d = r % stored;
+                st.put(h * sh.query_width() + (d < sh.dim ? d : sh.turned_at() + neighbours(d - sh.dim, sh.rot)), uq.data() + (size_t)r * sh.q_rank);
+            }
+            A81W41_TRY(finish(st, &L.uq));
+        }
         {   // the key up-projection of a head, transposed: it maps an unrotated query to latent space
             std::vector<float> uk, row(sh.dim);
             A81W41_TRY(src.matrix(mix + "uk", sh.heads * sh.dim, sh.rank, uk));
@@ -277,7 +293,7 @@ int TakosunModel<T>::allocate(int max_seq) {
     for (const LayerConfig& lc : cfg_.layers) {
         const LatentShape& sh = lc.mix;
         ld_down_ = std::max(ld_down_, sh.q_rank + sh.rank + sh.rot + sh.heads);
-        ld_q_ = std::max(ld_q_, sh.heads * (sh.dim + sh.rot));
+        ld_q_ = std::max(ld_q_, sh.heads * sh.query_width());
         ld_cq_ = std::max(ld_cq_, pad_k<T>(sh.q_rank));
         ld_attn_ = std::max(ld_attn_, pad_k<T>(sh.heads * sh.vdim));
         nope = std::max(nope, (size_t)sh.heads * pad_k<T>(sh.dim));
@@ -308,7 +324,7 @@ int TakosunModel<T>::allocate(int max_seq) {
     A81W41_TRY(allocate_array((size_t)(n_layers() + 1) * R * W, &states_));
     A81W41_TRY(allocate_array(R * ld_h_, &h_));
     A81W41_TRY(allocate_array(R * ld_down_, &down_));
-    A81W41_TRY(allocate_array(R * ld_q_, &q_));
+    A81W41_TRY(allocate_array((size_t)ld_q_, &q_));
     A81W41_TRY(allocate_array(R * ld_cq_, &c_q_));
     A81W41_TRY(allocate_array(R * nope, &nope_));
     A81W41_TRY(allocate_array(R * q_lat, &q_lat_));
@@ -362,13 +378,22 @@ AttendArgs<T> TakosunModel<T>::shared_attend(const Layer& L, const LatentShape& 
     return a;
 }
 
+// Queries of M tokens from their normed latents in c_q_, the unrotated and the rotated parts where the attention wants them.
+template <typename T>
+int TakosunModel<T>::form_queries(const Layer& L, const LatentShape& sh, int M, T* nope, int ld_nope, T* rotated, int ld_rot, hipStream_t s) {
+    LatentQueries<T> q;
+    q.heads = sh.heads, q.dim = sh.dim, q.rot = sh.rot, q.nope = nope, q.ld_nope = ld_nope, q.rotated = rotated, q.ld_rot = ld_rot;
+    q.cos_t = L.cos_t, q.sin_t = L.sin_t, q.pos_dev = pos, q.max_seq = max_seq();
+    A81W41_HIP_TRY(launch_dense_gemm_queries<T>(product(c_q_, ld_cq_, L.uq, nullptr, 0, M), q, s));
+    return 0;
+}
+
 // Attention in latent space: the key up-projection moves into the query, the value up-projection behind the sum.
 // Leaves the weighted latents in o_lat_.
 template <typename T>
 int TakosunModel<T>::attend_latent(const Layer& L, const LatentShape& sh, int M, hipStream_t s) {
-    const LatentRows in = latent_rows(L);
     const int ld_nope = pad_k<T>(sh.dim), ld_rank = pad_k<T>(sh.rank);
-    A81W41_HIP_TRY(launch_rotate_queries<T>(q_, ld_q_, in, sh, M, nope_, ld_nope, q_lat_ + sh.rank, sh.ld_cache, s));
+    A81W41_TRY(form_queries(L, sh, M, nope_, ld_nope, q_lat_ + sh.rank, sh.ld_cache, s));
     GemmArgs g = product(nope_, sh.heads * ld_nope, L.uk_t, q_lat_, sh.heads * sh.ld_cache, M);
     g.N = sh.rank, g.batches = sh.heads, g.a_step = ld_nope, g.w_step = (long long)sh.rank * L.uk_t.ld, g.c_step = sh.ld_cache;
     A81W41_HIP_TRY(launch_dense_gemm<T>(g, Epilogue::kElement, s));
@@ -401,7 +426,7 @@ int TakosunModel<T>::attend_formed(const Layer& L, const LatentShape& sh, int M,
         g.A = L.uv.data, g.lda = L.uv.ld, g.M = L.uv.rows, g.W = L.cache, g.ldw = sh.ld_cache, g.N = ctx, g.K = L.uv.ld;
         g.C = v_formed_, g.ldc = ld_v_;
         A81W41_HIP_TRY(launch_dense_gemm<T>(g, Epilogue::kElement, s));
-        A81W41_HIP_TRY(launch_rotate_queries<T>(q_, ld_q_, latent_rows(L), sh, M, nope_, dk, nope_ + sh.dim, dk, s));
+        A81W41_TRY(form_queries(L, sh, M, nope_, dk, nope_ + sh.dim, dk, s));
         AttendArgs<T> a;
         a.q = nope_, a.q_head = dk, a.q_token = sh.heads * dk, a.rows = M;
         a.k_own = k_formed_, a.k_own_head = sh.dim, a.ld_k_own = sh.heads * sh.dim, a.k_own_width = sh.dim;
@@ -423,7 +448,6 @@ int TakosunModel<T>::attention(const Layer& L, const LayerConfig& lc, int M, hip
     const float* gates = down_ + sh.q_rank + (own ? sh.rank + sh.rot : 0);
     A81W41_HIP_TRY(launch_dense_gemm<T>(product(h_, ld_h_, L.down, down_, ld_down_, M), Epilogue::kFloat, s));
     A81W41_HIP_TRY(launch_latent_rows<T>(latent_rows(L), sh, M, c_q_, ld_cq_, own ? L.cache : nullptr, s));
-    A81W41_HIP_TRY(launch_dense_gemm<T>(product(c_q_, ld_cq_, L.uq, q_, ld_q_, M), Epilogue::kFloat, s));
     // per key and head, latent space costs M (2 rank + rot) against M (dim + rot + vdim) and rank (dim + vdim) once
     const bool many = (long long)M * (2 * sh.rank - sh.dim - sh.vdim) > (long long)sh.rank * (sh.dim + sh.vdim);
     if (can_expand(sh) && (opt_attention_ == 3 || (opt_attention_ == 0 && many))) {

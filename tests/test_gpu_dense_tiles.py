@@ -284,3 +284,10 @@ def test_gated_units_of_large_gates(pkg, tmp_path):
         got = pkg.Model.load(str(tmp_path), 64, dtype).forward(ids, range(40))
         err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
         assert err.max() <= tol, (dtype, err.max())
+
+
+# queries turned and stored by the product: heads of an odd and of an even width, on 256 x 256 and 128 x 128 tiles and on small ones
+@pytest.mark.parametrize("heads,dim,rot", [(41, 95, 62), (40, 96, 64), (9, 33, 2)])
+def test_query_columns_on_large_tiles(pkg, heads, dim, rot):
+    cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(heads, dim, rot, 8, 70, 24, 0.1), None)])
+    _same_in_portions(pkg, cfg, 2100, 100)
