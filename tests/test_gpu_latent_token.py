@@ -46,3 +46,14 @@ def test_rows_behind_the_token_do_not_count(pkg, tmp_path):
     model.forward(np.full(30, 66, np.int32))  # leaves rows that are no numbers
     model.reset()
     _close(np.concatenate([model.forward(ids[i:i + 1]) for i in range(20)]), oracle.forward(ids), "stale rows")
+
+
+@pytest.mark.parametrize("q_rank", [4, 30, 2048, 2052])  # held by the threads: least, no whole float4s, most, one more
+@pytest.mark.parametrize("heads,rank,rot", [(2, 24, 6), (1, 30, 2)])
+def test_latents_held_and_not(pkg, tmp_path, q_rank, heads, rank, rot):
+    cfg = config(67, 64, 2, [layer(mixer(heads, 16, rot, 8, q_rank, rank, 0.25), dense(40)) for _ in range(3)])
+    w = tf.random_weights(cfg, 43)
+    write_model(str(tmp_path), cfg, w)
+    model, oracle = pkg.Model.load(str(tmp_path), 64, "bfloat16"), tf.TakosunOracle(cfg, w)
+    ids = np.random.default_rng(q_rank).integers(0, 67, 9).astype(np.int32)
+    _close(np.concatenate([model.forward(ids[:3])] + [model.forward(ids[i:i + 1]) for i in range(3, 9)]), oracle.forward(ids)[2:], q_rank)
