@@ -148,6 +148,7 @@ class StepRow {
     __device__ __forceinline__ explicit StepRow(const RowStep& p) : p_(p), parts_(p.width, p.norm_h.groups, threadIdx.x), fast_(parts_.fits()) {}
     __device__ __forceinline__ void load() {
         if (!fast_) return;
+        if (p_.before && p_.coef) coef_ = *p_.coef;
         // Without a branch a load: a thread without a part takes the row's first one and drops it.  A Takosun token, 16 such rows of 2048:
         // 254.6 us with a branch each, 249.2 so.
         auto part = [&](const float* a, int i) { return load4(a + max(i, 0)); };
@@ -176,7 +177,7 @@ class StepRow {
     __device__ __forceinline__ void finish(float* xs, int padded, float* inv, float* red) {
         if (!fast_) return slow(xs, padded, inv, red);
         const bool writer = blockIdx.x == 0 && blockIdx.y == 0;
-        const float coef = p_.before && p_.coef ? *p_.coef : 1.f;
+        const float coef = coef_;
         const bool normed = p_.y && p_.norm_y.w;
         const float inv_y = normed ? parts_.inverse_rms(y_, p_.norm_y.eps, red) : 0.f;
 #pragma unroll
@@ -234,6 +235,7 @@ class StepRow {
     const RowStep& p_;
     RowParts<kThreads, PARTS> parts_;
     bool fast_;
+    float coef_ = 1.f;
     float4 x_[kParts], y_[kParts], wy_[kParts], before_[kParts], wh_[kParts];
 };
 
@@ -274,10 +276,22 @@ struct HeadsEmit {
     }
 };
 
+// What a workgroup's first requests are made of stands ahead of the structs in the kernels' arguments: 14 leading dwords of scalars come with
+// the dispatch, the others with a load that the requests would wait for.  us a token behind a short prompt with the structs first / so:
+// Takosun, four layers, width 2048 241.5 / 234.6, 4096 480 / 465; Dimesun, two layers run twice, width 1024 151 / 145.  A launch of 784 rows
+// of 2048 behind a residual step 6.6 / 5.8 us, of which the mean's coefficient, asked for only behind the row, is a part.
+__device__ __forceinline__ void with_leading(RowStep& p, const float* x, const float* norm_h, const float* y, const float* norm_y, int width, int groups) {
+    p.x = x, p.norm_h.w = norm_h, p.y = y, p.norm_y.w = norm_y, p.width = width, p.norm_h.groups = groups;
+}
+#define LEADING_OF(p) (p).x, (p).norm_h.w, (p).y, (p).norm_y.w
+
 // emit gets W[n] . row, in pairs of n
 template <typename T, int PARTS, typename Emit>
-__global__ __launch_bounds__(kThreads) void gemv_step_kernel(RowStep p, const T* __restrict__ w, int ld, int N, Emit emit) {
+__global__ __launch_bounds__(kThreads) void gemv_step_kernel(const float* __restrict__ x, const float* __restrict__ norm_h, const float* __restrict__ y,
+                                                            const float* __restrict__ norm_y, const T* __restrict__ w, int width, int groups, int ld,
+                                                            int N, RowStep p, Emit emit) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    with_leading(p, x, norm_h, y, norm_y, width, groups);
     float *xs = smem, *red = xs + ld, *inv = red + kThreads / 64;
     StepRow<PARTS> row(p);
     row.load();
@@ -350,10 +364,12 @@ class NormedLatent {
 // Queries from their normed latent.  The last workgroups of the launch do other work of the same stage: one appends the
 // token's cache row, the others sum the states of the layers so far for the mean over depth.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void gemv_query_kernel(LatentRows in, LatentShape sh, const T* __restrict__ w, int ld, int N,
-                                                             float* __restrict__ q, T* __restrict__ cache, DepthAverage depth,
-                                                             int width, float* __restrict__ before, int main_groups) {
+__global__ __launch_bounds__(kThreads) void gemv_query_kernel(const float* __restrict__ down, const float* __restrict__ q_norm, const T* __restrict__ w,
+                                                             int q_rank, int ld, int N, int main_groups, float* __restrict__ q,
+                                                             T* __restrict__ cache, LatentRows in, LatentShape sh, DepthAverage depth, int width,
+                                                             float* __restrict__ before) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    in.down = down, in.q_norm = q_norm, sh.q_rank = q_rank;
     float *xs = smem, *red = xs + ld, *inv = red + kThreads / 64;
     const int t = threadIdx.x;
     if ((int)blockIdx.x >= main_groups) {
@@ -432,12 +448,19 @@ __global__ __launch_bounds__(kThreads) void gemv_query_kernel(LatentRows in, Lat
 // Query rows in latent space, one head per blockIdx.y: columns 0..rank from the unrotated part through the transposed key
 // up-projection, then the rotated part (first workgroup of the head).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void gemv_absorb_kernel(const float* __restrict__ q, LatentRows in, LatentShape sh,
-                                                              const T* __restrict__ uk_t, int ld, T* __restrict__ q_lat) {
+__global__ __launch_bounds__(kThreads) void gemv_absorb_kernel(const float* __restrict__ q, const T* __restrict__ uk_t, int ld, int rank, int dim, int rot,
+                                                              T* __restrict__ q_lat, const int* __restrict__ pos_dev, LatentRows in, LatentShape sh) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    in.pos_dev = pos_dev, sh.rank = rank, sh.dim = dim, sh.rot = rot;
     const int h = blockIdx.y, half = sh.rot >> 1;
     const float *src = q + (size_t)h * sh.query_width(), *turned = src + sh.turned_at();
     T* dst = q_lat + (size_t)h * sh.ld_cache;
+    const int N = sh.rank, chunks = ld * (int)sizeof(T) / 16, pairs = (N + 1) / 2;
+    const Deal d = deal_rows<T>(chunks, gridDim.x);
+    const PlainRows<T> rows{uk_t + (size_t)h * N * ld, ld, N};
+    Pair ahead;
+    request_first(ahead, rows, pairs, chunks, d);
+    copy_row(smem, src, sh.dim, ld);
     if (blockIdx.x == 0) {
         const int p = min(max(in.pos_dev[0], 0), in.max_seq - 1);
         for (int j = threadIdx.x; j < half; j += kThreads) {
@@ -447,12 +470,6 @@ __global__ __launch_bounds__(kThreads) void gemv_absorb_kernel(const float* __re
             dst[sh.rank + 2 * j + 1] = (T)(v * cs + u * sn);
         }
     }
-    const int N = sh.rank, chunks = ld * (int)sizeof(T) / 16, pairs = (N + 1) / 2;
-    const Deal d = deal_rows<T>(chunks, gridDim.x);
-    const PlainRows<T> rows{uk_t + (size_t)h * N * ld, ld, N};
-    Pair ahead;
-    request_first(ahead, rows, pairs, chunks, d);
-    copy_row(smem, src, sh.dim, ld);
     dense_lds_barrier();
     stream_pairs<T>(
         ahead, rows,
@@ -555,9 +572,8 @@ __device__ __forceinline__ void choose_experts(const ExpertRows& e, float* z, in
 
 // act = unit(gate, up) for the token's experts (blockIdx.y < top) and the dense or shared feed-forward (the last).
 template <typename T, int PARTS>
-__global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(RowStep p, const float* __restrict__ h, ExpertRows e,
-                                                               const T* __restrict__ experts, const T* __restrict__ dense, int ld,
-                                                               float* __restrict__ act) {
+__device__ __forceinline__ void gate_up(const RowStep& p, const float* __restrict__ h, const ExpertRows& e, const T* __restrict__ experts,
+                                        const T* __restrict__ dense, int ld, float* __restrict__ act) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     __shared__ int ids[kMaxTop];
     __shared__ float best[kMaxTop];
@@ -587,12 +603,30 @@ __global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(RowStep p, const
     stream_pairs<T>(ahead, rows, [&](int j, float gate, float up) { dst[j] = gated_unit(e.unit, gate, up); }, ff, xs, chunks, d);
 }
 
+// Behind a residual step, and on a row that is normed already.
+template <typename T, int PARTS>
+__global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(const float* __restrict__ x, const float* __restrict__ norm_h, const float* __restrict__ y,
+                                                               const float* __restrict__ norm_y, const T* __restrict__ dense, int width, int groups,
+                                                               int ld, int top, RowStep p, ExpertRows e, const T* __restrict__ experts,
+                                                               float* __restrict__ act) {
+    with_leading(p, x, norm_h, y, norm_y, width, groups);
+    e.top = top;
+    gate_up<T, PARTS>(p, nullptr, e, experts, dense, ld, act);
+}
+template <typename T>
+__global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(const float* __restrict__ logits, const float* __restrict__ bias, const float* __restrict__ h,
+                                                               const T* __restrict__ experts, int routed, int top, int ld, int width, RowStep p,
+                                                               ExpertRows e, const T* __restrict__ dense, float* __restrict__ act) {
+    e.logits = logits, e.bias = bias, e.experts = routed, e.top = top, p.width = width;
+    gate_up<T, 4>(p, h, e, experts, dense, ld, act);
+}
+
 // y[n] = mean over the token's experts of W_e[n] . act_e, plus the dense or shared feed-forward's.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void gemv_ff_down_kernel(ExpertRows e, const float* __restrict__ act, const T* __restrict__ experts,
-                                                               int ld, const T* __restrict__ dense, int ld_dense, int N,
-                                                               float* __restrict__ y) {
+__global__ __launch_bounds__(kThreads) void gemv_ff_down_kernel(const float* __restrict__ act, const T* __restrict__ dense, const T* __restrict__ experts,
+                                                               int dense_ff, int ld_dense, int top, int ld, int N, float* __restrict__ y, ExpertRows e) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    e.dense_ff = dense_ff, e.top = top;
     __shared__ int chosen[64];
     const int chunks = ld * (int)sizeof(T) / 16, chunks_dense = ld_dense * (int)sizeof(T) / 16, pairs = (N + 1) / 2;
     float* xs_dense = smem + e.top * ld;
@@ -761,10 +795,16 @@ class MixerPrologue {
 // y[n] = W_o[n] . mixer row + sum_k weights[k] W_e(k)[n] . act_k, as one row of W_o's and the chosen experts' chunks in turn;
 // the experts' weights are in the activations.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void gemv_mixer_down_kernel(MixerRow m, const T* __restrict__ wo, int ld_wo, ExpertRows e,
-                                                                  const float* __restrict__ act, const T* __restrict__ experts, int ld,
-                                                                  int N, float* __restrict__ y) {
+__global__ __launch_bounds__(kThreads) void gemv_mixer_down_kernel(const T* __restrict__ wo, const float* __restrict__ row_or_part,
+                                                                  const float* __restrict__ stats, const T* __restrict__ experts,
+                                                                  const int* __restrict__ picked, int ld_wo, int top, int ld, int N,
+                                                                  const float* __restrict__ act, float* __restrict__ y, MixerRow m, ExpertRows e) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    if (stats)
+        m.shares.part = row_or_part, m.shares.stats = stats;
+    else
+        m.row = row_or_part, m.shares.part = nullptr;
+    e.chosen = const_cast<int*>(picked), e.top = top;
     __shared__ int chosen[kMaxTop];
     const int t = threadIdx.x;
     const int chunks = ld * (int)sizeof(T) / 16, chunks_wo = ld_wo * (int)sizeof(T) / 16, all = chunks_wo + e.top * chunks;
@@ -863,9 +903,9 @@ template <typename T, typename Emit>
 hipError_t launch_step(const RowStep& p, const T* w, int ld, int N, const Emit& emit, hipStream_t s) {
     const dim3 grid(workgroups<T>(N, ld, kMaxGrid)), threads(kThreads);
     if (fits_two_parts(p))
-        hipLaunchKernelGGL((gemv_step_kernel<T, 2, Emit>), grid, threads, step_lds(ld, p), s, p, w, ld, N, emit);
+        hipLaunchKernelGGL((gemv_step_kernel<T, 2, Emit>), grid, threads, step_lds(ld, p), s, LEADING_OF(p), w, p.width, p.norm_h.groups, ld, N, p, emit);
     else
-        hipLaunchKernelGGL((gemv_step_kernel<T, 4, Emit>), grid, threads, step_lds(ld, p), s, p, w, ld, N, emit);
+        hipLaunchKernelGGL((gemv_step_kernel<T, 4, Emit>), grid, threads, step_lds(ld, p), s, LEADING_OF(p), w, p.width, p.norm_h.groups, ld, N, p, emit);
     return hipGetLastError();
 }
 
@@ -889,14 +929,14 @@ hipError_t launch_gemv_query(const LatentRows& in, const LatentShape& sh, const 
                              int width, float* before, hipStream_t s) {
     const int N = sh.heads * sh.query_width(), main_groups = workgroups<T>(N, ld, kMaxGrid);
     const int extra = (cache ? 1 : 0) + (width + kThreads - 1) / kThreads;
-    hipLaunchKernelGGL(gemv_query_kernel<T>, dim3(main_groups + extra), dim3(kThreads), (ld + kThreads / 64 + 1) * sizeof(float), s, in, sh,
-                       w, ld, N, q, cache, depth, width, before, main_groups);
+    hipLaunchKernelGGL(gemv_query_kernel<T>, dim3(main_groups + extra), dim3(kThreads), (ld + kThreads / 64 + 1) * sizeof(float), s, in.down,
+                       in.q_norm, w, sh.q_rank, ld, N, main_groups, q, cache, in, sh, depth, width, before);
     return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_gemv_absorb(const float* q, const LatentRows& in, const LatentShape& sh, const T* uk_t, int ld, T* q_lat, hipStream_t s) {
-    hipLaunchKernelGGL(gemv_absorb_kernel<T>, dim3(workgroups<T>(sh.rank, ld, 64), sh.heads), dim3(kThreads), ld * sizeof(float), s, q, in,
-                       sh, uk_t, ld, q_lat);
+    hipLaunchKernelGGL(gemv_absorb_kernel<T>, dim3(workgroups<T>(sh.rank, ld, 64), sh.heads), dim3(kThreads), ld * sizeof(float), s, q, uk_t,
+                       ld, sh.rank, sh.dim, sh.rot, q_lat, in.pos_dev, in, sh);
     return hipGetLastError();
 }
 template <typename T>
@@ -921,18 +961,20 @@ hipError_t launch_gemv_gate_up(const RowStep& p, const float* h, const ExpertRow
     // A row that is already normed is held in no parts: the workgroups that stream behind a router are two a CU, and the larger form
     // has the registers they want.  Dimesun, a token: rows of 4096 416 us with the smaller form and 413 with the larger, 2048 both 197,
     // 1536 167.0 and 166.3, 1024 133.5 and 133.1.
-    if (!h && fits_two_parts(p))
-        hipLaunchKernelGGL((gemv_gate_up_kernel<T, 2>), grid, threads, bytes, s, p, h, e, experts, dense, ld, act);
+    if (h)
+        hipLaunchKernelGGL(gemv_gate_up_kernel<T>, grid, threads, bytes, s, e.logits, e.bias, h, experts, e.experts, e.top, ld, p.width, p, e, dense, act);
+    else if (fits_two_parts(p))
+        hipLaunchKernelGGL((gemv_gate_up_kernel<T, 2>), grid, threads, bytes, s, LEADING_OF(p), dense, p.width, p.norm_h.groups, ld, e.top, p, e, experts, act);
     else
-        hipLaunchKernelGGL((gemv_gate_up_kernel<T, 4>), grid, threads, bytes, s, p, h, e, experts, dense, ld, act);
+        hipLaunchKernelGGL((gemv_gate_up_kernel<T, 4>), grid, threads, bytes, s, LEADING_OF(p), dense, p.width, p.norm_h.groups, ld, e.top, p, e, experts, act);
     return hipGetLastError();
 }
 template <typename T>
 hipError_t launch_gemv_ff_down(const ExpertRows& e, const float* act, const T* experts, int ld, const T* dense, int ld_dense, int N,
                                float* y, hipStream_t s) {
     const size_t lds = ((size_t)e.top * ld + (e.dense_ff ? ld_dense : 0)) * sizeof(float);
-    hipLaunchKernelGGL(gemv_ff_down_kernel<T>, dim3(workgroups<T>(N, e.dense_ff ? ld_dense : ld, kMaxGrid)), dim3(kThreads), lds, s, e, act,
-                       experts, ld, dense, ld_dense, N, y);
+    hipLaunchKernelGGL(gemv_ff_down_kernel<T>, dim3(workgroups<T>(N, e.dense_ff ? ld_dense : ld, kMaxGrid)), dim3(kThreads), lds, s, act,
+                       dense, experts, e.dense_ff, ld_dense, e.top, ld, N, y, e);
     return hipGetLastError();
 }
 
@@ -941,8 +983,8 @@ hipError_t launch_gemv_mixer_down(const MixerRow& m, const T* wo, int ld_wo, con
                                   int ld, int N, float* y, hipStream_t s) {
     const int row = ld_wo + e.top * ld, inv = m.shares.part ? m.heads * kMixerShares : m.heads;
     const size_t lds = (row + kThreads / 64 + inv) * sizeof(float);
-    hipLaunchKernelGGL(gemv_mixer_down_kernel<T>, dim3(workgroups<T>(N, row, kMaxGrid)), dim3(kThreads), lds, s, m, wo, ld_wo, e, act,
-                       experts, ld, N, y);
+    hipLaunchKernelGGL(gemv_mixer_down_kernel<T>, dim3(workgroups<T>(N, row, kMaxGrid)), dim3(kThreads), lds, s, wo,
+                       m.shares.part ? m.shares.part : m.row, m.shares.part ? m.shares.stats : nullptr, experts, e.chosen, ld_wo, e.top, ld, N, act, y, m, e);
     return hipGetLastError();
 }
 
