@@ -247,4 +247,8 @@ hipError_t launch_attention_one_token_split(const float* qkv, int n_q, int n_kv,
 hipError_t launch_silu_mul(const float* gate_up, float* out, int M, int inter, hipStream_t s);
 // silu(gate) * up as 80 B activation blocks of the [M][inter] result.  inter % 64 == 0, gate_up 16-byte aligned.
 hipError_t launch_silu_mul_quant(const float* gate_up, void* q_out, int M, int inter, hipStream_t s);
+// The last two into the block-scaled kernel's rows (A6).
+hipError_t launch_add_rmsnorm_a6(const float* x, const float* res_in, const float* w, float* res_out, void* a6, int M, int hidden,
+                                 float eps, hipStream_t s);
+hipError_t launch_silu_mul_a6(const float* gate_up, void* a6, int M, int inter, hipStream_t s);
 }  // namespace a81w41

@@ -126,15 +126,26 @@ int a81w41_qwen3::enqueue_pass(int M, const int* want, int n_want, hipStream_t s
     const bool quant_fused = M > 1 && prefill_fusion_usable(m);
     void* scratch = a81w41_context_activation_scratch_dev(m->ctx);
     const a81w41::GemmScratch& gws = a81w41::context_gemm_scratch(m->ctx);
-    // the contraction of rows that sit in the scratch as 80 B blocks: where the layer picks the block-scaled
-    // kernel, that one takes them in its own operand format
+    // Where a layer picks the block-scaled kernel, that one takes rows in its own operand format: the norms and SiLU*mul write it,
+    // the attention's blocks are converted.
+    void* a6 = a81w41::context_a6_scratch(m->ctx);
+    auto gemm_from_a6 = [&](a81w41_linear* lin, float* out, int N, int K) {
+        return a81w41::launch_gemm_fp6(a6, a81w41::linear_w6(lin), out, M, N, K, gws, s);
+    };
     auto gemm_from_scratch = [&](a81w41_linear* lin, float* out, int N, int K) -> hipError_t {
         if (a81w41::linear_block_scaled(lin, M)) {
-            void* a6 = a81w41::context_a6_scratch(m->ctx);
             if (hipError_t e = a81w41::launch_a80_to_a6(scratch, a6, M, K, s); e != hipSuccess) return e;
-            return a81w41::launch_gemm_fp6(a6, a81w41::linear_w6(lin), out, M, N, K, gws, s);
+            return gemm_from_a6(lin, out, N, K);
         }
         return a81w41::launch_gemm_fp32(scratch, a81w41_linear_weight_fp32_dev(lin), out, M, N, K, gws, s);
+    };
+    auto norm_and_gemm = [&](const float* x, const float* res, const float* w, a81w41_linear* lin, float* out, int N) -> hipError_t {
+        if (a81w41::linear_block_scaled(lin, M)) {
+            if (hipError_t e = a81w41::launch_add_rmsnorm_a6(x, res, w, m->x, a6, M, c.hidden, c.rms_eps, s); e != hipSuccess) return e;
+            return gemm_from_a6(lin, out, N, c.hidden);
+        }
+        if (hipError_t e = a81w41::launch_add_rmsnorm_quant(x, res, w, m->x, scratch, M, c.hidden, c.rms_eps, s); e != hipSuccess) return e;
+        return gemm_from_scratch(lin, out, N, c.hidden);
     };
     const bool attn_blocks = !m->opt_vector_attention && a81w41::attention_prefill_fits(M, c.n_q_heads, c.n_kv_heads);
     for (int l = 0; l < c.n_layers; l++) {
@@ -142,8 +153,7 @@ int a81w41_qwen3::enqueue_pass(int M, const int* want, int n_want, hipStream_t s
         const float* norm_in = pending ? pending : m->x;
         const float* norm_res = pending ? m->x : nullptr;
         if (quant_fused) {
-            Q_HIP(a81w41::launch_add_rmsnorm_quant(norm_in, norm_res, L.norm[0], m->x, scratch, M, c.hidden, c.rms_eps, s));
-            Q_HIP(gemm_from_scratch(L.lin[0], m->qkv, qkv_dim, c.hidden));
+            Q_HIP(norm_and_gemm(norm_in, norm_res, L.norm[0], L.lin[0], m->qkv, qkv_dim));
         } else {
             Q_HIP(a81w41::launch_add_rmsnorm(norm_in, norm_res, L.norm[0], m->x, m->h, M, c.hidden, c.rms_eps, s));
             Q_TRY(a81w41_linear_forward(L.lin[0], m->h, M, m->qkv, s));
@@ -160,10 +170,14 @@ int a81w41_qwen3::enqueue_pass(int M, const int* want, int n_want, hipStream_t s
             Q_TRY(a81w41_linear_forward(L.lin[1], m->attn, M, m->o, s));
         }
         if (quant_fused) {
-            Q_HIP(a81w41::launch_add_rmsnorm_quant(m->o, m->x, L.norm[1], m->x, scratch, M, c.hidden, c.rms_eps, s));
-            Q_HIP(gemm_from_scratch(L.lin[2], m->gate_up, 2 * c.intermediate, c.hidden));
-            Q_HIP(a81w41::launch_silu_mul_quant(m->gate_up, scratch, M, c.intermediate, s));
-            Q_HIP(gemm_from_scratch(L.lin[3], m->o, c.hidden, c.intermediate));
+            Q_HIP(norm_and_gemm(m->o, m->x, L.norm[1], L.lin[2], m->gate_up, 2 * c.intermediate));
+            if (a81w41::linear_block_scaled(L.lin[3], M)) {
+                Q_HIP(a81w41::launch_silu_mul_a6(m->gate_up, a6, M, c.intermediate, s));
+                Q_HIP(gemm_from_a6(L.lin[3], m->o, c.hidden, c.intermediate));
+            } else {
+                Q_HIP(a81w41::launch_silu_mul_quant(m->gate_up, scratch, M, c.intermediate, s));
+                Q_HIP(gemm_from_scratch(L.lin[3], m->o, c.hidden, c.intermediate));
+            }
         } else {
             Q_HIP(a81w41::launch_add_rmsnorm(m->o, m->x, L.norm[1], m->x, m->h, M, c.hidden, c.rms_eps, s));
             Q_TRY(a81w41_linear_forward(L.lin[2], m->h, M, m->gate_up, s));

@@ -14,6 +14,7 @@
 //                           activation quantiser of the linear that consumes the row
 //                           (quantize_row_q8_1_repack_fp32, quantized_gemx_kernels.cc:803-911), so the
 //                           fp32 row never goes to memory; the blocks are bit-identical to quantising it
+#include "a6_blocks.h"
 #include "a81w41_kernels.h"
 #include "quantize_common.h"
 
@@ -64,18 +65,31 @@ __device__ __forceinline__ void store_quantized_float4(uint8_t* __restrict__ blo
     }
 }
 
+// The same into A6, float4 j of row `row` of n4: rows as the block-scaled contraction reads them.  By way of 80 B blocks they took another
+// launch and another trip to memory: 322 rows, the norm of 4096 and silu * up of 12288 7.3 + 5.6 and 8.0 + 8.4 us, so 9.8 and 13.0.
+__device__ __forceinline__ void store_a6_float4(uint8_t* __restrict__ a6, int row, int j, int n4, float4 v) {
+    const Quant4 qz = quantize_float4_of_block32(v);
+    fp6::store_a6_block(a6, row, j >> 3, n4 >> 3, qz.packed, qz.d, qz.ssum, threadIdx.x & 63);
+}
+
+enum class RowsAs { kFloats, kBlocks, kA6 };
+
 // res_out = x + res_in (res_in may be null: res_out = x); norm_out = res_out / sqrt(mean(res_out^2) + eps) * w
 // (res_out may be the same buffer as x or res_in: every element is read and written by one thread).
 // One workgroup per row; a thread keeps up to 4 float4 of the row in registers (hidden <= 16 * THREADS),
-// longer rows are re-read from res_out.  With QUANT the normalised row is written as 80 B blocks to
-// q_out instead of as floats to norm_out.
-template <int THREADS, bool QUANT>
+// longer rows are re-read from res_out.  The normalised row is written as floats to norm_out, or as 80 B blocks or
+// A6 to q_out; A6 has whole panels, in which the rows from M on are zero.
+template <int THREADS, RowsAs AS>
 __global__ __launch_bounds__(THREADS) void add_rmsnorm_kernel(const float* x, const float* res_in, const float* __restrict__ w,
                                                             float* res_out, float* __restrict__ norm_out,
-                                                            uint8_t* __restrict__ q_out, int hidden, float eps) {
+                                                            uint8_t* __restrict__ q_out, int M, int hidden, float eps) {
     __shared__ float red[THREADS / 64];
     const size_t base = (size_t)blockIdx.x * hidden;
     const int n4 = hidden >> 2;  // hidden is a multiple of 64
+    if (AS == RowsAs::kA6 && (int)blockIdx.x >= M) {
+        for (int j = threadIdx.x; j < n4; j += THREADS) store_a6_float4(q_out, blockIdx.x, j, n4, make_float4(0.f, 0.f, 0.f, 0.f));
+        return;
+    }
     const float4* x4 = reinterpret_cast<const float4*>(x + base);
     const float4* r4 = res_in ? reinterpret_cast<const float4*>(res_in + base) : nullptr;
     float4* o4 = reinterpret_cast<float4*>(res_out + base);
@@ -100,12 +114,15 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_kernel(const float* x, co
     const float total = block_sum<THREADS>(ss, red);
     const float inv = 1.0f / sqrtf(total / (float)hidden + eps);
     const float4* w4 = reinterpret_cast<const float4*>(w);
-    float4* n4p = QUANT ? nullptr : reinterpret_cast<float4*>(norm_out + base);
+    float4* n4p = AS != RowsAs::kFloats ? nullptr : reinterpret_cast<float4*>(norm_out + base);
     auto scale_out = [&](int j, float4 v) {
         const float4 g = w4[j];
         const float4 n = make_float4((v.x * inv) * g.x, (v.y * inv) * g.y, (v.z * inv) * g.z, (v.w * inv) * g.w);
-        if (QUANT)  // j < n4 holds for whole groups of 8 lanes: n4 is a multiple of 16
+        // j < n4 holds for whole groups of 8 lanes: n4 is a multiple of 16
+        if (AS == RowsAs::kBlocks)
             store_quantized_float4(q_out, (long long)blockIdx.x * n4 + j, n);
+        else if (AS == RowsAs::kA6)
+            store_a6_float4(q_out, blockIdx.x, j, n4, n);
         else
             n4p[j] = n;
     };
@@ -726,20 +743,25 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__
     out[i] = (g * (1.0f / (1.0f + expf(-g)))) * u;
 }
 
-// The same product, four per thread, written as the 80 B blocks of the [M][inter] result.
-__global__ __launch_bounds__(256) void silu_mul_quant_kernel(const float4* __restrict__ gate_up, uint8_t* __restrict__ q_out,
+// The same product, four per thread, written as the 80 B blocks of the [M][inter] result, or as A6 with its rows from M on zero.
+template <RowsAs AS>
+__global__ __launch_bounds__(256) void silu_mul_quant_kernel(const float4* __restrict__ gate_up, uint8_t* __restrict__ q_out, int M,
                                                            int inter4, long long total4) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= total4) return;  // total4 is a multiple of 16: whole groups of 8 lanes leave together
     const long long m = i / inter4;
     const int j = (int)(i - m * inter4);
+    if (AS == RowsAs::kA6 && m >= M) return store_a6_float4(q_out, (int)m, j, inter4, make_float4(0.f, 0.f, 0.f, 0.f));
     const float4 g = gate_up[m * 2 * inter4 + j], u = gate_up[m * 2 * inter4 + inter4 + j];
     float4 v;
     v.x = (g.x * (1.0f / (1.0f + expf(-g.x)))) * u.x;
     v.y = (g.y * (1.0f / (1.0f + expf(-g.y)))) * u.y;
     v.z = (g.z * (1.0f / (1.0f + expf(-g.z)))) * u.z;
     v.w = (g.w * (1.0f / (1.0f + expf(-g.w)))) * u.w;
-    store_quantized_float4(q_out, i, v);
+    if (AS == RowsAs::kA6)
+        store_a6_float4(q_out, (int)m, j, inter4, v);
+    else
+        store_quantized_float4(q_out, i, v);
 }
 
 }  // namespace
@@ -748,11 +770,11 @@ hipError_t launch_add_rmsnorm(const float* x, const float* res_in, const float* 
                               int hidden, float eps, hipStream_t s) {
     // few rows: one wide workgroup per row, the row's latency is all there is to hide
     if (M <= 16)
-        hipLaunchKernelGGL((add_rmsnorm_kernel<1024, false>), dim3(M), dim3(1024), 0, s, x, res_in, w, res_out, norm_out, nullptr,
-                           hidden, eps);
+        hipLaunchKernelGGL((add_rmsnorm_kernel<1024, RowsAs::kFloats>), dim3(M), dim3(1024), 0, s, x, res_in, w, res_out, norm_out, nullptr,
+                           M, hidden, eps);
     else
-        hipLaunchKernelGGL((add_rmsnorm_kernel<256, false>), dim3(M), dim3(256), 0, s, x, res_in, w, res_out, norm_out, nullptr,
-                           hidden, eps);
+        hipLaunchKernelGGL((add_rmsnorm_kernel<256, RowsAs::kFloats>), dim3(M), dim3(256), 0, s, x, res_in, w, res_out, norm_out, nullptr,
+                           M, hidden, eps);
     return hipGetLastError();
 }
 
@@ -760,9 +782,16 @@ hipError_t launch_add_rmsnorm_quant(const float* x, const float* res_in, const f
                                     int hidden, float eps, hipStream_t s) {
     uint8_t* q = static_cast<uint8_t*>(q_out);
     if (M <= 16)
-        hipLaunchKernelGGL((add_rmsnorm_kernel<1024, true>), dim3(M), dim3(1024), 0, s, x, res_in, w, res_out, nullptr, q, hidden, eps);
+        hipLaunchKernelGGL((add_rmsnorm_kernel<1024, RowsAs::kBlocks>), dim3(M), dim3(1024), 0, s, x, res_in, w, res_out, nullptr, q, M, hidden, eps);
     else
-        hipLaunchKernelGGL((add_rmsnorm_kernel<256, true>), dim3(M), dim3(256), 0, s, x, res_in, w, res_out, nullptr, q, hidden, eps);
+        hipLaunchKernelGGL((add_rmsnorm_kernel<256, RowsAs::kBlocks>), dim3(M), dim3(256), 0, s, x, res_in, w, res_out, nullptr, q, M, hidden, eps);
+    return hipGetLastError();
+}
+
+hipError_t launch_add_rmsnorm_a6(const float* x, const float* res_in, const float* w, float* res_out, void* a6, int M, int hidden,
+                                 float eps, hipStream_t s) {
+    hipLaunchKernelGGL((add_rmsnorm_kernel<256, RowsAs::kA6>), dim3((M + 31) / 32 * 32), dim3(256), 0, s, x, res_in, w, res_out, nullptr,
+                       static_cast<uint8_t*>(a6), M, hidden, eps);
     return hipGetLastError();
 }
 
@@ -839,8 +868,15 @@ hipError_t launch_silu_mul(const float* gate_up, float* out, int M, int inter, h
 
 hipError_t launch_silu_mul_quant(const float* gate_up, void* q_out, int M, int inter, hipStream_t s) {
     const long long total4 = (long long)M * (inter / 4);
-    hipLaunchKernelGGL(silu_mul_quant_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<const float4*>(gate_up), static_cast<uint8_t*>(q_out), inter / 4, total4);
+    hipLaunchKernelGGL(silu_mul_quant_kernel<RowsAs::kBlocks>, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, s,
+                       reinterpret_cast<const float4*>(gate_up), static_cast<uint8_t*>(q_out), M, inter / 4, total4);
+    return hipGetLastError();
+}
+
+hipError_t launch_silu_mul_a6(const float* gate_up, void* a6, int M, int inter, hipStream_t s) {
+    const long long total4 = (long long)((M + 31) / 32 * 32) * (inter / 4);
+    hipLaunchKernelGGL(silu_mul_quant_kernel<RowsAs::kA6>, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, s,
+                       reinterpret_cast<const float4*>(gate_up), static_cast<uint8_t*>(a6), M, inter / 4, total4);
     return hipGetLastError();
 }
 
