@@ -65,22 +65,19 @@ constexpr int kTileWords = kTileM * kTileN;     // fp32 words of a partial tile
 // ---- operand preparation ------------------------------------------------------------------------
 
 // fp32 rows -> the reference's 80 B blocks (y80, may be null) and A6; rows M .. rows_padded-1 become zero blocks.
-// One float4 per thread, 8 lanes per 32-block (the arithmetic of quantize_row_q8_1_repack_fp32).
+// A float4 a thread, 8 lanes per 32-block (the arithmetic of quantize_row_q8_1_repack_fp32).
 template <bool ALIGNED>
 __global__ __launch_bounds__(256) void quantize_a6_kernel(const float* __restrict__ x, uint8_t* __restrict__ y80,
                                                           uint8_t* __restrict__ a6, int M, int rows_padded, int K) {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;  // one float4 each
-    const int per_row = K >> 2;
-    const int row = (int)(t / per_row);
-    const int c4 = (int)(t - (int64_t)row * per_row);
-    const int blk = c4 >> 3, j = c4 & 7;
+    const RowQuad own = row_quad(K >> 2);
+    const int row = own.row, c4 = own.j, blk = c4 >> 3, j = c4 & 7;
     const bool in_grid = row < rows_padded, real = row < M;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (real) {
         if (ALIGNED) {
-            v = reinterpret_cast<const float4*>(x)[t];
+            v = reinterpret_cast<const float4*>(x)[(int64_t)row * (K >> 2) + c4];
         } else {
-            const float* p = x + 4 * t;
+            const float* p = x + (int64_t)row * K + 4 * c4;
             v = make_float4(p[0], p[1], p[2], p[3]);
         }
     }
@@ -101,11 +98,8 @@ __global__ __launch_bounds__(256) void quantize_a6_kernel(const float* __restric
 // 80 B blocks (already quantised rows) -> A6.  Same thread mapping: thread (row, blk, j) takes dword j of the block's int8.
 __global__ __launch_bounds__(256) void a80_to_a6_kernel(const uint8_t* __restrict__ y80, uint8_t* __restrict__ a6, int M,
                                                         int rows_padded, int K) {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int per_row = K >> 2;
-    const int row = (int)(t / per_row);
-    const int c4 = (int)(t - (int64_t)row * per_row);
-    const int blk = c4 >> 3, j = c4 & 7;
+    const RowQuad own = row_quad(K >> 2);
+    const int row = own.row, blk = own.j >> 3, j = own.j & 7;
     if (row >= rows_padded) return;
     uint32_t packed = 0;
     float d = 0.f, ssum = 0.f;
@@ -459,8 +453,7 @@ hipError_t launch_w384_to_w6(const void* w384, void* w6, int N, int K, hipStream
 
 hipError_t launch_quantize_a6(const float* x, void* y80, void* a6, int M, int K, hipStream_t s) {
     const int rows_padded = (M + 31) / 32 * 32;
-    const long long threads = (long long)rows_padded * (K / 4);
-    const unsigned grid = (unsigned)((threads + 255) / 256);
+    const unsigned grid = row_quad_grid(rows_padded, K / 4);
     if ((reinterpret_cast<uintptr_t>(x) & 15) == 0)
         hipLaunchKernelGGL(quantize_a6_kernel<true>, dim3(grid), dim3(256), 0, s, x, static_cast<uint8_t*>(y80),
                            static_cast<uint8_t*>(a6), M, rows_padded, K);
@@ -472,8 +465,7 @@ hipError_t launch_quantize_a6(const float* x, void* y80, void* a6, int M, int K,
 
 hipError_t launch_a80_to_a6(const void* y80, void* a6, int M, int K, hipStream_t s) {
     const int rows_padded = (M + 31) / 32 * 32;
-    const long long threads = (long long)rows_padded * (K / 4);
-    hipLaunchKernelGGL(a80_to_a6_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, static_cast<const uint8_t*>(y80),
+    hipLaunchKernelGGL(a80_to_a6_kernel, dim3(row_quad_grid(rows_padded, K / 4)), dim3(256), 0, s, static_cast<const uint8_t*>(y80),
                        static_cast<uint8_t*>(a6), M, rows_padded, K);
     return hipGetLastError();
 }

@@ -66,7 +66,7 @@ __device__ __forceinline__ void store_quantized_float4(uint8_t* __restrict__ blo
 }
 
 // The same into A6, float4 j of row `row` of n4: rows as the block-scaled contraction reads them.  By way of 80 B blocks they took another
-// launch and another trip to memory: 322 rows, the norm of 4096 and silu * up of 12288 7.3 + 5.6 and 8.0 + 8.4 us, so 9.8 and 13.0.
+// launch and another trip to memory: 322 rows, the norm of 4096 and silu * up of 12288 7.3 + 5.6 and 8.0 + 8.4 us, so 9.8 and 11.1.
 __device__ __forceinline__ void store_a6_float4(uint8_t* __restrict__ a6, int row, int j, int n4, float4 v) {
     const Quant4 qz = quantize_float4_of_block32(v);
     fp6::store_a6_block(a6, row, j >> 3, n4 >> 3, qz.packed, qz.d, qz.ssum, threadIdx.x & 63);
@@ -743,25 +743,32 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__
     out[i] = (g * (1.0f / (1.0f + expf(-g)))) * u;
 }
 
-// The same product, four per thread, written as the 80 B blocks of the [M][inter] result, or as A6 with its rows from M on zero.
-template <RowsAs AS>
-__global__ __launch_bounds__(256) void silu_mul_quant_kernel(const float4* __restrict__ gate_up, uint8_t* __restrict__ q_out, int M,
+__device__ __forceinline__ float4 silu_mul4(float4 g, float4 u) {
+    return make_float4((g.x * (1.0f / (1.0f + expf(-g.x)))) * u.x, (g.y * (1.0f / (1.0f + expf(-g.y)))) * u.y,
+                       (g.z * (1.0f / (1.0f + expf(-g.z)))) * u.z, (g.w * (1.0f / (1.0f + expf(-g.w)))) * u.w);
+}
+
+// The same product, four per thread, written as the 80 B blocks of the [M][inter] result.
+__global__ __launch_bounds__(256) void silu_mul_quant_kernel(const float4* __restrict__ gate_up, uint8_t* __restrict__ q_out,
                                                            int inter4, long long total4) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= total4) return;  // total4 is a multiple of 16: whole groups of 8 lanes leave together
     const long long m = i / inter4;
     const int j = (int)(i - m * inter4);
-    if (AS == RowsAs::kA6 && m >= M) return store_a6_float4(q_out, (int)m, j, inter4, make_float4(0.f, 0.f, 0.f, 0.f));
-    const float4 g = gate_up[m * 2 * inter4 + j], u = gate_up[m * 2 * inter4 + inter4 + j];
-    float4 v;
-    v.x = (g.x * (1.0f / (1.0f + expf(-g.x)))) * u.x;
-    v.y = (g.y * (1.0f / (1.0f + expf(-g.y)))) * u.y;
-    v.z = (g.z * (1.0f / (1.0f + expf(-g.z)))) * u.z;
-    v.w = (g.w * (1.0f / (1.0f + expf(-g.w)))) * u.w;
-    if (AS == RowsAs::kA6)
-        store_a6_float4(q_out, (int)m, j, inter4, v);
-    else
-        store_quantized_float4(q_out, i, v);
+    store_quantized_float4(q_out, i, silu_mul4(gate_up[m * 2 * inter4 + j], gate_up[m * 2 * inter4 + inter4 + j]));
+}
+
+// The same as A6, its rows from M on zero.
+__global__ __launch_bounds__(256) void silu_mul_a6_kernel(const float4* __restrict__ gate_up, uint8_t* __restrict__ a6, int M, int rows_padded,
+                                                        int inter4) {
+    const fp6::RowQuad own = fp6::row_quad(inter4);
+    if (own.row >= rows_padded) return;  // whole waves
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (own.row < M) {
+        const float4* gates = gate_up + (size_t)own.row * 2 * inter4 + own.j;
+        v = silu_mul4(gates[0], gates[inter4]);
+    }
+    store_a6_float4(a6, own.row, own.j, inter4, v);
 }
 
 }  // namespace
@@ -868,15 +875,15 @@ hipError_t launch_silu_mul(const float* gate_up, float* out, int M, int inter, h
 
 hipError_t launch_silu_mul_quant(const float* gate_up, void* q_out, int M, int inter, hipStream_t s) {
     const long long total4 = (long long)M * (inter / 4);
-    hipLaunchKernelGGL(silu_mul_quant_kernel<RowsAs::kBlocks>, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<const float4*>(gate_up), static_cast<uint8_t*>(q_out), M, inter / 4, total4);
+    hipLaunchKernelGGL(silu_mul_quant_kernel, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, s,
+                       reinterpret_cast<const float4*>(gate_up), static_cast<uint8_t*>(q_out), inter / 4, total4);
     return hipGetLastError();
 }
 
 hipError_t launch_silu_mul_a6(const float* gate_up, void* a6, int M, int inter, hipStream_t s) {
-    const long long total4 = (long long)((M + 31) / 32 * 32) * (inter / 4);
-    hipLaunchKernelGGL(silu_mul_quant_kernel<RowsAs::kA6>, dim3((unsigned)((total4 + 255) / 256)), dim3(256), 0, s,
-                       reinterpret_cast<const float4*>(gate_up), static_cast<uint8_t*>(a6), M, inter / 4, total4);
+    const int rows_padded = (M + 31) / 32 * 32;
+    hipLaunchKernelGGL(silu_mul_a6_kernel, dim3(fp6::row_quad_grid(rows_padded, inter / 4)), dim3(256), 0, s,
+                       reinterpret_cast<const float4*>(gate_up), static_cast<uint8_t*>(a6), M, rows_padded, inter / 4);
     return hipGetLastError();
 }
 
