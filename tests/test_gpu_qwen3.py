@@ -292,3 +292,16 @@ def test_one_token_pass_on_narrow_models(pkg, synth, ora, hidden, inter):
     for got, ids in zip(here, passes):
         assert rel(got, cpu.forward(ids)) <= 2e-2
     assert np.array_equal(np.stack(here), _logits_with_option(gpu, "no_pair", 1, passes))
+
+
+@pytest.mark.parametrize("rows", [1409, 1440, 1503])  # one row in the last panel of 32, whole panels, a panel with one row missing
+def test_rows_written_for_the_block_scaled_kernel(pkg, rows):
+    """Norms and SiLU * up that write that kernel's operand format against fp32 rows through the layers' own quantiser: the same bits."""
+    cfg = dict(n_layers=1, hidden=1024, n_q_heads=8, n_kv_heads=2, intermediate=8192, vocab=512, max_seq=1536)
+    gpu = pkg.Qwen3Model(**cfg)
+    build(pkg.synth, None, cfg, 77, gpu_model=gpu)
+    ids = np.random.default_rng(rows).integers(0, 512, rows).astype(np.int32)
+    gpu.reset()
+    fused = gpu.forward(ids)
+    assert np.isfinite(fused).all()
+    assert np.array_equal(fused, _logits_with_option(gpu, "unfused", 1, [ids])[0])
