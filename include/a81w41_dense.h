@@ -15,6 +15,10 @@ extern "C" {
 /* C = A W^T: A [M][lda], W [N][ldw] elements, C [M][ldc] floats.  lda, ldw: at least K rounded up to 128 bytes, whole
  * multiples of 128 bytes; the columns of W beyond K are zero, those of A finite. */
 int a81w41_dense_gemm(const void *A, int lda, const void *W, int ldw, float *C, int ldc, int M, int N, int K, int bf16, void *stream);
+/* The same product with gated units: rows of W come as 16 gates, then their 16 ups, and so on (N a multiple of 32), and C [M][ldc >= N / 2]
+ * holds elements g / (1 + exp(-slope g)) (u + shift) of g = min(gate, limit), u = clamp(up, -limit, limit). */
+int a81w41_dense_gated(const void *A, int lda, const void *W, int ldw, void *C, int ldc, int M, int N, int K, float limit, float slope,
+                       float shift, int bf16, void *stream);
 /* Attention in latent space.  q [M heads][ld], cache [max_seq][ld] with rows [latent (rank) | rotated part (rot)] and zeros
  * up to ld (a multiple of 128 bytes); token m sees cache rows 0 .. pos + m.  out [M heads][rank] elements.
  * variant 0: the vector kernel; 1: matrix cores (bfloat16 only), the keys dealt to `splits` (1 .. 64) workgroups, with

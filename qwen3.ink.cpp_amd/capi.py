@@ -105,6 +105,7 @@ CORE_SIGNATURES = {
 # every symbol include/a81w41_dense.h declares
 DENSE_SIGNATURES = {
     "a81w41_dense_gemm": (_i, [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _i, _vp]),
+    "a81w41_dense_gated": (_i, [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, C.c_float, C.c_float, C.c_float, _i, _vp]),
     "a81w41_latent_attention": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _i, _i, C.c_float, _vp, _i, _i, _i, _vp, _vp, _vp]),
     "a81w41_formed_attention": (_i, [_vp, _vp, _vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _vp, _i, _i, C.c_float, _vp, _vp]),
     "a81w41_grouped_attention": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _i, _i, C.c_float, _i, _i, _vp, _i, _i, _i, _vp, _vp, _vp]),

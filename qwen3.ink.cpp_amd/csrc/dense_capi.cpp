@@ -21,6 +21,16 @@ int gemm(const void* A, int lda, const void* W, int ldw, float* C, int ldc, int 
     A81W41_HIP_TRY(launch_dense_gemm<T>(g, Epilogue::kFloat, s));
     return 0;
 }
+template <typename T>
+int gated(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N, int K, const GatedUnit& unit, hipStream_t s) {
+    constexpr int step = 128 / (int)sizeof(T);
+    if (lda % step || ldw % step || lda < pad_k<T>(K) || ldw < pad_k<T>(K) || ldc < N / 2)
+        return failf(A81W41_ERR_INVALID_ARG, "row strides must be whole multiples of 128 bytes and cover K");
+    GemmArgs g;
+    g.A = A, g.W = W, g.C = C, g.M = M, g.N = N, g.K = pad_k<T>(K), g.lda = lda, g.ldw = ldw, g.ldc = ldc, g.unit = unit;
+    A81W41_HIP_TRY(launch_dense_gemm<T>(g, Epilogue::kGatedPair, s));
+    return 0;
+}
 }  // namespace
 
 extern "C" {
@@ -29,6 +39,14 @@ int a81w41_dense_gemm(const void* A, int lda, const void* W, int ldw, float* C, 
     if (!A || !W || !C || M < 1 || N < 1 || K < 1 || !aligned16(A) || !aligned16(W)) return failf(A81W41_ERR_INVALID_ARG, "bad product");
     hipStream_t s = static_cast<hipStream_t>(stream);
     return is_bf16 ? gemm<bf16>(A, lda, W, ldw, C, ldc, M, N, K, s) : gemm<float>(A, lda, W, ldw, C, ldc, M, N, K, s);
+}
+
+int a81w41_dense_gated(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N, int K, float limit, float slope,
+                       float shift, int is_bf16, void* stream) {
+    if (!A || !W || !C || M < 1 || N < 32 || N % 32 || K < 1 || !aligned16(A) || !aligned16(W)) return failf(A81W41_ERR_INVALID_ARG, "bad product");
+    const GatedUnit unit{limit, slope, shift};
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    return is_bf16 ? gated<bf16>(A, lda, W, ldw, C, ldc, M, N, K, unit, s) : gated<float>(A, lda, W, ldw, C, ldc, M, N, K, unit, s);
 }
 
 int a81w41_latent_attention(const void* q, const void* cache, int ld, int rank, int rot, int heads, const int* pos_dev, int max_seq, int M,

@@ -9,8 +9,8 @@
 // What bounds it: bytes per product.  A 128 x 128 tile asks the L2 for 64 bytes a clock and CU at the matrix cores' full rate,
 // which is all the L2 gives, and reads LDS as fast as LDS goes; a 256 x 256 tile asks for half of the one and three quarters of
 // the other.  4095 x 12288 x 2048 in bfloat16 with the gated epilogue: 340 us with 128 x 128 tiles whose copies the compiler
-// waited for ahead of every step's first LDS read (see lds16), 190 us = 1.08 PFLOP/s with 256 x 256.  4095 x 2048 x 6144: 146 us and
-// 106 us, 2048 x 2048 x 2048: 46 us and 25 us.
+// waited for ahead of every step's first LDS read (see lds16), 209 us = 0.99 PFLOP/s with 256 x 256.  4095 x 2048 x 6144: 146 us and
+// 104 us, 2048 x 2048 x 2048: 46 us and 25 us.
 #include <type_traits>
 
 #include "dense_common.h"
@@ -27,14 +27,6 @@ __device__ __forceinline__ void mma(f32x16& acc, const lds16& a, const lds16& b,
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[2]), __uint_as_float(b[2]), acc, 0, 0, 0);
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[3]), __uint_as_float(b[3]), acc, 0, 0, 0);
 }
-
-// A unit that is rounded to bfloat16 next: the hardware's exponential and reciprocal, a unit of 24 bits off at most in what they return.
-// Of 36 us that the epilogue of 4095 x 12288 x 2048 took, 10 were the library's exponential and division.
-__device__ __forceinline__ float unit_of(const GatedUnit& p, float gate, float up, bf16*) {
-    const float g = fminf(gate, p.limit), u = fminf(fmaxf(up, -p.limit), p.limit);
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * p.slope * g)) * (u + p.shift);
-}
-__device__ __forceinline__ float unit_of(const GatedUnit& p, float gate, float up, float*) { return gated_unit(p, gate, up); }
 
 struct NoHeads {};
 
@@ -72,7 +64,7 @@ __device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, c
 #pragma unroll
         for (int v = 0; v < NV; v += 2) {
             const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[v]), __float_as_uint(x[v + 1]), false, false);
-            const float unit = unit_of(g.unit, __uint_as_float(both[0]), __uint_as_float(both[1]), static_cast<T*>(nullptr));
+            const float unit = gated_unit(g.unit, __uint_as_float(both[0]), __uint_as_float(both[1]));
             const int r = r0 + 8 * (v >> 2) + (v & 3) + odd;
             if (r < rows && col < g.N) dst[(size_t)(m0 + r) * g.ldc] = (T)unit;
         }
@@ -136,8 +128,7 @@ constexpr int kBandRows = 2048;
 // X: HeadRows<T> with the epilogue kHeads, LatentQueries<T> with kQueries, NoHeads with the others.  STAGES: how many steps LDS holds; all but one are under way.
 // PIPE: a step's operands are read one 16-byte column ahead of their products, also into the next step: the waves meet before a step's
 // last products, whose operands are in registers by then, so that its stage is free for new copies and the next step's first
-// reads run beside those products.  4095 x 12288 x 2048, gated: 200.6 us with the meeting between two steps, 189.5 so (with the unit
-// below).  Without PIPE the other workgroup of the CU fills the wait.
+// reads run beside those products.  4095 x 12288 x 2048 into floats: 211 us with the meeting between two steps, 204 so.  Without PIPE the other workgroup of the CU fills the wait.
 template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PIPE, Epilogue EPI, typename X>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(GemmArgs g, X heads) {
     constexpr int kThreads = 64 * WAVES_M * WAVES_N;

@@ -223,6 +223,14 @@ def dense_gemm(a, w, K: int):
     return out
 
 
+def dense_gated(a, w, K: int, limit: float = float("inf"), slope: float = 1.0, shift: float = 0.0):
+    """Parity hook a81w41_dense_gated: a [M][lda], w [N][ldw] with rows of 16 gates and 16 ups in turn -> [M][N / 2] of a's type."""
+    out = _torch().empty((a.shape[0], w.shape[0] // 2), dtype=a.dtype, device=a.device)
+    capi.check(capi.dense().a81w41_dense_gated(_dev_ptr(a), a.shape[1], _dev_ptr(w), w.shape[1], _dev_ptr(out), out.shape[1], a.shape[0],
+                                               w.shape[0], K, limit, slope, shift, _element(a), _stream()))
+    return out
+
+
 def latent_attention(q, cache, pos: int, rank: int, rot: int, heads: int, scale: float, variant: int = 0, splits: int = 1):
     """Parity hook a81w41_latent_attention: q [M*heads][ld], cache [max_seq][ld] -> [M*heads][rank] of q's type."""
     torch = _torch()

@@ -271,7 +271,7 @@ def test_experts_in_tiles_of_two_heights(pkg, n, experts, top, ff, width):
     _same_in_portions(pkg, cfg, n, 100)
 
 
-# a gated unit at the limits of its gate: the hardware's exponential and reciprocal against the library's in the 32-bit mode
+# a gated unit at the limits of its gate: exponentials past the range of a float, in both types
 def test_gated_units_of_large_gates(pkg, tmp_path):
     from oracle import takosun_forward as tf
     cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.dense(96))])
@@ -291,3 +291,39 @@ def test_gated_units_of_large_gates(pkg, tmp_path):
 def test_query_columns_on_large_tiles(pkg, heads, dim, rot):
     cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(heads, dim, rot, 8, 70, 24, 0.1), None)])
     _same_in_portions(pkg, cfg, 2100, 100)
+
+
+# The unit is formed in 32 bits ahead of its rounding to bfloat16: only a unit that lies within the error of that arithmetic of the middle
+# between two bfloat16 may be rounded the other way.  A product of three columns by ones puts any float of 24 bits together, exactly.
+# Relative errors in 2^-24: the exponential 2 (one unit in the last place) and 2 |slope g| of its rounded argument, one each of the sum,
+# the division and, with an up that is no constant, of u + shift and the product.  Gates end where 1.702 g is -85: from -88.7 on the exponential
+# is no float and the unit zero.
+@pytest.mark.parametrize("limit,slope,shift", [(float("inf"), 1.0, 0.0), (7.0, 1.702, 1.0)])
+@pytest.mark.parametrize("low,high", [(-4.0, 4.0), (-20.0, -4.0), (-50.0, -20.0)])
+@pytest.mark.parametrize("M", [320, 40])
+def test_gated_units_are_formed_in_32_bits(pkg, limit, slope, shift, low, high, M):
+    import torch
+    units, groups = 2048, 64
+    g = torch.Generator(device="cuda").manual_seed(M)
+    gate = torch.rand(groups, units, device="cuda", generator=g) * (high - low) + low
+    up = torch.rand(groups, units, device="cuda", generator=g) * 2 - 1 if shift else torch.ones(groups, units, device="cuda")
+
+    def columns(x):   # [groups][units] floats -> [units][3 groups], whose sums over a group's three columns are x
+        parts, rest = [], x
+        for _ in range(3):
+            parts.append(rest.bfloat16())
+            rest = rest - parts[-1].float()
+        assert not rest.any()
+        return torch.stack(parts, 1).permute(2, 0, 1).reshape(units, 3 * groups)
+
+    w = torch.stack([columns(gate).view(units // 16, 16, -1), columns(up).view(units // 16, 16, -1)], 1).reshape(2 * units, -1).contiguous()
+    rows = torch.arange(M, device="cuda") % groups
+    a = torch.zeros(M, groups, 3, device="cuda", dtype=torch.bfloat16)
+    a[torch.arange(M, device="cuda"), rows] = 1
+    got = pkg.ops.dense_gated(a.view(M, -1), w, 3 * groups, limit, slope, shift)
+    x, u = gate.double().clamp(max=limit), up.double().clamp(-limit, limit)
+    want = (x / (1 + (-float(np.float32(slope)) * x).exp()) * (u + shift))[rows]
+    units_off = 4 + 2 + (2 * slope * x[rows].abs() if slope != 1 else 0)
+    near = (want.abs() * 2.0 ** -24 * units_off + 2.0 ** -149)
+    ok = (got == (want - near).bfloat16()) | (got == (want + near).bfloat16())
+    assert ok.all(), ((~ok).sum().item(), gate[rows][~ok][:4].tolist(), got[~ok][:4].tolist(), want[~ok][:4].tolist())
