@@ -44,6 +44,7 @@ struct a81w41_qwen3 : a81w41_model {
     float *cos_t = nullptr, *sin_t = nullptr;
     // activations, sized for max_seq rows
     float *x = nullptr, *x2 = nullptr, *h = nullptr, *qkv = nullptr, *attn = nullptr, *o = nullptr, *gate_up = nullptr, *act = nullptr;
+    float* token_in = nullptr;  // embedding of the one-token pass, which may be there ahead of the pass
     float* attn_part = nullptr;    // split attention: n_q * kAttentionMaxSplits * 132 floats
     unsigned* attn_arrive = nullptr;  // ... and n_q arrival counters, zero between launches
     float attn_scale = 0.f;  // 1/sqrt(128) unless a scaling.bin said otherwise
@@ -221,7 +222,7 @@ int attention_step(a81w41_qwen3* m, LayerWeights& L, float* out, void* q_out, in
 }  // namespace
 
 bool a81w41_qwen3::token_row(a81w41::TokenRow* row) const {
-    *row = a81w41::TokenRow{embedding, a81w41::TableType::kFp16, cfg.hidden, o, cfg.hidden, cfg.vocab};
+    *row = a81w41::TokenRow{embedding, a81w41::TableType::kFp16, cfg.hidden, token_in, cfg.hidden, cfg.vocab};
     return one_token_pass_usable(this);
 }
 
@@ -245,8 +246,8 @@ int a81w41_qwen3::one_token_pass(hipStream_t s) {
     if (splits > fit) splits = fit;
     if (env_split > 0) splits = env_split;
     splits = splits < 1 ? 1 : (splits > a81w41::kAttentionMaxSplits ? a81w41::kAttentionMaxSplits : splits);
-    if (!row_given)  // pending = the embedding
-        Q_HIP(a81w41::launch_embed_rows(m->ids, m->embedding, a81w41::TableType::kFp16, c.hidden, m->o, 1, c.hidden, c.vocab, s));
+    if (!row_given)
+        Q_HIP(a81w41::launch_embed_rows(m->ids, m->embedding, a81w41::TableType::kFp16, c.hidden, m->token_in, 1, c.hidden, c.vocab, s));
     // The linears and the attention of the pass are one dependent chain (QwenDecoderLayer.cc:39-105).  As links of
     // an overlapping chain each of them starts while its predecessor runs and requests its first weight blocks
     // (or cache rows) before it waits for it; same kernels' arithmetic, same bits.
@@ -269,7 +270,7 @@ int a81w41_qwen3::one_token_pass(hipStream_t s) {
     a81w41::ChainLink link;
     unsigned grid = 0;
     auto next_link = [&]() { link = a81w41::chain_next(chain, &ls); };
-    const float* res_in = nullptr;
+    const float *res_in = nullptr, *pending = m->token_in;
     for (int l = 0; l < c.n_layers; l++) {
         LayerWeights& L = m->layers[l];
         a81w41::GemvPrologue p0;
@@ -279,7 +280,7 @@ int a81w41_qwen3::one_token_pass(hipStream_t s) {
         p0.eps = c.rms_eps;
         if (chain) {
             next_link();
-            Q_HIP(a81w41::launch_gemv_chain_add_norm(m->o, p0, scratch, a81w41_linear_weight_fp16_dev(L.lin[0]), m->qkv, qkv_dim,
+            Q_HIP(a81w41::launch_gemv_chain_add_norm(pending, p0, scratch, a81w41_linear_weight_fp16_dev(L.lin[0]), m->qkv, qkv_dim,
                                                      c.hidden, link, chain->cus, &grid, ls));
             a81w41::chain_launched(chain, grid);
             next_link();
@@ -296,7 +297,7 @@ int a81w41_qwen3::one_token_pass(hipStream_t s) {
             }
             a81w41::chain_launched(chain, grid);
         } else {
-            Q_HIP(a81w41::launch_gemv_add_norm(m->o, p0, scratch, a81w41_linear_weight_fp16_dev(L.lin[0]), m->qkv, qkv_dim,
+            Q_HIP(a81w41::launch_gemv_add_norm(pending, p0, scratch, a81w41_linear_weight_fp16_dev(L.lin[0]), m->qkv, qkv_dim,
                                                c.hidden, s));
             if (attn_fp32) {
                 Q_TRY(attention_step(m, L, m->attn, nullptr, splits, scale, s, nullptr));
@@ -334,6 +335,7 @@ int a81w41_qwen3::one_token_pass(hipStream_t s) {
             Q_HIP(a81w41::launch_gemv_fp16(scratch, a81w41_linear_weight_fp16_dev(L.lin[3]), m->o, c.hidden, c.intermediate, s));
         }
         res_in = m->x;
+        pending = m->o;
     }
     a81w41::GemvPrologue pf;
     pf.res_in = res_in;
@@ -342,12 +344,12 @@ int a81w41_qwen3::one_token_pass(hipStream_t s) {
     pf.eps = c.rms_eps;
     if (chain) {
         next_link();
-        Q_HIP(a81w41::launch_gemv_chain_add_norm(m->o, pf, scratch, a81w41_linear_weight_fp16_dev(m->lm_head), m->logits, c.vocab,
+        Q_HIP(a81w41::launch_gemv_chain_add_norm(pending, pf, scratch, a81w41_linear_weight_fp16_dev(m->lm_head), m->logits, c.vocab,
                                                  c.hidden, link, chain->cus, &grid, ls));
         a81w41::chain_launched(chain, grid);
         Q_HIP(a81w41::chain_end(chain));
     } else {
-        Q_HIP(a81w41::launch_gemv_add_norm(m->o, pf, scratch, a81w41_linear_weight_fp16_dev(m->lm_head), m->logits, c.vocab,
+        Q_HIP(a81w41::launch_gemv_add_norm(pending, pf, scratch, a81w41_linear_weight_fp16_dev(m->lm_head), m->logits, c.vocab,
                                            c.hidden, s));
     }
     if (!advance_given) Q_HIP(a81w41::launch_advance(m->pos, 1, s));
@@ -442,6 +444,7 @@ int a81w41_qwen3::create() {
     const size_t rows = c.max_seq;
     Q_TRY(dev_alloc(&m->x, rows * c.hidden));
     Q_TRY(dev_alloc(&m->x2, (size_t)c.hidden));  // second residual row of the one-token pass
+    Q_TRY(dev_alloc(&m->token_in, (size_t)c.hidden));
     Q_TRY(dev_alloc(&m->h, rows * c.hidden));
     Q_TRY(dev_alloc(&m->qkv, rows * m->qkv_dim()));
     Q_TRY(dev_alloc(&m->attn, rows * q_dim));
@@ -478,7 +481,7 @@ a81w41_qwen3::~a81w41_qwen3() {
         }
     }
     a81w41_linear_destroy(m->lm_head);
-    void* bufs[] = {m->final_norm, m->embedding, m->cos_t, m->sin_t, m->x, m->x2, m->h, m->qkv, m->attn, m->o,
+    void* bufs[] = {m->final_norm, m->embedding, m->cos_t, m->sin_t, m->x, m->x2, m->token_in, m->h, m->qkv, m->attn, m->o,
                     m->gate_up, m->act, m->attn_part, m->attn_arrive};
     for (void* b : bufs) (void)hipFree(b);
     a81w41_context_destroy(m->ctx);
@@ -588,7 +591,7 @@ size_t a81w41_qwen3_resident_bytes(const a81w41_qwen3* m, size_t* linear_weights
     other += 2 * (size_t)c.max_seq * kHeadDim * sizeof(float);  // rotation tables
     const size_t kv = 2 * (size_t)c.n_layers * c.n_kv_heads * c.max_seq * kHeadDim * 2;
     const size_t rows = c.max_seq;
-    size_t buf = (rows * c.hidden * 3 + (size_t)c.hidden + rows * m->qkv_dim() + rows * c.n_q_heads * kHeadDim +
+    size_t buf = (rows * c.hidden * 3 + 2 * (size_t)c.hidden + rows * m->qkv_dim() + rows * c.n_q_heads * kHeadDim +
                   rows * 3 * c.intermediate + (size_t)c.vocab) * sizeof(float);
     buf += (size_t)c.n_q_heads * a81w41::kAttentionMaxSplits * 132 * sizeof(float) + (size_t)c.n_q_heads * sizeof(unsigned);
     buf += (rows + 2 + (size_t)m->history_len) * sizeof(int);

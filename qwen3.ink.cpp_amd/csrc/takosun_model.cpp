@@ -136,7 +136,7 @@ class TakosunModel final : public DenseModel<T> {
    protected:
     int enqueue_pass(int M, const int* want, int n_want, hipStream_t s) override;
     bool token_row(TokenRow* row) const override {
-        *row = TokenRow{embed_.data, kTable, embed_.ld, states_, cfg_.width, cfg_.vocab};
+        *row = TokenRow{embed_.data, kTable, embed_.ld, token_in_, cfg_.width, cfg_.vocab};
         return one_token_fits_ && !opt_unfused_;
     }
 
@@ -190,6 +190,7 @@ class TakosunModel final : public DenseModel<T> {
     size_t part_rows_ = 0;
     int ld_part_ = 0;
     // of the one-token pass
+    float *token_in_ = nullptr;  // the embedding, which may be there ahead of the pass
     float *row_x_[2] = {nullptr, nullptr}, *row_mid_ = nullptr, *before_ = nullptr, *y_ff_ = nullptr;
     float *o_lat_row_ = nullptr, *attn_row_ = nullptr, *act_row_ = nullptr;
     int ld_act_row_ = 0;
@@ -340,7 +341,7 @@ int TakosunModel<T>::allocate(int max_seq) {
     part_rows_ = std::max((size_t)heads * kAttendMaxSplits, (size_t)8192);
     A81W41_TRY(allocate_array(part_rows_ * ld_part_, &part_));
     A81W41_TRY(allocate_array(part_rows_ * 2, &part_stats_));
-    for (float** row : {&row_x_[0], &row_x_[1], &row_mid_, &before_, &y_ff_}) A81W41_TRY(allocate_array(W, row));
+    for (float** row : {&token_in_, &row_x_[0], &row_x_[1], &row_mid_, &before_, &y_ff_}) A81W41_TRY(allocate_array(W, row));
     A81W41_TRY(allocate_array(o_lat, &o_lat_row_));
     A81W41_TRY(allocate_array((size_t)ld_attn_, &attn_row_));
     A81W41_TRY(allocate_array((size_t)slots * ld_act_row_, &act_row_));
@@ -547,9 +548,9 @@ int TakosunModel<T>::attend_one_token(const Layer& L, const LatentShape& sh, con
 template <typename T>
 int TakosunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
     const int W = cfg_.width, n = n_layers();
-    if (!row_given) A81W41_HIP_TRY(launch_embed_rows(ids, embed_.data, kTable, embed_.ld, states_, 1, W, cfg_.vocab, s));
+    if (!row_given) A81W41_HIP_TRY(launch_embed_rows(ids, embed_.data, kTable, embed_.ld, token_in_, 1, W, cfg_.vocab, s));
     RowStep step;  // what the next product's prologue does
-    step.x = states_, step.width = W, step.norm_h = norm(layers_[0].norm1);
+    step.x = token_in_, step.state = states_, step.width = W, step.norm_h = norm(layers_[0].norm1);
     for (int i = 0; i < n; i++) {
         const Layer& L = layers_[i];
         const LayerConfig& lc = cfg_.layers[i];

@@ -109,3 +109,31 @@ def test_generation_takes_the_first_maximum(pkg, tmp_path, vocab, width, dtype):
         assert token == int(logits.argmax())
         logits = model.forward([token])[0]
     assert model.position == 3 + 12
+
+
+# What a model's buffers hold behind a generation is what its last pass left there, not the token found behind it: the same tokens
+# handed in give the same buffers, of the prompt where no step follows, of the last step's token otherwise.
+@pytest.mark.parametrize("prompt", [1, 9])
+@pytest.mark.parametrize("new", [1, 2, 6])
+@pytest.mark.parametrize("unfused", [0, 1])
+@pytest.mark.parametrize("family", ["qwen3", "takosun"])
+def test_buffers_behind_a_generation(pkg, synth, ora, family, prompt, new, unfused):
+    ids = (np.arange(prompt) * 7 + 3).astype(np.int32)
+    if family == "qwen3":
+        models = [pkg.Qwen3Model(**TINY) for _ in range(2)]
+        for m in models:
+            build(synth, ora, TINY, 900, gpu_model=m)
+        names, width = ["residual", "block_out"], TINY["hidden"]
+    else:
+        models = [pkg.Model.random(SMALL, 40, "bfloat16", seed=3) for _ in range(2)]
+        names, width = [f"state{i}" for i in range(len(SMALL["layers"]) + 1)], SMALL["width"]
+    for m in models:
+        m.set_option("unfused", unfused)
+    found = models[0].generate_greedy(ids, new)[0]
+    models[1].forward(ids)
+    for token in found[:new - 1]:
+        models[1].forward([token])
+    rows = prompt if new == 1 else 1
+    for name in names:
+        got, want = (m.read_buffer(name, rows, width) for m in models)
+        assert np.isfinite(want).all() and want.any() and np.array_equal(got, want), name
