@@ -423,12 +423,15 @@ hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
         if (g.tiles) return launch_grouped<T, EPI>(g, heads, s);
     auto tiles = [&](int rows, int cols) { return (long long)((g.M + rows - 1) / rows) * ((g.N + cols - 1) / cols) * g.batches; };
     // One round of a tile for each CU, three quarters full or more; a tile has the larger one's stages and waves, so that its rows and
-    // weights are under way early.
+    // weights are under way early.  That takes some steps of K to pay: before the last of them are under way nothing fills the CU.
     auto one_round = [&](int rows, int cols) { return g.M > 64 && tiles(rows, cols) >= 192 && tiles(rows, cols) <= 256; };
+    const int steps = g.K * (int)sizeof(T) / 128;
     if constexpr (sizeof(T) == 2)
         if (large_tiles_preferred(tiles(256, 256), tiles(128, 128), g.K)) return launch_kernel<T, 256, 256, 2, 4, 2, true, EPI>(g, heads, s);
-    // us, so / with 128 x 128 tiles: 4095 rows, 2048 x 2048 39.6 / 41.1, 2048 x 6144 106 / 109; 2048 rows, 3104 x 2048 36.3 / 40.4
-    if (one_round(128, 256)) return launch_kernel<T, 128, 256, 2, 4, 3, true, EPI>(g, heads, s);
+    // us, so / with 128 x 128 tiles: 4095 rows, 2048 x 2048 39.6 / 41.1, 2048 x 6144 106 / 109; 2048 rows, 3104 x 2048 36.3 / 40.4.
+    // Over 45 drawn shapes a type, on average: bfloat16 up to 10 steps 1.02 of the time and up to 1.075 (1854 rows, 4203 x 640 21.4 /
+    // 20.1), 11 and more 0.98; float up to 4 steps 1.05 (951 rows, 6073 x 64 16.4 / 15.2), 6 and more 0.98.
+    if (steps >= (sizeof(T) == 2 ? 11 : 6) && one_round(128, 256)) return launch_kernel<T, 128, 256, 2, 4, 3, true, EPI>(g, heads, s);
     // 2048^3: 24.8 us with twice the waves and four stages, 33 us as two a CU
     if (one_round(128, 128)) return launch_kernel<T, 128, 128, 2, 4, 4, true, EPI>(g, heads, s);
     if (g.M > 64 && tiles(128, 128) > 256) {
@@ -437,8 +440,8 @@ hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
         return launch_kernel<T, 128, 128, 2, 2, 2, false, EPI>(g, heads, s);
     }
     // us, so / with 64 x 64 tiles: 1024 rows, 2048 x 2048 15.2 / 16.0, x 6144 45.1 / 49.2; 600 rows, 3072 x 1536 12.2 / 13.4; 180 rows, 9216
-    // x 1536 14.6 / 16.3
-    if (one_round(64, 128)) return launch_kernel<T, 64, 128, 2, 4, 3, true, EPI>(g, heads, s);
+    // x 1536 14.6 / 16.3; over 45 drawn shapes 0.98 on average, with one and two steps 1.03 (2674 rows, 553 x 128 5.8 / 5.5)
+    if (steps > 2 && one_round(64, 128)) return launch_kernel<T, 64, 128, 2, 4, 3, true, EPI>(g, heads, s);
     // So few tiles of 64 x 32 that no CU gets a second one (us, against 64 x 64 tiles with four stages): 33 rows, 784 x 2048 7.7 /
     // 12.5, 2048 x 6144 19 / 31; 256 rows, 2048 x 2048 10.2 / 13.5; with a second one 300 rows, 2048 x 2048 17.2 / 13.8, and 33
     // rows, 12288 x 2048 20 / 16.

@@ -263,6 +263,24 @@ def test_one_round_of_tiles(pkg, M, N, K, dtype):
     assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
 
 
+# The steps of K from which one round of 128 x 256 and of 64 x 128 tiles is taken, and those before: the same bits for a row in a call of
+# 33 rows, which goes through another kernel on either side.
+@pytest.mark.parametrize("M,N,dtype,steps", [(2045, 3100, "bfloat16", (10, 11, 12, 13)), (2045, 3100, "float32", (5, 6, 7)),
+                                             (1000, 2000, "bfloat16", (2, 3, 4)), (1000, 2000, "float32", (2, 3))])
+def test_one_round_from_some_steps_on(pkg, M, N, dtype, steps):
+    import torch
+    bf16 = dtype == "bfloat16"
+    for n in steps:
+        g, K = torch.Generator(device="cuda").manual_seed(n), n * (64 if bf16 else 32)
+        a = torch.randn(M, K, device="cuda", generator=g).to(getattr(torch, dtype))
+        w = torch.randn(N, K, device="cuda", generator=g).to(getattr(torch, dtype))
+        got = pkg.ops.dense_gemm(a, w, K)
+        # K products (exact in bfloat16) and K sums, rounded to 24 bits
+        bound = (1 if bf16 else 2) * K * 2.0 ** -24 * 4 * K ** 0.5
+        assert (got.double() - a.double() @ w.double().t()).abs().max().item() <= bound, n
+        assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:]), n
+
+
 # Experts' rows in tiles of 128 (one pass) and of 64 (portions): 128 x 256 and 128 x 128 tiles, 64 x 128 with two and three stages, 64 x 64;
 # experts with few rows or none, tables of few ids against many
 @pytest.mark.parametrize("n,experts,top,ff,width", [(2100, 8, 2, 600, 1088), (1100, 4, 1, 2048, 64), (700, 5, 3, 96, 2048), (1400, 16, 2, 520, 320)])
