@@ -49,6 +49,18 @@ struct HeadRows {
     float* rest = nullptr;
     int ld_rest = 0;
 };
+// Entry of the angle tables ([max_seq][pairs]) by which the token `d` places behind row m of a pass that starts at pos turns, from the
+// entry of row m's token on: tokens past the last place turn as that one.  base: entries ahead of row m's.
+struct AngleRows {
+    size_t base;
+    int left, pairs;
+    __host__ __device__ AngleRows(int pos, int m, int max_seq, int pairs) : pairs(pairs) {
+        const int first = pos < max_seq - m ? pos + m : max_seq - 1;
+        base = (size_t)first * pairs;
+        left = max_seq - 1 - first;
+    }
+    __host__ __device__ int behind(int d) const { return (d < left ? d : left) * pairs; }
+};
 // Columns of heads, each [dim | one zero if dim is odd | rot]: the first to nope, head h of row m at (m heads + h) ld_nope, the last
 // to rotated, at (m heads + h) ld_rot, turned in neighbouring pairs by the angles of the token at *pos_dev + m.
 template <typename T>

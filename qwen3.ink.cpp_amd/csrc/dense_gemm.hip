@@ -80,11 +80,13 @@ __device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, c
         const bool turns = __any(to.pair >= 0);
         float cs[NV], sn[NV];
         if (turns) {
-            const int pairs = turned_pairs(heads), own = max(to.pair, 0);
+            const AngleRows angles(pos, m0 + r0, heads.max_seq, turned_pairs(heads));
+            const size_t first = angles.base + max(to.pair, 0);
+            const float *cos_t = heads.cos_t + first, *sin_t = heads.sin_t + first;
 #pragma unroll
             for (int v = 0; v < NV; v++) {
-                const unsigned i = __umul24(min(pos + m0 + r0 + 8 * (v >> 2) + (v & 3), heads.max_seq - 1), pairs) + own;
-                cs[v] = heads.cos_t[i], sn[v] = heads.sin_t[i];
+                const int i = angles.behind(8 * (v >> 2) + (v & 3));
+                cs[v] = cos_t[i], sn[v] = sin_t[i];
             }
         }
         uint8_t* dst = to.dst;
