@@ -25,6 +25,11 @@ int a81w41_dense_gated(const void *A, int lda, const void *W, int ldw, void *C, 
  * part [splits M heads][rank rounded up to 4] and stats [splits M heads][2] floats as scratch. */
 int a81w41_latent_attention(const void *q, const void *cache, int ld, int rank, int rot, int heads, const int *pos_dev, int max_seq, int M,
                             float scale, void *out, int bf16, int variant, int splits, float *part, float *stats, void *stream);
+/* The same for one token over a short context, bfloat16, with the product behind it in the same launch: q [heads][ld] with zeros past
+ * rank + rot, uv [heads vdim][ld_uv] (ld_uv a multiple of 8, zeros past rank), gates [heads] floats (before the sigmoid), out [heads vdim]
+ * floats.  rank: a multiple of 8, at most 512; rot: 1 .. 64. */
+int a81w41_latent_token(const void *q, const void *cache, int ld, int rank, int rot, int heads, int vdim, const int *pos_dev, int max_seq,
+                        float scale, const void *uv, int ld_uv, const float *gates, float *out, void *stream);
 /* Attention on formed keys and values, bfloat16.  q [M][heads][dim + rot], k [max_seq][heads dim] and k_rot
  * [max_seq][ld_rot] (first rot columns), v_t [heads vdim][ld_v] transposed with ld_v a multiple of 64, at least max_seq;
  * gates [M][heads] floats (before the sigmoid), out [M][heads vdim].  dim, rot, ld_rot: multiples of 8. */

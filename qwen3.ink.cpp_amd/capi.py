@@ -107,6 +107,7 @@ DENSE_SIGNATURES = {
     "a81w41_dense_gemm": (_i, [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _i, _vp]),
     "a81w41_dense_gated": (_i, [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, C.c_float, C.c_float, C.c_float, _i, _vp]),
     "a81w41_latent_attention": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _i, _i, C.c_float, _vp, _i, _i, _i, _vp, _vp, _vp]),
+    "a81w41_latent_token": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _vp, _i, C.c_float, _vp, _i, _vp, _vp, _vp]),
     "a81w41_formed_attention": (_i, [_vp, _vp, _vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _vp, _i, _i, C.c_float, _vp, _vp]),
     "a81w41_grouped_attention": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _i, _i, C.c_float, _i, _i, _vp, _i, _i, _i, _vp, _vp, _vp]),
     "a81w41_matrix_memory_state": (_sz, [_i, _i, _i]),

@@ -83,6 +83,20 @@ int a81w41_latent_attention(const void* q, const void* cache, int ld, int rank, 
     return 0;
 }
 
+int a81w41_latent_token(const void* q, const void* cache, int ld, int rank, int rot, int heads, int vdim, const int* pos_dev, int max_seq,
+                        float scale, const void* uv, int ld_uv, const float* gates, float* out, void* stream) {
+    LatentShape sh;
+    sh.heads = heads, sh.rot = rot, sh.vdim = vdim, sh.rank = rank, sh.ld_cache = ld, sh.scale = scale;
+    if (!q || !cache || !pos_dev || !uv || !gates || !out || rank < 8 || heads < 1 || vdim < 1 || max_seq < 1 || !latent_token_fits(sh) ||
+        ld < rank + rot || ld % 64 || ld_uv < rank || ld_uv % 8 || !aligned16(q) || !aligned16(cache) || !aligned16(uv))
+        return failf(A81W41_ERR_INVALID_ARG, "bad attention shape");
+    LatentRows in;
+    in.pos_dev = pos_dev, in.max_seq = max_seq;
+    A81W41_HIP_TRY(launch_latent_token(static_cast<const bf16*>(q), in, sh, static_cast<const bf16*>(cache), static_cast<const bf16*>(uv), ld_uv,
+                                       gates, out, static_cast<hipStream_t>(stream)));
+    return 0;
+}
+
 int a81w41_formed_attention(const void* q, const void* k, const void* k_rot, int ld_rot, const void* v_t, int ld_v, const float* gates,
                             int heads, int dim, int rot, int vdim, const int* pos_dev, int max_seq, int M, float scale, void* out,
                             void* stream) {

@@ -245,6 +245,18 @@ def latent_attention(q, cache, pos: int, rank: int, rot: int, heads: int, scale:
     return out
 
 
+def latent_token(q, cache, pos: int, rank: int, rot: int, scale: float, uv, gates):
+    """Parity hook a81w41_latent_token: q [heads][ld], cache [max_seq][ld], uv [heads][vdim][ld_uv] (bfloat16), gates [heads] fp32
+    -> fp32 [heads][vdim]."""
+    torch = _torch()
+    heads, vdim, ld_uv = uv.shape
+    out = torch.empty((heads, vdim), dtype=torch.float32, device=q.device)
+    pos_dev = torch.tensor([pos], dtype=torch.int32, device=q.device)
+    capi.check(capi.dense().a81w41_latent_token(_dev_ptr(q), _dev_ptr(cache), q.shape[1], rank, rot, heads, vdim, _dev_ptr(pos_dev),
+                                                cache.shape[0], scale, _dev_ptr(uv), ld_uv, _dev_ptr(gates), _dev_ptr(out), _stream()))
+    return out
+
+
 def formed_attention(q, k, k_rot, v_t, gates, pos: int, vdim: int, scale: float):
     """Parity hook a81w41_formed_attention: q [M][heads][dim+rot], k [max_seq][heads*dim], k_rot [max_seq][ld],
     v_t [heads*vdim][ld_v] (bfloat16), gates [M][heads] fp32 -> bfloat16 [M][heads*vdim]."""

@@ -30,7 +30,7 @@ def _close(got, want, what):
 
 
 @pytest.mark.parametrize("name", SIZES)
-@pytest.mark.parametrize("start", [0, 6, 125, 509])  # tiles of eight keys, sixteen waves of them, the last context of this form
+@pytest.mark.parametrize("start", [0, 6, 125, 509])  # whole passes there and past the last context of this form; each key by itself below
 def test_contexts(pkg, tmp_path, name, start):
     model, oracle = _model(pkg, tmp_path, name)
     ids = np.random.default_rng(start).integers(0, 67, start + 6).astype(np.int32)
@@ -57,3 +57,48 @@ def test_latents_held_and_not(pkg, tmp_path, q_rank, heads, rank, rot):
     model, oracle = pkg.Model.load(str(tmp_path), 64, "bfloat16"), tf.TakosunOracle(cfg, w)
     ids = np.random.default_rng(q_rank).integers(0, 67, 9).astype(np.int32)
     _close(np.concatenate([model.forward(ids[:3])] + [model.forward(ids[i:i + 1]) for i in range(3, 9)]), oracle.forward(ids)[2:], q_rank)
+
+
+# Every key counts: key j has a latent of one 1 at j % rank, so that each output is a sum over few keys with small whole factors, and weights
+# are all alike or powers of two by the rotated part.  The sums are exact in 32 bits; what is not is the scale (log2 e rounded, so weights
+# of exponents up to 6 are off by 6 x 2^-23), a division and the gate's sigmoid: 1e-5 holds all of it, and a key left out moves an output by
+# more than ten times that.  Tiles of eight keys, sixteen waves of them, the second and later turns of a wave; rows behind the token are
+# no numbers.
+KEYS = [0, 6, 7, 8, 9, 62, 63, 64, 126, 127, 128, 129, 134, 135, 136, 254, 255, 256, 383, 384, 504, 510, 511, 512, 640]
+
+
+@pytest.mark.parametrize("rank,rot,vdim", [(8, 2, 8), (24, 64, 40), (56, 10, 33), (512, 64, 512)])
+@pytest.mark.parametrize("alike", [True, False])
+def test_every_key_counts(pkg, rank, rot, vdim, alike):
+    import torch
+    heads, seq, scale = 3, 700, float(np.log(2.0))
+    ld = (rank + rot + 63) // 64 * 64
+    q = torch.zeros(heads, ld, dtype=torch.bfloat16)
+    rows = torch.zeros(seq, ld, dtype=torch.bfloat16)
+    j = torch.arange(seq)
+    rows[j, j % rank] = 1
+    if not alike:
+        for h in range(heads):   # each head by another column
+            q[h, rank + (h + 1) % rot] = 1
+            rows[:, rank + (h + 1) % rot] = -((j * (2 * h + 5)) % 7).to(torch.bfloat16)
+    uv = torch.zeros(heads, vdim, (rank + 7) // 8 * 8, dtype=torch.bfloat16)
+    c = torch.arange(rank)
+    for v in range(vdim):
+        uv[:, v, :rank] = torch.where(c % vdim == v % rank, 1 + c % 128, 0).to(torch.bfloat16)
+    gates = torch.tensor([0.3, -1.2, 2.5])
+    for pos in KEYS:
+        def attended(left_out=None):
+            s = q.double() @ rows[:pos + 1].double().t() * scale
+            if left_out is not None:
+                s[:, left_out] = -float("inf")
+            o = s.softmax(1) @ rows[:pos + 1, :rank].double()
+            return (uv[..., :rank].double() @ o[..., None])[..., 0] * gates.double().sigmoid()[:, None]
+        cache = rows.clone()
+        cache[pos + 1:] = float("nan")
+        got = pkg.ops.latent_token(q.cuda(), cache.cuda(), pos, rank, rot, scale, uv.cuda(), gates.cuda()).cpu().double()
+        want = attended()
+        bound = 1e-5 * want.abs()
+        assert ((got - want).abs() <= bound).all(), (pos, ((got - want).abs() - bound).max().item())
+        if pos in (6, 8, 128, 512):   # the bound sees each key left out of the oracle
+            for left_out in range(pos + 1):
+                assert ((attended(left_out) - want).abs() > 10 * bound).any(1).all(), (pos, left_out)
