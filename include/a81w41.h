@@ -114,12 +114,13 @@ int a81w41_gemm_repack_A81W41_fp32(const void *A_repack_dev, const void *B_repac
 int a81w41_gemm_repack_A81W41_fp32_static(const void *A_repack_dev, const void *B_repack_dev,
                                           float *C_dev, int M, int N, int K, void *stream);
 
-/* Test hook, host only (no device is touched): walks the work list the 64 x 64-tile kernel would be
- * launched with for an M x N x K call on a device that holds `resident_workgroups` of its workgroups on
- * `cus` compute units.  Returns the number of
- * partial tiles the K split parks (>= 0) if every tile and every K chunk is covered exactly
- * once, the tile numbering is one-to-one and no two chunks share a partial tile; a negative
- * code names the violated property. */
+/* Test hook, host only (no device is touched): walks the work that a launch on 64 x 64 tiles would do
+ * for an M x N x K call on a device that holds `resident_workgroups` of the kernel without teams on
+ * `cus` compute units: that kernel's work list or, where teams of waves share a tile, their shares of K,
+ * with a scratch for this call alone and with a layer object's.  Returns the number of
+ * partial tiles the K split of a call without a layer object parks (>= 0) if every tile and every K
+ * chunk is covered exactly once, the tile numbering is one-to-one and no two chunks share a partial
+ * tile; a negative code names the violated property. */
 int a81w41_gemm_schedule_selfcheck(int M, int N, int K, int resident_workgroups, int cus);
 
 /* Test hook, host only: the same for the layer object's M > 32 kernel (128 x 128 tiles, the (tile,

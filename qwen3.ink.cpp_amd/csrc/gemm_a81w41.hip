@@ -403,6 +403,16 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4,
     tile_kernel_body(A, B, C, M, N, nb_k, sc, partials, arrivals, lds, s_arrived);
 }
 
+// The super-blocks of a team where a tile's K range goes to c parts of `teams` teams each.
+struct TeamShare {
+    int k0, n_sb, n_steps;  // the team's super-blocks; steps of every team of the part
+};
+__host__ __device__ __forceinline__ TeamShare team_share(int nb_k, int c, int ch, int teams, int team) {
+    const int from = nb_k * ch / c, all = nb_k * (ch + 1) / c - from;
+    const int begin = all * team / teams;
+    return {from + begin, all * (team + 1) / teams - begin, (all + teams - 1) / teams};
+}
+
 // Few tiles: a workgroup of TEAMS times four waves takes one tile, or one of `c` parts of its K range, each team of four
 // waves an equal share of the super-blocks with a ring of its own, and their sums meet in LDS.  One such workgroup of four teams
 // fills a CU like four workgroups of the kernel above, two of two teams likewise; the four would have to be parts of a tile's K range
@@ -425,9 +435,8 @@ __global__ __launch_bounds__(kTileThreads * TEAMS) __attribute__((amdgpu_waves_p
     int tx, ty;
     tile_xy(tau, tiles_m, tiles_n, band, tx, ty);
     const int m_base = ty * Geom::kTileM, n_base = tx * Geom::kTileN;
-    const int from = nb_k * ch / c, all = nb_k * (ch + 1) / c - from;
-    const int begin = all * team / TEAMS, n_sb = all * (team + 1) / TEAMS - begin, n_steps = (all + TEAMS - 1) / TEAMS;
-    const int k0 = from + begin;
+    const TeamShare share = team_share(nb_k, c, ch, TEAMS, team);
+    const int k0 = share.k0, n_sb = share.n_sb, n_steps = share.n_steps;
     const TileRead rd = tile_places(row0, col0, r, kh);
     const TileDma dma = tile_copies(A, B, M, N >> 3, nb_k, m_base, n_base, wave, lane);
     const bool wave_live = m_base + row0 < M;
@@ -721,6 +730,19 @@ const char* gemm_kernel_name(int M, int N, int K) {
         case 0: return "rows (2..8 rows resident in LDS, v_dot4, weights streamed once)";
         case 3: return "rows32 (int8 matrix ops, one row panel, K split inside the workgroup)";
         case 4: return "rows32_staged (int8 matrix ops, one row panel, K split inside the workgroup, wave-private LDS stages)";
+        default: break;
+    }
+    std::lock_guard<std::mutex> lock(g_dev_mutex);
+    DeviceInfo* d = nullptr;
+    Schedule sc;
+    int grid = 0, teams = 0;
+    if (device_info_locked(d) == hipSuccess) {
+        make_schedule(M, N, K, d->slots, d->cus, kMaxPartials, sc, grid);
+        teams = plan_teams(sc, K / 64, d->cus, false).teams;
+    }
+    switch (teams) {
+        case 2: return "tile64_teams (int8 matrix ops, 64 x 64 tiles, K split between two teams of four waves)";
+        case 4: return "tile64_teams (int8 matrix ops, 64 x 64 tiles, K split between four teams of four waves)";
         default: return "tile64 (int8 matrix ops, 64 x 64 tiles, LDS-staged)";
     }
 }
@@ -854,13 +876,57 @@ hipError_t launch_gemm_fp32(const void* A, const void* B, float* C, int M, int N
     }
 }
 
-// Host-side check of the work list a launch would walk (no device needed): every whole tile once, every
+namespace {
+// The numbering of a launch's tiles is one-to-one onto the tiles.
+bool tile_numbers_ok(const Schedule& sc) {
+    const int T = sc.tiles_m * sc.tiles_n;
+    std::vector<int> seen((size_t)T, 0);
+    for (int tau = 0; tau < T; tau++) {
+        int x = -1, y = -1;
+        tile_xy(tau, sc.tiles_m, sc.tiles_n, sc.band, x, y);
+        if (x < 0 || x >= sc.tiles_n || y < 0 || y >= sc.tiles_m || seen[(size_t)y * sc.tiles_n + x]++) return false;
+    }
+    return true;
+}
+
+// A launch of the team kernel: every super-block of every tile in one team's share of one part, shares within the steps that all
+// teams of the part take, parts as many as the last to arrive adds up, their places distinct and in the scratch.
+int team_plan_selfcheck(const Schedule& sc, int nb_k, const TeamPlan& plan) {
+    const int T = sc.tiles_m * sc.tiles_n, c = plan.c;
+    if ((plan.teams != 2 && plan.teams != 4) || c < 1 || c > 4) return -8;
+    std::vector<int> part_used((size_t)kMaxPartials, 0);
+    for (int block = 0; block < T * c; block++) {
+        const int ch = block / T, tau = block - ch * T, part = tau * c + ch;
+        if (c > 1 && (part >= kMaxPartials || part_used[part]++)) return -9;
+    }
+    std::vector<int> covered((size_t)nb_k, 0);
+    for (int ch = 0; ch < c; ch++)
+        for (int team = 0; team < plan.teams; team++) {
+            const TeamShare share = team_share(nb_k, c, ch, plan.teams, team);
+            if (share.n_sb < 0 || share.n_sb > share.n_steps) return -10;
+            for (int u = 0; u < share.n_sb; u++)
+                if (share.k0 + u < 0 || share.k0 + u >= nb_k || covered[share.k0 + u]++) return -11;
+        }
+    for (int k = 0; k < nb_k; k++)
+        if (covered[k] != 1) return -12;
+    return tile_numbers_ok(sc) ? 0 : -7;
+}
+}  // namespace
+
+// Host-side check of the work that a launch would do (no device needed), with a scratch that is there for every call and with one
+// that is there where K has to be split: the team kernel's shares, or the list of the kernel without teams, every whole tile once, every
 // chunk of every split tile once, partial-tile indices distinct and below the scratch size.
 int gemm_schedule_selfcheck(int M, int N, int K, int slots_fit, int cus) {
     Schedule sc;
     int grid = 0;
     if (!make_schedule(M, N, K, slots_fit, cus, kMaxPartials, sc, grid)) return -1;
     const int T = sc.tiles_m * sc.tiles_n, nb_k = K / 64;
+    const TeamPlan teams = plan_teams(sc, nb_k, cus, false);
+    if (teams.teams) {
+        for (const TeamPlan& plan : {teams, plan_teams(sc, nb_k, cus, true)})
+            if (const int bad = team_plan_selfcheck(sc, nb_k, plan)) return bad;
+        return teams.c > 1 ? T * teams.c : 0;
+    }
     if (sc.whole + sc.r != T || sc.items != sc.whole + sc.r * sc.c || sc.chunk * sc.c != nb_k) return -2;
     if (grid < 1 || grid > slots_fit) return -3;
     std::vector<int> covered((size_t)T, 0), part_used((size_t)kMaxPartials, 0);
@@ -877,13 +943,7 @@ int gemm_schedule_selfcheck(int M, int N, int K, int slots_fit, int cus) {
         }
     for (int t = 0; t < T; t++)
         if (covered[t] != nb_k) return -6;
-    // the tile numbering is one-to-one onto the tiles
-    std::vector<int> seen((size_t)T, 0);
-    for (int tau = 0; tau < T; tau++) {
-        int x = -1, y = -1;
-        tile_xy(tau, sc.tiles_m, sc.tiles_n, sc.band, x, y);
-        if (x < 0 || x >= sc.tiles_n || y < 0 || y >= sc.tiles_m || seen[(size_t)y * sc.tiles_n + x]++) return -7;
-    }
+    if (!tile_numbers_ok(sc)) return -7;
     return sc.r * sc.c;
 }
 

@@ -95,6 +95,21 @@ def test_gemm_schedule_covers_every_tile_and_chunk_once(pkg):
     assert L.a81w41_gemm_schedule_selfcheck(0, 64, 64, 1024, 256) < 0   # argument errors are negative too
 
 
+def test_gemm_schedule_follows_the_teams(pkg):
+    """Few tiles go to teams of waves on a tile: the check walks their shares, from one super-block of K on, with K that no ring or
+    part divides, and reports the partial tiles of that plan and not of the list that is not launched."""
+    L = pkg.capi.lib()
+    for K in (64, 128, 192, 256, 320, 704, 1408, 1472, 2048, 2112, 3712, 4096, 4160, 6144, 12288, 12352):
+        for N in (8, 72, 1024, 2504, 4096, 12288):
+            for M in (33, 40, 64, 65, 90, 120, 180, 250, 322):
+                for cus in (256, 64, 4):
+                    got = L.a81w41_gemm_schedule_selfcheck(M, N, K, 4 * cus, cus)
+                    assert 0 <= got <= 4096, (M, N, K, cus, got)
+    # 128 tiles: two parts of four teams, not the list's four; 64: four parts; 192 over 4608: none; K that is no multiple of 512: none
+    for M, N, K, parts in ((128, 4096, 4096, 256), (57, 4096, 12288, 256), (192, 4096, 4608, 0), (40, 2504, 3712, 0)):
+        assert L.a81w41_gemm_schedule_selfcheck(M, N, K, 1024, 256) == parts, (M, N, K)
+
+
 def test_block_scaled_gemm_plan_covers_every_unit_once(pkg):
     """The layer object's M > 32 kernel cuts the (tile, 32-block) units of a launch into equal contiguous runs:
     walked on the host for the layer's shapes and odd ones, for several device sizes."""
