@@ -551,7 +551,15 @@ struct DeviceInfo {
 DeviceInfo g_dev[kMaxDevices];
 std::mutex g_dev_mutex;
 
-// Occupancy and CU count of the current device (queried once per device); g_dev_mutex held.
+// The rings of the teams, and beside them the kernel's own word: more than the 64 KiB a kernel has unasked, with two teams too.
+template <int TEAMS>
+hipError_t allow_team_lds() {
+    static_assert(TEAMS * Geom::kLdsBytes + sizeof(unsigned) > 64 * 1024 && TEAMS * Geom::kLdsBytes + 16 <= 160 * 1024, "LDS of a CU");
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_a81w41_team_kernel<TEAMS>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               TEAMS * Geom::kLdsBytes);
+}
+
+// Occupancy and CU count of the current device, and what its kernels have to be allowed (once per device); g_dev_mutex held.
 hipError_t device_info_locked(DeviceInfo*& out) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -566,6 +574,7 @@ hipError_t device_info_locked(DeviceInfo*& out) {
         e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         if (e != hipSuccess) return e;
         if (per_cu < 1 || cus < 1) return hipErrorInvalidValue;
+        if ((e = allow_team_lds<2>()) != hipSuccess || (e = allow_team_lds<4>()) != hipSuccess) return e;
         d.cus = cus;
         d.slots = per_cu * cus;
     }
@@ -660,13 +669,7 @@ TeamPlan plan_teams(const Schedule& sc, int nb_k, int cus, bool may_split) {
 
 template <int TEAMS>
 hipError_t launch_teams(const void* A, const void* B, float* C, int M, int N, int nb_k, const Schedule& sc, int c, const GemmScratch& ws, hipStream_t s) {
-    const int lds = TEAMS * Geom::kLdsBytes;
-    if (lds > 64 * 1024) {  // asked per call: per device, no shared flag
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_a81w41_team_kernel<TEAMS>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(gemm_a81w41_team_kernel<TEAMS>, dim3(sc.tiles_m * sc.tiles_n * c), dim3(TEAMS * kTileThreads), lds, s,
+    hipLaunchKernelGGL(gemm_a81w41_team_kernel<TEAMS>, dim3(sc.tiles_m * sc.tiles_n * c), dim3(TEAMS * kTileThreads), TEAMS * Geom::kLdsBytes, s,
                        static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(B), M, N, nb_k, sc.tiles_m, sc.tiles_n, c, sc.band, C,
                        ws.partials, ws.arrivals);
     return hipGetLastError();
