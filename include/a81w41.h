@@ -98,7 +98,11 @@ int a81w41_gemv_repack_A81W41_fp16(const void *A_repack_dev, const void *B_repac
  * stream are ordered by the stream, calls on different streams use different scratches, so
  * no two launches share partial tiles -- with one caveat: a captured graph keeps the
  * scratch of the stream it was captured on wherever it is replayed, so its replays must
- * not overlap with K-split calls on that stream.  Results do not depend on timing. */
+ * not overlap with K-split calls on that stream.  Results do not depend on timing.
+ * A layer object's scratch is there from the start, so a81w41_linear_forward may split K where this call
+ * does not, so as not to need a scratch: at most as many tiles of 64 x 64 as half the CUs and K > 2048 no
+ * multiple of 512.  The two then sum in different orders and agree to the rounding of 32-bit sums;
+ * otherwise, where both run on 64 x 64 tiles, they agree in every bit. */
 int a81w41_gemm_repack_A81W41_fp32(const void *A_repack_dev, const void *B_repack_dev, float *C_dev,
                                    int M, int N, int K, void *stream);
 
@@ -214,7 +218,8 @@ void a81w41_linear_destroy(a81w41_linear *layer);
 size_t a81w41_linear_resident_bytes(const a81w41_linear *layer, size_t *fp16_blob, size_t *fp32_blob,
                                     size_t *block_scaled);
 /* Which kernel a forward call of M rows of this layer runs on (a static string for reports:
- * "gemv ...", "rows ...", "rows_fused ...", "rows32 ...", "rows32_staged ...", "tile64 ...", "block_scaled ..."). */
+ * "gemv ...", "rows ...", "rows_fused ...", "rows32 ...", "rows32_staged ...", "tile64 ...",
+ * "tile64_teams ...", "block_scaled ..."). */
 const char *a81w41_linear_kernel_name(const a81w41_linear *layer, int M);
 int a81w41_linear_in_features(const a81w41_linear *layer);  /* K */
 int a81w41_linear_out_features(const a81w41_linear *layer); /* N */

@@ -570,6 +570,23 @@ def test_current_stream_and_output_rows(pkg):
         assert type(out) is torch.Tensor and out.dtype is torch.float32 and out.shape == (2, 3, 24) and out.is_cuda and not out.requires_grad
 
 
+# A layer's scratch is there for every call, the free-standing call has none where it can do without: few tiles over a K past 2048 that is no
+# multiple of 512 are cut by the one and not by the other, and nothing else is.
+@pytest.mark.parametrize("M,N,K,alike", [(130, 136, 2048, True), (40, 2504, 1472, True), (40, 2504, 4096, True), (250, 4096, 4096, True),
+                                         (300, 4096, 2496, True), (90, 4104, 2496, True), (40, 2504, 3712, False), (90, 4096, 2496, False),
+                                         (64, 4096, 12352, False)])
+def test_layer_and_free_standing_call_on_few_tiles(pkg, ora, synth, torch, M, N, K, alike):
+    w4, scale, offset = synth.weight_files(N, K, seed=M)
+    layer = pkg.Linear.from_arrays(w4, scale, offset, N=N, K=K)
+    layer.set_kernel("int8")
+    x = dev(torch, synth.activations(M, K, seed=N, outliers=True))
+    got = layer.forward(x)
+    alone = pkg.ops.gemm_fp32(pkg.ops.quantize(x, True), dev(torch, ora.repack(w4, scale, offset, K, N, fp32=True)), M, N, K)
+    assert torch.equal(got, alone) == alike
+    # fp32 sums of K / 32 terms in another order: 2^-24 of the row each, with room for their cancellation
+    assert row_err(got.cpu().numpy(), alone.cpu().numpy()) < K / 32 * 2.0 ** -24 * 4 + 2e-6
+
+
 # Teams of four waves on one tile: two teams, four; a tile's K range whole, in two and in four parts (a layer's scratch; without it whole);
 # fewer super-blocks than teams, counts that no team divides, ragged rows and columns; between one and two tiles a CU.
 @pytest.mark.parametrize("M,N,K", [(40, 64, 64), (33, 72, 192), (64, 1000, 1408), (130, 136, 2048), (65, 520, 2112), (57, 4096, 2496),
