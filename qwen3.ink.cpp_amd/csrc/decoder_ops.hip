@@ -18,29 +18,8 @@ __device__ __forceinline__ float to_float(__half h) { return __half2float(h); }
 __device__ __forceinline__ float to_float(Bf16Bits b) { return __uint_as_float((unsigned)b.bits << 16); }
 __device__ __forceinline__ float to_float(float f) { return f; }
 
-// Eight values per load where the rows allow it (hidden and the row stride multiples of 8, 16-byte aligned).
-template <typename E>
-__global__ __launch_bounds__(256) void embed_rows_kernel(const int* __restrict__ ids, const E* __restrict__ table, int ld,
-                                                       float* __restrict__ out, int hidden, int vocab) {
-    const int m = blockIdx.x;
-    const int id = min(max(ids[m], 0), vocab - 1);
-    const E* row = table + (size_t)id * ld;
-    float* dst = out + (size_t)m * hidden;
-    if (sizeof(E) == 2 && ((hidden | ld) & 7) == 0) {
-        const uint4* row4 = reinterpret_cast<const uint4*>(row);
-        float4* dst4 = reinterpret_cast<float4*>(dst);
-        for (int j = threadIdx.x; j < (hidden >> 3); j += 256) {
-            const uint4 u = row4[j];
-            const E* e = reinterpret_cast<const E*>(&u);
-            dst4[2 * j] = make_float4(to_float(e[0]), to_float(e[1]), to_float(e[2]), to_float(e[3]));
-            dst4[2 * j + 1] = make_float4(to_float(e[4]), to_float(e[5]), to_float(e[6]), to_float(e[7]));
-        }
-    } else {
-        for (int j = threadIdx.x; j < hidden; j += 256) dst[j] = to_float(row[j]);
-    }
-}
-
-// One embedding row by a whole workgroup, as embed_rows_kernel writes it.
+// One embedding row by a whole workgroup.  Eight values per load where the rows allow it (hidden and the row stride multiples of 8, 16-byte
+// aligned).
 template <typename E>
 __device__ __forceinline__ void embed_row(const TokenRow& r, int id) {
     const E* row = static_cast<const E*>(r.table) + (size_t)id * r.ld;
@@ -63,6 +42,11 @@ __device__ __forceinline__ void embed_token(const TokenRow& r, int id) {
         case TableType::kBf16: return embed_row<Bf16Bits>(r, id);
         case TableType::kFp32: return embed_row<float>(r, id);
     }
+}
+// rows: that of the first of the tokens
+__global__ __launch_bounds__(256) void embed_rows_kernel(const int* __restrict__ ids, TokenRow rows) {
+    rows.out += (size_t)blockIdx.x * rows.hidden;
+    embed_token(rows, ids[blockIdx.x]);
 }
 
 // of two candidates the larger value, of equal values the lower index; a NaN is no candidate
@@ -163,20 +147,7 @@ __global__ void advance_kernel(int* __restrict__ pos_dev, int by) {
 
 hipError_t launch_embed_rows(const int* ids, const void* table, TableType type, int ld, float* out, int M, int hidden, int vocab,
                              hipStream_t s) {
-    switch (type) {
-        case TableType::kFp16:
-            hipLaunchKernelGGL(embed_rows_kernel<__half>, dim3(M), dim3(256), 0, s, ids, static_cast<const __half*>(table), ld, out,
-                               hidden, vocab);
-            break;
-        case TableType::kBf16:
-            hipLaunchKernelGGL(embed_rows_kernel<Bf16Bits>, dim3(M), dim3(256), 0, s, ids, static_cast<const Bf16Bits*>(table), ld,
-                               out, hidden, vocab);
-            break;
-        case TableType::kFp32:
-            hipLaunchKernelGGL(embed_rows_kernel<float>, dim3(M), dim3(256), 0, s, ids, static_cast<const float*>(table), ld, out,
-                               hidden, vocab);
-            break;
-    }
+    hipLaunchKernelGGL(embed_rows_kernel, dim3(M), dim3(256), 0, s, ids, TokenRow{table, type, ld, out, hidden, vocab});
     return hipGetLastError();
 }
 static hipError_t next_token(const float* logits, int n, int* next_id, int* history, int history_len, int* step_dev, int* pos_dev, int by,

@@ -421,8 +421,10 @@ hipError_t launch_grouped(const GemmArgs& g, const X& heads, hipStream_t s) {
 
 template <typename T, Epilogue EPI, typename X>
 hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
-    if constexpr (EPI == Epilogue::kGatedPair || EPI == Epilogue::kFloat)
-        if (g.tiles) return launch_grouped<T, EPI>(g, heads, s);
+    if (g.tiles) {
+        if constexpr (EPI == Epilogue::kGatedPair || EPI == Epilogue::kFloat) return launch_grouped<T, EPI>(g, heads, s);
+        return hipErrorInvalidValue;
+    }
     auto tiles = [&](int rows, int cols) { return (long long)((g.M + rows - 1) / rows) * ((g.N + cols - 1) / cols) * g.batches; };
     // One round of a tile for each CU, three quarters full or more; a tile has the larger one's stages and waves, so that its rows and
     // weights are under way early.  That takes some steps of K to pay: before the last of them are under way nothing fills the CU.
