@@ -78,7 +78,9 @@ struct GroupTile {
     int expert, first, row0, rows;
 };
 // How high the tiles are, for `rows` rows in all.  us of gate and up / down with 64 / 128 rows a tile, width 2048, units of 1024:
-// 256 rows for an expert on average 130.8 / 69.8 and 121.4 / 67.1, 128 rows 84.9 / 46.5 and 82.0 / 44.8, 75 rows 69.5 / 35.5 and 86.3 / 43.5.
+// 256 rows for an expert on average 137.3 / 77.3 and 128.5 / 68.7, 128 rows 88.5 / 48.5 and 90.3 / 47.6, 75 rows 72.3 / 38.6 and 91.4 / 45.7.
+// Narrower products would want the line later: width 1536, units of 768, 128 rows 51.8 / 31.2 and 62.9 / 37.3, 256 rows 81.4 / 49.8 and 74.6 / 41.3;
+// width 1024, units of 512, 256 rows 40.6 / 27.4 and 45.8 / 27.6.
 constexpr int kGroupTileRows = 64, kGroupTileManyRows = 128;
 inline int group_tile_rows(long long rows, int experts) { return rows >= 128LL * experts ? kGroupTileManyRows : kGroupTileRows; }
 struct GemmArgs {

@@ -400,16 +400,17 @@ hipError_t launch_grouped(const GemmArgs& g, const X& heads, hipStream_t s) {
     auto panels = [&](int width) { return (long long)((g.N + width - 1) / width); };
     if (g.tile_rows == kGroupTileManyRows) {
         // One 128 x 256 tile on a CU where its rounds of 256 come out seven tenths full or more, half of the experts' last tiles being
-        // there, otherwise two 128 x 128.  us, the second / the first: 2048 tokens of 4 experts out of 32, 2048 x 2048 gated 124.9 /
-        // 121.4, 1536 x 1536 66.1 / 63.5; 0.63 of two rounds full, 1024 x 1024 39.5 / 41.5.
+        // there, otherwise two 128 x 128.  us of gate and up + down, the second / the first: 2048 tokens of 4 experts out of 32, 2048 x 2048
+        // 128.7 + 70.5 / 128.5 + 68.7, 1536 x 1536 74.2 + 44.8 / 74.6 + 41.3; 0.63 of two rounds full, 1024 x 1024 45.4 + 27.4 / 47.6 + 28.2.
         const int whole = g.M / kGroupTileManyRows;
         const long long tiles = (whole + g.max_tiles) / 2 * panels(256), rounds = (tiles + 255) / 256;
         if (10 * tiles >= 7 * 256 * rounds) return launch_kernel<T, kGroupTileManyRows, 256, 2, 4, 3, true, EPI>(g, heads, s);
         return launch_kernel<T, kGroupTileManyRows, 128, 2, 2, 2, true, EPI>(g, heads, s);
     }
     // 64 x 128 tiles with two stages fit a CU three times, with three stages twice and have more of the weights under way, which counts where
-    // there are few rounds.  us with two / three: 600 tokens of 4 out of 32, 2048 x 2048 gated 80.5 / 69.5, 64 tokens 64.3 / 63.2, 16
-    // tokens, 1024 x 1024 15.7 / 12.1; 2048 tokens, 1024 x 1024 36.4 / 38.0.
+    // there are few rounds.  us of gate and up with two / three: 600 tokens of 4 out of 32, 2048 x 2048 82.4 / 72.3, 64 tokens 62.5 / 60.0,
+    // 16 tokens, 1024 x 1024 13.4 / 10.9.  Past the line prompts of 760 to 1020 tokens at width 2048 take 0.96 to 0.98 of the time with three as
+    // well; where 512 to 768 tiles are there, one round with two stages and two with three, 830 to 1020 tokens at width 1024 take 1.01 to 1.02 of it.
     if (g.N >= 1024) {
         if (g.max_tiles * panels(128) <= 1200) return launch_kernel<T, kGroupTileRows, 128, 2, 4, 3, true, EPI>(g, heads, s);
         return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, true, EPI>(g, heads, s);
