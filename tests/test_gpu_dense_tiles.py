@@ -245,7 +245,8 @@ def test_one_token_rows(pkg, width):
         assert np.linalg.norm(got[i] - want) <= 3e-5 * np.linalg.norm(want), i
 
 
-# One round of 128 x 256 tiles, of 64 x 256 and of 64 x 128, three stages each: fewer steps than stages, as many, more; ragged rows and columns
+# Sizes of one round of 128 x 256 tiles, of 64 x 256 and of 64 x 128, three stages each, ragged rows and columns: fewer steps than stages, as many
+# and more for 64 x 256; the others are taken from some steps on, below, and these K lie on both sides of the line
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 448])
 @pytest.mark.parametrize("M,N", [(2045, 3100), (300, 12280), (1000, 2000)])
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
@@ -279,6 +280,13 @@ def test_one_round_from_some_steps_on(pkg, M, N, dtype, steps):
         bound = (1 if bf16 else 2) * K * 2.0 ** -24 * 4 * K ** 0.5
         assert (got.double() - a.double() @ w.double().t()).abs().max().item() <= bound, n
         assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:]), n
+
+
+# One round of 128 x 256 tiles over enough steps for it, with the epilogues of a prompt: queries turned and stored, gated units, columns of
+# heads with what is no head's behind them; the same rows in portions go through small tiles.
+def test_epilogues_on_one_round_of_tiles(pkg):
+    _same_in_portions(pkg, tx.config(64, 704, 1, [tx.layer(tx.mixer(16, 128, 64, 8, 704, 24, 0.1), tx.dense(1552))]), 2045, 100)
+    _same_in_portions(pkg, dx.config(64, 704, [dx.attention(16, 4, 128, 128, 70, 0.09, rot_dims=64, mlp=None)], (0, 1, 1)), 2045, 100)
 
 
 # Experts' rows in tiles of 128 (one pass) and of 64 (portions): 128 x 256 and 128 x 128 tiles, 64 x 128 with two and three stages, 64 x 64;
