@@ -86,10 +86,10 @@ __device__ __forceinline__ void store_a6_block(uint8_t* __restrict__ a6, int row
         if (chunk == 0) {
             v = make_uint4(dw[0], dw[1], dw[2], dw[3]);
         } else {
-            // the scaled sum as three bf16 pieces: hi | mid in the high piece's copy (read by lanes 0..31 of the
-            // contraction kernel), lo in the low piece's copy (lanes 32..63)
+            // the scaled sum as three bf16 pieces, as the contraction multiplies them: hi | hi in the high piece's copy, mid | lo in
+            // the low piece's
             const uint2 s3 = split_bf16x3(ssum);
-            v = make_uint4(dw[4], dw[5], __float_as_uint(d), piece == 0 ? s3.x : s3.y);
+            v = make_uint4(dw[4], dw[5], __float_as_uint(d), piece == 0 ? __builtin_amdgcn_perm(s3.x, s3.x, 0x01000100u) : s3.x >> 16 | s3.y << 16);
         }
         uint8_t* dst = a6 + ((size_t)(row >> 5) * nb + blk) * kPanelA + piece * 1024 + chunk * 512 + (row & 31) * 16;
         *reinterpret_cast<uint4*>(dst) = v;

@@ -23,8 +23,8 @@
 //   W6: per (32-column panel, 32-block) 1 KiB: chunk 0 = [32 columns][16 B] fp6 codes k = 0..20 (+2 bits),
 //       chunk 1 = [32 columns][16 B] rest of the codes (8 B), dW (fp32), mW as two bf16 pieces (hi | lo << 16).
 //   A6: per (32-row panel, 32-block) 2 KiB: piece 0 (qh) then piece 1 (ql), each laid out like a W6 panel
-//       with dA (fp32) and two of the scaled sum's three bf16 pieces in chunk 1: hi | mid in piece 0's copy, lo in
-//       piece 1's (the two lane halves of the contraction kernel exchange them).
+//       with dA (fp32) and two of the scaled sum's bf16 pieces in chunk 1, as the min term multiplies them: hi | hi in
+//       piece 0's copy, mid | lo in piece 1's.
 // A lane reads its operand with two 16-byte loads; lanes of a half-wave read consecutive 16 bytes.
 //
 // Tiling: 128 x 256 tiles of C per workgroup, 8 waves of 64 x 64 (two row panels against two column panels),
@@ -165,6 +165,11 @@ __host__ __device__ __forceinline__ int run_owner(const Plan& p, long long u) { 
 // Dwords 0..5 are the matrix op's operand (a 32 x 6-bit operand occupies six registers; the op does not look at
 // the other two), dwords 6 and 7 the two parameters.
 typedef v8i Frag;
+// An operand in eight registers one behind the other: the matrix op takes the first six where they are.  Without this the compiler loads the second
+// half elsewhere, copies two registers of it and waits for that load in the middle of the block ahead of the one that uses it.  2047 rows, 12288 x
+// 4096, us a call: 277; with the min terms' operands as they are read (instead of selected by lane half and exchanged between the
+// halves) 271; and with this 264.
+__device__ __forceinline__ void whole(Frag& f) { asm("" : "+v"(f)); }
 
 __device__ __forceinline__ Frag read_frag(const uint8_t* p) {
     const v4i lo = *reinterpret_cast<const v4i*>(p), hi = *reinterpret_cast<const v4i*>(p + 512);
@@ -184,6 +189,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // E8M0 block scales: patterns are integers / 8 on both sides (2^3 each); the qh piece counts 16-fold
     const int scale_a = 127 + 3 + 4 * (1 - h), scale_b = 127 + 3;
     const uint32_t lane_a = (uint32_t)h * 1024u + (uint32_t)r * 16u, lane_b = (uint32_t)r * 16u;
+
+    const uint32_t min_select = h ? 0x01000100u : 0x03020100u;
 
     // Workgroups are dealt to the 8 XCDs round robin; run = (XCD, index inside it) makes an XCD's runs
     // neighbours in the unit space, so that the row tiles of a column panel (which share its weights) and
@@ -226,25 +233,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             for (int j = 0; j < 2; j++) acc[i][j] = v16f{0};
         const bool rows_live = kTileM * ty + 64 * wr < M;  // else every row of this wave is past M
 
-        // min terms of up to four 32-blocks (zero pieces where the run ends early): lane half 0 brings blocks 0 and 1,
-        // half 1 blocks 2 and 3, four K slots per block: (s_hi, s_hi, s_mid, s_lo) against (w_hi, w_lo, w_hi, w_hi).
-        // Lanes 0..31 read hi | mid of a scaled sum, lanes 32..63 its lo: ya = this lane's word for the half's own
-        // two blocks, za = its word for the other half's two blocks, which the partner lane (same row, other half)
-        // needs; one exchange per block gives every lane all three pieces of its own blocks.
-        auto min_terms = [&](const uint32_t (&ya)[2][2], const uint32_t (&za)[2][2], const uint32_t (&yb)[2][2]) {
-            v4i opa[2], opb[2];
+        // Min terms of up to four 32-blocks, each with two K slots of either lane half: half 0 brings (s_hi, s_hi) against (w_hi, w_lo), half 1
+        // (s_mid, s_lo) against (w_hi, w_hi).  An activation operand's last word is that as it was read; blocks that are not there have zeros.
+        v4i opa[2], opb[2];
+        auto keep_min = [&](int k, const Frag (&fa)[2], const Frag (&fb)[2]) {
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-#pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    const uint32_t got = (uint32_t)__shfl_xor((int)za[i][k], 32, 64);
-                    const uint32_t himid = h ? got : ya[i][k], lo = h ? ya[i][k] : got;
-                    opa[i][2 * k] = (int)__builtin_amdgcn_perm(himid, himid, 0x01000100u);  // hi, hi
-                    opa[i][2 * k + 1] = (int)((himid >> 16) | (lo << 16));                       // mid, lo
-                    opb[i][2 * k] = (int)yb[i][k];                                                  // hi, lo
-                    opb[i][2 * k + 1] = (int)__builtin_amdgcn_perm(yb[i][k], yb[i][k], 0x01000100u);  // hi, hi
-                }
+                opa[i][k] = fa[i][7];
+                opb[i][k] = (int)__builtin_amdgcn_perm((uint32_t)fb[i][7], (uint32_t)fb[i][7], min_select);
             }
+        };
+        auto min_terms = [&]() {
             typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
             auto bf = [](const v4i& v) { return __builtin_bit_cast(v8bf, v); };
 #pragma unroll
@@ -276,28 +275,32 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         if (rows_live) {
             Frag fa[2][2], fb[2][2];  // two sets: the one in use and the next step's, in flight
             load_step(0, fa[0], fb[0]);
-            for (int step0 = 0; step0 < n_steps; step0 += 4) {
-                uint32_t ya[2][2] = {{0, 0}, {0, 0}}, za[2][2] = {{0, 0}, {0, 0}}, yb[2][2] = {{0, 0}, {0, 0}};
+            auto block = [&](int k, int step) {
+                __builtin_amdgcn_sched_barrier(0);
+                load_step(step + 1, fa[(k + 1) & 1], fb[(k + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+                whole(fa[k & 1][0]);
+                whole(fb[k & 1][0]);
+                whole(fa[k & 1][1]);
+                whole(fb[k & 1][1]);
+                keep_min(k, fa[k & 1], fb[k & 1]);
+                compute(fa[k & 1], fb[k & 1]);
+            };
+            int step = 0;
+            for (; step + 4 <= n_steps; step += 4) {
 #pragma unroll
-                for (int u4 = 0; u4 < 4; u4++) {
-                    const int step = step0 + u4;
-                    if (step >= n_steps) break;  // uniform over the workgroup
-                    load_step(step + 1, fa[(u4 + 1) & 1], fb[(u4 + 1) & 1]);
-                    const Frag(&ca)[2] = fa[u4 & 1];
-                    const Frag(&cb)[2] = fb[u4 & 1];
-                    if ((u4 >> 1) == h) {  // this lane half's block: keep its min-term pieces
+                for (int k = 0; k < 4; k++) block(k, step + k);
+                min_terms();
+            }
+            if (step < n_steps) {
 #pragma unroll
-                        for (int i = 0; i < 2; i++) {
-                            ya[i][u4 & 1] = (uint32_t)ca[i][7];
-                            yb[i][u4 & 1] = (uint32_t)cb[i][7];
-                        }
-                    } else {  // the other half's block: the partner lane needs this lane's word of its scaled sums
-#pragma unroll
-                        for (int i = 0; i < 2; i++) za[i][u4 & 1] = (uint32_t)ca[i][7];
-                    }
-                    compute(ca, cb);
+                for (int k = 0; k < 4; k++) {
+                    if (step + k < n_steps)
+                        block(k, step + k);
+                    else
+                        opa[0][k] = opa[1][k] = opb[0][k] = opb[1][k] = 0;
                 }
-                min_terms(ya, za, yb);
+                min_terms();
             }
         }
 
