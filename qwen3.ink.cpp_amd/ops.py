@@ -30,12 +30,13 @@ def _stream():
 
 
 def _float_rows(x, cols: int):
-    """Uninitialised float32 [...][cols] beside x [...][k].  A plain float tensor makes it in 1.5 us, torch.empty in 2.5."""
+    """Uninitialised float32 [...][cols] beside x [...][k].  For two dimensions of a plain float tensor the sizes go to the call as they are: 1.1 us,
+    as a shape that is cut out of x's and put together 1.9; torch.empty takes 2.5.  A call of one row, 1024 x 4096, which the host's
+    way to the launch bounds: 7.2 us, so 6.5."""
     torch = _torch()
-    shape = x.shape[:-1] + (cols,)
     if type(x) is torch.Tensor and x.dtype is torch.float32:
-        return x.new_empty(shape)
-    return torch.empty(shape, dtype=torch.float32, device=x.device)
+        return x.new_empty(x.size(0), cols) if x.dim() == 2 else x.new_empty(x.shape[:-1] + (cols,))
+    return torch.empty(x.shape[:-1] + (cols,), dtype=torch.float32, device=x.device)
 
 
 def _np_ptr(a: np.ndarray):
