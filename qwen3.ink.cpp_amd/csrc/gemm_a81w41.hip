@@ -213,16 +213,18 @@ __device__ __forceinline__ void tile_epilogue(const TileProd& F, v16f& acc) {
 // Work list of one launch.  Tiles are numbered so that column panels x = 8*j + c go to the
 // workgroups with index = c (mod 8), which share an XCD and its L2, with the row tiles of a
 // panel next to each other.  Items [0, whole) are whole tiles; the remaining r tiles (the last,
-// partial round of the persistent grid) have their K range cut into c chunks each, item
+// partial round of the persistent grid) have their K range cut into c chunks each, equal but for one super-block, item
 // whole + ch*r + tr being chunk ch of tile whole + tr.  Workgroup b takes items b, b + grid, ...
 // Workgroups are dispatched in index order and the SIMDs favour the older of two resident
 // waves, so the low-index workgroups, which get the extra items, are also the faster ones.
 struct Schedule {
     int tiles_m, tiles_n;
-    int whole, r, c, chunk;
+    int whole, r, c;
     int items;
     int band;  // row tiles per band (see tile_xy)
 };
+
+__host__ __device__ __forceinline__ int chunk_start(int nb_k, int c, int ch) { return nb_k * ch / c; }
 
 // Within an XCD (c = tau mod 8) the tiles are walked band by band: `band` row tiles high, all of the
 // XCD's column panels wide, row tiles of a panel next to each other.  The workgroups of an XCD that
@@ -284,8 +286,8 @@ __device__ __forceinline__ void tile_kernel_body(const uint8_t* __restrict__ A, 
             const int k = item - sc.whole;
             const int tr = k % sc.r, ch = k / sc.r;
             tau = sc.whole + tr;
-            k0 = ch * sc.chunk;
-            n_sb = sc.chunk;
+            k0 = chunk_start(nb_k, sc.c, ch);
+            n_sb = chunk_start(nb_k, sc.c, ch + 1) - k0;
             part = tr * sc.c + ch;
         }
         int tx, ty;
@@ -396,10 +398,10 @@ __device__ __forceinline__ void tile_kernel_body(const uint8_t* __restrict__ A, 
 // split scratch, needed at the end of a tile only, follow.
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_a81w41_tile64_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int nb_k, int tiles_m, int tiles_n, int whole,
-    int r, int c, int chunk, int band, float* __restrict__ C, float* __restrict__ partials, unsigned* __restrict__ arrivals) {
+    int r, int c, int band, float* __restrict__ C, float* __restrict__ partials, unsigned* __restrict__ arrivals) {
     extern __shared__ __align__(16) uint8_t lds[];  // kRing stages
     __shared__ unsigned s_arrived;
-    const Schedule sc = {tiles_m, tiles_n, whole, r, c, chunk, whole + r * c, band};
+    const Schedule sc = {tiles_m, tiles_n, whole, r, c, whole + r * c, band};
     tile_kernel_body(A, B, C, M, N, nb_k, sc, partials, arrivals, lds, s_arrived);
 }
 
@@ -587,9 +589,13 @@ __global__ void clear_counters_kernel(unsigned* p, int n) {
     if (i < n) p[i] = 0u;
 }
 
+// Without a scratch for every call K is cut only where its super-blocks divide evenly into rings.  With one (any_split), chunks are equal but for one
+// super-block and have sixteen or more.
+constexpr int kMinChunk = 16;
+
 // The schedule of one launch (see Schedule): a pure function of the shape and of the device's size.
 // Returns false when the K split the shape calls for needs more than max_partials partial tiles.
-bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials, Schedule& sc, int& grid) {
+bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials, bool any_split, Schedule& sc, int& grid) {
     const int nb_k = K / 64;
     sc.tiles_m = (M + Geom::kTileM - 1) / Geom::kTileM;
     sc.tiles_n = (N + Geom::kTileN - 1) / Geom::kTileN;
@@ -611,7 +617,7 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     // Split the last, partial round: in two, so that the chunks go to the first (faster) half
     // of the grid; in four when even then less than 3/4 of the grid would have one.
     int c = 1;
-    auto valid = [&](int cc) { return cc >= 1 && cc <= 16 && nb_k % (Geom::kRing * cc) == 0 && (long long)sc.r * cc <= kMaxPartials; };
+    auto valid = [&](int cc) { return cc >= 1 && cc <= 16 && (any_split ? nb_k >= kMinChunk * cc : nb_k % (Geom::kRing * cc) == 0) && (long long)sc.r * cc <= kMaxPartials; };
     if (sc.r > 0) {
         if (valid(2)) c = 2;
         if (valid(4) && sc.r * 4 <= slots * 3 / 4) c = 4;
@@ -631,7 +637,6 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     const int env_band = tuning_env_int("A81W41_GEMM_BAND");
     if (env_band > 0) sc.band = env_band < sc.tiles_m ? env_band : sc.tiles_m;
     sc.c = c;
-    sc.chunk = nb_k / c;
     sc.items = sc.whole + sc.r * c;
     grid = sc.items < slots ? sc.items : slots;
     return sc.r * c <= max_partials;
@@ -667,6 +672,16 @@ TeamPlan plan_teams(const Schedule& sc, int nb_k, int cus, bool may_split) {
     return own_four && nb_k >= 64 && (nb_k >= 96 || 8 * T <= 7 * cus) ? TeamPlan{} : TeamPlan{4, 1};
 }
 
+// Whether a K range that the schedule leaves whole, for want of a divisor, is cut all the same where there is a scratch.  Between one and two and a
+// half tiles a CU whole tiles leave many CUs with one while others have two, or a few tiles to a round of their own.  us whole / cut: 168 rows,
+// 6176 x 3904 39.1 / 32.0; 774 rows, 1464 x 3776 41.8 / 35.8; 1030 rows, 2096 x 4288 68.2 / 55.3; 332 rows, 5024 x 3776 41.0 / 40.7; over 70 drawn
+// shapes 1.14 times as fast, the worst 34.1 / 34.7 (406 rows, 4264 x 2944).  With more tiles chunks are no better than whole ones: 1543 rows, 1720 x
+// 2880 54.2 / 55.9, 1164 rows, 2320 x 2176 37.5 / 44.5; nor with short ranges: 1154 rows, 1288 x 1152 19.6 / 21.9.
+bool cut_anyhow(const Schedule& sc, int nb_k, int cus) {
+    const int T = sc.tiles_m * sc.tiles_n;
+    return sc.c == 1 && nb_k >= 40 && T > cus && 2 * T <= 5 * cus;
+}
+
 template <int TEAMS>
 hipError_t launch_teams(const void* A, const void* B, float* C, int M, int N, int nb_k, const Schedule& sc, int c, const GemmScratch& ws, hipStream_t s) {
     hipLaunchKernelGGL(gemm_a81w41_team_kernel<TEAMS>, dim3(sc.tiles_m * sc.tiles_n * c), dim3(TEAMS * kTileThreads), TEAMS * Geom::kLdsBytes, s,
@@ -684,15 +699,20 @@ hipError_t launch_tiles(const void* A, const void* B, float* C, int M, int N, in
     }
     Schedule sc;
     int grid = 0;
-    const bool fits = make_schedule(M, N, K, d->slots, d->cus, ws.max_partials, sc, grid);
+    const bool fits = make_schedule(M, N, K, d->slots, d->cus, ws.max_partials, false, sc, grid);
     const int nb_k = K / 64;
     const TeamPlan teams = plan_teams(sc, nb_k, d->cus, ws.any_split);
     if (teams.teams ? teams.c > 1 && sc.tiles_m * sc.tiles_n * teams.c > ws.max_partials : !fits) return hipErrorInvalidValue;
     if (teams.teams == 4) return launch_teams<4>(A, B, C, M, N, nb_k, sc, teams.c, ws, s);
     if (teams.teams == 2) return launch_teams<2>(A, B, C, M, N, nb_k, sc, 1, ws, s);
+    if (ws.any_split && cut_anyhow(sc, nb_k, d->cus)) {
+        Schedule cut;
+        int cut_grid = 0;
+        if (make_schedule(M, N, K, d->slots, d->cus, ws.max_partials, true, cut, cut_grid)) sc = cut, grid = cut_grid;
+    }
     hipLaunchKernelGGL(gemm_a81w41_tile64_kernel, dim3(grid), dim3(kTileThreads), Geom::kLdsBytes, s,
                        static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(B), M, N, nb_k, sc.tiles_m, sc.tiles_n, sc.whole,
-                       sc.r, sc.c, sc.chunk, sc.band, C, ws.partials, ws.arrivals);
+                       sc.r, sc.c, sc.band, C, ws.partials, ws.arrivals);
     return hipGetLastError();
 }
 
@@ -740,7 +760,7 @@ const char* gemm_kernel_name(int M, int N, int K) {
     Schedule sc;
     int grid = 0, teams = 0;
     if (device_info_locked(d) == hipSuccess) {
-        make_schedule(M, N, K, d->slots, d->cus, kMaxPartials, sc, grid);
+        make_schedule(M, N, K, d->slots, d->cus, kMaxPartials, false, sc, grid);
         teams = plan_teams(sc, K / 64, d->cus, false).teams;
     }
     switch (teams) {
@@ -858,7 +878,7 @@ int gemm_partial_tiles(int M, int N, int K) {
     if (device_info_locked(d) != hipSuccess) return -1;
     Schedule sc;
     int grid = 0;
-    make_schedule(M, N, K, d->slots, d->cus, kMaxPartials, sc, grid);
+    make_schedule(M, N, K, d->slots, d->cus, kMaxPartials, false, sc, grid);
     const TeamPlan teams = plan_teams(sc, K / 64, d->cus, false);
     if (teams.teams) return teams.c > 1 ? sc.tiles_m * sc.tiles_n * teams.c : 0;
     return sc.r * sc.c;
@@ -914,23 +934,11 @@ int team_plan_selfcheck(const Schedule& sc, int nb_k, const TeamPlan& plan) {
         if (covered[k] != 1) return -12;
     return tile_numbers_ok(sc) ? 0 : -7;
 }
-}  // namespace
 
-// Host-side check of the work that a launch would do (no device needed), with a scratch that is there for every call and with one
-// that is there where K has to be split: the team kernel's shares, or the list of the kernel without teams, every whole tile once, every
-// chunk of every split tile once, partial-tile indices distinct and below the scratch size.
-int gemm_schedule_selfcheck(int M, int N, int K, int slots_fit, int cus) {
-    Schedule sc;
-    int grid = 0;
-    if (!make_schedule(M, N, K, slots_fit, cus, kMaxPartials, sc, grid)) return -1;
-    const int T = sc.tiles_m * sc.tiles_n, nb_k = K / 64;
-    const TeamPlan teams = plan_teams(sc, nb_k, cus, false);
-    if (teams.teams) {
-        for (const TeamPlan& plan : {teams, plan_teams(sc, nb_k, cus, true)})
-            if (const int bad = team_plan_selfcheck(sc, nb_k, plan)) return bad;
-        return teams.c > 1 ? T * teams.c : 0;
-    }
-    if (sc.whole + sc.r != T || sc.items != sc.whole + sc.r * sc.c || sc.chunk * sc.c != nb_k) return -2;
+// A launch of the kernel without teams: every super-block of every tile in one item, parts' places distinct and in the scratch.
+int schedule_walk(const Schedule& sc, int grid, int nb_k, int slots_fit) {
+    const int T = sc.tiles_m * sc.tiles_n;
+    if (sc.whole + sc.r != T || sc.items != sc.whole + sc.r * sc.c) return -2;
     if (grid < 1 || grid > slots_fit) return -3;
     std::vector<int> covered((size_t)T, 0), part_used((size_t)kMaxPartials, 0);
     for (int b = 0; b < grid; b++)
@@ -940,14 +948,36 @@ int gemm_schedule_selfcheck(int M, int N, int K, int slots_fit, int cus) {
             } else {
                 const int k = item - sc.whole, tr = k % sc.r, ch = k / sc.r, part = tr * sc.c + ch;
                 if (part < 0 || part >= kMaxPartials || part_used[part]++) return -4;
-                if (ch * sc.chunk + sc.chunk > nb_k) return -5;
-                covered[sc.whole + tr] += sc.chunk;
+                const int n_sb = chunk_start(nb_k, sc.c, ch + 1) - chunk_start(nb_k, sc.c, ch);
+                if (n_sb < 1) return -5;
+                covered[sc.whole + tr] += n_sb;
             }
         }
     for (int t = 0; t < T; t++)
         if (covered[t] != nb_k) return -6;
-    if (!tile_numbers_ok(sc)) return -7;
-    return sc.r * sc.c;
+    return tile_numbers_ok(sc) ? 0 : -7;
+}
+}  // namespace
+
+// Host-side check of the work that a launch would do (no device needed), with a scratch that is there for every call and with one
+// that is there where K has to be split: the team kernel's shares, or the list of the kernel without teams, every whole tile once, every
+// chunk of every split tile once, partial-tile indices distinct and below the scratch size.
+int gemm_schedule_selfcheck(int M, int N, int K, int slots_fit, int cus) {
+    Schedule sc;
+    int grid = 0;
+    if (!make_schedule(M, N, K, slots_fit, cus, kMaxPartials, false, sc, grid)) return -1;
+    const int T = sc.tiles_m * sc.tiles_n, nb_k = K / 64;
+    const TeamPlan teams = plan_teams(sc, nb_k, cus, false);
+    if (teams.teams) {
+        for (const TeamPlan& plan : {teams, plan_teams(sc, nb_k, cus, true)})
+            if (const int bad = team_plan_selfcheck(sc, nb_k, plan)) return bad;
+        return teams.c > 1 ? T * teams.c : 0;
+    }
+    if (const int bad = schedule_walk(sc, grid, nb_k, slots_fit)) return bad;
+    const int parts = sc.r * sc.c;
+    if (cut_anyhow(sc, nb_k, cus) && make_schedule(M, N, K, slots_fit, cus, kMaxPartials, true, sc, grid))
+        if (const int bad = schedule_walk(sc, grid, nb_k, slots_fit)) return bad;
+    return parts;
 }
 
 }  // namespace a81w41

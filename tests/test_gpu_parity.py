@@ -609,3 +609,26 @@ def test_teams_of_waves_on_a_tile(pkg, ora, synth, torch, M, N, K):
     # the last of several parts to arrive adds them in order, whoever it is
     for _ in range(5):
         assert torch.equal(layer.forward(xd), got)
+
+
+# Between one and two and a half tiles a CU, over 40 super-blocks and more that no ring divides, a layer cuts K: the fewest tiles and
+# the most, the shortest range, one round and a round with a few tiles behind it (cut in two and in four), ragged rows and columns.
+@pytest.mark.parametrize("M,N,K", [(69, 8232, 2624), (330, 5440, 2624), (179, 5888, 3712), (600, 4096, 2560 + 64), (570, 4200, 4288),
+                                   (33, 16392, 2688)])
+def test_k_cut_where_no_ring_divides_it(pkg, ora, synth, torch, M, N, K):
+    w4, scale, offset = synth.weight_files(N, K, seed=M)
+    layer = pkg.Linear.from_arrays(w4, scale, offset, N=N, K=K)
+    layer.set_kernel("int8")
+    b16, b32 = (ora.repack(w4, scale, offset, K, N, fp32=f) for f in (False, True))
+    x = synth.activations(M, K, seed=N, outliers=True)
+    xd = dev(torch, x)
+    got = layer.forward(xd)
+    alone = pkg.ops.gemm_fp32(pkg.ops.quantize(xd, True), dev(torch, b32), M, N, K)
+    rows = sorted({0, 31, 32, 63, M // 2, M - 1} & set(range(M)))
+    want = np.concatenate([ora.linear_forward(np.concatenate([x[m:m + 1]] * 2), b16, b32, N)[:1] for m in rows])
+    # fp32 sums of K / 32 terms in another order: 2^-24 of the row each, with room for their cancellation
+    for y in (got, alone):
+        assert row_err(y.cpu().numpy()[rows], want) < K / 32 * 2.0 ** -24 * 4 + 2e-6
+    assert not torch.equal(got, alone)   # the free-standing call, which has no scratch, does not cut these
+    for _ in range(5):   # the last of several parts to arrive adds them in order, whoever it is
+        assert torch.equal(layer.forward(xd), got)
