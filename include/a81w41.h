@@ -101,7 +101,7 @@ int a81w41_gemv_repack_A81W41_fp16(const void *A_repack_dev, const void *B_repac
  * not overlap with K-split calls on that stream.  Results do not depend on timing.
  * A layer object's scratch is there from the start, so a81w41_linear_forward may split K where this call
  * does not, so as not to need a scratch: at most as many tiles of 64 x 64 as half the CUs and K > 2048 no
- * multiple of 512, or between one and two and a half tiles a CU and K >= 2560 no multiple of 512.  The two
+ * multiple of 512, or between one and two tiles a CU and K >= 2560 no multiple of 512.  The two
  * then sum in different orders and agree to the rounding of 32-bit sums;
  * otherwise, where both run on 64 x 64 tiles, they agree in every bit. */
 int a81w41_gemm_repack_A81W41_fp32(const void *A_repack_dev, const void *B_repack_dev, float *C_dev,

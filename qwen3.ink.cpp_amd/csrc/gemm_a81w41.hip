@@ -219,12 +219,12 @@ __device__ __forceinline__ void tile_epilogue(const TileProd& F, v16f& acc) {
 // waves, so the low-index workgroups, which get the extra items, are also the faster ones.
 struct Schedule {
     int tiles_m, tiles_n;
-    int whole, r, c;
+    int whole, r, c, chunk;  // chunk: super-blocks of a part, the first nb_k - c * chunk parts have one more
     int items;
     int band;  // row tiles per band (see tile_xy)
 };
 
-__host__ __device__ __forceinline__ int chunk_start(int nb_k, int c, int ch) { return nb_k * ch / c; }
+__host__ __device__ __forceinline__ int chunk_start(const Schedule& sc, int nb_k, int ch) { return ch * sc.chunk + min(ch, nb_k - sc.c * sc.chunk); }
 
 // Within an XCD (c = tau mod 8) the tiles are walked band by band: `band` row tiles high, all of the
 // XCD's column panels wide, row tiles of a panel next to each other.  The workgroups of an XCD that
@@ -286,8 +286,8 @@ __device__ __forceinline__ void tile_kernel_body(const uint8_t* __restrict__ A, 
             const int k = item - sc.whole;
             const int tr = k % sc.r, ch = k / sc.r;
             tau = sc.whole + tr;
-            k0 = chunk_start(nb_k, sc.c, ch);
-            n_sb = chunk_start(nb_k, sc.c, ch + 1) - k0;
+            k0 = chunk_start(sc, nb_k, ch);
+            n_sb = chunk_start(sc, nb_k, ch + 1) - k0;
             part = tr * sc.c + ch;
         }
         int tx, ty;
@@ -398,10 +398,10 @@ __device__ __forceinline__ void tile_kernel_body(const uint8_t* __restrict__ A, 
 // split scratch, needed at the end of a tile only, follow.
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_a81w41_tile64_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M, int N, int nb_k, int tiles_m, int tiles_n, int whole,
-    int r, int c, int band, float* __restrict__ C, float* __restrict__ partials, unsigned* __restrict__ arrivals) {
+    int r, int c, int chunk, int band, float* __restrict__ C, float* __restrict__ partials, unsigned* __restrict__ arrivals) {
     extern __shared__ __align__(16) uint8_t lds[];  // kRing stages
     __shared__ unsigned s_arrived;
-    const Schedule sc = {tiles_m, tiles_n, whole, r, c, whole + r * c, band};
+    const Schedule sc = {tiles_m, tiles_n, whole, r, c, chunk, whole + r * c, band};
     tile_kernel_body(A, B, C, M, N, nb_k, sc, partials, arrivals, lds, s_arrived);
 }
 
@@ -589,6 +589,22 @@ __global__ void clear_counters_kernel(unsigned* p, int n) {
     if (i < n) p[i] = 0u;
 }
 
+// One round of whole tiles, none of them cut, rather than parts that meet in memory (2.5 us for two): where K is short or where up to
+// three or up to four tiles a CU come out even enough.  us cut / whole, by tiles a CU (256 CUs) and super-blocks of K:
+//   up to 2, 16: 310 rows, 2368 x 1024 15.9 / 15.6 (1.2), 672 rows, 2264 x 1024 19.4 / 17.1 (1.5); 8: 525 rows, 2704 x 512 15.1 / 11.5 (1.5);
+//     but 24: 423 rows, 4112 x 1536 20.5 / 21.4
+//   up to 2.5, 24: 226 rows, 9248 x 1536 26.8 / 25.0; but 32: 312 rows, 6584 x 2048 29.5 / 30.9
+//   up to 3: 391 rows, 6032 x 1536 31.3 / 25.9 (2.6), 203 rows, 11464 x 3072 48.1 / 43.5 (2.8), 849 rows, 3344 x 512 20.9 / 14.7 (2.9)
+//   up to 3.4, where three a CU and a few in quarters are better: 709 rows, 4304 x 2048 36.9 / 40.1 (3.2)
+//   up to 4: 801 rows, 4752 x 1024 28.8 / 25.7 (3.8), 683 rows, 5904 x 512 20.3 / 17.1 (4)
+// A whole round is four workgroups a CU whatever is cut elsewhere: at two a CU, as ranges that no ring divides were, a few tiles had a round of their
+// own (1030 rows, 2096 x 4288 68.2 us, so 56; 243 rows, 8584 x 768 18.7 and 16.6).
+bool one_whole_round(int T, int nb_k, int cus) {
+    if (T <= 2 * cus) return T > cus && nb_k <= 16;
+    if (2 * T <= 5 * cus) return nb_k <= 24;
+    return nb_k < 192 && (T < 3 * cus || (5 * T >= 17 * cus && T <= 4 * cus));
+}
+
 // Without a scratch for every call K is cut only where its super-blocks divide evenly into rings.  With one (any_split), chunks are equal but for one
 // super-block and have sixteen or more.
 constexpr int kMinChunk = 16;
@@ -604,7 +620,7 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     // tiles T per CU (measured at N = 4096, M = 128..1536): up to 2 per CU, four (finer K split over
     // more workgroups); up to 2.67, two (one round of two-per-CU tiles plus a split remainder beats a
     // sparse round of slower ones: 640 rows 144 against 155 us); up to 4, three (832 rows 179 against
-    // 201 us); from 4 on, four.
+    // 201 us); from 4 on, four.  Whole tiles, which are all there at once, are four.
     const int fit = slots_fit / cus;
     int per_cu = fit;
     if (T > 2 * cus && T < 4 * cus) per_cu = 3 * T <= 8 * cus ? 2 : 3;
@@ -618,7 +634,7 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     // of the grid; in four when even then less than 3/4 of the grid would have one.
     int c = 1;
     auto valid = [&](int cc) { return cc >= 1 && cc <= 16 && (any_split ? nb_k >= kMinChunk * cc : nb_k % (Geom::kRing * cc) == 0) && (long long)sc.r * cc <= kMaxPartials; };
-    if (sc.r > 0) {
+    if (sc.r > 0 && (any_split || !one_whole_round(T, nb_k, cus))) {
         if (valid(2)) c = 2;
         if (valid(4) && sc.r * 4 <= slots * 3 / 4) c = 4;
         // a launch that does not fill the chip once, over a long K: quarters still leave 48 steps per chunk
@@ -637,8 +653,10 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     const int env_band = tuning_env_int("A81W41_GEMM_BAND");
     if (env_band > 0) sc.band = env_band < sc.tiles_m ? env_band : sc.tiles_m;
     sc.c = c;
+    sc.chunk = nb_k / c;
     sc.items = sc.whole + sc.r * c;
-    grid = sc.items < slots ? sc.items : slots;
+    const int room = c == 1 && T <= fit * cus ? fit * cus : slots;
+    grid = sc.items < room ? sc.items : room;
     return sc.r * c <= max_partials;
 }
 
@@ -665,21 +683,20 @@ TeamPlan plan_teams(const Schedule& sc, int nb_k, int cus, bool may_split) {
     if (sc.c > 1) may_split = true;
     if (mode == 9) return {};
     if (mode == 2 || mode == 4) return {mode, 1};
-    if (T > cus) return T <= 2 * cus && 16 * T >= 27 * cus && nb_k <= 40 && sc.c > 1 ? TeamPlan{2, 1} : TeamPlan{};
+    if (T > cus) return T <= 2 * cus && 16 * T >= 27 * cus && nb_k <= 40 && nb_k % (2 * Geom::kRing) == 0 ? TeamPlan{2, 1} : TeamPlan{};
     if (nb_k <= 32) return own_four && nb_k > 24 && 2 * T <= cus ? TeamPlan{} : TeamPlan{2, 1};
     if (4 * T <= cus) return {4, may_split ? 4 : 1};
     if (2 * T <= cus) return own_four && nb_k < 64 ? TeamPlan{} : TeamPlan{4, may_split ? 2 : 1};
     return own_four && nb_k >= 64 && (nb_k >= 96 || 8 * T <= 7 * cus) ? TeamPlan{} : TeamPlan{4, 1};
 }
 
-// Whether a K range that the schedule leaves whole, for want of a divisor, is cut all the same where there is a scratch.  Between one and two and a
-// half tiles a CU whole tiles leave many CUs with one while others have two, or a few tiles to a round of their own.  us whole / cut: 168 rows,
-// 6176 x 3904 39.1 / 32.0; 774 rows, 1464 x 3776 41.8 / 35.8; 1030 rows, 2096 x 4288 68.2 / 55.3; 332 rows, 5024 x 3776 41.0 / 40.7; over 70 drawn
-// shapes 1.14 times as fast, the worst 34.1 / 34.7 (406 rows, 4264 x 2944).  With more tiles chunks are no better than whole ones: 1543 rows, 1720 x
-// 2880 54.2 / 55.9, 1164 rows, 2320 x 2176 37.5 / 44.5; nor with short ranges: 1154 rows, 1288 x 1152 19.6 / 21.9.
+// Whether a K range that the schedule leaves whole, for want of a divisor, is cut all the same where there is a scratch.  Between one and two
+// tiles a CU whole ones leave many CUs with one while others have two.  us whole / cut: 168 rows, 6176 x 3904 39.1 / 32.0; 774 rows, 1464 x 3776
+// 41.8 / 35.8; 332 rows, 5024 x 3776 41.0 / 40.7; over 58 drawn shapes 1.14 times as fast, the worst 34.1 / 34.7 (406 rows, 4264 x 2944).  Not
+// over short ranges: 1154 rows, 1288 x 1152 19.6 / 21.9; with more tiles see one_whole_round.
 bool cut_anyhow(const Schedule& sc, int nb_k, int cus) {
     const int T = sc.tiles_m * sc.tiles_n;
-    return sc.c == 1 && nb_k >= 40 && T > cus && 2 * T <= 5 * cus;
+    return sc.c == 1 && nb_k >= 40 && T > cus && T <= 2 * cus;
 }
 
 template <int TEAMS>
@@ -712,7 +729,7 @@ hipError_t launch_tiles(const void* A, const void* B, float* C, int M, int N, in
     }
     hipLaunchKernelGGL(gemm_a81w41_tile64_kernel, dim3(grid), dim3(kTileThreads), Geom::kLdsBytes, s,
                        static_cast<const uint8_t*>(A), static_cast<const uint8_t*>(B), M, N, nb_k, sc.tiles_m, sc.tiles_n, sc.whole,
-                       sc.r, sc.c, sc.band, C, ws.partials, ws.arrivals);
+                       sc.r, sc.c, sc.chunk, sc.band, C, ws.partials, ws.arrivals);
     return hipGetLastError();
 }
 
@@ -948,7 +965,7 @@ int schedule_walk(const Schedule& sc, int grid, int nb_k, int slots_fit) {
             } else {
                 const int k = item - sc.whole, tr = k % sc.r, ch = k / sc.r, part = tr * sc.c + ch;
                 if (part < 0 || part >= kMaxPartials || part_used[part]++) return -4;
-                const int n_sb = chunk_start(nb_k, sc.c, ch + 1) - chunk_start(nb_k, sc.c, ch);
+                const int n_sb = chunk_start(sc, nb_k, ch + 1) - chunk_start(sc, nb_k, ch);
                 if (n_sb < 1) return -5;
                 covered[sc.whole + tr] += n_sb;
             }

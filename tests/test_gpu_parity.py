@@ -611,11 +611,14 @@ def test_teams_of_waves_on_a_tile(pkg, ora, synth, torch, M, N, K):
         assert torch.equal(layer.forward(xd), got)
 
 
-# Between one and two and a half tiles a CU, over 40 super-blocks and more that no ring divides, a layer cuts K: the fewest tiles and
-# the most, the shortest range, one round and a round with a few tiles behind it (cut in two and in four), ragged rows and columns.
-@pytest.mark.parametrize("M,N,K", [(69, 8232, 2624), (330, 5440, 2624), (179, 5888, 3712), (600, 4096, 2560 + 64), (570, 4200, 4288),
-                                   (33, 16392, 2688)])
-def test_k_cut_where_no_ring_divides_it(pkg, ora, synth, torch, M, N, K):
+# Between one and two tiles a CU, over 40 super-blocks and more that no ring divides, a layer cuts K: the fewest tiles and the most, the
+# shortest range, ragged rows and columns.  Whole rounds, which neither cuts: the fewest tiles and the most of up to two, two and a half, three and
+# four a CU, with their longest ranges, and three and a fifth, where the rest is in quarters.
+@pytest.mark.parametrize("M,N,K,cut", [(69, 8232, 2624, True), (330, 5440, 2624, True), (179, 5888, 3712, True), (33, 16392, 2688, True),
+                                       (33, 16392, 1024, False), (512, 4096, 512, False), (513, 3640, 1536, False), (640, 4096, 1536, False),
+                                       (641, 3720, 4096, False), (192, 16320, 576, False), (780, 4104, 2048, False), (868, 3976, 1088, False),
+                                       (1024, 4096, 512, False)])
+def test_k_ranges_of_one_round(pkg, ora, synth, torch, M, N, K, cut):
     w4, scale, offset = synth.weight_files(N, K, seed=M)
     layer = pkg.Linear.from_arrays(w4, scale, offset, N=N, K=K)
     layer.set_kernel("int8")
@@ -629,6 +632,6 @@ def test_k_cut_where_no_ring_divides_it(pkg, ora, synth, torch, M, N, K):
     # fp32 sums of K / 32 terms in another order: 2^-24 of the row each, with room for their cancellation
     for y in (got, alone):
         assert row_err(y.cpu().numpy()[rows], want) < K / 32 * 2.0 ** -24 * 4 + 2e-6
-    assert not torch.equal(got, alone)   # the free-standing call, which has no scratch, does not cut these
+    assert torch.equal(got, alone) != cut   # the free-standing call, which has no scratch, does not cut them
     for _ in range(5):   # the last of several parts to arrive adds them in order, whoever it is
         assert torch.equal(layer.forward(xd), got)
