@@ -589,7 +589,7 @@ __global__ void clear_counters_kernel(unsigned* p, int n) {
     if (i < n) p[i] = 0u;
 }
 
-// One round of whole tiles, none of them cut, rather than parts that meet in memory (2.5 us for two): where K is short or where up to
+// Whole tiles, none of them cut, rather than parts that meet in memory (2.5 us for two): where K is short or where up to
 // three or up to four tiles a CU come out even enough.  us cut / whole, by tiles a CU (256 CUs) and super-blocks of K:
 //   up to 2, 16: 310 rows, 2368 x 1024 15.9 / 15.6 (1.2), 672 rows, 2264 x 1024 19.4 / 17.1 (1.5); 8: 525 rows, 2704 x 512 15.1 / 11.5 (1.5);
 //     but 24: 423 rows, 4112 x 1536 20.5 / 21.4
@@ -597,9 +597,14 @@ __global__ void clear_counters_kernel(unsigned* p, int n) {
 //   up to 3: 391 rows, 6032 x 1536 31.3 / 25.9 (2.6), 203 rows, 11464 x 3072 48.1 / 43.5 (2.8), 849 rows, 3344 x 512 20.9 / 14.7 (2.9)
 //   up to 3.4, where three a CU and a few in quarters are better: 709 rows, 4304 x 2048 36.9 / 40.1 (3.2)
 //   up to 4: 801 rows, 4752 x 1024 28.8 / 25.7 (3.8), 683 rows, 5904 x 512 20.3 / 17.1 (4)
+//   more, by what the last round has: 898 rows, 7296 x 512 30.0 / 23.5 (2.7), 812 rows, 8304 x 512 30.6 / 23.8 (2.6), 617 rows, 10680 x 1024 41.7 /
+//     36.3 (2.5), 694 rows, 10024 x 1536 57.1 / 51.0 (2.7), 1139 rows, 4312 x 1024 32.9 / 31.0 (0.8); but 939 rows, 4584 x 1024 28.1 / 29.6 (0.2),
+//     1169 rows, 10728 x 512 39.0 / 40.3 (0.5)
 // A whole round is four workgroups a CU whatever is cut elsewhere: at two a CU, as ranges that no ring divides were, a few tiles had a round of their
 // own (1030 rows, 2096 x 4288 68.2 us, so 56; 243 rows, 8584 x 768 18.7 and 16.6).
-bool one_whole_round(int T, int nb_k, int cus) {
+bool whole_tiles_preferred(int T, int nb_k, int cus) {
+    const int last = T % (4 * cus);
+    if (T > 4 * cus) return (nb_k <= 8 && 2 * last >= cus) || (nb_k <= 24 && 4 * last >= 3 * cus);
     if (T <= 2 * cus) return T > cus && nb_k <= 16;
     if (2 * T <= 5 * cus) return nb_k <= 24;
     return nb_k < 192 && (T < 3 * cus || (5 * T >= 17 * cus && T <= 4 * cus));
@@ -634,7 +639,7 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     // of the grid; in four when even then less than 3/4 of the grid would have one.
     int c = 1;
     auto valid = [&](int cc) { return cc >= 1 && cc <= 16 && (any_split ? nb_k >= kMinChunk * cc : nb_k % (Geom::kRing * cc) == 0) && (long long)sc.r * cc <= kMaxPartials; };
-    if (sc.r > 0 && (any_split || !one_whole_round(T, nb_k, cus))) {
+    if (sc.r > 0 && (any_split || !whole_tiles_preferred(T, nb_k, cus))) {
         if (valid(2)) c = 2;
         if (valid(4) && sc.r * 4 <= slots * 3 / 4) c = 4;
         // a launch that does not fill the chip once, over a long K: quarters still leave 48 steps per chunk
@@ -693,7 +698,7 @@ TeamPlan plan_teams(const Schedule& sc, int nb_k, int cus, bool may_split) {
 // Whether a K range that the schedule leaves whole, for want of a divisor, is cut all the same where there is a scratch.  Between one and two
 // tiles a CU whole ones leave many CUs with one while others have two.  us whole / cut: 168 rows, 6176 x 3904 39.1 / 32.0; 774 rows, 1464 x 3776
 // 41.8 / 35.8; 332 rows, 5024 x 3776 41.0 / 40.7; over 58 drawn shapes 1.14 times as fast, the worst 34.1 / 34.7 (406 rows, 4264 x 2944).  Not
-// over short ranges: 1154 rows, 1288 x 1152 19.6 / 21.9; with more tiles see one_whole_round.
+// over short ranges: 1154 rows, 1288 x 1152 19.6 / 21.9; with more tiles see whole_tiles_preferred.
 bool cut_anyhow(const Schedule& sc, int nb_k, int cus) {
     const int T = sc.tiles_m * sc.tiles_n;
     return sc.c == 1 && nb_k >= 40 && T > cus && T <= 2 * cus;

@@ -613,12 +613,13 @@ def test_teams_of_waves_on_a_tile(pkg, ora, synth, torch, M, N, K):
 
 # Between one and two tiles a CU, over 40 super-blocks and more that no ring divides, a layer cuts K: the fewest tiles and the most, the
 # shortest range, ragged rows and columns.  Whole rounds, which neither cuts: the fewest tiles and the most of up to two, two and a half, three and
-# four a CU, with their longest ranges, and three and a fifth, where the rest is in quarters.
+# four a CU and of a second round, with their longest ranges, and three and a fifth and a second round of few, where the rest is in quarters.
 @pytest.mark.parametrize("M,N,K,cut", [(69, 8232, 2624, True), (330, 5440, 2624, True), (179, 5888, 3712, True), (33, 16392, 2688, True),
                                        (33, 16392, 1024, False), (512, 4096, 512, False), (513, 3640, 1536, False), (640, 4096, 1536, False),
                                        (641, 3720, 4096, False), (192, 16320, 576, False), (780, 4104, 2048, False), (868, 3976, 1088, False),
-                                       (1024, 4096, 512, False)])
-def test_k_ranges_of_one_round(pkg, ora, synth, torch, M, N, K, cut):
+                                       (1024, 4096, 512, False), (1100, 4136, 512, False), (1216, 4096, 1536, False),
+                                       (1160, 4096, 1024, False)])
+def test_k_ranges_whole_and_cut(pkg, ora, synth, torch, M, N, K, cut):
     w4, scale, offset = synth.weight_files(N, K, seed=M)
     layer = pkg.Linear.from_arrays(w4, scale, offset, N=N, K=K)
     layer.set_kernel("int8")
