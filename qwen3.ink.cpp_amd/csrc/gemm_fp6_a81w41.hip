@@ -165,10 +165,10 @@ __host__ __device__ __forceinline__ int run_owner(const Plan& p, long long u) { 
 // Dwords 0..5 are the matrix op's operand (a 32 x 6-bit operand occupies six registers; the op does not look at
 // the other two), dwords 6 and 7 the two parameters.
 typedef v8i Frag;
-// An operand in eight registers one behind the other: the matrix op takes the first six where they are.  Without this the compiler loads the second
-// half elsewhere, copies two registers of it and waits for that load in the middle of the block ahead of the one that uses it.  2047 rows, 12288 x
-// 4096, us a call: 277; with the min terms' operands as they are read (instead of selected by lane half and exchanged between the
-// halves) 271; and with this 264.
+// An operand in eight registers one behind the other: the matrix op takes the first six where they are.  Without this the compiler loads some
+// second halves elsewhere and copies them (36 copies in four blocks instead of 14).  2047 rows, 12288 x 4096, us a call with its quantiser, weights in
+// the memory-side cache: 283 with min terms exchanged through LDS and loads wherever the compiler put them; with one instruction an exchange and a
+// block's loads at its start 273; and with this 270.
 __device__ __forceinline__ void whole(Frag& f) { asm("" : "+v"(f)); }
 
 __device__ __forceinline__ Frag read_frag(const uint8_t* p) {
@@ -185,12 +185,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave >> 2, wc = wave & 3;  // this wave's 64 rows (panels 2 wr, 2 wr + 1) x 64 columns (panels 2 wc, 2 wc + 1) of the tile
-    const int r = lane & 31, h = lane >> 5;
+    const int h = lane >> 5;
     // E8M0 block scales: patterns are integers / 8 on both sides (2^3 each); the qh piece counts 16-fold
     const int scale_a = 127 + 3 + 4 * (1 - h), scale_b = 127 + 3;
-    const uint32_t lane_a = (uint32_t)h * 1024u + (uint32_t)r * 16u, lane_b = (uint32_t)r * 16u;
-
-    const uint32_t min_select = h ? 0x01000100u : 0x03020100u;
 
     // Workgroups are dealt to the 8 XCDs round robin; run = (XCD, index inside it) makes an XCD's runs
     // neighbours in the unit space, so that the row tiles of a column panel (which share its weights) and
@@ -208,21 +205,24 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         // Operands come straight from memory into registers (the 8 waves of the workgroup share them through the
         // vector cache): per 32-block, two 16-byte loads per 32 x 32 operand.  Panels past the last one alias it;
         // what is computed from them is never stored.
+        int lane_now = lane;
+        asm volatile("" : "+v"(lane_now));
+        const uint32_t lane_b = (uint32_t)(lane_now & 31) * 16u, lane_a = lane_b + (uint32_t)(lane_now & 32) * 32u;
         const uint8_t* pa[2];
         const uint8_t* pb[2];
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const int panel_a = min(kTileM / 32 * ty + 2 * wr + i, panels_m - 1);
             const int panel_b = min(kTileN / 32 * tx + 2 * wc + i, panels_n - 1);
-            pa[i] = A6 + ((size_t)panel_a * nb + k0) * kPanelA;  // wave-uniform
-            pb[i] = W6 + ((size_t)panel_b * nb + k0) * kPanelB;
+            pa[i] = A6 + ((size_t)panel_a * nb + k0) * kPanelA + lane_a;
+            pb[i] = W6 + ((size_t)panel_b * nb + k0) * kPanelB + lane_b;
         }
         auto load_step = [&](int step, Frag (&fa)[2], Frag (&fb)[2]) {
             const int s = min(step, n_steps - 1);  // past the end the last block is read again
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                fa[i] = read_frag(pa[i] + (size_t)s * kPanelA + lane_a);
-                fb[i] = read_frag(pb[i] + (size_t)s * kPanelB + lane_b);
+                fa[i] = read_frag(pa[i] + (size_t)s * kPanelA);
+                fb[i] = read_frag(pb[i] + (size_t)s * kPanelB);
             }
         };
 
@@ -233,19 +233,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             for (int j = 0; j < 2; j++) acc[i][j] = v16f{0};
         const bool rows_live = kTileM * ty + 64 * wr < M;  // else every row of this wave is past M
 
-        // Min terms of up to four 32-blocks, each with two K slots of either lane half: half 0 brings (s_hi, s_hi) against (w_hi, w_lo), half 1
-        // (s_mid, s_lo) against (w_hi, w_hi).  An activation operand's last word is that as it was read; blocks that are not there have zeros.
-        v4i opa[2], opb[2];
-        auto keep_min = [&](int k, const Frag (&fa)[2], const Frag (&fb)[2]) {
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                opa[i][k] = fa[i][7];
-                opb[i][k] = (int)__builtin_amdgcn_perm((uint32_t)fb[i][7], (uint32_t)fb[i][7], min_select);
-            }
+        // Min terms of up to four 32-blocks (zeros for blocks that are not there): lane half 0 brings blocks 0 and 1, half 1 blocks 2 and 3, four K
+        // slots a block, (s_hi, s_hi, s_mid, s_lo) against (w_hi, w_lo, w_hi, w_hi).  Of a scaled sum lanes 0..31 read (s_hi, s_hi), lanes 32..63
+        // (s_mid, s_lo): block k's words of the upper half and block k + 2's of the lower one change places, one instruction, and are the
+        // operand.  Which slot a product has decides how the sum is rounded, 2e-7 of a call, and a Qwen3 prompt, whose rows are
+        // rounded to 8 bits ahead of every linear, makes 0.012 of that: its logits were others with two slots of a block in either half, which
+        // needs no exchange and is no faster (2047 rows, 12288 x 4096: 269 and 270 us).
+        uint32_t ya[2][4], yb[2][2];
+        auto keep_min = [&](int i, int k, int word_a, int word_b) {
+            ya[i][k] = (uint32_t)word_a;
+            yb[i][k & 1] = k < 2 || h ? (uint32_t)word_b : yb[i][k & 1];
         };
         auto min_terms = [&]() {
             typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
             auto bf = [](const v4i& v) { return __builtin_bit_cast(v8bf, v); };
+            v4i opa[2], opb[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const auto own = __builtin_amdgcn_permlane32_swap(ya[i][k], ya[i][k + 2], false, false);
+                    opa[i][2 * k] = (int)own[0];
+                    opa[i][2 * k + 1] = (int)own[1];
+                    opb[i][2 * k] = (int)yb[i][k];                                                                    // hi, lo
+                    opb[i][2 * k + 1] = (int)__builtin_amdgcn_perm(yb[i][k], yb[i][k], 0x01000100u);  // hi, hi
+                }
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -283,7 +295,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 whole(fb[k & 1][0]);
                 whole(fa[k & 1][1]);
                 whole(fb[k & 1][1]);
-                keep_min(k, fa[k & 1], fb[k & 1]);
+#pragma unroll
+                for (int i = 0; i < 2; i++) keep_min(i, k, fa[k & 1][i][7], fb[k & 1][i][7]);
                 compute(fa[k & 1], fb[k & 1]);
             };
             int step = 0;
@@ -294,16 +307,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             }
             if (step < n_steps) {
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    if (step + k < n_steps)
-                        block(k, step + k);
-                    else
-                        opa[0][k] = opa[1][k] = opb[0][k] = opb[1][k] = 0;
+                for (int k = 0; k < 4; k++) keep_min(0, k, 0, 0), keep_min(1, k, 0, 0);
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    if (step + k < n_steps) block(k, step + k);
                 }
                 min_terms();
             }
         }
 
+        // What follows, like the operands' places above, starts again from the thread's number: kept over the blocks, its row, lane half and
+        // addresses would be registers more than there are.
+        int me = tid;
+        asm volatile("" : "+v"(me));
         // Result registers of sub-tile (i, j): register v, lane (r, h): column 32 j + r, row 32 i + 8 (v/4) + 4 h + v%4.
         const int m_base = kTileM * ty + 64 * wr, n_base = kTileN * tx + 64 * wc;
         auto store_tile = [&](const v16f (&x)[2][2]) {
@@ -312,11 +328,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             for (int i = 0; i < 2; i++)
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
-                    const int n = n_base + 32 * j + r;
+                    const int n = n_base + 32 * j + (me & 31);
                     if (n >= N) continue;
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        const int m = m_base + 32 * i + 8 * (v >> 2) + 4 * h + (v & 3);
+                        const int m = m_base + 32 * i + 8 * (v >> 2) + (me >> 3 & 4) + (v & 3);
                         if (m < M) C[(size_t)m * N + n] = x[i][j][v];
                     }
                 }
@@ -333,7 +349,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int b = run;
             const int slot = run_start(plan, b) >= tile_u0 ? 2 * b : 2 * b + 1;
             // element (register quad q, thread) of a partial tile at [slot][q][thread][4]: 4 KiB per wave-wide access
-            float* mine = partials + (size_t)slot * kTileWords + 4 * tid;
+            float* mine = partials + (size_t)slot * kTileWords + 4 * me;
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -345,7 +361,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                     }
             wait_vmcnt<0>();
             __syncthreads();
-            if (tid == 0) s_arrived = atomicAdd(&arrivals[first], 1u);
+            if (me == 0) s_arrived = atomicAdd(&arrivals[first], 1u);
             __syncthreads();
             if (s_arrived == (unsigned)(last - first)) {
                 v16f sum[2][2];
@@ -362,7 +378,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                         continue;
                     }
                     const int cs = run_start(plan, c) >= tile_u0 ? 2 * c : 2 * c + 1;
-                    const float* p = partials + (size_t)cs * kTileWords + 4 * tid;
+                    const float* p = partials + (size_t)cs * kTileWords + 4 * me;
                     v4f l[16];
 #pragma unroll
                     for (int q = 0; q < 16; q++) l[q] = load16_agent(p + (size_t)q * 4 * kThreads);
@@ -374,7 +390,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                         for (int e = 0; e < 4; e++) sum[q >> 3][(q >> 2) & 1][4 * (q & 3) + e] += l[q][e];
                 }
                 store_tile(sum);
-                if (tid == 0) __hip_atomic_store(&arrivals[first], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (me == 0) __hip_atomic_store(&arrivals[first], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             __syncthreads();  // s_arrived is free again
         }

@@ -1,4 +1,4 @@
-"""Two pins of the block-scaled (fp6 matrix op) kernel that its fp32 outputs on zero-mean activations do not give.
+"""Three pins of the block-scaled (fp6 matrix op) kernel that its fp32 outputs on zero-mean activations do not give.
 
 1. Its block dots are the reference's integers (quantized_gemx_kernels.cc:430-457,509: int32 dot, then
    cvtepi32_ps).  The kernel never holds them as integers, so they are made visible: weight scale 1, min 0,
@@ -8,7 +8,11 @@
 2. Its min terms fma(mW, sA, acc) (quantized_gemx_kernels.cc:509-512) run on bf16 pieces (three for the
    scaled sum, two for the min).  With zero-mean weights (min = -7.5 scale) and rows that are not zero-mean the min
    term is far larger than the result it cancels down to; the error must stay inside the path's 1e-4 bar
-   with room to spare."""
+   with room to spare.
+3. The order of its sums: a product's K slot in the min terms' matrix op decides how they are rounded (2e-7 of a call), and a prompt
+   whose rows are rounded to 8 bits ahead of every linear makes 1e-2 of that.  A call's bits are held."""
+import zlib
+
 import numpy as np
 import pytest
 
@@ -101,3 +105,17 @@ def test_min_terms_with_zero_mean_weights_and_biased_rows(pkg, ora, synth, name,
           f"int8 {errs['int8']:.2e}]")
     assert errs["int8"] <= 1e-5
     assert errs["block_scaled"] <= 4e-5          # the path's bar is 1e-4: a factor 2.5 in hand (observed 2.0e-5 .. 2.6e-5)
+
+
+# Of sums on 256 CUs (the cut of the work into runs goes by them).  Runs of one to four blocks past a multiple of four and of many, tiles of one run
+# and of several, one panel and ragged ones.
+@pytest.mark.parametrize("M,N,K,bits", [(33, 8, 64, 1823667629), (130, 136, 448, 2408502087), (65, 1000, 2048, 2921864782),
+                                        (100, 512, 12288, 529302396), (322, 1024, 4096, 2724076504)])
+def test_sums_keep_their_order(pkg, synth, M, N, K, bits):
+    import torch
+
+    w4, scale, _ = synth.weight_files(N, K, M + N)
+    layer = pkg.Linear.from_arrays(w4, scale * np.float32(1.0371), np.float32(-7.3) * scale, N=N, K=K)
+    layer.set_kernel("block_scaled")
+    x = torch.from_numpy(np.float32(0.5) + synth.activations(M, K, K + 1)).cuda()
+    assert zlib.crc32(layer.forward(x).cpu().numpy().tobytes()) == bits
