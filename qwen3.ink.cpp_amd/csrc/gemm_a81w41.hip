@@ -594,9 +594,14 @@ __global__ void clear_counters_kernel(unsigned* p, int n) {
 //   up to 2, 16: 310 rows, 2368 x 1024 15.9 / 15.6 (1.2), 672 rows, 2264 x 1024 19.4 / 17.1 (1.5); 8: 525 rows, 2704 x 512 15.1 / 11.5 (1.5);
 //     but 24: 423 rows, 4112 x 1536 20.5 / 21.4
 //   up to 2.5, 24: 226 rows, 9248 x 1536 26.8 / 25.0; but 32: 312 rows, 6584 x 2048 29.5 / 30.9
-//   up to 3: 391 rows, 6032 x 1536 31.3 / 25.9 (2.6), 203 rows, 11464 x 3072 48.1 / 43.5 (2.8), 849 rows, 3344 x 512 20.9 / 14.7 (2.9)
-//   up to 3.4, where three a CU and a few in quarters are better: 709 rows, 4304 x 2048 36.9 / 40.1 (3.2)
-//   up to 4: 801 rows, 4752 x 1024 28.8 / 25.7 (3.8), 683 rows, 5904 x 512 20.3 / 17.1 (4)
+//   up to 3: 391 rows, 6032 x 1536 31.3 / 25.9 (2.6), 203 rows, 11464 x 3072 48.1 / 43.5 (2.8), 849 rows, 3344 x 512 20.9 / 14.7 (2.9),
+//     1573 rows, 1888 x 10752 149.7 / 147.0 (2.9)
+//   up to 3.5, where three a CU and a few in quarters are better: 709 rows, 4304 x 2048 36.9 / 40.1 (3.2), 484 rows, 6968 x 1536 29.5 / 30.6 (3.4),
+//     422 rows, 8064 x 6656 100.9 / 108.2 (3.4), 419 rows, 8088 x 10752 153.9 / 163.8 (3.5); but 16, from 3.4 on: 860 rows, 3992 x 1024 25.0 / 23.1,
+//     and 8: 225 rows, 14264 x 512 17.2 / 15.9.  (At 8 and 16 whole tiles were not timed below 3.4.)
+//   up to 4: 411 rows, 8320 x 6144 102.9 / 98.8 (3.6), 398 rows, 8232 x 10752 164.8 / 161.9 (3.5), 801 rows, 4752 x 1024 28.8 / 25.7 (3.8), 683 rows,
+//     5904 x 512 20.3 / 17.1 (4)
+//   up to 3 and to 4, 192 and more: not timed, cut
 //   more, by what the last round has: 898 rows, 7296 x 512 30.0 / 23.5 (2.7), 812 rows, 8304 x 512 30.6 / 23.8 (2.6), 617 rows, 10680 x 1024 41.7 /
 //     36.3 (2.5), 694 rows, 10024 x 1536 57.1 / 51.0 (2.7), 1139 rows, 4312 x 1024 32.9 / 31.0 (0.8); but 939 rows, 4584 x 1024 28.1 / 29.6 (0.2),
 //     1169 rows, 10728 x 512 39.0 / 40.3 (0.5)
@@ -607,7 +612,8 @@ bool whole_tiles_preferred(int T, int nb_k, int cus) {
     if (T > 4 * cus) return (nb_k <= 8 && 2 * last >= cus) || (nb_k <= 24 && 4 * last >= 3 * cus);
     if (T <= 2 * cus) return T > cus && nb_k <= 16;
     if (2 * T <= 5 * cus) return nb_k <= 24;
-    return nb_k < 192 && (T < 3 * cus || (5 * T >= 17 * cus && T <= 4 * cus));
+    if (nb_k >= 192) return false;
+    return T < 3 * cus || 2 * T > 7 * cus || (5 * T >= 17 * cus && nb_k <= 16);
 }
 
 // Without a scratch for every call K is cut only where its super-blocks divide evenly into rings.  With one (any_split), chunks are equal but for one

@@ -110,6 +110,27 @@ def test_gemm_schedule_follows_the_teams(pkg):
         assert L.a81w41_gemm_schedule_selfcheck(M, N, K, 1024, 256) == parts, (M, N, K)
 
 
+# Which tiles of a launch are cut on 256 CUs, by parts (0: none).  T tiles of 64 x 64, K in super-blocks of 64.
+@pytest.mark.parametrize("M,N,K,parts", [
+    # up to two a CU: whole up to 16 super-blocks (T = 257, 427), halves of all beyond
+    (33, 16392, 1024, 0), (420, 3904, 1024, 0), (420, 3904, 1536, 854),
+    # up to two and a half (T = 640): whole up to 24, beyond two a CU and the other 128 in halves
+    (640, 4096, 1536, 0), (640, 4096, 2048, 256), (600, 4096, 2560, 256),
+    # up to three (T = 649, 767): whole below 192
+    (641, 3720, 4096, 0), (641, 3720, 11776, 0), (641, 3720, 12288, 274), (830, 3776, 2048, 0),
+    # a few more than three (T = 816, 845, 870): three a CU and the rest cut
+    (709, 4304, 2048, 192), (780, 4104, 2048, 308), (780, 4104, 512, 154), (950, 3712, 1024, 408),
+    # up to three and a half (T = 880, 882, 888, 891, 896): whole up to 16 only
+    (868, 3976, 1024, 0), (350, 9464, 1024, 0), (529, 6304, 1536, 246), (691, 5120, 4608, 224), (868, 4096, 2560, 256), (868, 4096, 11264, 512),
+    # up to four (T = 897, 912, 1024): whole below 192
+    (830, 4416, 4096, 0), (1024, 3592, 11776, 0), (1024, 4096, 512, 0),
+    # more: cut where the last round has few (126, 191 tiles), whole where it has more (146, 192), cut over long ranges: 192 in quarters, 256 in halves
+    (1472, 3200, 512, 252), (1100, 4136, 512, 0), (960, 5184, 1024, 764), (1030, 4096, 1024, 256), (1160, 4096, 1024, 0), (1216, 4096, 4096, 768),
+    (1280, 4096, 4096, 512)])
+def test_gemm_schedule_cuts_what_it_should(pkg, M, N, K, parts):
+    assert pkg.capi.lib().a81w41_gemm_schedule_selfcheck(M, N, K, 1024, 256) == parts
+
+
 def test_block_scaled_gemm_plan_covers_every_unit_once(pkg):
     """The layer object's M > 32 kernel cuts the (tile, 32-block) units of a launch into equal contiguous runs:
     walked on the host for the layer's shapes and odd ones, for several device sizes."""
