@@ -616,11 +616,8 @@ bool whole_tiles_preferred(int T, int nb_k, int cus) {
     return T < 3 * cus || 2 * T > 7 * cus || (5 * T >= 17 * cus && nb_k <= 16);
 }
 
-// Without a scratch for every call K is cut only where its super-blocks divide evenly into rings.  With one (any_split), chunks are equal but for one
-// super-block and have sixteen or more.
-constexpr int kMinChunk = 16;
-
-// The schedule of one launch (see Schedule): a pure function of the shape and of the device's size.
+// The schedule of one launch (see Schedule): a pure function of the shape and of the device's size.  Without a scratch for every call K is
+// cut only where its super-blocks divide evenly into rings; with one (any_split, see cut_anyhow) chunks are equal but for one super-block.
 // Returns false when the K split the shape calls for needs more than max_partials partial tiles.
 bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials, bool any_split, Schedule& sc, int& grid) {
     const int nb_k = K / 64;
@@ -644,7 +641,7 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     // Split the last, partial round: in two, so that the chunks go to the first (faster) half
     // of the grid; in four when even then less than 3/4 of the grid would have one.
     int c = 1;
-    auto valid = [&](int cc) { return cc >= 1 && cc <= 16 && (any_split ? nb_k >= kMinChunk * cc : nb_k % (Geom::kRing * cc) == 0) && (long long)sc.r * cc <= kMaxPartials; };
+    auto valid = [&](int cc) { return cc >= 1 && cc <= 16 && (any_split || nb_k % (Geom::kRing * cc) == 0) && (long long)sc.r * cc <= kMaxPartials; };
     if (sc.r > 0 && (any_split || !whole_tiles_preferred(T, nb_k, cus))) {
         if (valid(2)) c = 2;
         if (valid(4) && sc.r * 4 <= slots * 3 / 4) c = 4;
