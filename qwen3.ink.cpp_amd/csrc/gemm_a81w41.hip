@@ -634,7 +634,8 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     if (T > 2 * cus && T < 4 * cus) per_cu = 3 * T <= 8 * cus ? 2 : 3;
     if (per_cu > fit) per_cu = fit;
     const int env_per_cu = tuning_env_int("A81W41_GEMM_PER_CU");
-    if (env_per_cu >= 1 && env_per_cu <= fit) per_cu = env_per_cu;
+    const bool set_per_cu = env_per_cu >= 1 && env_per_cu <= fit;
+    if (set_per_cu) per_cu = env_per_cu;
     const int slots = per_cu * cus;
     sc.whole = (T / slots) * slots;
     sc.r = T - sc.whole;
@@ -648,9 +649,9 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
         // a launch that does not fill the chip once, over a long K: quarters still leave 48 steps per chunk
         // (down_proj at 322 rows: 75.6 against 79.8 us)
         if (valid(4) && sc.whole == 0 && nb_k / 4 >= 48) c = 4;
-        const int env_c = tuning_env_int("A81W41_GEMM_SPLIT");
-        if (env_c > 0 && valid(env_c)) c = env_c;
     }
+    const int env_c = tuning_env_int("A81W41_GEMM_SPLIT");
+    if (sc.r > 0 && env_c > 0 && valid(env_c)) c = env_c;
     if (c == 1) {
         sc.whole = T;
         sc.r = 0;
@@ -663,7 +664,7 @@ bool make_schedule(int M, int N, int K, int slots_fit, int cus, int max_partials
     sc.c = c;
     sc.chunk = nb_k / c;
     sc.items = sc.whole + sc.r * c;
-    const int room = c == 1 && T <= fit * cus ? fit * cus : slots;
+    const int room = c == 1 && !set_per_cu ? fit * cus : slots;
     grid = sc.items < room ? sc.items : room;
     return sc.r * c <= max_partials;
 }
