@@ -124,11 +124,11 @@ int a81w41_gemm_repack_A81W41_fp32_static(const void *A_repack_dev, const void *
  * `cus` compute units: that kernel's work list or, where teams of waves share a tile, their shares of K,
  * with a scratch for this call alone and with a layer object's.  Returns the number of
  * partial tiles the K split of a call without a layer object parks (>= 0) if every tile and every K
- * chunk is covered exactly once, the tile numbering is one-to-one and no two chunks share a partial
- * tile; a negative code names the violated property. */
+ * chunk is covered exactly once, the tile numbering is one-to-one, no two chunks share a partial
+ * tile and a layer object's launch is cut where it should be; a negative code names the violated property. */
 int a81w41_gemm_schedule_selfcheck(int M, int N, int K, int resident_workgroups, int cus);
 
-/* Test hook, host only: the same for the layer object's M > 32 kernel (128 x 128 tiles, the (tile,
+/* Test hook, host only: the same for the layer object's M > 32 kernel (128 x 256 tiles, the (tile,
  * 32-block) units of a launch cut into equal contiguous runs): every unit exactly once, contributor
  * ranges and partial-tile slots consistent.  Returns the number of tiles shared between workgroups. */
 int a81w41_gemm_fp6_plan_selfcheck(int M, int N, int K, int resident_workgroups);

@@ -987,7 +987,8 @@ int schedule_walk(const Schedule& sc, int grid, int nb_k, int slots_fit) {
 
 // Host-side check of the work that a launch would do (no device needed), with a scratch that is there for every call and with one
 // that is there where K has to be split: the team kernel's shares, or the list of the kernel without teams, every whole tile once, every
-// chunk of every split tile once, partial-tile indices distinct and below the scratch size.
+// chunk of every split tile once, partial-tile indices distinct and below the scratch size; -8 if a list that a layer object's scratch is there
+// to have cut (cut_anyhow) comes out whole, though it does not fill its last round.
 int gemm_schedule_selfcheck(int M, int N, int K, int slots_fit, int cus) {
     Schedule sc;
     int grid = 0;
@@ -1001,8 +1002,11 @@ int gemm_schedule_selfcheck(int M, int N, int K, int slots_fit, int cus) {
     }
     if (const int bad = schedule_walk(sc, grid, nb_k, slots_fit)) return bad;
     const int parts = sc.r * sc.c;
-    if (cut_anyhow(sc, nb_k, cus) && make_schedule(M, N, K, slots_fit, cus, kMaxPartials, true, sc, grid))
+    if (cut_anyhow(sc, nb_k, cus)) {
+        const bool fits = make_schedule(M, N, K, slots_fit, cus, kMaxPartials, true, sc, grid);
+        if (!fits || (sc.c == 1 && T % (slots_fit / cus * cus) != 0)) return -8;
         if (const int bad = schedule_walk(sc, grid, nb_k, slots_fit)) return bad;
+    }
     return parts;
 }
 

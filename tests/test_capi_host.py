@@ -131,6 +131,19 @@ def test_gemm_schedule_cuts_what_it_should(pkg, M, N, K, parts):
     assert pkg.capi.lib().a81w41_gemm_schedule_selfcheck(M, N, K, 1024, 256) == parts
 
 
+def test_gemm_schedule_of_a_layer_cuts_ranges_that_no_ring_divides(pkg):
+    """Between one and two tiles a CU a layer object's launch is cut from 40 super-blocks on, in halves and from 192 on in quarters, with remainders
+    of one to three; the check walks it and reports -8 if it was left whole."""
+    L = pkg.capi.lib()
+    for blocks in (41, 42, 43, 58, 61, 190, 191, 193, 194, 195, 209, 301):
+        for cus in (256, 64):
+            for M in (33, 70, 330, 1000, 2047):
+                rows = -(-M // 64)
+                for tiles in {cus // rows + 1, 3 * cus // (2 * rows), 2 * cus // rows}:
+                    # 0: a call without a layer does not cut them
+                    assert L.a81w41_gemm_schedule_selfcheck(M, 64 * tiles - 8, 64 * blocks, 4 * cus, cus) == 0, (M, tiles, blocks, cus)
+
+
 def test_block_scaled_gemm_plan_covers_every_unit_once(pkg):
     """The layer object's M > 32 kernel cuts the (tile, 32-block) units of a launch into equal contiguous runs:
     walked on the host for the layer's shapes and odd ones, for several device sizes."""

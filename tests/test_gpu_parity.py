@@ -172,8 +172,8 @@ def test_gemv_extreme_codes(pkg, ora, torch):
                                    # ... and with wave-private LDS stages on wide ones: ragged N, K not a multiple of
                                    # the ring or of the waves, shared K, more panels than workgroup slots
                                    (8, 4096, 12288), (7, 2056, 8192), (9, 8200, 64), (17, 9000, 320), (32, 8192, 1024), (20, 72000, 256), (25, 12288, 4096), (21, 1032, 320),
-                                   # more tiles than workgroup slots (768): whole rounds plus a K-split partial
-                                   # round, ragged rows and columns; 513..682 tiles: the two-per-CU schedule
+                                   # more tiles than one a CU over short K, ragged rows and columns: whole tiles, or (8 super-blocks, some teams) shared
+                                   # by two teams; rounds of which only a part is cut are in test_k_ranges_by_parts
                                    (256, 16384, 256), (322, 12288, 256), (1030, 4104, 256), (384, 24576, 512), (640, 4096, 256)])
 def test_gemm_parity(pkg, ora, synth, torch, M, N, K):
     w4, s, o = synth.weight_files(N, K, 79)
@@ -612,8 +612,8 @@ def test_teams_of_waves_on_a_tile(pkg, ora, synth, torch, M, N, K):
 
 
 # Between one and two tiles a CU, over 40 super-blocks and more that no ring divides, a layer cuts K: the fewest tiles and the most, the
-# shortest range, ragged rows and columns.  Whole rounds, which neither cuts: the fewest tiles and the most of up to two, two and a half, three and
-# four a CU and of a second round, with their longest ranges, and three and a fifth and a second round of few, where the rest is in quarters.
+# shortest range, ragged rows and columns.  The others both calls treat alike: whole tiles of up to two, two and a half, three and four a CU and of a
+# second round (with 576 and 1088 values of K because no ring divides them), 512 tiles that two teams share, and 780 rows with their last tiles in quarters.
 @pytest.mark.parametrize("M,N,K,cut", [(69, 8232, 2624, True), (330, 5440, 2624, True), (179, 5888, 3712, True), (33, 16392, 2688, True),
                                        (33, 16392, 1024, False), (512, 4096, 512, False), (513, 3640, 1536, False), (640, 4096, 1536, False),
                                        (641, 3720, 4096, False), (192, 16320, 576, False), (780, 4104, 2048, False), (868, 3976, 1088, False),
@@ -636,3 +636,17 @@ def test_k_ranges_whole_and_cut(pkg, ora, synth, torch, M, N, K, cut):
     assert torch.equal(got, alone) != cut   # the free-standing call, which has no scratch, does not cut them
     for _ in range(5):   # the last of several parts to arrive adds them in order, whoever it is
         assert torch.equal(layer.forward(xd), got)
+
+
+# The same with what a launch cuts pinned, by parts (0: none) of a call that has no scratch of its own.  Whole where rings divide K: 427 and 767 tiles, 882 over 16
+# super-blocks, 897 over 32.  Cut: halves of all, two tiles a CU and 128 in halves, three a CU and the rest in halves, a second round in quarters and in halves.
+# Cut by a layer only: quarters, one to three of them a super-block longer.
+@pytest.mark.parametrize("M,N,K,parts,cut", [(420, 3904, 1024, 0, False), (830, 3776, 2048, 0, False), (868, 3976, 1024, 0, False),
+                                             (830, 4416, 2048, 0, False), (420, 3904, 1536, 854, False), (600, 4096, 2560, 256, False),
+                                             (529, 6304, 1536, 246, False), (868, 4096, 2560, 256, False), (1030, 4096, 1024, 256, False),
+                                             (1280, 4096, 4096, 512, False), (330, 2728, 12352, 0, True), (450, 2104, 12416, 0, True),
+                                             (700, 1528, 12480, 0, True)])
+def test_k_ranges_by_parts(pkg, ora, synth, torch, M, N, K, parts, cut):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert pkg.capi.lib().a81w41_gemm_schedule_selfcheck(M, N, K, 4 * cus, cus) == parts
+    test_k_ranges_whole_and_cut(pkg, ora, synth, torch, M, N, K, cut)
