@@ -683,8 +683,9 @@ struct TeamPlan {
 //   half of the CUs, two parts of four teams: 128, K = 4096 16.6 / 16.2; 96, K = 4608 20.3 / 17.9; K = 3072, the schedule's own four 14.5 / 15.2
 //   T <= CUs, four teams: 256, K = 4096 23.6 / 21.3, K = 3072 19.9 / 17.7; 192, K = 4608 24.9 / 23.0; the schedule's own four, 192, K = 4096
 //     19.4 / 20.4, 250, K = 12288 51 / 55
-//   up to two tiles a CU, two teams where the schedule cuts K: 432, K = 1536 18.0 / 16.7; 448, K = 2048 21.9 / 20.8; 288, K = 1536 15.5 / 16.4,
-//     448, K = 704, which it does not cut, 10.6 / 11.6
+//   from 27/16 to two tiles a CU, K up to 2560 that two teams share in whole rings: against halves, 432, K = 1536 18.0 / 16.7; 448, K = 2048 21.9 / 20.8;
+//     480, K = 2560 30.1 / 28.5; against whole tiles, 484, K = 1024 15.7 / 15.4, but 460, K = 512 11.1 / 11.5 (with the line at K = 1024 that would
+//     be the better side; not drawn); not below, 288, K = 1536 15.5 / 16.4, nor in uneven shares, 448, K = 704 10.6 / 11.6
 // K that is no multiple of 512 the schedule did not cut: 40 rows, 2504 x 3712 25.6 / 11.8, 90 rows 25.9 / 14.6, 180 rows 26.0 / 15.8.
 TeamPlan plan_teams(const Schedule& sc, int nb_k, int cus, bool may_split) {
     const int T = sc.tiles_m * sc.tiles_n, mode = tuning_env_int("A81W41_GEMM_TEAMS");  // tuning builds: 9 = never, else how many
@@ -701,8 +702,9 @@ TeamPlan plan_teams(const Schedule& sc, int nb_k, int cus, bool may_split) {
 
 // Whether a K range that the schedule leaves whole, for want of a divisor, is cut all the same where there is a scratch.  Between one and two
 // tiles a CU whole ones leave many CUs with one while others have two.  us whole / cut: 168 rows, 6176 x 3904 39.1 / 32.0; 774 rows, 1464 x 3776
-// 41.8 / 35.8; 332 rows, 5024 x 3776 41.0 / 40.7; over 58 drawn shapes 1.14 times as fast, the worst 34.1 / 34.7 (406 rows, 4264 x 2944).  Not
-// over short ranges: 1154 rows, 1288 x 1152 19.6 / 21.9; with more tiles see whole_tiles_preferred.
+// 41.8 / 35.8; 332 rows, 5024 x 3776 41.0 / 40.7; in quarters 1623 rows, 1112 x 13184 129.9 / 126.3; over 87 drawn shapes with K up to 12224 1.12 times as
+// fast, 0.99 to 1.34, over 20 with more 1.19, 1.06 to 1.53.  Not over short ranges: 1154 rows, 1288 x 1152 19.6 / 21.9; with more tiles see
+// whole_tiles_preferred.
 bool cut_anyhow(const Schedule& sc, int nb_k, int cus) {
     const int T = sc.tiles_m * sc.tiles_n;
     return sc.c == 1 && nb_k >= 40 && T > cus && T <= 2 * cus;
