@@ -274,8 +274,9 @@ struct MemoryArgs {
     const float* norm = nullptr;                       // [heads vdim]
     float* state = nullptr;
     const int* pos_dev = nullptr;
-    // prompt kernels: [chunks][heads][chunk_size], [chunks + 1][heads], [chunks][heads][2]
+    // prompt kernels: [chunks][heads][chunk_size], [chunks + 1][heads], [chunks][heads][2], and the gates of a chunk's tokens [chunks][heads][3][kMemoryChunk]
     float *chunk_states = nullptr, *chunk_m = nullptr, *chunk_stats = nullptr;
+    double* chunk_gates = nullptr;
 };
 // Token by token, any sizes: o [M][heads vdim] as it is.
 hipError_t launch_memory_steps(const MemoryArgs& a, float* o, hipStream_t s);

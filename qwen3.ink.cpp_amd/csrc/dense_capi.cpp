@@ -161,10 +161,15 @@ static MemoryShape memory_shape(int heads, int dim, int vdim) {
 
 size_t a81w41_matrix_memory_state(int heads, int dim, int vdim) { return memory_shape(heads, dim, vdim).state_size(); }
 
+// Floats of the chunks' states, scales and stats; behind them, at a whole double, come the gates.
+static size_t memory_chunk_floats(const MemoryShape& sh, size_t chunks) {
+    return (chunks * sh.heads * sh.chunk_size() + (3 * chunks + 1) * sh.heads + 1) / 2 * 2;
+}
+
 size_t a81w41_matrix_memory_scratch(int heads, int dim, int vdim, int M) {
     const MemoryShape sh = memory_shape(heads, dim, vdim);
     const size_t chunks = (M + kMemoryChunk - 1) / kMemoryChunk, H = heads;
-    return std::max(chunks * H * sh.chunk_size() + (3 * chunks + 1) * H, (size_t)M * H * vdim);
+    return std::max(memory_chunk_floats(sh, chunks) + 2 * chunks * H * 3 * kMemoryChunk, (size_t)M * H * vdim);
 }
 
 int a81w41_matrix_memory(const float* in, int ld_in, int M, int heads, int dim, int vdim, float cap, float eps, const float* bias_i,
@@ -188,6 +193,7 @@ int a81w41_matrix_memory(const float* in, int ld_in, int M, int heads, int dim, 
     a.chunk_states = scratch;
     a.chunk_m = scratch + chunks * heads * a.sh.chunk_size();
     a.chunk_stats = a.chunk_m + (chunks + 1) * heads;
+    a.chunk_gates = reinterpret_cast<double*>(scratch + memory_chunk_floats(a.sh, chunks));
     A81W41_HIP_TRY(launch_memory_chunks<float>(a, out, heads * vdim, s));
     return 0;
 }

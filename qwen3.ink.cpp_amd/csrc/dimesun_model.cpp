@@ -242,6 +242,7 @@ class DimesunModel final : public DenseModel<T> {
     float *part_ = nullptr, *part_stats_ = nullptr;  // shares of the attention
     size_t part_rows_ = 0;
     float *chunk_states_ = nullptr, *chunk_m_ = nullptr, *chunk_stats_ = nullptr;
+    double* chunk_gates_ = nullptr;
     int *chosen_ = nullptr, *src_rows_ = nullptr, *slot_rows_ = nullptr, *n_tiles_ = nullptr;
     float* expert_weights_ = nullptr;
     GroupTile* tiles_ = nullptr;
@@ -386,6 +387,7 @@ int DimesunModel<T>::allocate(int max_seq) {
         A81W41_TRY(allocate_array(chunks * chunk_states, &chunk_states_));
         A81W41_TRY(allocate_array((chunks + 1) * memory_heads, &chunk_m_));
         A81W41_TRY(allocate_array(chunks * memory_heads * 2, &chunk_stats_));
+        A81W41_TRY(allocate_array(chunks * memory_heads * 3 * kMemoryChunk, &chunk_gates_));
     }
     if (top) {
         A81W41_TRY(allocate_array(R * act, &act_));
@@ -437,7 +439,7 @@ MemoryArgs DimesunModel<T>::memory_args(const Layer& L, const MemoryShape& sh, c
     MemoryArgs a;
     a.sh = sh, a.in = in_, a.ld_in = ld_in, a.M = M, a.bias_i = L.bias_i, a.bias_f = L.bias_f, a.norm = L.memory_norm;
     a.state = kept.state, a.pos_dev = pos;
-    a.chunk_states = chunk_states_, a.chunk_m = chunk_m_, a.chunk_stats = chunk_stats_;
+    a.chunk_states = chunk_states_, a.chunk_m = chunk_m_, a.chunk_stats = chunk_stats_, a.chunk_gates = chunk_gates_;
     return a;
 }
 

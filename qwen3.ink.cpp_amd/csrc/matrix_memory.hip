@@ -204,6 +204,10 @@ __global__ __launch_bounds__(kThreads) void memory_outer_kernel(MemoryArgs a) {
             st[0] = (float)most;
             st[1] = (float)g.b;
         }
+        if (blockIdx.z == 0) {
+            double* to = a.chunk_gates + ((size_t)chunk * sh.heads + h) * 3 * C + lane;
+            to[0] = g.b, to[C] = g.a, to[2 * C] = g.most;
+        }
     }
     dense_lds_barrier();
     for (int first = 0; first < kLoads; first += kBatch) {
@@ -247,22 +251,22 @@ __global__ __launch_bounds__(kThreads) void memory_outer_kernel(MemoryArgs a) {
 
 // The chain over chunks for W neighbouring elements of a head's S and n: chunk_states becomes the state before each chunk,
 // the state itself the one after the last; chunk_m the scales.
+//
+// What bounds it: the trips of one element's chain.  kAhead chunks of it are under way, and what a chunk's sums are scaled by is formed
+// ahead, a chunk a lane: read and formed by every thread inside the chain, 8 heads of 128 x 256 over 32 chunks took 18.7 us, now 16.4; 141
+// chunks of 32 x 64 and 2 heads 49.9, now 25.8.
 template <int W>
 __global__ __launch_bounds__(kThreads) void memory_chain_kernel(MemoryArgs a, int chunks) {
-    constexpr int kAhead = 4;
+    constexpr int kAhead = 8, kScales = 64;
+    __shared__ float keep[kScales], add[kScales];
     const MemoryShape sh = a.sh;
-    const int h = blockIdx.y, pos = max(a.pos_dev[0], 0);
+    const int h = blockIdx.y, pos = max(a.pos_dev[0], 0), lane = threadIdx.x & 63;
     const size_t e = ((size_t)blockIdx.x * kThreads + threadIdx.x) * W, s_size = (size_t)sh.dim * sh.vdim, size = sh.chunk_size();
     const size_t nm = (size_t)h * (sh.dim + 1);
-    float m = state_nm(a, pos)[nm + sh.dim];
-    const bool scale_writer = e == 0;
-    if (e >= size) return;
-    const bool in_s = e < s_size;  // W > 1: the parts are whole multiples of W
+    const bool mine = e < size, in_s = e < s_size;  // W > 1: the parts are whole multiples of W
     const float* from = in_s ? a.state + h * s_size + e : state_nm(a, pos) + nm + (e - s_size);
     float* to = in_s ? a.state + h * s_size + e : state_nm(a, pos + a.M) + nm + (e - s_size);
-    float cur[W];
-#pragma unroll
-    for (int w = 0; w < W; w++) cur[w] = from[w];
+    alignas(16) float cur[W], next[kAhead][W];
     const size_t step = (size_t)sh.heads * size;
     float* at = a.chunk_states + h * size + e;
     auto load = [&](float* dst, int c) {
@@ -272,184 +276,234 @@ __global__ __launch_bounds__(kThreads) void memory_chain_kernel(MemoryArgs a, in
         else
             dst[0] = src[0];
     };
-    alignas(16) float next[kAhead][W];
+    if (mine) {
 #pragma unroll
-    for (int u = 0; u < kAhead; u++) load(next[u], u);
-    for (int c0 = 0; c0 < chunks; c0 += kAhead) {
-        alignas(16) float now[kAhead][W];
+        for (int w = 0; w < W; w++) cur[w] = from[w];
 #pragma unroll
-        for (int u = 0; u < kAhead; u++)
-#pragma unroll
-            for (int w = 0; w < W; w++) now[u][w] = next[u][w];
-        if (c0 + kAhead < chunks) {
-#pragma unroll
-            for (int u = 0; u < kAhead; u++) load(next[u], c0 + kAhead + u);
+        for (int u = 0; u < kAhead; u++) load(next[u], u);
+    }
+    float m = state_nm(a, pos)[nm + sh.dim];
+    for (int first = 0; first < chunks; first += kScales) {
+        const int n = min(kScales, chunks - first);
+        if (first) dense_lds_barrier();  // nobody still reads the scales before
+        if (threadIdx.x < 64) {
+            const float* st = a.chunk_stats + 2 * ((size_t)(first + min(lane, n - 1)) * sh.heads + h);
+            const float most_own = st[0], sum_own = st[1];
+            float before = m;
+            for (int c = 0; c < n; c++) {
+                if (lane == c) before = m;
+                const float most = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(most_own), c));
+                m = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sum_own), c)) + fmaxf(m, most);
+            }
+            const float most = fmaxf(before, most_own);
+            keep[lane] = expf(before - most);
+            add[lane] = expf(most_own - most);
+            if (blockIdx.x == 0 && lane < n) a.chunk_m[(size_t)(first + lane) * sh.heads + h] = before;
         }
+        dense_lds_barrier();
+        if (!mine) continue;
+        for (int c0 = first; c0 < first + n; c0 += kAhead) {
+            alignas(16) float now[kAhead][W];
 #pragma unroll
-        for (int u = 0; u < kAhead; u++) {
-            const int c = c0 + u;
-            if (c >= chunks) break;
-            const float* st = a.chunk_stats + 2 * ((size_t)c * sh.heads + h);
-            const float most = fmaxf(m, st[0]), keep = expf(m - most), add = expf(st[0] - most);
-            if (scale_writer) a.chunk_m[(size_t)c * sh.heads + h] = m;
-            if constexpr (W == 4)
-                store4(at + c * step, *reinterpret_cast<const float4*>(cur));
-            else
-                at[c * step] = cur[0];
+            for (int u = 0; u < kAhead; u++)
 #pragma unroll
-            for (int w = 0; w < W; w++) cur[w] = fmaf(keep, cur[w], add * now[u][w]);
-            m = st[1] + most;
+                for (int w = 0; w < W; w++) now[u][w] = next[u][w];
+            if (c0 + kAhead < chunks) {
+#pragma unroll
+                for (int u = 0; u < kAhead; u++) load(next[u], c0 + kAhead + u);
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; u++) {
+                const int c = c0 + u;
+                if (c >= chunks) break;
+                if constexpr (W == 4)
+                    store4(at + c * step, *reinterpret_cast<const float4*>(cur));
+                else
+                    at[c * step] = cur[0];
+#pragma unroll
+                for (int w = 0; w < W; w++) cur[w] = fmaf(keep[c - first], cur[w], add[c - first] * now[u][w]);
+            }
         }
     }
+    if (mine) {
 #pragma unroll
-    for (int w = 0; w < W; w++) to[w] = cur[w];
-    if (scale_writer) a.chunk_m[(size_t)chunks * sh.heads + h] = m;
+        for (int w = 0; w < W; w++) to[w] = cur[w];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.chunk_m[(size_t)chunks * sh.heads + h] = m;
 }
 
-// Outputs of a chunk for one head, 64 tokens x vdim columns in the accumulators: 64 x 32 VF per wave.  q and k come through
-// LDS, 64 columns at a time; rows of S and v go from memory to the matrix operands, requested ahead of the barriers.
+// Outputs of 32 tokens of a chunk for one head, 32 tokens x vdim columns in the accumulators: 32 x 32 VF per wave.  q and k come
+// through LDS, 64 columns at a time; rows of S and v go from memory to the matrix operands, S kAhead x 32 columns of q ahead.
+//
+// What bounds it: where chunks are few one workgroup's way, products in 32 bits (two fifths) and what waits for them; where they are many also
+// the single floats of S and v, an instruction for two rows.  So a workgroup has half a chunk, two of them fit a CU, the halves with
+// all keys come first, rows of v follow those of S in one ring, scores are weighted by all waves, and gates are as memory_outer_kernel left them.
+// us, so / with a chunk a workgroup, S and v requested just ahead of their use and gates formed again: 8 heads of 128 + 256
+// columns, 1 chunk 18.9 / 36.2, 3 chunks 19.9 / 36.7, 13 chunks 22.1 / 41.2, 32 chunks 34.0 / 44.7; 64 + 128, 32 chunks 20.1 / 28.7; 4 heads
+// of 256 + 512, 11 chunks 46.6 / 85.
 constexpr int kStep = 64;          // columns of q and k in LDS at a time
 constexpr int kLd = kStep + 4;     // floats of an LDS row: sixteen-byte reads of neighbouring rows spread over the banks
+constexpr int kOut = 32;           // tokens of a workgroup
+static_assert(2 * kOut == C, "a chunk has two halves");
 template <typename T, int W, int WAVES, int VF>
-__global__ __launch_bounds__(64 * WAVES) void memory_outputs_kernel(MemoryArgs a, int chunks, T* __restrict__ out, int ld_out) {
-    constexpr int kT = 64 * WAVES, kPer = kStep / W, kLoads = C * kPer / kT;
+__global__ __launch_bounds__(64 * WAVES, W == 4 && WAVES == 8 && VF == 1 ? 4 : 2) void memory_outputs_kernel(MemoryArgs a, int chunks, T* __restrict__ out, int ld_out) {
+    constexpr int kT = 64 * WAVES, kPer = kStep / W, kLoadsQ = kOut * kPer / kT, kLoadsK = C * kPer / kT;
     constexpr int kTeam = kT / C;  // threads that share a token's sums
-    __shared__ __attribute__((aligned(16))) float qs[C * kLd], ks[C * kLd];  // ks holds the weighted scores afterwards
-    __shared__ double log_a[C], log_most[C];                                // a_s, M_t
-    __shared__ float start[C], floor_t[C], den[C], inv[C], squares[C][WAVES], n_part[kStep];
+    __shared__ __attribute__((aligned(16))) float qs[kOut * kLd], ks[C * kLd];
+    __shared__ __attribute__((aligned(16))) float scored[2][kOut * kLd];  // the scores' shares [token][key], then weighted in the first
+    __shared__ double log_a[C], log_most[kOut];                         // a_s, M_t
+    __shared__ float start[kOut], floor_t[kOut], den[kOut], inv[kOut], squares[kOut][WAVES], n_part[kStep];
     const MemoryShape sh = a.sh;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, l31 = lane & 31, half = lane >> 5;
-    const int chunk = blockIdx.x, h = blockIdx.y, m0 = chunk * C, count = min(C, a.M - m0);
-    const float m_start = a.chunk_m[(size_t)chunk * sh.heads + h];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), l31 = lane & 31, half = lane >> 5;
+    const int late = 1 - (int)blockIdx.z, chunk = blockIdx.x, h = blockIdx.y, m0 = chunk * C, t0 = late * kOut;
+    const int count = min(C, a.M - m0), rows = min(kOut, count - t0), keys = min(count, t0 + kOut);  // rows: of this half
+    // the scale after the last chunk goes to the state only now: the chain's workgroups all read the old one
+    if (!late && chunk == chunks - 1 && t == 0)
+        state_nm(a, max(a.pos_dev[0], 0) + a.M)[(size_t)h * (sh.dim + 1) + sh.dim] = a.chunk_m[(size_t)chunks * sh.heads + h];
+    if (rows <= 0) return;
     const float* S = a.chunk_states + ((size_t)chunk * sh.heads + h) * sh.chunk_size();
     const float* n = S + (size_t)sh.dim * sh.vdim;
     const int col0 = wave * 32 * VF + l31;
-    float q_part[kLoads][W], k_part[kLoads][W], n_own = 0.f;
+    float q_part[kLoadsQ][W], k_part[kLoadsK][W], n_own = 0.f;
     auto request = [&](int d0) {
 #pragma unroll
-        for (int u = 0; u < kLoads; u++) {
+        for (int u = 0; u < kLoadsQ; u++) {
             const int i = t + u * kT, s = i / kPer, d = d0 + i % kPer * W;
-            const float* row = a.in + (size_t)(m0 + min(s, count - 1)) * a.ld_in + h * sh.dim + d;
-            const bool real = s < count && d < sh.dim;
-            read_part<W>(q_part[u], row + sh.at_q, real);
-            read_part<W>(k_part[u], row + sh.at_k, real);
+            read_part<W>(q_part[u], a.in + (size_t)(m0 + t0 + min(s, rows - 1)) * a.ld_in + h * sh.dim + d + sh.at_q, s < rows && d < sh.dim);
+        }
+#pragma unroll
+        for (int u = 0; u < kLoadsK; u++) {
+            const int i = t + u * kT, s = i / kPer, d = d0 + i % kPer * W;
+            read_part<W>(k_part[u], a.in + (size_t)(m0 + min(s, keys - 1)) * a.ld_in + h * sh.dim + d + sh.at_k, s < keys && d < sh.dim);
         }
         if (t < kStep) n_own = d0 + t < sh.dim ? n[d0 + t] : 0.f;
     };
-    constexpr int kHalf = kStep / 16;  // operand steps of eight columns: half of those of a pass
-    float b[kHalf][VF][4];
-    auto request_states = [&](int d0) {
+    // Parts of 32 rows, kHalf operand steps of eight: those of S, in pairs, and two of v.  kAhead parts are under way.
+    constexpr int kHalf = kStep / 16, kAhead = VF == 1 ? 2 : 1;
+    const int parts = (sh.dim + 31) / 32, first_v = (parts + 1) / 2 * 2;
+    const float* v_rows = a.in + (size_t)m0 * a.ld_in + sh.at_v + h * sh.vdim;
+    float b[kAhead][kHalf][VF][4];
+    auto request_part = [&](float (&to)[kHalf][VF][4], int p) {
+        const bool values = p >= first_v;
+        if (p >= first_v + late + 1) return;  // keys that come later count nothing
+        const float* src = values ? v_rows : S;
+        const int ld = values ? a.ld_in : sh.vdim, row0 = 32 * (values ? p - first_v : p), last = values ? count - 1 : sh.dim - 1;
 #pragma unroll
         for (int kk = 0; kk < kHalf; kk++)
 #pragma unroll
             for (int f = 0; f < VF; f++)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    b[kk][f][j] = S[(size_t)min(d0 + 4 * (2 * kk + half) + j, sh.dim - 1) * sh.vdim + min(col0 + 32 * f, sh.vdim - 1)];
+                    to[kk][f][j] = src[(size_t)min(row0 + 4 * (2 * kk + half) + j, last) * ld + min(col0 + 32 * f, sh.vdim - 1)];
     };
     request(0);
-    if (wave == 0) {
-        const ChunkGates g = chunk_gates(a, m0, count, h);
-        const double most = fmax((double)m_start, g.most);
-        log_a[lane] = g.a;
-        log_most[lane] = most;
-        start[lane] = expf((float)((double)m_start - most));
-        floor_t[lane] = expf(-(float)(g.b + most));
+    if (wave == WAVES - 1) {
+        const double* g = a.chunk_gates + ((size_t)chunk * sh.heads + h) * 3 * C;
+        const float m_start = a.chunk_m[(size_t)chunk * sh.heads + h];
+        log_a[lane] = g[C + lane];
+        if (lane < kOut) {
+            const double most = fmax((double)m_start, g[2 * C + t0 + lane]);
+            log_most[lane] = most;
+            start[lane] = expf((float)((double)m_start - most));
+            floor_t[lane] = expf(-(float)(g[t0 + lane] + most));
+        }
     }
-    // the scale after the last chunk goes to the state only now: the chain's workgroups all read the old one
-    if (chunk == chunks - 1 && t == 0)
-        state_nm(a, max(a.pos_dev[0], 0) + a.M)[(size_t)h * (sh.dim + 1) + sh.dim] = a.chunk_m[(size_t)chunks * sh.heads + h];
-    f32x16 acc[2][VF], score;
+#pragma unroll
+    for (int u = 0; u < kAhead; u++) request_part(b[u], u);
+    f32x16 acc[VF], score;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
         score[i] = 0.f;
 #pragma unroll
-        for (int f = 0; f < VF; f++) acc[0][f][i] = acc[1][f][i] = 0.f;
+        for (int f = 0; f < VF; f++) acc[f][i] = 0.f;
     }
-    // this wave's piece of the scores, tokens st.. and keys ss..; the waves from 4 on take every second operand step
-    const int st = (wave & 1) * 32, ss = (wave >> 1 & 1) * 32;
+    // The scores of 32 keys: of two waves each has every second operand step, or one wave has all.
+    constexpr int kShares = WAVES == 4 ? 1 : 2;
+    const int ss = (wave & 1) * 32, share = wave >> 1;
+    const bool scores = wave < 2 * kShares && ss <= t0;
     float nq = 0.f;  // of token t / kTeam, a share of the columns
+    const bool sums = t < kOut * kTeam;
     for (int d0 = 0; d0 < sh.dim; d0 += kStep) {
-        request_states(d0);
         if (d0) dense_lds_barrier();  // nobody still reads the columns before
 #pragma unroll
-        for (int u = 0; u < kLoads; u++) {
+        for (int u = 0; u < kLoadsQ; u++) {
             const int i = t + u * kT, at = i / kPer * kLd + i % kPer * W;
 #pragma unroll
             for (int e = 0; e < W; e++) q_part[u][e] *= sh.q_scale;
             write_part<W>(qs + at, q_part[u]);
-            write_part<W>(ks + at, k_part[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kLoadsK; u++) {
+            const int i = t + u * kT;
+            write_part<W>(ks + i / kPer * kLd + i % kPer * W, k_part[u]);
         }
         if (t < kStep) n_part[t] = n_own;
         dense_lds_barrier();
         if (d0 + kStep < sh.dim) request(d0 + kStep);
 #pragma unroll
         for (int part = 0; part < 2; part++) {
-            if (part) request_states(d0 + kStep / 2);
-            if (d0 + part * (kStep / 2) >= sh.dim) break;
+            const int p = d0 / 32 + part;
+            if (p < parts) {
 #pragma unroll
-            for (int kk = 0; kk < kHalf; kk++) {
-                const int step = part * kHalf + kk, at = 4 * (2 * step + half);
-                alignas(16) float q[2][4], k[4];
+                for (int kk = 0; kk < kHalf; kk++) {
+                    const int step = part * kHalf + kk, at = 4 * (2 * step + half);
+                    alignas(16) float q[4], k[4];
+                    *reinterpret_cast<float4*>(q) = load4(qs + l31 * kLd + at);
 #pragma unroll
-                for (int i = 0; i < 2; i++) *reinterpret_cast<float4*>(q[i]) = load4(qs + (i * 32 + l31) * kLd + at);
+                    for (int f = 0; f < VF; f++)
 #pragma unroll
-                for (int f = 0; f < VF; f++)
+                        for (int j = 0; j < 4; j++) acc[f] = mfma32(q[j], b[part % kAhead][kk][f][j], acc[f]);
+                    if (scores && (kShares == 1 || (step & 1) == share)) {
+                        *reinterpret_cast<float4*>(k) = load4(ks + (ss + l31) * kLd + at);
 #pragma unroll
-                    for (int j = 0; j < 4; j++)
-#pragma unroll
-                        for (int i = 0; i < 2; i++) acc[i][f] = mfma32(q[i][j], b[kk][f][j], acc[i][f]);
-                // a piece whose keys all come later counts nothing
-                if (ss <= st && (WAVES == 4 || (step & 1) == wave >> 2)) {
-                    *reinterpret_cast<float4*>(k) = load4(ks + (ss + l31) * kLd + at);
-#pragma unroll
-                    for (int j = 0; j < 4; j++) score = mfma32(st ? q[1][j] : q[0][j], k[j], score);
+                        for (int j = 0; j < 4; j++) score = mfma32(q[j], k[j], score);
+                    }
                 }
             }
+            request_part(b[part % kAhead], p + kAhead);
         }
+        if (sums) {
 #pragma unroll
-        for (int c = 0; c < kStep / kTeam; c++) {
-            const int d = t % kTeam + kTeam * c;
-            nq = fmaf(qs[t / kTeam * kLd + d], n_part[d], nq);
-        }
-    }
-    // the first rows of v, while the scores are weighted
-    constexpr int kRowsAhead = 4;
-    const float* v_rows = a.in + sh.at_v + h * sh.vdim;
-    float v[kRowsAhead][VF][4];
-    auto request_values = [&](int kk0) {
-#pragma unroll
-        for (int kk = 0; kk < kRowsAhead; kk++)
-#pragma unroll
-            for (int f = 0; f < VF; f++)
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    v[kk][f][j] = v_rows[(size_t)(m0 + min(4 * (2 * (kk0 + kk) + half) + j, count - 1)) * a.ld_in + min(col0 + 32 * f, sh.vdim - 1)];
-    };
-    request_values(0);
-    dense_lds_barrier();
-    float* weighted = ks;  // [token][key]
-    for (int turn = 0; turn < WAVES / 4; turn++) {
-        if (wave >> 2 == turn) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int token = st + 8 * (i >> 2) + 4 * half + (i & 3), key = ss + l31;
-                float& w = weighted[token * kLd + key];
-                const float own = key <= token ? score[i] * expf((float)(log_a[key] - log_most[token])) : 0.f;
-                w = turn ? w + own : own;
+            for (int c = 0; c < kStep / kTeam; c++) {
+                const int d = t % kTeam + kTeam * c;
+                nq = fmaf(qs[t / kTeam * kLd + d], n_part[d], nq);
             }
         }
-        dense_lds_barrier();
     }
+    float gate[VF][16];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int f = 0; f < VF; f++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
-            const float w = start[i * 32 + 8 * (r >> 2) + 4 * half + (r & 3)];
-#pragma unroll
-            for (int f = 0; f < VF; f++) acc[i][f][r] *= w;
+            const int token = min(8 * (r >> 2) + 4 * half + (r & 3), rows - 1);
+            gate[f][r] = a.in[(size_t)(m0 + t0 + token) * a.ld_in + sh.at_g + h * sh.vdim + min(col0 + 32 * f, sh.vdim - 1)];
         }
-    {
+    if (scores) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) scored[share][(8 * (i >> 2) + 4 * half + (i & 3)) * kLd + ss + l31] = score[i];
+    }
+    dense_lds_barrier();
+    float* const weighted = scored[0];
+    for (int i = t; i < kOut * C / 4; i += kT) {
+        const int token = i / (C / 4), key0 = i % (C / 4) * 4, at = token * kLd + key0;
+        float w[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const bool seen = key0 + e <= t0 + token;
+            const float decay = expf((float)(log_a[key0 + e] - log_most[token]));
+            w[e] = seen ? scored[0][at + e] * decay : 0.f;
+            if (kShares == 2) w[e] += seen ? scored[1][at + e] * decay : 0.f;
+        }
+        store4(weighted + at, make_float4(w[0], w[1], w[2], w[3]));
+    }
+    dense_lds_barrier();
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const float w = start[8 * (r >> 2) + 4 * half + (r & 3)];
+#pragma unroll
+        for (int f = 0; f < VF; f++) acc[f][r] *= w;
+    }
+    if (sums) {
         const int token = t / kTeam;
         float sum = nq * start[token];
 #pragma unroll
@@ -458,65 +512,50 @@ __global__ __launch_bounds__(64 * WAVES) void memory_outputs_kernel(MemoryArgs a
         if (t % kTeam == 0) den[token] = 1.0f / (fmaxf(fabsf(sum), floor_t[token]) + kMemoryFloor);
     }
 #pragma unroll
-    for (int kk0 = 0; kk0 < C / 8; kk0 += kRowsAhead) {
-        if (kk0) request_values(kk0);
+    for (int u = 0; u < 2; u++) {
+        if (u > late) break;
 #pragma unroll
-        for (int kk = 0; kk < kRowsAhead; kk++) {
-            const int at = 4 * (2 * (kk0 + kk) + half);
-            alignas(16) float p[2][4];
-#pragma unroll
-            for (int i = 0; i < 2; i++) *reinterpret_cast<float4*>(p[i]) = load4(weighted + (i * 32 + l31) * kLd + at);
+        for (int kk = 0; kk < kHalf; kk++) {
+            alignas(16) float p[4];
+            *reinterpret_cast<float4*>(p) = load4(weighted + l31 * kLd + 32 * u + 4 * (2 * kk + half));
 #pragma unroll
             for (int f = 0; f < VF; f++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    if (kk0 + kk < C / 16) acc[0][f] = mfma32(p[0][j], v[kk][f][j], acc[0][f]);
-                    acc[1][f] = mfma32(p[1][j], v[kk][f][j], acc[1][f]);
-                }
+                for (int j = 0; j < 4; j++) acc[f] = mfma32(p[j], b[u % kAhead][kk][f][j], acc[f]);
         }
+        if (u + kAhead < 2) request_part(b[u % kAhead], first_v + u + kAhead);
     }
     dense_lds_barrier();
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int r = 0; r < 16; r++) {
+        const int token = 8 * (r >> 2) + 4 * half + (r & 3);
+        const float d = den[token];
+        float sum = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int token = i * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-            const float d = den[token];
-            float sum = 0.f;
-#pragma unroll
-            for (int f = 0; f < VF; f++) {
-                acc[i][f][r] *= d;
-                if (col0 + 32 * f < sh.vdim) sum = fmaf(acc[i][f][r], acc[i][f][r], sum);
-            }
-            sum = dense_wave_sum(sum, 32);
-            if (l31 == 0) squares[token][wave] = sum;
+        for (int f = 0; f < VF; f++) {
+            acc[f][r] *= d;
+            if (col0 + 32 * f < sh.vdim) sum = fmaf(acc[f][r], acc[f][r], sum);
         }
-    __syncthreads();
-    if (t < C) {
+        sum = dense_wave_sum(sum, 32);
+        if (l31 == 0) squares[token][wave] = sum;
+    }
+    dense_lds_barrier();
+    if (t < kOut) {
         float sum = 0.f;
         for (int w = 0; w < WAVES; w++) sum += squares[t][w];
         inv[t] = 1.0f / sqrtf(sum / (float)sh.vdim + sh.eps);
     }
-    __syncthreads();
+    dense_lds_barrier();
 #pragma unroll
     for (int f = 0; f < VF; f++) {
         const int col = col0 + 32 * f;
         if (col >= sh.vdim) continue;
         const float w = a.norm[h * sh.vdim + col];
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            float gate[16];
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int token = min(i * 32 + 8 * (r >> 2) + 4 * half + (r & 3), count - 1);
-                gate[r] = a.in[(size_t)(m0 + token) * a.ld_in + sh.at_g + h * sh.vdim + col];
-            }
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int token = i * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-                if (token < count)
-                    out[(size_t)(m0 + token) * ld_out + h * sh.vdim + col] = (T)(acc[i][f][r] * inv[token] * w * sigmoid(gate[r]));
-            }
+        for (int r = 0; r < 16; r++) {
+            const int token = 8 * (r >> 2) + 4 * half + (r & 3);
+            if (token < rows)
+                out[(size_t)(m0 + t0 + token) * ld_out + h * sh.vdim + col] = (T)(acc[f][r] * inv[token] * w * sigmoid(gate[f][r]));
         }
     }
 }
@@ -534,7 +573,7 @@ hipError_t launch_chunks(const MemoryArgs& a, T* out, int ld_out, hipStream_t s)
     const int parts = (int)(sh.chunk_size() / W);
     hipLaunchKernelGGL(memory_outer_kernel<W>, dim3(chunks, sh.heads, tiles), dim3(kThreads), 0, s, a);
     hipLaunchKernelGGL(memory_chain_kernel<W>, dim3((parts + kThreads - 1) / kThreads, sh.heads), dim3(kThreads), 0, s, a, chunks);
-    const dim3 grid(chunks, sh.heads);
+    const dim3 grid(chunks, sh.heads, 2);
     if (sh.vdim <= 128)
         hipLaunchKernelGGL((memory_outputs_kernel<T, W, 4, 1>), grid, dim3(256), 0, s, a, chunks, out, ld_out);
     else if (sh.vdim <= 256)

@@ -189,6 +189,20 @@ def test_matrix_memory(pkg, heads, dim, vdim, gates):
         close(got, want, 5e-5, (variants, sizes))
 
 
+@pytest.mark.parametrize("T", [31, 32, 33, 64, 95, 97])
+@pytest.mark.parametrize("heads,dim,vdim", [(1, 32, 128), (2, 96, 256), (1, 64, 129), (2, 30, 264)])
+def test_matrix_memory_halves_of_a_chunk(pkg, heads, dim, vdim, T):
+    """The chunked form's workgroups take 32 tokens each: the last of a half, a half of its own and one more."""
+    import torch
+    cap, eps = 15.0, 0.3
+    rows, bi, bf, norm = _memory_rows(T, heads, dim, vdim, T + dim, *GATES["mixed"])
+    want = _memory_reference(rows, heads, dim, vdim, cap, eps, bi, bf, norm)
+    dev = [torch.from_numpy(x).cuda() for x in (bi, bf, norm)]
+    state = pkg.ops.matrix_memory_state(heads, dim, vdim)
+    got = pkg.ops.matrix_memory(torch.from_numpy(rows).cuda(), heads, dim, vdim, cap, eps, *dev, state, 0, 1).cpu().numpy()
+    close(got, want, 5e-5, (T, heads, dim, vdim))   # as test_matrix_memory: sums of 32-bit products of up to 97 tokens
+
+
 def test_matrix_memory_finds_a_far_token(pkg):
     """One key among hundreds is asked for again, across chunks and portions: a lost or decayed state would not have it."""
     import torch
