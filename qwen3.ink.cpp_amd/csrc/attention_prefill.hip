@@ -1,8 +1,8 @@
 // Causal GQA attention for many new tokens at once (the prompt pass) on the matrix cores:
 // QK^T * scale, causal mask, softmax, PV (QwenAttention.cc:150-195) over the fp16 KV cache.
 //
-// One workgroup per (tile of 32 query tokens, KV head) with G x S waves: the G query heads of the
-// KV group share every staged key / value tile, and the key tiles of a head are dealt round-robin
+// One workgroup per (tile of 32 query tokens, G query heads of a KV head) with G x S waves: the heads
+// share every staged key / value tile, and the key tiles of a head are dealt round-robin
 // to S waves, which shortens the serial walk over the context S times.  Each wave keeps the
 // running-maximum ("online") softmax of its share in fp32; the S shares are merged at the end.
 //
@@ -14,7 +14,7 @@
 // registers plus one exchange with lane q of the other half, and the rescaling factor of the
 // running output is a per-lane scalar.  The same registers feed the second product directly:
 // its contraction index may run over the keys in any order as long as V^T uses the same one,
-// so the value tile is staged transposed in LDS in exactly the order the P registers have.
+// and transposing LDS reads give V^T in exactly the order the P registers have.
 //
 // The cache holds fp16, which the matrix cores take as it is.  The fp32 queries and
 // probabilities are split into two fp16 terms (x = hi + lo, |lo| <= 2^-11 |hi|) and multiplied
@@ -39,22 +39,45 @@ namespace {
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
 constexpr int kHeadDim = 128;
 constexpr int kTile = 32;         // query tokens per workgroup, keys per step
-constexpr int kKStride = 272;     // bytes per key row of the staged key tile (256 + 16: conflict-free 16-byte reads)
-// Bytes per head-dim row of the transposed value tile (32 keys * 2 + 8).  18 words: the rows 8 apart that
-// the lanes of a wave write together fall into alternating halves of the 32 banks, and the 8-byte operand
-// reads of 32 consecutive rows cover every bank once.
-constexpr int kVStride = 72;
-constexpr int kTileLdsBytes = kTile * kKStride + kHeadDim * kVStride;  // one key tile + one transposed value tile
-constexpr int kMergeSlotBytes = 64 * 64 * 4;                           // one wave's 128 x 32 fp32 output
+constexpr int kRowBytes = 256;    // of a staged key or value
+constexpr int kKeyBytes = kTile * kRowBytes, kTileBytes = 2 * kKeyBytes;  // 32 keys, then their values, as the cache has them
+constexpr int kQueryBytes = kTile * kHeadDim * 4;                        // a head's 32 queries in fp32
+constexpr int kBlockBytes = 64 * 16 * 4;                                 // 32 head dims of one wave's 128 x 32 fp32 output
 constexpr float kLowest = -3.0e38f;
 
-// Position of key `key` (0..31 inside the tile) along the contraction index of the second product:
-// register v = 4g + i of half kh holds key 8g + 4kh + i; chunk c = g >> 1 takes registers 8c..8c+7.
-__device__ __forceinline__ int value_slot(int key) {
-    const int g = key >> 3, kh = (key >> 2) & 1, i = key & 3;
-    return ((g >> 1) * 2 + kh) * 8 + 4 * (g & 1) + i;
+// Sixteen-byte chunk c of a staged row sits at place c ^ this.  Keys are read 32 rows at one chunk, values by transposing
+// reads of four rows and four chunks: either way the places of a read cover the banks.
+__device__ __forceinline__ int key_swap(int key) { return key & 15; }
+__device__ __forceinline__ int value_swap(int key) { return (key & 3) << 2; }
+
+__device__ __forceinline__ void copy16(const void* src, void* lds_base) {  // lane l's sixteen bytes land at lds_base + 16 l
+    __builtin_amdgcn_global_load_lds(src, (lds_ptr_t)lds_base, 16, 0, 0);
+}
+// This wave's copies are in LDS and its LDS reads done, then every wave's.
+__device__ __forceinline__ void wait_and_meet() {
+    __builtin_amdgcn_s_waitcnt(0x0070);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// A^T operands of 32 keys' values: two steps of 16 keys for the lane's head dim.  `at`: where the lane's four dims of key 4 (lane / 32) +
+// lane % 16 / 4 sit.  Reads and their wait in one: ahead of the builtin the compiler would wait for the copies under way.
+__device__ __forceinline__ void read_values(uint32_t at, v2u (&v)[4]) {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4\n"
+        "ds_read_b64_tr_b16 %1, %4 offset:2048\n"
+        "ds_read_b64_tr_b16 %2, %4 offset:4096\n"
+        "ds_read_b64_tr_b16 %3, %4 offset:6144\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+        : "v"(at)
+        : "memory");
 }
 
 __device__ __forceinline__ void split_fp16(const float (&x)[8], v8h& hi, v8h& lo) {
@@ -70,27 +93,30 @@ __device__ __forceinline__ void split_fp16(const float (&x)[8], v8h& hi, v8h& lo
 __device__ __forceinline__ float fast_exp(float x) { return __expf(x); }
 
 // G = query heads per KV head, S = key splits: wave (h, sp) = (wave % G, wave / G) owns query head
-// kvh*G + h and every S-th key tile starting at sp.  A round stages S consecutive key / value
-// tiles; at the end the S partial (maximum, sum, output) triples of a head are merged through LDS.
+// kvh*G + h and every S-th key tile starting at sp.  The queries, and a round of S tiles ahead of the one that is worked on, are copied
+// global -> LDS directly; at the end the S partial (maximum, sum, output) triples of a head meet through LDS, where
+// each of its waves takes a share of the head dims, merges, quantises and stores it.
+//
+// What bounds it: the way of the workgroup with the most keys, a round's wait, matrix ops and softmax one after the other.
+// us, so / with tiles that went through registers and were transposed on their way to LDS, two waits a round, queries read row by row and one
+// wave a head merging and quantising: 180 tokens, 16 heads on 4, 9.0 / 14.8; 322 tokens, 32 on 8, 13.2 / 23.1; 900 tokens, 12 on 3, 24.5 / 39.4;
+// 2048 tokens, 32 on 8, 152 / 205; the same bits.
 template <int G, int S>
-__global__ __launch_bounds__(64 * G * S) void attention_prefill_kernel(const float* __restrict__ q, int q_row_stride,
-                                                                      const __half* __restrict__ k_cache,
-                                                                      const __half* __restrict__ v_cache,
-                                                                      const int* __restrict__ pos_dev, float* __restrict__ out,
-                                                                      int out_row_stride, uint8_t* __restrict__ q_out, int n_q,
-                                                                      int M, int max_seq, float scale) {
-    constexpr int kThreads = 64 * G * S;
-    constexpr int kKPieces = S * kTile * 16;       // 16-byte pieces (key, 8 head dims) of the S staged key tiles
-    constexpr int kKItems = kKPieces / kThreads;
-    constexpr int kVPieces = S * (kTile / 2) * 16; // (pair of adjacent keys, 8 head dims) of the S value tiles
-    constexpr int kVItems = (kVPieces + kThreads - 1) / kThreads;
-    static_assert(kKItems * kThreads == kKPieces, "key tile pieces must divide over the workgroup");
+__global__ __launch_bounds__(64 * G * S, G * S / 4) void attention_prefill_kernel(const float* __restrict__ q, int q_row_stride,
+                                                                                 const __half* __restrict__ k_cache,
+                                                                                 const __half* __restrict__ v_cache,
+                                                                                 const int* __restrict__ pos_dev, float* __restrict__ out,
+                                                                                 int out_row_stride, uint8_t* __restrict__ q_out, int n_q,
+                                                                                 int M, int max_seq, float scale) {
+    constexpr int kBuf = S * kTileBytes;     // a round's tiles
+    constexpr int kCopies = kTileBytes / 1024;  // of a tile, dealt to the G waves
+    constexpr int kOwn = 4 / S;              // 32-blocks of head dims that a wave finishes
     extern __shared__ __align__(16) uint8_t lds[];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 31, kh = lane >> 5;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 31, kh = lane >> 5;
     const int h = wave % G, sp = wave / G;
     // gridDim.z workgroups share a KV head when its group of query heads is larger than G
     const int kvh = blockIdx.y, head = kvh * (n_q / (int)gridDim.y) + (int)blockIdx.z * G + h;
-    const int m0 = blockIdx.x * kTile;
+    const int m0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * kTile;  // the longest rows first
     const int pos0 = pos_dev[0];
     const int m_last = min(m0 + kTile, M) - 1;                  // last real token of the tile
     const int n_keys = min(pos0 + m_last, max_seq - 1) + 1;     // keys the tile's last token sees
@@ -98,67 +124,54 @@ __global__ __launch_bounds__(64 * G * S) void attention_prefill_kernel(const flo
     const int n_rounds = (n_tiles + S - 1) / S;
     const int m = m0 + r;                                       // this lane's query token
     const int last_key = min(pos0 + min(m, m_last), n_keys - 1);  // it sees keys 0..last_key
-    const uint8_t* k_lds = lds + sp * kTileLdsBytes;            // this wave's tile of the round
-    const uint8_t* v_lds = k_lds + kTile * kKStride;
+    const int first_last_key = min(pos0 + m0, n_keys - 1);      // what every token of the tile sees
 
+    const uint8_t* k_base = reinterpret_cast<const uint8_t*>(k_cache) + (size_t)kvh * max_seq * kRowBytes;
+    const uint8_t* v_base = reinterpret_cast<const uint8_t*>(v_cache) + (size_t)kvh * max_seq * kRowBytes;
+    auto copy_tile = [&](int round) {  // this wave's share of its tile; rows past the context repeat the last one (they are masked)
+        const int tile = round * S + sp;
+        if (tile >= n_tiles) return;
+        uint8_t* to = lds + (round & 1) * kBuf + sp * kTileBytes;
+#pragma unroll
+        for (int i = 0; i < (kCopies + G - 1) / G; i++) {
+            const int n = i * G + h, key = 4 * (n & 7) + (lane >> 4), place = lane & 15;
+            const size_t row = (size_t)min(tile * kTile + key, n_keys - 1) * kRowBytes;
+            if (n < 8)
+                copy16(k_base + row + 16 * (place ^ key_swap(key)), to + n * 1024);
+            else
+                copy16(v_base + row + 16 * (place ^ value_swap(key)), to + n * 1024);
+        }
+    };
+    copy_tile(0);
+    // The queries pass where round 1 will be: chunk c of row i at place c ^ i.
+    uint8_t* const q_lds = lds + kBuf + h * kQueryBytes;
+#pragma unroll
+    for (int i = 0; i < 16 / S; i++) {
+        const int n = i * S + sp, row = 2 * n + kh;
+        const float* src = q + (size_t)min(m0 + row, M - 1) * q_row_stride + (size_t)head * kHeadDim;
+        copy16(src + 4 * (r ^ row), q_lds + n * 1024);
+    }
+    wait_and_meet();
     // this lane's query row as B operands: step d covers head dims 16d + 8kh .. + 7
     v8h q_hi[8], q_lo[8];
-    {
-        const float* row = q + (size_t)min(m, M - 1) * q_row_stride + (size_t)head * kHeadDim + 8 * kh;
 #pragma unroll
-        for (int d = 0; d < 8; d++) {
-            const float4 a = *reinterpret_cast<const float4*>(row + 16 * d);
-            const float4 b = *reinterpret_cast<const float4*>(row + 16 * d + 4);
-            const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-            split_fp16(x, q_hi[d], q_lo[d]);
-        }
+    for (int d = 0; d < 8; d++) {
+        const v4f a = *reinterpret_cast<const v4f*>(q_lds + r * 512 + 16 * ((4 * d + 2 * kh) ^ r));
+        const v4f b = *reinterpret_cast<const v4f*>(q_lds + r * 512 + 16 * ((4 * d + 2 * kh + 1) ^ r));
+        const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        split_fp16(x, q_hi[d], q_lo[d]);
     }
 
-    const __half* k_base = k_cache + (size_t)kvh * max_seq * kHeadDim;
-    const __half* v_base = v_cache + (size_t)kvh * max_seq * kHeadDim;
-    uint4 k_reg[kKItems], v_reg[kVItems][2];
-    auto fetch = [&](int round) {  // rows past the context repeat the last one (they are masked)
-        const int key0 = round * S * kTile;
+    // where this lane's transposing reads of 32-block b of the head dims start in a tile of values
+    uint32_t value_at[4];
+    {
+        const int i = lane & 15, key = 4 * kh + (i >> 2);
 #pragma unroll
-        for (int it = 0; it < kKItems; it++) {
-            const int piece = tid + it * kThreads, key = piece >> 4, sub = piece & 15;  // key: 0 .. 32 S - 1
-            k_reg[it] = *reinterpret_cast<const uint4*>(k_base + (size_t)min(key0 + key, n_keys - 1) * kHeadDim + 8 * sub);
+        for (int b = 0; b < 4; b++) {
+            const int c = 4 * b + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+            value_at[b] = kKeyBytes + key * kRowBytes + 16 * (c ^ value_swap(key)) + 8 * (i & 1);
         }
-#pragma unroll
-        for (int it = 0; it < kVItems; it++) {
-            const int piece = tid + it * kThreads;
-            if (piece < kVPieces) {
-                const int tl = piece >> 8, sub = (piece >> 4) & 15, pair = piece & 15;
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    v_reg[it][j] = *reinterpret_cast<const uint4*>(
-                        v_base + (size_t)min(key0 + tl * kTile + 2 * pair + j, n_keys - 1) * kHeadDim + 8 * sub);
-            }
-        }
-    };
-    auto stage = [&]() {
-#pragma unroll
-        for (int it = 0; it < kKItems; it++) {
-            const int piece = tid + it * kThreads, tl = piece >> 9, key = (piece >> 4) & 31, sub = piece & 15;
-            *reinterpret_cast<uint4*>(lds + tl * kTileLdsBytes + key * kKStride + 16 * sub) = k_reg[it];
-        }
-#pragma unroll
-        for (int it = 0; it < kVItems; it++) {
-            const int piece = tid + it * kThreads;
-            if (piece < kVPieces) {  // keys 2 pair and 2 pair + 1 sit next to each other along the contraction index
-                const int tl = piece >> 8, sub = (piece >> 4) & 15, pair = piece & 15;
-                const uint32_t a[4] = {v_reg[it][0].x, v_reg[it][0].y, v_reg[it][0].z, v_reg[it][0].w};
-                const uint32_t b[4] = {v_reg[it][1].x, v_reg[it][1].y, v_reg[it][1].z, v_reg[it][1].w};
-                uint8_t* col = lds + tl * kTileLdsBytes + kTile * kKStride + (8 * sub) * kVStride + 2 * value_slot(2 * pair);
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const uint32_t lo = (a[e >> 1] >> (16 * (e & 1))) & 0xffffu, hi = (b[e >> 1] >> (16 * (e & 1))) & 0xffffu;
-                    *reinterpret_cast<uint32_t*>(col + e * kVStride) = lo | (hi << 16);
-                }
-            }
-        }
-    };
-
+    }
     v16f o_acc[4];
 #pragma unroll
     for (int b = 0; b < 4; b++)
@@ -166,33 +179,37 @@ __global__ __launch_bounds__(64 * G * S) void attention_prefill_kernel(const flo
         for (int v = 0; v < 16; v++) o_acc[b][v] = 0.f;
     float m_run = kLowest, l_run = 0.f;
 
-    fetch(0);
     for (int round = 0; round < n_rounds; round++) {  // uniform over the workgroup
-        __syncthreads();  // every wave is done with the previous round's tiles
-        stage();
-        __syncthreads();
-        if (round + 1 < n_rounds) fetch(round + 1);
+        wait_and_meet();  // the round's tiles are in LDS, and nobody still reads what the next ones replace
+        copy_tile(round + 1);
         const int tile = round * S + sp;
-        if (tile >= n_tiles) continue;  // uniform over the wave; the barriers are outside
+        if (tile >= n_tiles) continue;  // uniform over the wave
+        const uint8_t* k_lds = lds + (round & 1) * kBuf + sp * kTileBytes;
 
         v16f s_acc;
 #pragma unroll
         for (int v = 0; v < 16; v++) s_acc[v] = 0.f;
 #pragma unroll
         for (int d = 0; d < 8; d++) {
-            const v8h a = *reinterpret_cast<const v8h*>(k_lds + r * kKStride + 32 * d + 16 * kh);
+            const v8h a = *reinterpret_cast<const v8h*>(k_lds + r * kRowBytes + 16 * ((2 * d + kh) ^ key_swap(r)));
             s_acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, q_hi[d], s_acc, 0, 0, 0);
             s_acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, q_lo[d], s_acc, 0, 0, 0);
         }
 
         float sc[16];
         float t_max = kLowest;
+        if (tile * kTile + kTile - 1 <= first_last_key) {
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int key = tile * kTile + 8 * (v >> 2) + 4 * kh + (v & 3);
-            sc[v] = key <= last_key ? s_acc[v] * scale : kLowest;
-            t_max = fmaxf(t_max, sc[v]);
+            for (int v = 0; v < 16; v++) sc[v] = s_acc[v] * scale;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                const int key = tile * kTile + 8 * (v >> 2) + 4 * kh + (v & 3);
+                sc[v] = key <= last_key ? s_acc[v] * scale : kLowest;
+            }
         }
+#pragma unroll
+        for (int v = 0; v < 16; v++) t_max = fmaxf(t_max, sc[v]);
         t_max = fmaxf(t_max, __shfl_xor(t_max, 32, 64));
         const float m_new = fmaxf(m_run, t_max);
         // a token that sees none of this tile's keys and none before it (only possible in a wave
@@ -207,11 +224,13 @@ __global__ __launch_bounds__(64 * G * S) void attention_prefill_kernel(const flo
         }
         p_sum += __shfl_xor(p_sum, 32, 64);
         l_run = l_run * alpha + p_sum;
+        if (__any(m_new > m_run)) {
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) o_acc[b][v] *= alpha;
+        }
         m_run = m_new;
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) o_acc[b][v] *= alpha;
 
         v8h p_hi[2], p_lo[2];
 #pragma unroll
@@ -220,13 +239,14 @@ __global__ __launch_bounds__(64 * G * S) void attention_prefill_kernel(const flo
                                 p[8 * c + 4], p[8 * c + 5], p[8 * c + 6], p[8 * c + 7]};
             split_fp16(x, p_hi[c], p_lo[c]);
         }
+        const uint32_t v_at = (uint32_t)(uintptr_t)(lds_ptr_t)k_lds;
 #pragma unroll
         for (int b = 0; b < 4; b++) {
+            v2u part[4];
+            read_values(v_at + value_at[b], part);
 #pragma unroll
             for (int c = 0; c < 2; c++) {
-                const uint8_t* src = v_lds + (32 * b + r) * kVStride + (2 * c + kh) * 16;  // 8-byte aligned
-                const uint2 a0 = *reinterpret_cast<const uint2*>(src), a1 = *reinterpret_cast<const uint2*>(src + 8);
-                const uint4 a4 = make_uint4(a0.x, a0.y, a1.x, a1.y);
+                const uint4 a4 = make_uint4(part[2 * c][0], part[2 * c][1], part[2 * c + 1][0], part[2 * c + 1][1]);
                 const v8h a = __builtin_bit_cast(v8h, a4);
                 o_acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, p_hi[c], o_acc[b], 0, 0, 0);
                 o_acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, p_lo[c], o_acc[b], 0, 0, 0);
@@ -235,80 +255,70 @@ __global__ __launch_bounds__(64 * G * S) void attention_prefill_kernel(const flo
     }
 
     // ---- merge the S partial results of each head ------------------------------------------------
-    // LDS now holds: the outputs being handed over (one 16 KiB slot per sending wave), then the
-    // running maxima and sums of all waves.
-    float* stat = reinterpret_cast<float*>(lds + kMergeSlotBytes * G * (S / 2 > 0 ? S / 2 : 1));
-    __syncthreads();  // the staged tiles are dead
-    if (kh == 0) {
-        stat[(sp * G + h) * 32 + r] = m_run;
-        stat[(S * G + sp * G + h) * 32 + r] = l_run;
-    }
-    __syncthreads();
-    float m_fin = kLowest;
-#pragma unroll
-    for (int j = 0; j < S; j++) m_fin = fmaxf(m_fin, stat[(j * G + h) * 32 + r]);  // finite: tile 0 holds key 0
-    float l_tot = 0.f;
-#pragma unroll
-    for (int j = 0; j < S; j++)
-        l_tot += stat[(S * G + j * G + h) * 32 + r] * fast_exp(stat[(j * G + h) * 32 + r] - m_fin);
-    const float f = fast_exp(m_run - m_fin);  // 0 for a wave that had no visible key
-#pragma unroll
-    for (int b = 0; b < 4; b++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) o_acc[b][v] *= f;
-#pragma unroll
-    for (int stride = S / 2; stride >= 1; stride >>= 1) {  // sp in [stride, 2 stride) hands over to sp - stride
-        float4* slot = reinterpret_cast<float4*>(lds + (size_t)((sp % stride) * G + h) * kMergeSlotBytes);
-        if (sp >= stride && sp < 2 * stride) {
-#pragma unroll
-            for (int b = 0; b < 4; b++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-                    slot[(4 * b + g) * 64 + lane] =
-                        make_float4(o_acc[b][4 * g], o_acc[b][4 * g + 1], o_acc[b][4 * g + 2], o_acc[b][4 * g + 3]);
+    // LDS now holds 32-block b of wave w's scaled output at (w 4 + b) kBlockBytes, then the running maxima and sums of all waves.
+    float l_tot = l_run;
+    if constexpr (S > 1) {
+        float* stat = reinterpret_cast<float*>(lds + 4 * G * S * kBlockBytes);
+        wait_and_meet();  // the staged tiles are dead
+        if (kh == 0) {
+            stat[(sp * G + h) * 32 + r] = m_run;
+            stat[(S * G + sp * G + h) * 32 + r] = l_run;
         }
-        __syncthreads();
-        if (sp < stride) {
+        wait_and_meet();
+        float m_fin = kLowest;
 #pragma unroll
-            for (int b = 0; b < 4; b++)
+        for (int j = 0; j < S; j++) m_fin = fmaxf(m_fin, stat[(j * G + h) * 32 + r]);  // finite: tile 0 holds key 0
+        l_tot = 0.f;
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const float4 t = slot[(4 * b + g) * 64 + lane];
-                    o_acc[b][4 * g] += t.x;
-                    o_acc[b][4 * g + 1] += t.y;
-                    o_acc[b][4 * g + 2] += t.z;
-                    o_acc[b][4 * g + 3] += t.w;
-                }
+        for (int j = 0; j < S; j++)
+            l_tot += stat[(S * G + j * G + h) * 32 + r] * fast_exp(stat[(j * G + h) * 32 + r] - m_fin);
+        const float f = fast_exp(m_run - m_fin);  // 0 for a wave that had no visible key
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            v4f* slot = reinterpret_cast<v4f*>(lds + ((sp * G + h) * 4 + b) * kBlockBytes);
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                slot[g * 64 + lane] = v4f{o_acc[b][4 * g] * f, o_acc[b][4 * g + 1] * f, o_acc[b][4 * g + 2] * f, o_acc[b][4 * g + 3] * f};
         }
-        __syncthreads();
+        wait_and_meet();
     }
-
-    if (sp != 0) return;  // whole waves
     const float inv = 1.0f / l_tot;
-    if (q_out == nullptr) {
-        if (m <= m_last) {
-            float* dst = out + (size_t)m * out_row_stride + (size_t)head * kHeadDim + 4 * kh;
-#pragma unroll
-            for (int b = 0; b < 4; b++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-                    *reinterpret_cast<float4*>(dst + 32 * b + 8 * g) =
-                        make_float4(o_acc[b][4 * g] * inv, o_acc[b][4 * g + 1] * inv, o_acc[b][4 * g + 2] * inv,
-                                    o_acc[b][4 * g + 3] * inv);
-        }
-        return;
-    }
     // 32-block b of this head: values 8g + 4kh + i (g, i = 0..3) here, the rest in lane ^ 32.  All lanes
     // take part in the exchanges; rows past the last token store nothing.
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
+    for (int own = 0; own < kOwn; own++) {
+        const int b = sp * kOwn + own;
         float val[16];
+        if constexpr (S > 1) {
+            auto slot = [&](int j) { return reinterpret_cast<const v4f*>(lds + ((j * G + h) * 4 + b) * kBlockBytes); };
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                v4f sum = slot(0)[g * 64 + lane];
+                if constexpr (S == 2) {
+                    sum += slot(1)[g * 64 + lane];
+                } else {
+                    static_assert(S == 4, "the order of the sums");
+                    sum = (sum + slot(2)[g * 64 + lane]) + (slot(1)[g * 64 + lane] + slot(3)[g * 64 + lane]);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) val[4 * g + i] = sum[i] * inv;
+            }
+        } else {
+#pragma unroll
+            for (int v = 0; v < 16; v++) val[v] = o_acc[own][v] * inv;
+        }
+        if (q_out == nullptr) {
+            if (m <= m_last) {
+                float* dst = out + (size_t)m * out_row_stride + (size_t)head * kHeadDim + 4 * kh;
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *reinterpret_cast<float4*>(dst + 32 * b + 8 * g) = make_float4(val[4 * g], val[4 * g + 1], val[4 * g + 2], val[4 * g + 3]);
+            }
+            continue;
+        }
         float amax = 0.f;
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            val[v] = o_acc[b][v] * inv;
-            amax = fmaxf(amax, fabsf(val[v]));
-        }
+        for (int v = 0; v < 16; v++) amax = fmaxf(amax, fabsf(val[v]));
         amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
         const float d = amax / 127.f;                           // the quantiser's arithmetic, step by step
         const float id = (amax != 0.0f) ? 127.f / amax : 0.0f;
@@ -339,11 +349,12 @@ __global__ __launch_bounds__(64 * G * S) void attention_prefill_kernel(const flo
     }
 }
 
+// Two rounds of tiles; one and the queries; or the waves' outputs and statistics.
 template <int G, int S>
 constexpr size_t prefill_lds_bytes() {
-    constexpr size_t staging = (size_t)S * kTileLdsBytes;
-    constexpr size_t merge = (size_t)kMergeSlotBytes * G * (S / 2 > 0 ? S / 2 : 1) + (size_t)2 * S * G * 32 * sizeof(float);
-    return staging > merge ? staging : merge;
+    constexpr size_t round = (size_t)S * kTileBytes, rest = (size_t)G * kQueryBytes > round ? (size_t)G * kQueryBytes : round;
+    constexpr size_t merge = S > 1 ? (size_t)4 * G * S * kBlockBytes + (size_t)2 * S * G * 32 * sizeof(float) : 0;
+    return round + rest > merge ? round + rest : merge;
 }
 
 template <int G, int S>
@@ -377,16 +388,15 @@ hipError_t launch_attention_prefill(const float* q, int q_row_stride, const void
     uint8_t* qo = static_cast<uint8_t*>(q_out);
     const __half* kc = static_cast<const __half*>(k_cache);
     const __half* vc = static_cast<const __half*>(v_cache);
-    // G heads x S key splits per workgroup, at most 8 waves: a wave needs about 220 registers per
-    // lane (64 for its query, 64 for its output), which rules out four waves per SIMD.  The whole
-    // group in one workgroup shares each staged tile among the most heads; with few query tiles that
-    // leaves most of the chip idle (322 tokens, 8 KV heads: 88 workgroups), so the group is then cut
-    // into workgroups of fewer heads and more key splits until there are at least 128 (322 tokens: 23.6 -> 21.2 us
-    // with two heads per workgroup; one head per workgroup: 32.6 us, and 10.2 against 11.3 us at 64 tokens).
+    // G heads x S key splits per workgroup, at most 8 waves: a wave needs about 200 registers per lane (64 for its query, 64 for
+    // its output).  One head and four splits where every workgroup gets a CU; two heads, whose tiles two waves share, while the longest
+    // workgroup counts; the whole group where there are many rounds.  us with 1 / 2 / 4 heads: 180 tokens, 16 heads on 4, 9.0 / 10.0 / 12.4;
+    // 322 tokens, 8 on 2 10.8 / 11.9 / 16.6, 32 on 8 (352, 176, 88 workgroups) 18.5 / 13.2 / 17.4; 900 tokens, 12 on 3 31.9 / 24.5 / 35.8;
+    // 2048 tokens, 8 on 2 76 / 45 / 72, 32 on 8 252 / 157 / 152; 3000 tokens - / 244 / 234.
     // A81W41_ATTENTION_HEADS=<G> fixes the heads per workgroup (measurement aid, tuning builds only).
     static const int env_g = tuning_env_int("A81W41_ATTENTION_HEADS");
-    int g = group;
-    while (g > 1 && tiles * n_kv * (group / g) < 128) g >>= 1;
+    int g = 1;
+    while (g < group && (long long)tiles * n_kv * (group / g) > (g == 1 ? 256 : 1024)) g <<= 1;
     if (env_g > 0 && env_g <= group && group % env_g == 0) g = env_g;
     if (heads_per_workgroup > 0) {
         if (heads_per_workgroup > group || group % heads_per_workgroup) return hipErrorInvalidValue;

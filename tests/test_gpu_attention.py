@@ -86,6 +86,22 @@ def test_every_split_of_a_head_group(pkg, synth, torch, M, pos, n_q, n_kv, max_s
         assert row_err(got, want) < TOL, variant
 
 
+@pytest.mark.parametrize("M,pos", [(31, 0), (33, 64), (64, 33), (65, 127), (97, 96)])
+@pytest.mark.parametrize("n_q,n_kv", [(8, 1), (2, 2)])
+def test_edges_of_tiles_and_rounds(pkg, synth, torch, n_q, n_kv, M, pos):
+    """One query more and less than a tile, contexts that end in the middle of a round of the key splits, for every number of
+    heads a workgroup takes; keys behind the context hold what no token may see."""
+    scale = 1.0 / np.sqrt(128.0)
+    q, k, v = make(synth, M, pos, n_q, n_kv, M + pos + 40, 900 + M)
+    want = reference(q, k[:, :M + pos].astype(np.float32), v[:, :M + pos].astype(np.float32), pos, n_q, n_kv, scale)
+    k[:, M + pos:], v[:, M + pos:] = 60000.0, np.nan
+    for variant in (2, 3, 4, 5, 6):
+        if variant > 2 and (1 << (variant - 3)) > n_q // n_kv:
+            continue
+        got = run(pkg, torch, q, k, v, pos, n_q, n_kv, scale, variant, row_pad=4)
+        assert row_err(got, want) < TOL, variant
+
+
 def test_sharp_and_flat_rows(pkg, synth, torch):
     """Scores far apart (one key dominates) and all equal (uniform weights): the running-maximum
     bookkeeping across tiles and the masked entries of partial tiles."""
