@@ -3,7 +3,7 @@
 //   expanded  a key is [own part | part shared by all heads], values come transposed ([value column][key]).
 //
 // A workgroup of KG x QW waves takes 32 QW query rows.  A wave owns 32 of them; KG waves share them, each with every KG-th tile of 64
-// keys, and meet at the end: a workgroup of two groups keeps two waves on every SIMD while its rows, and with them the
+// keys (or 32), and meet at the end: a workgroup of several groups keeps two waves on every SIMD while its rows, and with them the
 // rows past the diagonal, stay few.  Scores are formed transposed, S^T = K Q^T (v_mfma_f32_32x32x16_bf16 with the keys
 // as rows), so that a lane holds scores of query l % 32 only.  Row r of a 32-key product is key r with bits 2 and 3
 // exchanged: register v of lane half h is then key 16 (v / 8) + 8 h + v % 8, and eight registers are, as they stand, the
@@ -13,13 +13,15 @@
 //
 // A tile is copied global -> LDS by direct 16-byte loads, the next one while this one is worked on; in the rows form only while its
 // scores and weights are formed, as the compiler waits for every copy under way ahead of the first transposing read of values.
-// Chunk c of key k sits at place c ^ k % 16, or, where rows are an odd number of 128 bytes, c ^ k / 2 % 8; chunk c of a transposed
-// value column d at c ^ d / 2 % 8: sixteen rows read at one chunk column cover the 256 bytes of all banks.
+// Chunk c of key k sits at place c ^ (4 (k % 4) + k / 4 % 4), or, where rows are an odd number of 128 bytes, c ^ k / 2 % 8; chunk c of a
+// transposed value column d at c ^ d / 2 % 8, of half a row at c ^ d / 4 % 4: sixteen rows read at one chunk column, and four rows that a transposing read
+// takes four chunks of, cover the 256 bytes of all banks.  With c ^ k % 16 those four rows met in eight places, and more than half of
+// the cycles of LDS were conflicts: 2048 rows in chunks of 1024, 16 heads on 4 of 128 + 128 columns 28.8 us, so 26.7.
 //
 // What bounds it: matrix ops and softmax of a SIMD's two waves, one after the other; then LDS, which gives an operand of 1 KiB
-// for every matrix op.  4095 rows of 16 heads, 192 + 128 columns: 120 us = 712 TFLOP/s, against 537 us with 16 x 16 matrix ops,
-// heads' rows dealt out one head after the other and one workgroup of four waves on a CU; 2048 rows in chunks of 1024, 16 heads
-// on 4 of 128 + 128 columns: 31 us against 71 us.
+// for every matrix op; of a short prompt's workgroup its start and end.  So queries, the row's gate and the first tile are one trip, and rows are
+// stored sixteen bytes a lane.  4095 rows of 16 heads, 192 + 128 columns: 114 us = 750 TFLOP/s, 118 with queries awaited ahead of
+// the first tile's copies, the gate behind the last and stores of eight bytes.
 #include "dense_common.h"
 
 namespace a81w41 {
@@ -30,11 +32,14 @@ typedef __attribute__((ext_vector_type(8))) short s16x8;
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLowest = -1e30f;
-constexpr int kTile = 64;      // keys
 
 template <int DK>
 __device__ __forceinline__ int place_of_key(int k) {
-    return DK % 128 ? (k >> 1) & 7 : k & 15;
+    return DK % 128 ? (k >> 1) & 7 : (k & 3) << 2 | (k >> 2 & 3);
+}
+template <int CV>  // a row of CV chunks
+__device__ __forceinline__ int place_of_value(int d) {
+    return CV == 8 ? (d >> 1) & 7 : (d >> 2) & 3;
 }
 // the value of the lane 32 away
 __device__ __forceinline__ float other_half(float v) {
@@ -43,13 +48,14 @@ __device__ __forceinline__ float other_half(float v) {
 }
 
 // DK: columns of a tile row; the scores take those from KEY0 on (rows form: the key part, 0 otherwise).  DV: value columns.
-template <int DK, int DV, int KEY0, int KG, int QW, bool EXPANDED>
+// kTile: keys of a tile, 64 or 32.
+template <int DK, int DV, int KEY0, int KG, int QW, int kTile, bool EXPANDED>
 __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kernel(AttendArgs<bf16> a) {
-    constexpr int CK = DK / 8, KS = (DK - KEY0) / 16, VF = DV / 32, kRows = 32 * QW;
+    constexpr int CK = DK / 8, CV = kTile / 8, KT = kTile / 32, KS = (DK - KEY0) / 16, VF = DV / 32, kRows = 32 * QW;
     constexpr int kKeyBytes = kTile * DK * 2, kBuf = kKeyBytes + (EXPANDED ? DV * kTile * 2 : 0);
-    constexpr int NK = kTile * CK / 64 / QW, NV = EXPANDED ? DV * 8 / 64 / QW : 0;  // copies of a wave and tile
-    static_assert(DK % 64 == 0 && DV % 32 == 0 && KEY0 % 64 == 0 && kTile * CK % (64 * QW) == 0 && DV * 8 % (64 * QW) == 0, "tile sizes");
-    static_assert(KG == 1 || 64 * 4 * (16 * VF + 2) * QW <= 2 * KG * kBuf, "the groups meet in LDS");
+    constexpr int NK = kTile * CK / 64 / QW, NV = EXPANDED ? DV * CV / 64 / QW : 0;  // copies of a wave and tile
+    static_assert(DK % 64 == 0 && DV % 32 == 0 && KEY0 % 64 == 0 && kTile * CK % (64 * QW) == 0 && DV * CV % (64 * QW) == 0, "tile sizes");
+    static_assert((KG - 1) * 64 * 4 * (16 * VF + 2) * QW <= 2 * KG * kBuf, "the groups meet in LDS");
     __shared__ __attribute__((aligned(128))) uint8_t lds[2 * KG * kBuf];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l31 = lane & 31, half = lane >> 5;
     const int qw = wave % QW, kg = wave / QW;
@@ -98,7 +104,7 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
     if constexpr (EXPANDED) {
 #pragma unroll
         for (int n = 0; n < NV; n++) {
-            const int q = (n * QW + qw) * 64 + lane, r = q >> 3, c = (q & 7) ^ ((r >> 1) & 7);
+            const int q = (n * QW + qw) * 64 + lane, r = q / CV, c = (q % CV) ^ place_of_value<CV>(r);
             value_src[n] = a.v_t + ((size_t)z * a.dv + min(r, a.dv - 1)) * a.ld_v + key_begin + kg * kTile + c * 8;
         }
     }
@@ -131,17 +137,21 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
     const int lowest_limit = last_key(min(wave_row0, a.rows - 1)), highest_limit = last_key(min(wave_row0 + 31, a.rows - 1));
     const int highest_first = chunk_begin(highest_limit);
     const float scale = fabsf(a.scale) * kLog2e;
+    // They, the row's gate and the first tile are one trip.
     bf16x8 qf[KS];
+    const float gate = a.head_gate ? a.head_gate[(size_t)my_row * a.ld_gate + z] : 0.f;
     {
         const bf16* src = a.q + z * a.q_head + (size_t)my_token * a.q_token + (my_row - my_token * a.rows_per_token) * a.ld_q;
         const unsigned sign = a.scale < 0.f ? 0x80008000u : 0u;
+        uint4 u[KS];
+#pragma unroll
+        for (int k = 0; k < KS; k++) u[k] = *reinterpret_cast<const uint4*>(src + min(2 * k + half, all_chunks - 1) * 8);
+        if (kg < n_tiles) copy_tile(kg, 0);
 #pragma unroll
         for (int k = 0; k < KS; k++) {
-            const int c = 2 * k + half;
-            uint4 u = make_uint4(0, 0, 0, 0);
-            if (c < all_chunks) u = *reinterpret_cast<const uint4*>(src + c * 8);
-            u = make_uint4(u.x ^ sign, u.y ^ sign, u.z ^ sign, u.w ^ sign);
-            qf[k] = *reinterpret_cast<const bf16x8*>(&u);
+            const unsigned keep = 2 * k + half < all_chunks ? ~0u : 0u;
+            u[k] = make_uint4((u[k].x ^ sign) & keep, (u[k].y ^ sign) & keep, (u[k].z ^ sign) & keep, (u[k].w ^ sign) & keep);
+            qf[k] = *reinterpret_cast<const bf16x8*>(&u[k]);
         }
     }
     f32x16 acc[VF];
@@ -168,7 +178,6 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
             }
     }
 
-    if (kg < n_tiles) copy_tile(kg, 0);
     for (int turn = 0; turn < n_turns; turn++) {
         const int tile = turn * KG + kg, key0 = key_begin + tile * kTile;
         // the tile is in LDS, everybody's copies of it; and nobody still reads the other buffer
@@ -180,9 +189,9 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
         if (tile >= n_tiles || key0 > highest_limit) continue;
         const uint8_t* kb = my_lds + (turn & 1) * kBuf;
         const uint8_t* vb = kb + kKeyBytes;
-        f32x16 sc[2];
+        f32x16 sc[KT];
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < KT; t++) {
 #pragma unroll
             for (int v = 0; v < 16; v++) sc[t][v] = 0.f;
 #pragma unroll
@@ -193,7 +202,7 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
         }
         if (key0 + kTile - 1 > lowest_limit || key0 < highest_first || key0 + kTile > key_end) {
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+            for (int t = 0; t < KT; t++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
                     const int key = key0 + 32 * t + 16 * (v >> 3) + 8 * half + (v & 7);
@@ -202,7 +211,7 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
         }
         float top = sc[0][0];
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int t = 0; t < KT; t++)
 #pragma unroll
             for (int v = 0; v < 16; v++) top = fmaxf(top, sc[t][v]);
         top = fmaxf(top, other_half(top)) * scale;
@@ -216,13 +225,13 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
         auto weights_sum = [&]() {
             float add[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+            for (int t = 0; t < KT; t++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) add[v & 3] += sc[t][v];
             return (add[0] + add[1]) + (add[2] + add[3]);
         };
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int t = 0; t < KT; t++)
 #pragma unroll
             for (int v = 0; v < 16; v++) sc[t][v] = __builtin_amdgcn_exp2f(fmaf(sc[t][v], scale, -mx));
         float add = weights_sum();
@@ -231,24 +240,24 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
         // in the exponential's instruction is free but moves the last bits of sums).
         if (__builtin_expect(__any(add != add), 0)) {
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+            for (int t = 0; t < KT; t++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) sc[t][v] = fmaxf(sc[t][v], 0.f);
             add = weights_sum();
         }
         sum += add;
-        bf16x8 pf[4];
+        bf16x8 pf[2 * KT];
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int t = 0; t < KT; t++)
 #pragma unroll
             for (int v = 0; v < 16; v++) pf[2 * t + (v >> 3)][v & 7] = (bf16)sc[t][v];
 #pragma unroll
-        for (int u = 0; u < 4; u++)
+        for (int u = 0; u < 2 * KT; u++)
 #pragma unroll
             for (int f = 0; f < VF; f++) {
                 bf16x8 vf;
                 if constexpr (EXPANDED) {
-                    vf = *reinterpret_cast<const bf16x8*>(vb + (f * 32 + l31) * (kTile * 2) + (((2 * u + half) ^ ((l31 >> 1) & 7)) << 4));
+                    vf = *reinterpret_cast<const bf16x8*>(vb + (f * 32 + l31) * (kTile * 2) + (((2 * u + half) ^ place_of_value<CV>(l31)) << 4));
                 } else {
                     const uint8_t* at = kb + (f >> 2) * 256 + u * 16 * (DK * 2);
                     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(at + value_at[f & 3][0]));
@@ -261,31 +270,43 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
     }
 
     sum += other_half(sum);
-    if constexpr (KG > 1) {  // the second group hands its share of the keys over; value column of register (f, v) at (f 16 + v)
-        static_assert(KG == 2, "two groups meet");
-        float* part = reinterpret_cast<float*>(lds) + (size_t)qw * (16 * VF + 2) * 64 + lane;
+    if constexpr (KG > 1) {  // the other groups hand their shares of the keys over, the first adds them one by one; registers (f, v .. v + 3) at 4 f + v / 4
+        constexpr int kPart = (16 * VF + 2) * 64, kStats = 16 * VF * 64;
+        float* part = reinterpret_cast<float*>(lds) + (size_t)qw * kPart;
         __syncthreads();
-        if (kg == 1) {
-            part[0] = mx, part[64] = sum;
+        if (kg > 0) {
+            float* own = part + (kg - 1) * QW * kPart;
+            own[kStats + lane] = mx, own[kStats + 64 + lane] = sum;
 #pragma unroll
             for (int f = 0; f < VF; f++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) part[(2 + f * 16 + v) * 64] = acc[f][v];
+                for (int v = 0; v < 16; v += 4)
+                    reinterpret_cast<f32x4*>(own)[(4 * f + v / 4) * 64 + lane] = f32x4{acc[f][v], acc[f][v + 1], acc[f][v + 2], acc[f][v + 3]};
         }
         __syncthreads();
-        if (kg == 1) return;
-        const float other = part[0], m = fmaxf(mx, other), mine = __builtin_amdgcn_exp2f(mx - m), theirs = __builtin_amdgcn_exp2f(other - m);
-        sum = sum * mine + part[64] * theirs;
-        mx = m;
+        if (kg > 0) return;
 #pragma unroll
-        for (int f = 0; f < VF; f++)
+        for (int k = 1; k < KG; k++, part += QW * kPart) {
+            const float other = part[kStats + lane], m = fmaxf(mx, other);
+            const float mine = __builtin_amdgcn_exp2f(mx - m), theirs = __builtin_amdgcn_exp2f(other - m);
+            sum = sum * mine + part[kStats + 64 + lane] * theirs;
+            mx = m;
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[f][v] = acc[f][v] * mine + part[(2 + f * 16 + v) * 64] * theirs;
+            for (int f = 0; f < VF; f++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    if (v % 4 == 0) {
+                        const f32x4 add = reinterpret_cast<const f32x4*>(part)[(4 * f + v / 4) * 64 + lane];
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[f][v + i] = acc[f][v + i] * mine + add[i] * theirs;
+                    }
+                }
+        }
     }
     // register (f, v) holds value column 32 f + 8 (v / 4) + 4 half + v % 4 of query l % 32
-    const int r = wave_row0 + l31;
-    if (r >= a.rows) return;
     if (a.splits > 1) {
+        const int r = wave_row0 + l31;
+        if (r >= a.rows) return;
         const size_t at = ((size_t)blockIdx.z * gridDim.x + z) * a.rows + r;
         if (half == 0) {
             a.part_stats[2 * at] = mx;
@@ -302,30 +323,40 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
         return;
     }
     float inv = 1.0f / sum;
-    if (a.head_gate) inv *= sigmoid(a.head_gate[(size_t)r * a.ld_gate + z]);
-    bf16* dst = a.out + z * a.out_head + (size_t)my_token * a.out_token + (r - my_token * a.rows_per_token) * a.ld_out;
-    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-    const bool whole = ((a.dv | a.ld_out | a.out_token) & 3) == 0 && (a.out_head & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 7) == 0;
+    if (a.head_gate) inv *= sigmoid(gate);
+    bf16* dst = a.out + z * a.out_head + (size_t)my_token * a.out_token + (my_row - my_token * a.rows_per_token) * a.ld_out;
+    const bool real = wave_row0 + l31 < a.rows;
+    // Eight neighbouring columns a lane: of two fours the halves of a row trade one.
+    const bool whole = ((a.dv | a.ld_out | a.out_token) & 7) == 0 && (a.out_head & 7) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 #pragma unroll
     for (int f = 0; f < VF; f++)
 #pragma unroll
-        for (int v = 0; v < 16; v += 4) {
-            const int d = 32 * f + 2 * v + 4 * half;
+        for (int v = 0; v < 16; v += 8) {
             if (whole) {
-                if (d < a.dv)
-                    *reinterpret_cast<bf16x4*>(dst + d) =
-                        bf16x4{(bf16)(acc[f][v] * inv), (bf16)(acc[f][v + 1] * inv), (bf16)(acc[f][v + 2] * inv), (bf16)(acc[f][v + 3] * inv)};
+                unsigned first[2], second[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const bf16x2 x = {(bf16)(acc[f][v + 2 * i] * inv), (bf16)(acc[f][v + 2 * i + 1] * inv)};
+                    const bf16x2 y = {(bf16)(acc[f][v + 4 + 2 * i] * inv), (bf16)(acc[f][v + 5 + 2 * i] * inv)};
+                    const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y), false, false);
+                    first[i] = both[0], second[i] = both[1];
+                }
+                const int d = 32 * f + 2 * v + 8 * half;
+                if (real && d < a.dv) *reinterpret_cast<lds16*>(dst + d) = lds16{first[0], first[1], second[0], second[1]};
             } else {
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (d + i < a.dv) dst[d + i] = (bf16)(acc[f][v + i] * inv);
+                for (int i = 0; i < 8; i++) {
+                    const int d = 32 * f + 2 * v + (i & 4) * 2 + 4 * half + (i & 3);
+                    if (real && d < a.dv) dst[d] = (bf16)(acc[f][v + i] * inv);
+                }
             }
         }
 }
 
-template <int DK, int DV, int KEY0, int KG, int QW, bool EXPANDED>
+template <int DK, int DV, int KEY0, int KG, int QW, int kTile, bool EXPANDED>
 hipError_t launch_kernel(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
-    hipLaunchKernelGGL((attend_prompt_kernel<DK, DV, KEY0, KG, QW, EXPANDED>), dim3(heads, (a.rows + 32 * QW - 1) / (32 * QW), a.splits),
+    hipLaunchKernelGGL((attend_prompt_kernel<DK, DV, KEY0, KG, QW, kTile, EXPANDED>), dim3(heads, (a.rows + 32 * QW - 1) / (32 * QW), a.splits),
                        dim3(64 * KG * QW), 0, s, a);
     return hipGetLastError();
 }
@@ -338,18 +369,24 @@ constexpr int kQW = kAttendPromptRows / 32;
 // 8 heads on 2, 256 + 256 columns, 330 rows 29.1 / 29.7, 2000 rows 121 / 128.
 hipError_t launch_attend_rows_prompt(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
     const int widest = a.k_own_width > a.v_width ? a.k_own_width : a.v_width;
-    if (widest <= 64) return launch_kernel<128, 64, 64, 2, kQW, false>(a, heads, s);
-    if (widest <= 128) return launch_kernel<256, 128, 128, 2, kQW, false>(a, heads, s);
-    return launch_kernel<512, 256, 256, 1, kQW, false>(a, heads, s);
+    if (widest <= 64) return launch_kernel<128, 64, 64, 2, kQW, 64, false>(a, heads, s);
+    if (widest <= 128) return launch_kernel<256, 128, 128, 2, kQW, 64, false>(a, heads, s);
+    return launch_kernel<512, 256, 256, 1, kQW, 64, false>(a, heads, s);
 }
 
 // The widest form takes all 512 registers and spills 50 of them, addresses of copies, whose reloads wait for the copies before.  It is
 // the faster one all the same (us, against 16 x 16): 8 heads, 192 + 64 and 256 columns, 330 rows 36 / 51, 2000 rows 159 / 212.
 hipError_t launch_attend_expanded(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
     const int dk = a.k_own_width + a.k_shared_width;
-    if (dk <= 128 && a.dv <= 64) return launch_kernel<128, 64, 0, 2, kQW, true>(a, heads, s);
-    if (dk <= 192 && a.dv <= 128) return launch_kernel<192, 128, 0, 2, kQW, true>(a, heads, s);
-    return launch_kernel<320, 256, 0, 1, kQW, true>(a, heads, s);
+    // Workgroups of 64 rows where there are no more than two for a CU, their keys in four groups of 32: a long prompt's last rows then have
+    // half as many turns.  us, so / with 128 rows in two groups of 64: 8 heads, 500 rows 16.5 / 20, 900 rows 22 / 28, 2048 rows 37 / 49; 16 heads, 2048
+    // rows 50 / 52; 12 heads, 180 rows 13 / 14.  More of them copy more: every workgroup has its keys to itself.
+    const bool few = (long long)heads * ((a.rows + 63) / 64) <= 512;
+    if (dk <= 128 && a.dv <= 64)
+        return few ? launch_kernel<128, 64, 0, 4, 2, 32, true>(a, heads, s) : launch_kernel<128, 64, 0, 2, kQW, 64, true>(a, heads, s);
+    if (dk <= 192 && a.dv <= 128)
+        return few ? launch_kernel<192, 128, 0, 4, 2, 32, true>(a, heads, s) : launch_kernel<192, 128, 0, 2, kQW, 64, true>(a, heads, s);
+    return launch_kernel<320, 256, 0, 1, kQW, 64, true>(a, heads, s);
 }
 
 }  // namespace a81w41

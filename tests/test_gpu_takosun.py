@@ -165,6 +165,13 @@ def test_formed_attention(pkg, M, heads, dim, rot, vdim, pos):
     close(got.float().cpu().numpy().reshape(M, heads, vdim), want, 0.02)
 
 
+@pytest.mark.parametrize("M,heads,dim,rot,vdim,pos", [
+    (64, 512, 24, 8, 40, 5),                                             # the most heads whose 64 rows have a workgroup of their own
+    (129, 171, 40, 24, 33, 3), (257, 103, 128, 64, 128, 30), (65, 257, 16, 16, 8, 0)])   # and more: 128 rows a workgroup
+def test_formed_attention_rows_of_a_workgroup(pkg, M, heads, dim, rot, vdim, pos):
+    test_formed_attention(pkg, M, heads, dim, rot, vdim, pos)
+
+
 # ---- the model -------------------------------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
