@@ -79,6 +79,19 @@ __device__ __forceinline__ ColumnPlace column_place(const LatentQueries<T>& p, i
     if (!turned && c >= p.dim) to.rows = 0;
     return to;
 }
+// whether `together` columns (2 or 4) from a multiple of them on are stored next to each other and aligned to all of them
+template <typename T>
+__device__ __forceinline__ bool columns_go_together(const HeadRows<T>& p, int n, int together) {
+    const uintptr_t elements = reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(p.cache);
+    const bool rest = n <= p.heads * p.dim + p.kv_heads * (p.dim + p.vdim) ||
+                      ((p.ld_rest & (together - 1)) == 0 && (reinterpret_cast<uintptr_t>(p.rest) & (together * sizeof(float) - 1)) == 0);
+    return rest && ((n | p.dim | p.vdim | p.ld_cache) & (together - 1)) == 0 && (elements & (together * sizeof(T) - 1)) == 0;
+}
+template <typename T>
+__device__ __forceinline__ bool columns_go_together(const LatentQueries<T>& p, int n, int together) {
+    const uintptr_t elements = reinterpret_cast<uintptr_t>(p.nope) | reinterpret_cast<uintptr_t>(p.rotated);
+    return ((n | p.dim | p.rot | p.ld_nope | p.ld_rot) & (together - 1)) == 0 && (elements & (together * sizeof(T) - 1)) == 0;
+}
 template <typename T>
 __device__ __forceinline__ int turned_pairs(const HeadRows<T>& p) {
     return p.rot_pairs;
@@ -91,6 +104,16 @@ __device__ __forceinline__ int turned_pairs(const LatentQueries<T>& p) {
 // One direct copy global -> LDS of 16 bytes per lane: lane l's bytes land at lds_base + 16 l (lds_base uniform).
 __device__ __forceinline__ void copy16_to_lds(const void* global_src, void* lds_base) {
     __builtin_amdgcn_global_load_lds(global_src, (dense_lds_ptr)lds_base, 16, 0, 0);
+}
+
+// The same from a uniform base: lane l's source is `at` + `step` bytes (32 bits, step uniform) behind it, with no address of 64 bits
+// to form.
+typedef __amdgpu_buffer_rsrc_t CopySource;
+__device__ __forceinline__ CopySource copy_source(const void* base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xffffffff, 0x00027000);
+}
+__device__ __forceinline__ void copy16_to_lds(CopySource from, void* lds_base, unsigned at, int step) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (dense_lds_ptr)lds_base, 16, at, step, 0, 0);
 }
 
 // A barrier that orders LDS only: requested global loads stay in flight.

@@ -1,16 +1,17 @@
-// C = A W^T on the matrix cores for weights in bfloat16 (v_mfma_f32_32x32x16_bf16) or float
-// (v_mfma_f32_32x32x2_f32: true 32-bit products and sums).
+// C = A W^T on the matrix cores for weights in bfloat16 (v_mfma_f32_16x16x32_bf16) or float
+// (v_mfma_f32_16x16x4_f32: true 32-bit products and sums).
 //
-// A workgroup takes a BM x BN tile, each of its waves an equal part of it in 32 x 32 pieces.  K goes in steps of 128 bytes
-// per row; a step's rows are copied global -> LDS by direct 16-byte loads into one of STAGES stages, later steps' copies in
-// flight while one is multiplied.  A fragment is the same 16 bytes per lane for both types: lane l holds row l & 31,
-// chunk 2 kk + (l >> 5).
+// A workgroup takes a BM x BN tile, each of its waves an equal part of it in 16 x 16 pieces.  K goes in steps of 128 bytes
+// per row; a step's rows are copied global -> LDS by direct 16-byte loads into one of several stages, later steps' copies in
+// flight while one is multiplied.  A fragment is the same 16 bytes per lane for both types: lane l holds row l & 15,
+// chunk 4 phase + (l >> 4).
 //
-// What bounds it: bytes per product.  A 128 x 128 tile asks the L2 for 64 bytes a clock and CU at the matrix cores' full rate,
-// which is all the L2 gives, and reads LDS as fast as LDS goes; a 256 x 256 tile asks for half of the one and three quarters of
-// the other.  4095 x 12288 x 2048 in bfloat16 with the gated epilogue: 340 us with 128 x 128 tiles whose copies the compiler
-// waited for ahead of every step's first LDS read (see lds16), 209 us = 0.99 PFLOP/s with 256 x 256.  4095 x 2048 x 6144: 146 us and
-// 104 us, 2048 x 2048 x 2048: 46 us and 25 us.
+// What bounds it: where tiles are large the card's power: 4095 x 12288 x 2048 on random data runs at 1.6 to 1.8 GHz, on zeros, whose products
+// cost less of it, it takes three quarters of the time.  So what counts is that no clock goes by without a matrix op and that a product costs few reads.  A step of 256 x 256 x 64
+// has 2048 clocks of matrix ops a SIMD and takes 2340; with reads and copies in bursts between them 3300, since 64 copies in a row occupy
+// the CU's way to its caches for 1000 clocks; with branches around copies and 64-bit addresses 2530.  16 x 16 pieces take 3 to 5 % less than 32 x 32 at equal clocks.  Then
+// the weights' first trip: tiles whose LDS has room take W a stage further ahead than A.  us, so / as bursts: 4095 x 12288 x 2048 in bfloat16
+// 159 / 194, gated 168 / 203, 4095 x 2048 x 6144 82 / 105, x 2048 33 / 40, 2048^3 20.4 / 24.4, 8192^3 750 / 940 (1.47 PFLOP/s; the library 145, -, 83, 34, 21, 670).
 #include <type_traits>
 
 #include "dense_common.h"
@@ -18,14 +19,13 @@
 namespace a81w41 {
 namespace {
 
-__device__ __forceinline__ void mma(f32x16& acc, const lds16& a, const lds16& b, bf16*) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&a), *reinterpret_cast<const bf16x8*>(&b), acc, 0, 0, 0);
+// 16 x 16 pieces: a fragment is sixteen rows of 64 bytes, lane l holds row l & 15, chunk l >> 4.
+__device__ __forceinline__ void mma(f32x4& acc, const lds16& a, const lds16& b, bf16*) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&a), *reinterpret_cast<const bf16x8*>(&b), acc, 0, 0, 0);
 }
-__device__ __forceinline__ void mma(f32x16& acc, const lds16& a, const lds16& b, float*) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[0]), __uint_as_float(b[0]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[1]), __uint_as_float(b[1]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[2]), __uint_as_float(b[2]), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[3]), __uint_as_float(b[3]), acc, 0, 0, 0);
+__device__ __forceinline__ void mma(f32x4& acc, const lds16& a, const lds16& b, float*) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[e]), __uint_as_float(b[e]), acc, 0, 0, 0);
 }
 
 struct NoHeads {};
@@ -51,74 +51,169 @@ __device__ __forceinline__ void wait_copies_and_meet() {
     asm volatile("" ::: "memory");
 }
 
-// NV registers of a 32 x 32 product: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4 from row0 on, column l % 32 from
-// col0 on; rows from `rows` on are not stored.
-template <typename T, Epilogue EPI, int NV, typename V, typename X>
-__device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, const V& x, int m0, int rows, int row0, int col0, long long batch) {
-    const int lane = threadIdx.x & 63, col = col0 + (lane & 31), r0 = row0 + 4 * (lane >> 5);
-    if constexpr (EPI == Epilogue::kGatedPair) {
-        // Lanes 16 .. 31 and 48 .. 63 hold the ups of the 16 lanes before them.  Of two rows v, v + 1 the gates of the second and the
-        // ups of the first trade places: every lane then has both of one row, and no unit is formed twice.
-        const int odd = (lane >> 4) & 1;
-        T* dst = static_cast<T*>(g.C) + (col >> 5) * 16 + (col & 15);
-#pragma unroll
-        for (int v = 0; v < NV; v += 2) {
-            const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[v]), __float_as_uint(x[v + 1]), false, false);
-            const float unit = gated_unit(g.unit, __uint_as_float(both[0]), __uint_as_float(both[1]));
-            const int r = r0 + 8 * (v >> 2) + (v & 3) + odd;
-            if (r < rows && col < g.N) dst[(size_t)(m0 + r) * g.ldc] = (T)unit;
-        }
-        return;
+// Lanes whose numbers differ in the given low bit trade: of a pair one gives x and takes y's place of the other.
+template <int BIT>
+__device__ __forceinline__ void trade(float& x, float& y) {
+    const bool set = threadIdx.x & BIT;
+    const float mine = set ? x : y;
+    const float other = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mine), BIT == 1 ? 0xB1 : 0x4E, 0xf, 0xf, true));
+    x = set ? other : x;
+    y = set ? y : other;
+}
+// Of G pieces side by side lane l holds column l % 16 of each; then columns 0 .. G - 1 of group l % 16 / G of piece l % G.
+template <int G>
+__device__ __forceinline__ void gather_columns(float (&x)[G]) {
+    if constexpr (G == 4) {
+        trade<1>(x[0], x[1]), trade<1>(x[2], x[3]);
+        trade<2>(x[0], x[2]), trade<2>(x[1], x[3]);
+    } else if constexpr (G == 2) {
+        trade<1>(x[0], x[1]);
     }
+}
+template <int G>
+__device__ __forceinline__ int gathered_column(int lane) {
+    return 16 * (lane & (G - 1)) + (lane & 15 & ~(G - 1));
+}
+template <typename T, int G>
+__device__ __forceinline__ void store_columns(void* dst, const float (&x)[G]) {  // aligned to all of them
+    struct alignas(G * sizeof(T)) {
+        T e[G];
+    } all;
+#pragma unroll
+    for (int i = 0; i < G; i++) all.e[i] = (T)x[i];
+    __builtin_memcpy(__builtin_assume_aligned(dst, G * sizeof(T)), &all, sizeof(all));
+}
+
+// A wave's part of a tile, FM x FN pieces of 16 x 16: register v of lane l holds row 4 (l / 16) + v, column l % 16 of a piece.  Rows from
+// `rows` on are not stored.  Where the target's rows are aligned for it a lane stores G neighbouring columns at a time, sixteen lanes 16 G of a
+// row: an instruction then writes whole lines, with single columns half a line of floats or a quarter of one of elements of 16 bits.
+template <typename T, Epilogue EPI, int FM, int FN, typename X>
+__device__ __forceinline__ void store_tile(const GemmArgs& g, const X& heads, const f32x4 (&acc)[FM][FN], int m0, int rows, int row0, int col0, long long batch) {
+    const int lane = threadIdx.x & 63, l15 = lane & 15, r0 = row0 + 4 * (lane >> 4);
     if constexpr (EPI == Epilogue::kHeads || EPI == Epilogue::kQueries) {
-        // The column's place once, then, where the piece has columns that turn, the rows' angles all at a time; a piece without skips
-        // them, and rows follow by adding.  2048 x 3104 x 2048 with kHeads, 64 of 128 columns of a head turning: 51.5 us with an address
-        // for every element, 45.7 so.  4095 x 3072 x 768 with kQueries, 64 of 192: 38.7 us; in 32 bits first and turned by a launch of
-        // its own 32.6 + 21.5 us, with an address for every element no less than that.
-        const int pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1);
-        const ColumnPlace to = column_place(heads, min(col, g.N - 1), m0 + r0, pos);
-        const bool turns = __any(to.pair >= 0);
-        float cs[NV], sn[NV];
-        if (turns) {
-            const AngleRows angles(pos, m0 + r0, heads.max_seq, turned_pairs(heads));
-            const size_t first = angles.base + max(to.pair, 0);
-            const float *cos_t = heads.cos_t + first, *sin_t = heads.sin_t + first;
+        constexpr int G = FN < 4 ? FN : 4;
+        const int pos = min(max(heads.pos_dev[0], 0), heads.max_seq - 1), pairs = turned_pairs(heads);
+        if (columns_go_together(heads, g.N, G)) {
 #pragma unroll
-            for (int v = 0; v < NV; v++) {
-                const int i = angles.behind(8 * (v >> 2) + (v & 3));
-                cs[v] = cos_t[i], sn[v] = sin_t[i];
+            for (int j = 0; j < FN; j += G) {
+                const int col = col0 + 16 * j + gathered_column<G>(lane);
+                const ColumnPlace to = column_place(heads, min(col, g.N - 1), m0 + r0, pos);
+                const bool turns = __any(to.pair >= 0);
+                const int high = col < g.N ? min(rows - r0, to.rows) : 0;
+                float cs[2][4][G / 2], sn[2][4][G / 2];  // the rows' angles of this i and the next
+                auto request = [&](int i, int to_set) {
+                    if (!turns || i >= FM) return;
+                    const AngleRows angles(pos, m0 + r0 + 16 * i, heads.max_seq, pairs);
+                    const size_t first = angles.base + max(to.pair, 0);
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+#pragma unroll
+                        for (int p = 0; p < G / 2; p++) {
+                            const size_t at = first + angles.behind(v) + (to.pair + p < pairs ? p : 0);
+                            cs[to_set][v][p] = heads.cos_t[at], sn[to_set][v][p] = heads.sin_t[at];
+                        }
+                };
+                request(0, 0);
+#pragma unroll
+                for (int i = 0; i < FM; i++) {
+                    request(i + 1, (i + 1) & 1);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        float x[G];
+#pragma unroll
+                        for (int e = 0; e < G; e++) x[e] = acc[i][j + e][v];
+                        gather_columns<G>(x);
+                        if (turns) {
+#pragma unroll
+                            for (int p = 0; p < G / 2; p++) {
+                                const float c = cs[i & 1][v][p], n = sn[i & 1][v][p], u = x[2 * p], w = x[2 * p + 1];
+                                const bool own = to.pair >= 0 && to.pair + p < pairs;
+                                x[2 * p] = own ? u * c - w * n : u;
+                                x[2 * p + 1] = own ? w * c + u * n : w;
+                            }
+                        }
+                        uint8_t* dst = to.dst + (16 * i + v) * (long long)to.step;
+                        if (16 * i + v < high) {
+                            if (to.as_float)
+                                store_columns<float, G>(dst, x);
+                            else
+                                store_columns<T, G>(dst, x);
+                        }
+                    }
+                }
             }
+            return;
         }
-        uint8_t* dst = to.dst;
-        const int high = col < g.N ? min(rows - r0, to.rows) : 0;
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
-            if (v) dst += (v & 3) ? to.step : 5 * to.step;
-            float y = x[v];
-            if (turns) {
-                const float other = swap_neighbours(y), turned = to.second ? y * cs[v] + other * sn[v] : y * cs[v] - other * sn[v];
-                y = to.pair >= 0 ? turned : y;
-            }
-            if (8 * (v >> 2) + (v & 3) < high) {
-                if (to.as_float)
-                    *reinterpret_cast<float*>(dst) = y;
-                else
-                    *reinterpret_cast<T*>(dst) = (T)y;
+        for (int j = 0; j < FN; j++) {
+            const int col = col0 + 16 * j + l15;
+            const ColumnPlace to = column_place(heads, min(col, g.N - 1), m0 + r0, pos);
+            const int high = col < g.N ? min(rows - r0, to.rows) : 0;
+#pragma unroll
+            for (int i = 0; i < FM; i++) {
+                const AngleRows angles(pos, m0 + r0 + 16 * i, heads.max_seq, pairs);
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float x = acc[i][j][v], other = swap_neighbours(x);
+                    float y = x;
+                    if (to.pair >= 0) {
+                        const size_t at = angles.base + angles.behind(v) + to.pair;
+                        const float c = heads.cos_t[at], n = heads.sin_t[at];
+                        y = to.second ? x * c + other * n : x * c - other * n;
+                    }
+                    uint8_t* dst = to.dst + (16 * i + v) * (long long)to.step;
+                    if (16 * i + v < high) {
+                        if (to.as_float)
+                            *reinterpret_cast<float*>(dst) = y;
+                        else
+                            *reinterpret_cast<T*>(dst) = (T)y;
+                    }
+                }
             }
         }
         return;
     }
+    // units have half as many columns as the product
+    using E = std::conditional_t<EPI == Epilogue::kFloat, float, T>;
+    constexpr bool kGated = EPI == Epilogue::kGatedPair;
+    constexpr int kPieces = kGated ? FN / 2 : FN, G = kPieces < 4 ? kPieces : 4;
+    const int N = kGated ? g.N / 2 : g.N, first = kGated ? col0 / 2 : col0;
+    E* const C = static_cast<E*>(g.C) + (g.tiles ? 0 : batch * g.c_step);
+    const bool together = ((g.ldc | N) & (G - 1)) == 0 && (reinterpret_cast<uintptr_t>(C) & (G * sizeof(E) - 1)) == 0;
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-        const int r = r0 + 8 * (v >> 2) + (v & 3);
-        const size_t row = m0 + r;
-        if (r < rows && col < g.N) {
-            if constexpr (EPI == Epilogue::kFloat) {
-                (static_cast<float*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = x[v];
-            } else {
-                float f = x[v];
-                if constexpr (EPI == Epilogue::kHeadGate) f *= sigmoid(g.head_gate[row * g.ld_gate + batch]);
-                (static_cast<T*>(g.C) + (g.tiles ? 0 : batch * g.c_step))[row * g.ldc + col] = (T)f;
+    for (int i = 0; i < FM; i++) {
+        float gate[4];
+        if constexpr (EPI == Epilogue::kHeadGate) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) gate[v] = sigmoid(g.head_gate[(size_t)(m0 + min(r0 + 16 * i + v, rows - 1)) * g.ld_gate + batch]);
+        }
+#pragma unroll
+        for (int j = 0; j < kPieces; j += G) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = r0 + 16 * i + v;
+                float x[G];
+#pragma unroll
+                for (int e = 0; e < G; e++) {
+                    if constexpr (kGated)
+                        x[e] = gated_unit(g.unit, acc[i][2 * (j + e)][v], acc[i][2 * (j + e) + 1][v]);
+                    else if constexpr (EPI == Epilogue::kHeadGate)
+                        x[e] = acc[i][j + e][v] * gate[v];
+                    else
+                        x[e] = acc[i][j + e][v];
+                }
+                E* const row = C + (size_t)(m0 + r) * g.ldc;
+                if (together) {
+                    gather_columns<G>(x);
+                    const int col = first + 16 * j + gathered_column<G>(lane);
+                    if (r < rows && col < N) store_columns<E, G>(row + col, x);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < G; e++) {
+                        const int col = first + 16 * (j + e) + l15;
+                        if (r < rows && col < N) row[col] = (E)x[e];
+                    }
+                }
             }
         }
     }
@@ -127,20 +222,22 @@ __device__ __forceinline__ void store_piece(const GemmArgs& g, const X& heads, c
 // Rows of tiles that are walked together: an XCD's workgroups then share these rows and a few column panels in its L2.
 constexpr int kBandRows = 2048;
 
-// X: HeadRows<T> with the epilogue kHeads, LatentQueries<T> with kQueries, NoHeads with the others.  STAGES: how many steps LDS holds; all but one are under way.
-// PIPE: a step's operands are read one 16-byte column ahead of their products, also into the next step: the waves meet before a step's
-// last products, whose operands are in registers by then, so that its stage is free for new copies and the next step's first
-// reads run beside those products.  4095 x 12288 x 2048 into floats: 211 us with the meeting between two steps, 204 so.  Without PIPE the other workgroup of the CU fills the wait.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PIPE, Epilogue EPI, typename X>
+// X: HeadRows<T> with the epilogue kHeads, LatentQueries<T> with kQueries, NoHeads with the others.  STAGES: how many steps LDS holds.
+// A step has two phases of 64 bytes a row.  A phase's operands are read while the phase before it is multiplied, also over the end of a step:
+// the waves meet ahead of a step's second phase, whose operands are in registers by then, so that its stage is free for new copies.
+// PIPED: reads and copies go one by one between the matrix ops, kFirst of a stage's copies in that second phase and the rest in the next step's
+// first; requested in a row they kept every wave of the CU waiting for its turn at the caches while the matrix cores idled.
+// Without, for tiles of which a CU has several, a step's copies come first and other workgroups fill the wait.
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, bool PIPED, Epilogue EPI, typename X>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(GemmArgs g, X heads) {
     constexpr int kThreads = 64 * WAVES_M * WAVES_N;
-    constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 32, FN = WN / 32;
-    constexpr int LA = BM * 8 / kThreads, LB = BN * 8 / kThreads;  // direct copies per thread and stage
-    constexpr int kStage = (BM + BN) * 128;
-    static_assert(STAGES >= 2 && (STAGES - 1) * (LA + LB) < 64, "copies a wait can leave outstanding");
-    __shared__ __attribute__((aligned(128))) uint8_t lds[STAGES * kStage];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l31 = lane & 31, half = lane >> 5;
+    constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 16, FN = WN / 16;
+    constexpr int LA = BM * 8 / kThreads, LB = BN * 8 / kThreads, L = LA + LB;  // direct copies per thread and stage
+    constexpr int kStageA = BM * 128, kStageW = BN * 128;
+    static_assert(SA >= 2 && (SA == SW || (PIPED && SW == SA + 1)) && SW * L < 64, "copies a wait can leave outstanding");
+    __shared__ __attribute__((aligned(128))) uint8_t lds[SA * kStageA + SW * kStageW];
+    uint8_t* const lds_w = lds + SA * kStageA;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l15 = lane & 15;
     // Tiles dealt to the XCDs in contiguous runs, in bands of kBandRows rows and inside one column panel after the other.  A grouped
     // product's go expert by expert, column panel by column panel: an XCD then reads the rows of a few experts once and their weights
     // once.  With the rows of all experts for one panel after the other (8192 rows of 4 KB, 32 experts, 16 panels) the rows were read from
@@ -166,111 +263,144 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(G
         rows = g.M - m0;
     }
     const int n0 = nt * BN;
-    const uint8_t* A = reinterpret_cast<const uint8_t*>(static_cast<const T*>(g.A) + (g.tiles ? 0 : batch * g.a_step));
-    const uint8_t* W = reinterpret_cast<const uint8_t*>(static_cast<const T*>(g.W) + batch * g.w_step);
-    const uint8_t *a_src[LA], *b_src[LB];
+    // A tile's rows by 32-bit offsets from the first; gathered rows from the start of A, which models keep under 4 GB
+    const T* const A = static_cast<const T*>(g.A) + (g.tiles ? 0 : batch * g.a_step) + (g.a_rows ? 0 : (size_t)m0 * g.lda);
+    const T* const W = static_cast<const T*>(g.W) + batch * g.w_step + (size_t)n0 * g.ldw;
+    const CopySource from_a = copy_source(A), from_w = copy_source(W);
+    unsigned a_at[LA], w_at[LB];
 #pragma unroll
     for (int i = 0; i < LA; i++) {
-        const int c = i * kThreads + tid, r = c >> 3;
-        int row = m0 + min(r, rows - 1);
-        if (g.a_rows) row = g.a_rows[row];
-        a_src[i] = A + (size_t)row * g.lda * sizeof(T) + (((c & 7) ^ place_of_row(r)) << 4);
+        const int c = i * kThreads + tid, r = c >> 3, row = min(r, rows - 1);
+        a_at[i] = (unsigned)(g.a_rows ? g.a_rows[m0 + row] : row) * (g.lda * (unsigned)sizeof(T)) + (((c & 7) ^ place_of_row(r)) << 4);
     }
 #pragma unroll
     for (int i = 0; i < LB; i++) {
         const int c = i * kThreads + tid, r = c >> 3;
-        b_src[i] = W + (size_t)min(n0 + r, g.N - 1) * g.ldw * sizeof(T) + (((c & 7) ^ place_of_row(r)) << 4);
+        w_at[i] = (unsigned)min(r, g.N - 1 - n0) * (g.ldw * (unsigned)sizeof(T)) + (((c & 7) ^ place_of_row(r)) << 4);
     }
-    auto copy_step = [&](int step, int stage) {
-        uint8_t* base = lds + stage * kStage + wave * 1024;
-#pragma unroll
-        for (int i = 0; i < LA; i++) copy16_to_lds(a_src[i] + (size_t)step * 128, base + i * kThreads * 16);
-#pragma unroll
-        for (int i = 0; i < LB; i++) copy16_to_lds(b_src[i] + (size_t)step * 128, base + BM * 128 + i * kThreads * 16);
+    auto copy_a = [&](int i, int step, int stage) {
+        copy16_to_lds(from_a, lds + stage * kStageA + wave * 1024 + i * kThreads * 16, a_at[i], step * 128);
     };
-    f32x16 acc[FM][FN];
+    auto copy_w = [&](int i, int step, int stage) {
+        copy16_to_lds(from_w, lds_w + stage * kStageW + wave * 1024 + i * kThreads * 16, w_at[i], step * 128);
+    };
+    f32x4 acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
-        for (int j = 0; j < FN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+        for (int j = 0; j < FN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int wm = (wave % WAVES_M) * WM, wn = (wave / WAVES_M) * WN;
     const int n_steps = g.K * (int)sizeof(T) / 128;
+    constexpr int kReads = FM + FN, kOps = FM * FN;
     lds16 a[2][FM], b[2][FN];
-    auto read = [&](int kk, const uint8_t* sa) {
-        const uint8_t* sb = sa + BM * 128;
-#pragma unroll
-        for (int i = 0; i < FM; i++) {
-            const int r = wm + i * 32 + l31;
-            a[kk & 1][i] = *reinterpret_cast<const lds16*>(sa + r * 128 + (((2 * kk + half) ^ place_of_row(r)) << 4));
-        }
-#pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const int r = wn + j * 32 + l31;
-            b[kk & 1][j] = *reinterpret_cast<const lds16*>(sb + r * 128 + (((2 * kk + half) ^ place_of_row(r)) << 4));
-        }
+    const int own_row = l15 * 128, own_place[2] = {((lane >> 4) ^ place_of_row(l15)) << 4, ((4 + (lane >> 4)) ^ place_of_row(l15)) << 4};
+    auto read_one = [&](int r, int phase, const uint8_t* sa, const uint8_t* sw) {  // fragment r of the phase, A's first
+        if (r < FM)
+            a[phase][r < FM ? r : 0] = *reinterpret_cast<const lds16*>(sa + wm * 128 + r * 2048 + own_row + own_place[phase]);
+        else
+            b[phase][r < FM ? 0 : r - FM] = *reinterpret_cast<const lds16*>(sw + wn * 128 + (r - FM) * 2048 + own_row + own_place[phase]);
     };
-    auto multiply = [&](int kk) {
+    if constexpr (PIPED) {
+        // Of the copies that a step makes room for, A's before W's, this many go beside its second phase, the rest beside the next step's first;
+        // with two stages of A all, which need the time.
+        constexpr int kFirst = SA == 2 ? L : (2 * L + 2) / 3;
+        // copies that a step leaves under way when it waits for the next one's
+        constexpr int kAfter = (SA - 2) * L + (SW > SA ? LB : 0);
+        auto copy_one = [&](int i, int step, int stage_a, int stage_w) {
+            if (i < LA)
+                copy_a(i < LA ? i : 0, step + SA, stage_a);
+            else
+                copy_w(i < LA ? 0 : i - LA, step + SW, stage_w);
+        };
+        // as if steps -SW .. -1 had made room: W's further stage first, and of the last of them kFirst copies
+        if constexpr (SW > SA) {
 #pragma unroll
-        for (int i = 0; i < FM; i++)
+            for (int i = 0; i < LB; i++) copy_w(i, 0, 0);
+        }
+        const bool whole = n_steps >= SW;
+        for (int step = -SA; step < 0; step++)
 #pragma unroll
-            for (int j = 0; j < FN; j++) mma(acc[i][j], a[kk & 1][i], b[kk & 1][j], static_cast<T*>(nullptr));
-    };
-    if constexpr (PIPE) {
-        for (int step = 0; step < STAGES && step < n_steps; step++) copy_step(step, step);
-        if (n_steps >= STAGES)
-            wait_copies_and_meet<(STAGES - 1) * (LA + LB)>();
+            for (int i = 0; i < L; i++)
+                if ((step < -1 || i < kFirst || !whole) && (i < LA ? step + SA : step + SW) < n_steps) copy_one(i, step, step + SA, step + SW);
+        if (whole)
+            wait_copies_and_meet<kAfter + kFirst>();
         else
             wait_copies_and_meet<0>();
-        read(0, lds);
-        int stage = 0;
-        for (int step = 0; step < n_steps; step++) {
-            const uint8_t* sa = lds + stage * kStage;
-            const int next = stage + 1 < STAGES ? stage + 1 : 0;
 #pragma unroll
-            for (int kk = 0; kk < 3; kk++) {
+        for (int r = 0; r < kReads; r++) read_one(r, 0, lds, lds_w);
+        int step = 0, sa = 0, sw = 0;
+        // REST: copies of what the step before made room for are left; A, W: this step's stages are filled again; AHEAD: copies stay under
+        // way at the meeting
+        auto one_step = [&](auto rest, auto fill_a, auto fill_w, auto ahead, bool more) {
+            constexpr int kRest = decltype(rest)::value ? L - kFirst : 0;
+            constexpr int kFillA = decltype(fill_a)::value ? kFirst : 0, kFillW = decltype(fill_w)::value ? kFirst : 0;
+            const int next_a = sa + 1 < SA ? sa + 1 : 0, next_w = sw + 1 < SW ? sw + 1 : 0;
+            const int before_a = sa ? sa - 1 : SA - 1, before_w = sw ? sw - 1 : SW - 1;
+            auto phase = [&](auto which, int c0, int copies, int of_step, int stage_a, int stage_w, const uint8_t* from_sa, const uint8_t* from_sw) {
+                constexpr int P = decltype(which)::value;
+                const int all = kReads + copies;
                 __builtin_amdgcn_sched_barrier(0);
-                read(kk + 1, sa);
+#pragma unroll
+                for (int o = 0; o < kOps; o++) {
+#pragma unroll
+                    for (int x = 0; x < all; x++) {
+                        if ((all <= kOps ? x : x * kOps / all) != o) continue;
+                        if (x < kReads)
+                            read_one(x, 1 - P, from_sa, from_sw);
+                        else if (P == 0 || (c0 + x - kReads < LA ? kFillA : kFillW))
+                            copy_one(c0 + x - kReads, of_step, stage_a, stage_w);
+                    }
+                    mma(acc[o / FN][o % FN], a[P][o / FN], b[P][o % FN], static_cast<T*>(nullptr));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            phase(std::integral_constant<int, 0>{}, kFirst, kRest, step - 1, before_a, before_w, lds + sa * kStageA, lds_w + sw * kStageW);
+            if (more) {
                 __builtin_amdgcn_sched_barrier(0);
-                multiply(kk);
+                wait_copies_and_meet<decltype(ahead)::value ? kAfter : 0>();
             }
-            __builtin_amdgcn_sched_barrier(0);
-            if (step + 1 < n_steps) {
-                if (step + STAGES <= n_steps)
-                    wait_copies_and_meet<(STAGES - 2) * (LA + LB)>();
-                else
-                    wait_copies_and_meet<0>();
-                if (step + STAGES < n_steps) copy_step(step + STAGES, stage);
-                read(0, lds + next * kStage);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            multiply(3);
-            stage = next;
+            phase(std::integral_constant<int, 1>{}, 0, kFillA > kFillW ? kFillA : kFillW, step, sa, sw, lds + next_a * kStageA, lds_w + next_w * kStageW);
+            sa = next_a, sw = next_w;
+            step++;
+        };
+        constexpr std::true_type yes;
+        constexpr std::false_type no;
+        while (step < n_steps - SW) one_step(yes, yes, yes, yes, true);
+        if constexpr (SW > SA) {  // the last rows of A are still to come, no more of W
+            static_assert(kFirst == L, "nothing is left to the next step");
+            if (whole) one_step(no, yes, no, yes, step + 1 < n_steps);
+        } else {
+            if (whole) one_step(yes, no, no, yes, step + 1 < n_steps);
         }
+        while (step < n_steps) one_step(no, no, no, no, step + 1 < n_steps);
     } else {
-        for (int step = 0; step < STAGES - 1 && step < n_steps; step++) copy_step(step, step);
+        auto copy_step = [&](int step, int stage) {
+#pragma unroll
+            for (int i = 0; i < LA; i++) copy_a(i, step, stage);
+#pragma unroll
+            for (int i = 0; i < LB; i++) copy_w(i, step, stage);
+        };
+        for (int step = 0; step < SA - 1 && step < n_steps; step++) copy_step(step, step);
         int stage = 0;
         for (int step = 0; step < n_steps; step++) {
             // the copies of the step are in LDS, later ones may be under way; and nobody still reads the stage before it
-            if (step + STAGES - 2 < n_steps)
-                wait_copies_and_meet<(STAGES - 2) * (LA + LB)>();
+            if (step + SA - 2 < n_steps)
+                wait_copies_and_meet<(SA - 2) * L>();
             else
                 wait_copies_and_meet<0>();
-            if (step + STAGES - 1 < n_steps) copy_step(step + STAGES - 1, stage ? stage - 1 : STAGES - 1);
-            const uint8_t* sa = lds + stage * kStage;
-            stage = stage + 1 < STAGES ? stage + 1 : 0;
+            if (step + SA - 1 < n_steps) copy_step(step + SA - 1, stage ? stage - 1 : SA - 1);
+            const uint8_t *sa = lds + stage * kStageA, *sw = lds_w + stage * kStageW;
+            stage = stage + 1 < SA ? stage + 1 : 0;
 #pragma unroll
-            for (int kk = 0; kk < 4; kk++) {
-                read(kk, sa);
-                multiply(kk);
+            for (int phase = 0; phase < 2; phase++) {
+#pragma unroll
+                for (int r = 0; r < kReads; r++) read_one(r, phase, sa, sw);
+#pragma unroll
+                for (int o = 0; o < kOps; o++) mma(acc[o / FN][o % FN], a[phase][o / FN], b[phase][o % FN], static_cast<T*>(nullptr));
             }
         }
     }
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) store_piece<T, EPI, 16>(g, heads, acc[i][j], m0, rows, wm + i * 32, n0 + wn + j * 32, batch);
+    store_tile<T, EPI, FM, FN>(g, heads, acc, m0, rows, wm, n0 + wn, batch);
 }
 
 // Few rows, so few tiles that a CU has one at most: what counts is that the weights are under way and that a step is short.  64
@@ -283,7 +413,7 @@ template <typename T, Epilogue EPI, typename X>
 __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X heads) {
     constexpr int SA = 10, SW = 20, kStageA = 64 * 128, kStageW = 32 * 128;
     __shared__ __attribute__((aligned(128))) uint8_t lds[SA * kStageA + SW * kStageW];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l31 = lane & 31, half = lane >> 5;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l15 = lane & 15;
     // row tiles of a column panel next to each other on one XCD
     const int n_mt = (g.M + 63) / 64;
     const int q = gridDim.x >> 3, r8 = gridDim.x & 7, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
@@ -333,25 +463,25 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
         }
         return;
     }
-    f32x16 acc;
+    f32x4 acc[2][2];
 #pragma unroll
-    for (int v = 0; v < 16; v++) acc[v] = 0.f;
-    lds16 a[2][4], w[2][4];
+    for (int o = 0; o < 4; o++) acc[o / 2][o % 2] = f32x4{0.f, 0.f, 0.f, 0.f};
+    lds16 a[2][4], w[2][4];  // of a step: phase 0's two fragments, then phase 1's
     int slot_a = 0, slot_w = 0;
     auto read = [&](lds16 (&x)[4], lds16 (&y)[4]) {
-        const uint8_t *pa = lds + slot_a * kStageA + wave * 4096 + l31 * 128, *pw = lds_w + slot_w * kStageW + l31 * 128;
+        const uint8_t *pa = lds + slot_a * kStageA + wave * 4096 + l15 * 128, *pw = lds_w + slot_w * kStageW + l15 * 128;
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-            const int at = ((2 * kk + half) ^ place_of_row(l31)) << 4;
-            x[kk] = *reinterpret_cast<const lds16*>(pa + at);
-            y[kk] = *reinterpret_cast<const lds16*>(pw + at);
+        for (int n = 0; n < 4; n++) {
+            const int at = n % 2 * 2048 + (((n / 2 * 4 + (lane >> 4)) ^ place_of_row(l15)) << 4);
+            x[n] = *reinterpret_cast<const lds16*>(pa + at);
+            y[n] = *reinterpret_cast<const lds16*>(pw + at);
         }
         slot_a = slot_a + 1 < SA ? slot_a + 1 : 0;
         slot_w = slot_w + 1 < SW ? slot_w + 1 : 0;
     };
     auto multiply = [&](const lds16 (&x)[4], const lds16 (&y)[4]) {
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) mma(acc, x[kk], y[kk], static_cast<T*>(nullptr));
+        for (int o = 0; o < 8; o++) mma(acc[o / 2 % 2][o % 2], x[o / 4 * 2 + o / 2 % 2], y[o / 4 * 2 + o % 2], static_cast<T*>(nullptr));
     };
     // meet: the step is in LDS; its reads then run beside the products of the step before
     wait_copies_and_meet<0>();
@@ -367,7 +497,7 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
         multiply(a[1], w[1]);
     }
     if (n_steps & 1) multiply(a[0], w[0]);
-    store_piece<T, EPI, 16>(g, heads, acc, m0, rows, wave * 32, n0, batch);
+    store_tile<T, EPI, 2, 2>(g, heads, acc, m0, rows, wave * 32, n0, batch);
 }
 
 // 256 x 256 tiles, one workgroup per CU, or 128 x 128, two per CU.  At K = 2048 a round of 256 large tiles takes 65 us whether
@@ -380,10 +510,10 @@ bool large_tiles_preferred(long long large, long long small, int K) {
     return rounds * (rounds > 1 && K <= 2048 ? 769 : 750) <= small;
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool PIPE, Epilogue EPI, typename X>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, bool PIPED, Epilogue EPI, typename X>
 hipError_t launch_kernel(const GemmArgs& g, const X& heads, hipStream_t s) {
     const int n_mt = g.tiles ? g.max_tiles : (g.M + BM - 1) / BM, n_nt = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((dense_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, STAGES, PIPE, EPI, X>), dim3(n_mt * n_nt, g.batches),
+    hipLaunchKernelGGL((dense_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, SA, SW, PIPED, EPI, X>), dim3(n_mt * n_nt, g.batches),
                        dim3(64 * WAVES_M * WAVES_N), 0, s, g, heads);
     return hipGetLastError();
 }
@@ -404,20 +534,20 @@ hipError_t launch_grouped(const GemmArgs& g, const X& heads, hipStream_t s) {
         // 128.7 + 70.5 / 128.5 + 68.7, 1536 x 1536 74.2 + 44.8 / 74.6 + 41.3; 0.63 of two rounds full, 1024 x 1024 45.4 + 27.4 / 47.6 + 28.2.
         const int whole = g.M / kGroupTileManyRows;
         const long long tiles = (whole + g.max_tiles) / 2 * panels(256), rounds = (tiles + 255) / 256;
-        if (10 * tiles >= 7 * 256 * rounds) return launch_kernel<T, kGroupTileManyRows, 256, 2, 4, 3, true, EPI>(g, heads, s);
-        return launch_kernel<T, kGroupTileManyRows, 128, 2, 2, 2, true, EPI>(g, heads, s);
+        if (10 * tiles >= 7 * 256 * rounds) return launch_kernel<T, kGroupTileManyRows, 256, 2, 4, 3, 3, true, EPI>(g, heads, s);
+        return launch_kernel<T, kGroupTileManyRows, 128, 2, 2, 2, 2, true, EPI>(g, heads, s);
     }
     // 64 x 128 tiles with two stages fit a CU three times, with three stages twice and have more of the weights under way, which counts where
     // there are few rounds.  us of gate and up with two / three: 600 tokens of 4 out of 32, 2048 x 2048 82.4 / 72.3, 64 tokens 62.5 / 60.0,
     // 16 tokens, 1024 x 1024 13.4 / 10.9.  Past the line prompts of 760 to 1020 tokens at width 2048 take 0.96 to 0.98 of the time with three as
     // well; where 512 to 768 tiles are there, one round with two stages and two with three, 830 to 1020 tokens at width 1024 take 1.01 to 1.02 of it.
     if (g.N >= 1024) {
-        if (g.max_tiles * panels(128) <= 1200) return launch_kernel<T, kGroupTileRows, 128, 2, 4, 3, true, EPI>(g, heads, s);
-        return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, true, EPI>(g, heads, s);
+        if (g.max_tiles * panels(128) <= 1200) return launch_kernel<T, kGroupTileRows, 128, 2, 4, 3, 3, true, EPI>(g, heads, s);
+        return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, 2, true, EPI>(g, heads, s);
     }
     // see launch_by_size: 1000 tiles, 512 x 512 14.7 us with four stages, 11.6 with two
-    if (g.max_tiles * panels(64) > 512) return launch_kernel<T, kGroupTileRows, 64, 2, 2, 2, false, EPI>(g, heads, s);
-    return launch_kernel<T, kGroupTileRows, 64, 2, 2, 4, false, EPI>(g, heads, s);
+    if (g.max_tiles * panels(64) > 512) return launch_kernel<T, kGroupTileRows, 64, 2, 2, 2, 2, false, EPI>(g, heads, s);
+    return launch_kernel<T, kGroupTileRows, 64, 2, 2, 4, 4, false, EPI>(g, heads, s);
 }
 
 template <typename T, Epilogue EPI, typename X>
@@ -432,21 +562,21 @@ hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
     auto one_round = [&](int rows, int cols) { return g.M > 64 && tiles(rows, cols) >= 192 && tiles(rows, cols) <= 256; };
     const int steps = g.K * (int)sizeof(T) / 128;
     if constexpr (sizeof(T) == 2)
-        if (large_tiles_preferred(tiles(256, 256), tiles(128, 128), g.K)) return launch_kernel<T, 256, 256, 2, 4, 2, true, EPI>(g, heads, s);
+        if (large_tiles_preferred(tiles(256, 256), tiles(128, 128), g.K)) return launch_kernel<T, 256, 256, 2, 4, 2, 3, true, EPI>(g, heads, s);
     // us, so / with 128 x 128 tiles: 4095 rows, 2048 x 2048 39.6 / 41.1, 2048 x 6144 106 / 109; 2048 rows, 3104 x 2048 36.3 / 40.4.
     // Over 45 drawn shapes a type, on average: bfloat16 up to 10 steps 1.02 of the time and up to 1.075 (1854 rows, 4203 x 640 21.4 /
     // 20.1), 11 and more 0.98; float up to 4 steps 1.05 (951 rows, 6073 x 64 16.4 / 15.2), 6 and more 0.98.
-    if (steps >= (sizeof(T) == 2 ? 11 : 6) && one_round(128, 256)) return launch_kernel<T, 128, 256, 2, 4, 3, true, EPI>(g, heads, s);
+    if (steps >= (sizeof(T) == 2 ? 11 : 6) && one_round(128, 256)) return launch_kernel<T, 128, 256, 2, 4, 3, 3, true, EPI>(g, heads, s);
     // 2048^3: 24.8 us with twice the waves and four stages, 33 us as two a CU
-    if (one_round(128, 128)) return launch_kernel<T, 128, 128, 2, 4, 4, true, EPI>(g, heads, s);
+    if (one_round(128, 128)) return launch_kernel<T, 128, 128, 2, 4, 4, 4, true, EPI>(g, heads, s);
     if (g.M > 64 && tiles(128, 128) > 256) {
         // 300 rows, 12288 x 2048 26.7 / 36.8
-        if (one_round(64, 256)) return launch_kernel<T, 64, 256, 2, 4, 3, true, EPI>(g, heads, s);
-        return launch_kernel<T, 128, 128, 2, 2, 2, false, EPI>(g, heads, s);
+        if (one_round(64, 256)) return launch_kernel<T, 64, 256, 2, 4, 3, 3, true, EPI>(g, heads, s);
+        return launch_kernel<T, 128, 128, 2, 2, 2, 2, false, EPI>(g, heads, s);
     }
     // us, so / with 64 x 64 tiles: 1024 rows, 2048 x 2048 15.2 / 16.0, x 6144 45.1 / 49.2; 600 rows, 3072 x 1536 12.2 / 13.4; 180 rows, 9216
     // x 1536 14.6 / 16.3; over 45 drawn shapes 0.98 on average, with one and two steps 1.03 (2674 rows, 553 x 128 5.8 / 5.5)
-    if (steps > 2 && one_round(64, 128)) return launch_kernel<T, 64, 128, 2, 4, 3, true, EPI>(g, heads, s);
+    if (steps > 2 && one_round(64, 128)) return launch_kernel<T, 64, 128, 2, 4, 3, 3, true, EPI>(g, heads, s);
     // So few tiles of 64 x 32 that no CU gets a second one (us, against 64 x 64 tiles with four stages): 33 rows, 784 x 2048 7.7 /
     // 12.5, 2048 x 6144 19 / 31; 256 rows, 2048 x 2048 10.2 / 13.5; with a second one 300 rows, 2048 x 2048 17.2 / 13.8, and 33
     // rows, 12288 x 2048 20 / 16.
@@ -454,8 +584,8 @@ hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
     // 64 x 64 tiles with four stages fit a CU twice, with two stages five times: more tiles than 512 would go in rounds.  bfloat16,
     // us with four / two: 1030 rows, 544 tiles, 2048 x 1024 15.9 / 12.2, 2048 x 6144 63 / 50; in one round, 400 rows, 448 tiles, 4096 x
     // 4096 27.5 / 34.  float, 1030 rows, 2048 x 1024: 60.5 / 56.9.
-    if (tiles(64, 64) > 512) return launch_kernel<T, 64, 64, 2, 2, 2, false, EPI>(g, heads, s);
-    return launch_kernel<T, 64, 64, 2, 2, 4, false, EPI>(g, heads, s);
+    if (tiles(64, 64) > 512) return launch_kernel<T, 64, 64, 2, 2, 2, 2, false, EPI>(g, heads, s);
+    return launch_kernel<T, 64, 64, 2, 2, 4, 4, false, EPI>(g, heads, s);
 }
 
 }  // namespace

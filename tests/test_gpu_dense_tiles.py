@@ -264,6 +264,21 @@ def test_one_round_of_tiles(pkg, M, N, K, dtype):
     assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
 
 
+# 256 x 256 tiles, whose rings of A and W have two and three stages: fewer steps than stages, as many, more; rows of C that take four columns
+# at a time and rows that do not.
+@pytest.mark.parametrize("N", [4096, 4094, 4093])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 9])
+def test_rings_of_two_lengths(pkg, N, steps):
+    import torch
+    g, K, M = torch.Generator(device="cuda").manual_seed(steps), 64 * steps, 4090
+    a = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = torch.randn(N, K, device="cuda", generator=g).bfloat16()
+    got = pkg.ops.dense_gemm(a, w, K)
+    # K products, exact, and K sums, rounded to 24 bits
+    assert (got.double() - a.double() @ w.double().t()).abs().max().item() <= K * 2.0 ** -24 * 4 * K ** 0.5
+    assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
+
+
 # The steps of K from which one round of 128 x 256 and of 64 x 128 tiles is taken, and those before: the same bits for a row in a call of
 # 33 rows, which goes through another kernel on either side.
 @pytest.mark.parametrize("M,N,dtype,steps", [(2045, 3100, "bfloat16", (10, 11, 12, 13)), (2045, 3100, "float32", (5, 6, 7)),
