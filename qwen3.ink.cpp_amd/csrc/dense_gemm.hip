@@ -222,19 +222,19 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const X& heads, co
 // Rows of tiles that are walked together: an XCD's workgroups then share these rows and a few column panels in its L2.
 constexpr int kBandRows = 2048;
 
-// X: HeadRows<T> with the epilogue kHeads, LatentQueries<T> with kQueries, NoHeads with the others.  STAGES: how many steps LDS holds.
+// X: HeadRows<T> with the epilogue kHeads, LatentQueries<T> with kQueries, NoHeads with the others.  SA, SW: how many steps' rows and weights LDS holds.
 // A step has two phases of 64 bytes a row.  A phase's operands are read while the phase before it is multiplied, also over the end of a step:
 // the waves meet ahead of a step's second phase, whose operands are in registers by then, so that its stage is free for new copies.
-// PIPED: reads and copies go one by one between the matrix ops, kFirst of a stage's copies in that second phase and the rest in the next step's
-// first; requested in a row they kept every wave of the CU waiting for its turn at the caches while the matrix cores idled.
-// Without, for tiles of which a CU has several, a step's copies come first and other workgroups fill the wait.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, bool PIPED, Epilogue EPI, typename X>
+// Reads and copies go one by one between the matrix ops, kFirst of a stage's copies in that second phase and the rest in the next step's
+// first; requested in a row they kept every wave of the CU waiting for its turn at the caches while the matrix cores idled.  That holds where
+// a CU has several workgroups as well: 64 x 64 tiles with a step's copies in a row took 1.2 to 1.3 times as long.
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, Epilogue EPI, typename X>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(GemmArgs g, X heads) {
     constexpr int kThreads = 64 * WAVES_M * WAVES_N;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 16, FN = WN / 16;
     constexpr int LA = BM * 8 / kThreads, LB = BN * 8 / kThreads, L = LA + LB;  // direct copies per thread and stage
     constexpr int kStageA = BM * 128, kStageW = BN * 128;
-    static_assert(SA >= 2 && (SA == SW || (PIPED && SW == SA + 1)) && SW * L < 64, "copies a wait can leave outstanding");
+    static_assert(SA >= 2 && (SA == SW || SW == SA + 1) && SW * L < 64, "copies a wait can leave outstanding");
     __shared__ __attribute__((aligned(128))) uint8_t lds[SA * kStageA + SW * kStageW];
     uint8_t* const lds_w = lds + SA * kStageA;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l15 = lane & 15;
@@ -300,106 +300,78 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(G
         else
             b[phase][r < FM ? 0 : r - FM] = *reinterpret_cast<const lds16*>(sw + wn * 128 + (r - FM) * 2048 + own_row + own_place[phase]);
     };
-    if constexpr (PIPED) {
-        // Of the copies that a step makes room for, A's before W's, this many go beside its second phase, the rest beside the next step's first;
-        // with two stages of A all, which need the time.
-        constexpr int kFirst = SA == 2 ? L : (2 * L + 2) / 3;
-        // copies that a step leaves under way when it waits for the next one's
-        constexpr int kAfter = (SA - 2) * L + (SW > SA ? LB : 0);
-        auto copy_one = [&](int i, int step, int stage_a, int stage_w) {
-            if (i < LA)
-                copy_a(i < LA ? i : 0, step + SA, stage_a);
-            else
-                copy_w(i < LA ? 0 : i - LA, step + SW, stage_w);
-        };
-        // as if steps -SW .. -1 had made room: W's further stage first, and of the last of them kFirst copies
-        if constexpr (SW > SA) {
-#pragma unroll
-            for (int i = 0; i < LB; i++) copy_w(i, 0, 0);
-        }
-        const bool whole = n_steps >= SW;
-        for (int step = -SA; step < 0; step++)
-#pragma unroll
-            for (int i = 0; i < L; i++)
-                if ((step < -1 || i < kFirst || !whole) && (i < LA ? step + SA : step + SW) < n_steps) copy_one(i, step, step + SA, step + SW);
-        if (whole)
-            wait_copies_and_meet<kAfter + kFirst>();
+    // Of the copies that a step makes room for, A's before W's, this many go beside its second phase, the rest beside the next step's first;
+    // with two stages of A all, which need the time.
+    constexpr int kFirst = SA == 2 ? L : (2 * L + 2) / 3;
+    // copies that a step leaves under way when it waits for the next one's
+    constexpr int kAfter = (SA - 2) * L + (SW > SA ? LB : 0);
+    auto copy_one = [&](int i, int step, int stage_a, int stage_w) {
+        if (i < LA)
+            copy_a(i < LA ? i : 0, step + SA, stage_a);
         else
-            wait_copies_and_meet<0>();
+            copy_w(i < LA ? 0 : i - LA, step + SW, stage_w);
+    };
+    // as if steps -SW .. -1 had made room: W's further stage first, and of the last of them kFirst copies
+    if constexpr (SW > SA) {
 #pragma unroll
-        for (int r = 0; r < kReads; r++) read_one(r, 0, lds, lds_w);
-        int step = 0, sa = 0, sw = 0;
-        // REST: copies of what the step before made room for are left; A, W: this step's stages are filled again; AHEAD: copies stay under
-        // way at the meeting
-        auto one_step = [&](auto rest, auto fill_a, auto fill_w, auto ahead, bool more) {
-            constexpr int kRest = decltype(rest)::value ? L - kFirst : 0;
-            constexpr int kFillA = decltype(fill_a)::value ? kFirst : 0, kFillW = decltype(fill_w)::value ? kFirst : 0;
-            const int next_a = sa + 1 < SA ? sa + 1 : 0, next_w = sw + 1 < SW ? sw + 1 : 0;
-            const int before_a = sa ? sa - 1 : SA - 1, before_w = sw ? sw - 1 : SW - 1;
-            auto phase = [&](auto which, int c0, int copies, int of_step, int stage_a, int stage_w, const uint8_t* from_sa, const uint8_t* from_sw) {
-                constexpr int P = decltype(which)::value;
-                const int all = kReads + copies;
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int o = 0; o < kOps; o++) {
-#pragma unroll
-                    for (int x = 0; x < all; x++) {
-                        if ((all <= kOps ? x : x * kOps / all) != o) continue;
-                        if (x < kReads)
-                            read_one(x, 1 - P, from_sa, from_sw);
-                        else if (P == 0 || (c0 + x - kReads < LA ? kFillA : kFillW))
-                            copy_one(c0 + x - kReads, of_step, stage_a, stage_w);
-                    }
-                    mma(acc[o / FN][o % FN], a[P][o / FN], b[P][o % FN], static_cast<T*>(nullptr));
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            };
-            phase(std::integral_constant<int, 0>{}, kFirst, kRest, step - 1, before_a, before_w, lds + sa * kStageA, lds_w + sw * kStageW);
-            if (more) {
-                __builtin_amdgcn_sched_barrier(0);
-                wait_copies_and_meet<decltype(ahead)::value ? kAfter : 0>();
-            }
-            phase(std::integral_constant<int, 1>{}, 0, kFillA > kFillW ? kFillA : kFillW, step, sa, sw, lds + next_a * kStageA, lds_w + next_w * kStageW);
-            sa = next_a, sw = next_w;
-            step++;
-        };
-        constexpr std::true_type yes;
-        constexpr std::false_type no;
-        while (step < n_steps - SW) one_step(yes, yes, yes, yes, true);
-        if constexpr (SW > SA) {  // the last rows of A are still to come, no more of W
-            static_assert(kFirst == L, "nothing is left to the next step");
-            if (whole) one_step(no, yes, no, yes, step + 1 < n_steps);
-        } else {
-            if (whole) one_step(yes, no, no, yes, step + 1 < n_steps);
-        }
-        while (step < n_steps) one_step(no, no, no, no, step + 1 < n_steps);
-    } else {
-        auto copy_step = [&](int step, int stage) {
-#pragma unroll
-            for (int i = 0; i < LA; i++) copy_a(i, step, stage);
-#pragma unroll
-            for (int i = 0; i < LB; i++) copy_w(i, step, stage);
-        };
-        for (int step = 0; step < SA - 1 && step < n_steps; step++) copy_step(step, step);
-        int stage = 0;
-        for (int step = 0; step < n_steps; step++) {
-            // the copies of the step are in LDS, later ones may be under way; and nobody still reads the stage before it
-            if (step + SA - 2 < n_steps)
-                wait_copies_and_meet<(SA - 2) * L>();
-            else
-                wait_copies_and_meet<0>();
-            if (step + SA - 1 < n_steps) copy_step(step + SA - 1, stage ? stage - 1 : SA - 1);
-            const uint8_t *sa = lds + stage * kStageA, *sw = lds_w + stage * kStageW;
-            stage = stage + 1 < SA ? stage + 1 : 0;
-#pragma unroll
-            for (int phase = 0; phase < 2; phase++) {
-#pragma unroll
-                for (int r = 0; r < kReads; r++) read_one(r, phase, sa, sw);
-#pragma unroll
-                for (int o = 0; o < kOps; o++) mma(acc[o / FN][o % FN], a[phase][o / FN], b[phase][o % FN], static_cast<T*>(nullptr));
-            }
-        }
+        for (int i = 0; i < LB; i++) copy_w(i, 0, 0);
     }
+    const bool whole = n_steps >= SW;
+    for (int step = -SA; step < 0; step++)
+#pragma unroll
+        for (int i = 0; i < L; i++)
+            if ((step < -1 || i < kFirst || !whole) && (i < LA ? step + SA : step + SW) < n_steps) copy_one(i, step, step + SA, step + SW);
+    if (whole)
+        wait_copies_and_meet<kAfter + kFirst>();
+    else
+        wait_copies_and_meet<0>();
+#pragma unroll
+    for (int r = 0; r < kReads; r++) read_one(r, 0, lds, lds_w);
+    int step = 0, sa = 0, sw = 0;
+    // REST: copies of what the step before made room for are left; A, W: this step's stages are filled again; AHEAD: copies stay under
+    // way at the meeting
+    auto one_step = [&](auto rest, auto fill_a, auto fill_w, auto ahead, bool more) {
+        constexpr int kRest = decltype(rest)::value ? L - kFirst : 0;
+        constexpr int kFillA = decltype(fill_a)::value ? kFirst : 0, kFillW = decltype(fill_w)::value ? kFirst : 0;
+        const int next_a = sa + 1 < SA ? sa + 1 : 0, next_w = sw + 1 < SW ? sw + 1 : 0;
+        const int before_a = sa ? sa - 1 : SA - 1, before_w = sw ? sw - 1 : SW - 1;
+        auto phase = [&](auto which, int c0, int copies, int of_step, int stage_a, int stage_w, const uint8_t* from_sa, const uint8_t* from_sw) {
+            constexpr int P = decltype(which)::value;
+            const int all = kReads + copies;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int o = 0; o < kOps; o++) {
+#pragma unroll
+                for (int x = 0; x < all; x++) {
+                    if ((all <= kOps ? x : x * kOps / all) != o) continue;
+                    if (x < kReads)
+                        read_one(x, 1 - P, from_sa, from_sw);
+                    else if (P == 0 || (c0 + x - kReads < LA ? kFillA : kFillW))
+                        copy_one(c0 + x - kReads, of_step, stage_a, stage_w);
+                }
+                mma(acc[o / FN][o % FN], a[P][o / FN], b[P][o % FN], static_cast<T*>(nullptr));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        phase(std::integral_constant<int, 0>{}, kFirst, kRest, step - 1, before_a, before_w, lds + sa * kStageA, lds_w + sw * kStageW);
+        if (more) {
+            __builtin_amdgcn_sched_barrier(0);
+            wait_copies_and_meet<decltype(ahead)::value ? kAfter : 0>();
+        }
+        phase(std::integral_constant<int, 1>{}, 0, kFillA > kFillW ? kFillA : kFillW, step, sa, sw, lds + next_a * kStageA, lds_w + next_w * kStageW);
+        sa = next_a, sw = next_w;
+        step++;
+    };
+    constexpr std::true_type yes;
+    constexpr std::false_type no;
+    while (step < n_steps - SW) one_step(yes, yes, yes, yes, true);
+    if constexpr (SW > SA) {  // the last rows of A are still to come, no more of W
+        static_assert(kFirst == L, "nothing is left to the next step");
+        if (whole) one_step(no, yes, no, yes, step + 1 < n_steps);
+    } else {
+        if (whole) one_step(yes, no, no, yes, step + 1 < n_steps);
+    }
+    while (step < n_steps) one_step(no, no, no, no, step + 1 < n_steps);
     store_tile<T, EPI, FM, FN>(g, heads, acc, m0, rows, wm, n0 + wn, batch);
 }
 
@@ -500,20 +472,50 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
     store_tile<T, EPI, 2, 2>(g, heads, acc, m0, rows, wave * 32, n0, batch);
 }
 
-// 256 x 256 tiles, one workgroup per CU, or 128 x 128, two per CU.  At K = 2048 a round of 256 large tiles takes 65 us whether
-// it is full or not, small tiles 44 us per 512 of them.  Over several rounds small ones overlap the end of one with the start of the
-// next, which counts where rounds are short: with exactly 768 of them a round, us with small / large, 2047 rows, 12288 x 1024 66 / 69,
-// x 2048 117 / 120, x 4096 227 / 224; 3000 rows, 8192 x 512 40.8 / 43.2, x 2048 118 / 122, x 6144 331 / 329.  With a few more they
-// begin one more round (2048 rows, 12320 x 2048, 776 a round, 131 / 125); one round, 2047 rows, 6144 x 1024 39.8 / 36.4.
-bool large_tiles_preferred(long long large, long long small, int K) {
-    const long long rounds = (large + 255) / 256;
-    return rounds * (rounds > 1 && K <= 2048 ? 769 : 750) <= small;
+// The kernels of a product without a list of tiles.  One is chosen by an estimate of its time, fitted to what each of them took.
+enum class Form { k256x256, k128x256, k128x128, k64x128, k64x64FourStages, k64x64TwoStages, kFew };
+struct FormTime {
+    Form form;
+    int rows, cols, per_cu;  // the tile, and how many of them fit a CU
+    // us: of a launch; of each tile of the CU that has most of them, and of each of the tile's steps of K; of each round of per_cu tiles a CU
+    float launch, tile, step, round, round_step;
+};
+// Fitted to 1418 products of 65 to 4074 rows, 256 to 12224 columns and 128 to 6144 of K in bfloat16, 536 of 65 to 4079, 256 to 12224 and 64
+// to 3072 in float, drawn evenly in the logarithm of each, every form timed on every product; 30 % of them were held back and come out
+// alike.  The form chosen takes 1.024 (bfloat16) and 1.014 (float) of the time of the best one for the product on average, where the
+// rules by counts of tiles that stood here before took 1.09 and 1.08; of 1014 and 491 products of 5.5 us or more, 13 and 12 take more
+// than 1.05 of the time that those rules gave them, the most 1.17 and 1.11.  On 200 and 80 more they gave 1.05 and 1.05 of what the estimate
+// gives.  One row to 64: 1.12 and 1.03.
+constexpr FormTime kTimesBf16[] = {{Form::k256x256, 256, 256, 1, 0.458f, 11.19f, 1.222f, 0, 0},
+                                   {Form::k128x256, 128, 256, 1, 0.637f, 6.33f, 0.649f, 0, 0},
+                                   {Form::k128x128, 128, 128, 1, 1.003f, 4.283f, 0.482f, 0, 0},
+                                   {Form::k64x128, 64, 128, 2, 2.251f, 1.026f, 0.245f, 0.513f, 0.051f},
+                                   {Form::kFew, 64, 32, 1, 1.338f, 1.852f, 0.199f, 0, 0},
+                                   {Form::k64x64FourStages, 64, 64, 2, 1.078f, 0.319f, 0.183f, 1.76f, 0.072f},
+                                   {Form::k64x64TwoStages, 64, 64, 5, 3.306f, 0.2f, 0.16f, 0.378f, 0.107f}};
+// The matrix ops of a step are 16 times as long in float and hide everything else: larger tiles gain nothing and round worse.
+constexpr FormTime kTimesFloat[] = {{Form::kFew, 64, 32, 1, 2.344f, 2.212f, 0.306f, 0, 0},
+                                    {Form::k64x64FourStages, 64, 64, 2, 2.612f, 0.92f, 0.44f, 0.51f, 0.073f},
+                                    {Form::k64x64TwoStages, 64, 64, 5, 3.133f, 0.784f, 0.427f, 0.017f, 0.103f}};
+
+template <size_t N>
+Form fastest_form(const FormTime (&times)[N], const GemmArgs& g, int steps) {
+    constexpr long long kCus = 256;
+    Form best{};
+    float least = INFINITY;
+    for (const FormTime& f : times) {
+        const long long tiles = (long long)((g.M + f.rows - 1) / f.rows) * ((g.N + f.cols - 1) / f.cols) * g.batches;
+        const float most = (tiles + kCus - 1) / kCus, rounds = (tiles + kCus * f.per_cu - 1) / (kCus * f.per_cu);
+        const float time = f.launch + most * (f.tile + f.step * steps) + rounds * (f.round + f.round_step * steps);
+        if (time < least) least = time, best = f.form;
+    }
+    return best;
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, bool PIPED, Epilogue EPI, typename X>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, Epilogue EPI, typename X>
 hipError_t launch_kernel(const GemmArgs& g, const X& heads, hipStream_t s) {
     const int n_mt = g.tiles ? g.max_tiles : (g.M + BM - 1) / BM, n_nt = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((dense_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, SA, SW, PIPED, EPI, X>), dim3(n_mt * n_nt, g.batches),
+    hipLaunchKernelGGL((dense_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, SA, SW, EPI, X>), dim3(n_mt * n_nt, g.batches),
                        dim3(64 * WAVES_M * WAVES_N), 0, s, g, heads);
     return hipGetLastError();
 }
@@ -534,20 +536,21 @@ hipError_t launch_grouped(const GemmArgs& g, const X& heads, hipStream_t s) {
         // 128.7 + 70.5 / 128.5 + 68.7, 1536 x 1536 74.2 + 44.8 / 74.6 + 41.3; 0.63 of two rounds full, 1024 x 1024 45.4 + 27.4 / 47.6 + 28.2.
         const int whole = g.M / kGroupTileManyRows;
         const long long tiles = (whole + g.max_tiles) / 2 * panels(256), rounds = (tiles + 255) / 256;
-        if (10 * tiles >= 7 * 256 * rounds) return launch_kernel<T, kGroupTileManyRows, 256, 2, 4, 3, 3, true, EPI>(g, heads, s);
-        return launch_kernel<T, kGroupTileManyRows, 128, 2, 2, 2, 2, true, EPI>(g, heads, s);
+        if (10 * tiles >= 7 * 256 * rounds) return launch_kernel<T, kGroupTileManyRows, 256, 2, 4, 3, 3, EPI>(g, heads, s);
+        return launch_kernel<T, kGroupTileManyRows, 128, 2, 2, 2, 2, EPI>(g, heads, s);
     }
     // 64 x 128 tiles with two stages fit a CU three times, with three stages twice and have more of the weights under way, which counts where
     // there are few rounds.  us of gate and up with two / three: 600 tokens of 4 out of 32, 2048 x 2048 82.4 / 72.3, 64 tokens 62.5 / 60.0,
     // 16 tokens, 1024 x 1024 13.4 / 10.9.  Past the line prompts of 760 to 1020 tokens at width 2048 take 0.96 to 0.98 of the time with three as
     // well; where 512 to 768 tiles are there, one round with two stages and two with three, 830 to 1020 tokens at width 1024 take 1.01 to 1.02 of it.
     if (g.N >= 1024) {
-        if (g.max_tiles * panels(128) <= 1200) return launch_kernel<T, kGroupTileRows, 128, 2, 4, 3, 3, true, EPI>(g, heads, s);
-        return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, 2, true, EPI>(g, heads, s);
+        if (g.max_tiles * panels(128) <= 1200) return launch_kernel<T, kGroupTileRows, 128, 2, 4, 3, 3, EPI>(g, heads, s);
+        return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, 2, EPI>(g, heads, s);
     }
-    // see launch_by_size: 1000 tiles, 512 x 512 14.7 us with four stages, 11.6 with two
-    if (g.max_tiles * panels(64) > 512) return launch_kernel<T, kGroupTileRows, 64, 2, 2, 2, 2, false, EPI>(g, heads, s);
-    return launch_kernel<T, kGroupTileRows, 64, 2, 2, 4, 4, false, EPI>(g, heads, s);
+    // Four stages fit a CU twice, two stages five times: past 512 tiles the first go in rounds.  kTimesBf16 has 7.0 / 7.5 us for 512 tiles
+    // of 8 steps, 11.1 / 9.0 for 513.
+    if (g.max_tiles * panels(64) > 512) return launch_kernel<T, kGroupTileRows, 64, 2, 2, 2, 2, EPI>(g, heads, s);
+    return launch_kernel<T, kGroupTileRows, 64, 2, 2, 4, 4, EPI>(g, heads, s);
 }
 
 template <typename T, Epilogue EPI, typename X>
@@ -556,36 +559,19 @@ hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
         if constexpr (EPI == Epilogue::kGatedPair || EPI == Epilogue::kFloat) return launch_grouped<T, EPI>(g, heads, s);
         return hipErrorInvalidValue;
     }
-    auto tiles = [&](int rows, int cols) { return (long long)((g.M + rows - 1) / rows) * ((g.N + cols - 1) / cols) * g.batches; };
-    // One round of a tile for each CU, three quarters full or more; a tile has the larger one's stages and waves, so that its rows and
-    // weights are under way early.  That takes some steps of K to pay: before the last of them are under way nothing fills the CU.
-    auto one_round = [&](int rows, int cols) { return g.M > 64 && tiles(rows, cols) >= 192 && tiles(rows, cols) <= 256; };
     const int steps = g.K * (int)sizeof(T) / 128;
-    if constexpr (sizeof(T) == 2)
-        if (large_tiles_preferred(tiles(256, 256), tiles(128, 128), g.K)) return launch_kernel<T, 256, 256, 2, 4, 2, 3, true, EPI>(g, heads, s);
-    // us, so / with 128 x 128 tiles: 4095 rows, 2048 x 2048 39.6 / 41.1, 2048 x 6144 106 / 109; 2048 rows, 3104 x 2048 36.3 / 40.4.
-    // Over 45 drawn shapes a type, on average: bfloat16 up to 10 steps 1.02 of the time and up to 1.075 (1854 rows, 4203 x 640 21.4 /
-    // 20.1), 11 and more 0.98; float up to 4 steps 1.05 (951 rows, 6073 x 64 16.4 / 15.2), 6 and more 0.98.
-    if (steps >= (sizeof(T) == 2 ? 11 : 6) && one_round(128, 256)) return launch_kernel<T, 128, 256, 2, 4, 3, 3, true, EPI>(g, heads, s);
-    // 2048^3: 24.8 us with twice the waves and four stages, 33 us as two a CU
-    if (one_round(128, 128)) return launch_kernel<T, 128, 128, 2, 4, 4, 4, true, EPI>(g, heads, s);
-    if (g.M > 64 && tiles(128, 128) > 256) {
-        // 300 rows, 12288 x 2048 26.7 / 36.8
-        if (one_round(64, 256)) return launch_kernel<T, 64, 256, 2, 4, 3, 3, true, EPI>(g, heads, s);
-        return launch_kernel<T, 128, 128, 2, 2, 2, 2, false, EPI>(g, heads, s);
+    Form form;
+    if constexpr (sizeof(T) == 2) form = fastest_form(kTimesBf16, g, steps);
+    else form = fastest_form(kTimesFloat, g, steps);
+    if constexpr (sizeof(T) == 2) {
+        if (form == Form::k256x256) return launch_kernel<T, 256, 256, 2, 4, 2, 3, EPI>(g, heads, s);
+        if (form == Form::k128x256) return launch_kernel<T, 128, 256, 2, 4, 3, 3, EPI>(g, heads, s);
+        if (form == Form::k128x128) return launch_kernel<T, 128, 128, 2, 4, 4, 4, EPI>(g, heads, s);
+        if (form == Form::k64x128) return launch_kernel<T, 64, 128, 2, 4, 3, 3, EPI>(g, heads, s);
     }
-    // us, so / with 64 x 64 tiles: 1024 rows, 2048 x 2048 15.2 / 16.0, x 6144 45.1 / 49.2; 600 rows, 3072 x 1536 12.2 / 13.4; 180 rows, 9216
-    // x 1536 14.6 / 16.3; over 45 drawn shapes 0.98 on average, with one and two steps 1.03 (2674 rows, 553 x 128 5.8 / 5.5)
-    if (steps > 2 && one_round(64, 128)) return launch_kernel<T, 64, 128, 2, 4, 3, 3, true, EPI>(g, heads, s);
-    // So few tiles of 64 x 32 that no CU gets a second one (us, against 64 x 64 tiles with four stages): 33 rows, 784 x 2048 7.7 /
-    // 12.5, 2048 x 6144 19 / 31; 256 rows, 2048 x 2048 10.2 / 13.5; with a second one 300 rows, 2048 x 2048 17.2 / 13.8, and 33
-    // rows, 12288 x 2048 20 / 16.
-    if (tiles(64, 32) <= 256) return launch_few<T, EPI>(g, heads, s);
-    // 64 x 64 tiles with four stages fit a CU twice, with two stages five times: more tiles than 512 would go in rounds.  bfloat16,
-    // us with four / two: 1030 rows, 544 tiles, 2048 x 1024 15.9 / 12.2, 2048 x 6144 63 / 50; in one round, 400 rows, 448 tiles, 4096 x
-    // 4096 27.5 / 34.  float, 1030 rows, 2048 x 1024: 60.5 / 56.9.
-    if (tiles(64, 64) > 512) return launch_kernel<T, 64, 64, 2, 2, 2, 2, false, EPI>(g, heads, s);
-    return launch_kernel<T, 64, 64, 2, 2, 4, 4, false, EPI>(g, heads, s);
+    if (form == Form::kFew) return launch_few<T, EPI>(g, heads, s);
+    if (form == Form::k64x64TwoStages) return launch_kernel<T, 64, 64, 2, 2, 2, 2, EPI>(g, heads, s);
+    return launch_kernel<T, 64, 64, 2, 2, 4, 4, EPI>(g, heads, s);
 }
 
 }  // namespace

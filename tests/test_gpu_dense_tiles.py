@@ -279,6 +279,26 @@ def test_rings_of_two_lengths(pkg, N, steps):
     assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
 
 
+# The tile that the estimate of times takes, in each of its forms: as few steps as lead to it and one more, ragged rows and columns: 256 x 256;
+# 128 x 256; 128 x 128; 64 x 128; 64 x 64 with four stages and with two; the last two in float
+@pytest.mark.parametrize("M,N,steps", [(4090, 4093, 3), (4090, 4093, 4), (1921, 4093, 2), (2045, 4093, 3), (1000, 3100, 8), (1025, 3100, 9),
+                                       (300, 12280, 2), (129, 6136, 3), (3000, 6136, 8), (65, 6136, 1), (65, 6136, 3), (65, 6136, 4),
+                                       (500, 4093, 5), (129, 12280, 1), (1025, 1990, 2), (2045, 8000, 3)])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_each_form_of_tile(pkg, M, N, steps, dtype):
+    import torch
+    bf16 = dtype == "bfloat16"
+    K = steps * (64 if bf16 else 32)
+    g = torch.Generator(device="cuda").manual_seed(M + steps)
+    a = torch.randn(M, K, device="cuda", generator=g).to(getattr(torch, dtype))
+    w = torch.randn(N, K, device="cuda", generator=g).to(getattr(torch, dtype))
+    got = pkg.ops.dense_gemm(a, w, K)
+    # K products (exact in bfloat16) and K sums, rounded to 24 bits
+    bound = (1 if bf16 else 2) * K * 2.0 ** -24 * 4 * K ** 0.5
+    assert (got.double() - a.double() @ w.double().t()).abs().max().item() <= bound
+    assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
+
+
 # The steps of K from which one round of 128 x 256 and of 64 x 128 tiles is taken, and those before: the same bits for a row in a call of
 # 33 rows, which goes through another kernel on either side.
 @pytest.mark.parametrize("M,N,dtype,steps", [(2045, 3100, "bfloat16", (10, 11, 12, 13)), (2045, 3100, "float32", (5, 6, 7)),
