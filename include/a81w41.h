@@ -133,6 +133,10 @@ int a81w41_gemm_schedule_selfcheck(int M, int N, int K, int resident_workgroups,
  * ranges and partial-tile slots consistent.  Returns the number of tiles shared between workgroups. */
 int a81w41_gemm_fp6_plan_selfcheck(int M, int N, int K, int resident_workgroups);
 
+/* Test hook, host only: what a one-token pass reads ahead of a layer's 320 B blocks within `room` bytes (gate | up: the launch whose
+ * output is their product).  Returns the bytes, *extent: how far into the blocks they reach. */
+long long a81w41_gemv_ahead_selfcheck(int N, int K, int gate_up, long long room, long long *extent);
+
 /* The int32 block dots both kernels form before scaling (iacc_low / iacc_high,
  * quantized_gemx_kernels.cc:161-168 and :430-457), exposed for parity checks:
  * out_dev[(m*N + n)*(K/32) + 2*sb + h], h = 0 low / 1 high 32-block.

@@ -6,6 +6,7 @@
 #include <stdlib.h>
 
 #include "chain.h"
+#include "weights_ahead.h"
 
 namespace a81w41 {
 
@@ -70,6 +71,8 @@ bool gemv_pair_fits(int N, int K);
 hipError_t launch_gemv_add_norm_silu_pair(const float* x, const GemvPrologue& pro, const void* B_gate_up, int N, int K,
                                           hipStream_t s);
 int gemv_waves_per_group_log2(int nb_n, int nb_k, bool paired_output);
+// At most `budget` bytes of what such a launch reads first: the same share of the first weights of each of its workgroups.
+WeightsAhead::Part gemv_weights_ahead(const void* B, int N, int K, bool paired_output, size_t budget);
 
 // ---- chains of overlapping launches, host side (chain.hip; the device side is in chain.h) ----------------------
 // Between chain_begin and chain_end every launch is a link: it goes to the stream chain_next names (the caller's
@@ -234,7 +237,8 @@ hipError_t launch_attention_prefill(const float* q, int q_row_stride, const void
 hipError_t launch_attention_one_token(const float* qkv, int n_q, int n_kv, const float* q_w, const float* k_w,
                                       const float* cos_t, const float* sin_t, const int* pos_dev, void* k_cache, void* v_cache,
                                       float* out, void* q_out, int max_seq, float eps, float scale, hipStream_t s,
-                                      const ChainLink* link = nullptr);  // link: the launch is a link of a chain (chain.h)
+                                      const ChainLink* link = nullptr,  // the launch is a link of a chain (chain.h)
+                                      const WeightsAhead* ahead = nullptr);  // weights read beside it; not in a chain
 // The same with the context of every head cut into `splits` (<= kAttentionMaxSplits) shares, one workgroup
 // each, for long contexts.  partials: n_q * splits * 132 floats; arrivals: n_q counters, zero before the
 // first launch (every launch leaves them zero).  Launches that share them must not overlap in time.
@@ -243,7 +247,7 @@ hipError_t launch_attention_one_token_split(const float* qkv, int n_q, int n_kv,
                                             const float* cos_t, const float* sin_t, const int* pos_dev, void* k_cache,
                                             void* v_cache, float* out, void* q_out, float* partials, unsigned* arrivals,
                                             int splits, int max_seq, float eps, float scale, hipStream_t s,
-                                            const ChainLink* link = nullptr);
+                                            const ChainLink* link = nullptr, const WeightsAhead* ahead = nullptr);
 hipError_t launch_silu_mul(const float* gate_up, float* out, int M, int inter, hipStream_t s);
 // silu(gate) * up as 80 B activation blocks of the [M][inter] result.  inter % 64 == 0, gate_up 16-byte aligned.
 hipError_t launch_silu_mul_quant(const float* gate_up, void* q_out, int M, int inter, hipStream_t s);

@@ -363,6 +363,13 @@ int a81w41_gemm_fp6_plan_selfcheck(int M, int N, int K, int resident_workgroups)
     return a81w41::gemm_fp6_plan_selfcheck(M, N, K, resident_workgroups);
 }
 
+long long a81w41_gemv_ahead_selfcheck(int N, int K, int gate_up, long long room, long long* extent) {
+    if (!shape_ok(N, K) || room < 0 || !extent) return fail(A81W41_ERR_INVALID_ARG, "bad arguments") * -100;
+    const a81w41::WeightsAhead::Part part = a81w41::gemv_weights_ahead(nullptr, N, K, gate_up != 0, (size_t)room);
+    *extent = (long long)part.extent();
+    return (long long)part.size();
+}
+
 int a81w41_gemv_repack_A80W40(const void* A_repack_dev, const void* B_repack_dev, float* C_dev, int M, int N,
                               int K, void* stream) {
     if (int st = contract_args_ok(A_repack_dev, B_repack_dev, C_dev, M, N, K)) return st;

@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "weights_ahead.h"
+
 namespace a81w41 {
 
 using bf16 = __bf16;
@@ -310,6 +312,9 @@ template <typename T>
 hipError_t launch_gemv_step_heads(const RowStep& p, const T* w, int ld, int N, const HeadRows<T>& heads, hipStream_t s);
 template <typename T>
 hipError_t launch_gemv_plain(const float* x, int K, const T* w, int ld, int N, float* C, hipStream_t s);
+// At most `room` bytes of the weights that launch_gemv_plain or launch_gemv_step reads first.
+template <typename T>
+WeightsAhead::Part gemv_rows_ahead(const T* w, int ld, int N, size_t room);
 // Queries; also the token's cache row (cache may be null) and before = sum_{j < depth.n} coef[j] states[j].
 template <typename T>
 hipError_t launch_gemv_query(const LatentRows& in, const LatentShape& sh, const T* w, int ld, float* q, T* cache, const DepthAverage& depth,
@@ -328,7 +333,7 @@ hipError_t launch_gemv_values(const float* o_lat, int ld_o, const LatentShares& 
 // [heads][ld_cache] against the rows of `cache`.
 bool latent_token_fits(const LatentShape& sh);
 hipError_t launch_latent_token(const bf16* q_lat, const LatentRows& in, const LatentShape& sh, const bf16* cache, const bf16* uv, int ld_uv,
-                               const float* gates, float* attn, hipStream_t s);
+                               const float* gates, float* attn, const WeightsAhead& ahead, hipStream_t s);
 // The feed-forwards a token uses: `top` of `experts` by table (0: none), and one every token uses (dense_ff 0: none).
 struct ExpertRows {
     const int *ids = nullptr, *table = nullptr;
@@ -345,6 +350,9 @@ struct ExpertRows {
 template <typename T>
 hipError_t launch_gemv_gate_up(const RowStep& p, const float* h, const ExpertRows& e, const T* experts, const T* dense, int ld, float* act,
                                hipStream_t s);
+// The same of what it reads of one feed-forward of `ff` units, or of `slots` experts `slot_step` elements apart.
+template <typename T>
+WeightsAhead::Part gemv_gate_up_ahead(const T* w, int ld, int ff, int slots, size_t slot_step, size_t room);
 template <typename T>
 hipError_t launch_gemv_ff_down(const ExpertRows& e, const float* act, const T* experts, int ld, const T* dense, int ld_dense, int N,
                                float* y, hipStream_t s);

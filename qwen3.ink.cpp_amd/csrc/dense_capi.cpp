@@ -83,6 +83,18 @@ int a81w41_latent_attention(const void* q, const void* cache, int ld, int rank, 
     return 0;
 }
 
+long long a81w41_dense_ahead_selfcheck(int rows, int ld, int gate_up, long long room, int is_bf16, long long* extent) {
+    if (rows < 1 || ld < 64 || ld % 64 || room < 0 || !extent) return -100 * failf(A81W41_ERR_INVALID_ARG, "bad arguments");
+    auto part_of = [&](auto type) {
+        using T = decltype(type);
+        const T* none = nullptr;
+        return gate_up ? gemv_gate_up_ahead<T>(none, ld, rows, 0, 0, (size_t)room) : gemv_rows_ahead<T>(none, ld, rows, (size_t)room);
+    };
+    const WeightsAhead::Part part = is_bf16 ? part_of(bf16{}) : part_of(0.f);
+    *extent = (long long)part.extent();
+    return (long long)part.size();
+}
+
 int a81w41_latent_token(const void* q, const void* cache, int ld, int rank, int rot, int heads, int vdim, const int* pos_dev, int max_seq,
                         float scale, const void* uv, int ld_uv, const float* gates, float* out, void* stream) {
     LatentShape sh;
@@ -93,7 +105,7 @@ int a81w41_latent_token(const void* q, const void* cache, int ld, int rank, int 
     LatentRows in;
     in.pos_dev = pos_dev, in.max_seq = max_seq;
     A81W41_HIP_TRY(launch_latent_token(static_cast<const bf16*>(q), in, sh, static_cast<const bf16*>(cache), static_cast<const bf16*>(uv), ld_uv,
-                                       gates, out, static_cast<hipStream_t>(stream)));
+                                       gates, out, WeightsAhead{}, static_cast<hipStream_t>(stream)));
     return 0;
 }
 

@@ -889,6 +889,12 @@ int workgroups(int N, int ld, int limit) {
 }
 constexpr int kMaxGrid = 1024;
 
+// Units of a workgroup's lane groups, the first ones; as many as fit.
+template <typename T>
+int lane_groups(int ld) {
+    return kThreads / lanes_of(ld * (int)sizeof(T) / 16);
+}
+
 size_t step_lds(int ld, const RowStep& p) {
     const int groups = p.norm_y.groups > p.norm_h.groups ? p.norm_y.groups : p.norm_h.groups;
     return (ld + kThreads / 64 + groups) * sizeof(float);
@@ -923,6 +929,27 @@ template <typename T>
 hipError_t launch_gemv_plain(const float* x, int K, const T* w, int ld, int N, float* C, hipStream_t s) {
     hipLaunchKernelGGL(gemv_plain_kernel<T>, dim3(workgroups<T>(N, ld, kMaxGrid)), dim3(kThreads), ld * sizeof(float), s, x, K, w, ld, N, C);
     return hipGetLastError();
+}
+template <typename T>
+WeightsAhead::Part gemv_rows_ahead(const T* w, int ld, int N, size_t room) {
+    const int rows = 2 * lane_groups<T>(ld);  // of a workgroup's round
+    WeightsAhead::Part part;
+    part.base = reinterpret_cast<const uint8_t*>(w);
+    part.step = part.bytes = (unsigned)(rows * ld * sizeof(T));
+    part.block_step = part.step;
+    part.count = (int)std::min<size_t>(N / rows, room / part.bytes);
+    return part;
+}
+template <typename T>
+WeightsAhead::Part gemv_gate_up_ahead(const T* w, int ld, int ff, int slots, size_t slot_step, size_t room) {
+    const int rows = std::min(lane_groups<T>(ld), 16);  // sixteen rows of gate and sixteen of up in turn
+    WeightsAhead::Part part;
+    part.base = reinterpret_cast<const uint8_t*>(w);
+    part.step = part.bytes = (unsigned)(rows * ld * sizeof(T));
+    part.block = 16 / rows, part.block_step = (size_t)32 * ld * sizeof(T), part.also = (size_t)16 * ld * sizeof(T);
+    part.slots = slots, part.slot_step = slot_step * sizeof(T);
+    part.count = (int)std::min<size_t>(ff / 16 * part.block, room / (2 * part.bytes * (size_t)std::max(slots, 1)));
+    return part;
 }
 template <typename T>
 hipError_t launch_gemv_query(const LatentRows& in, const LatentShape& sh, const T* w, int ld, float* q, T* cache, const DepthAverage& depth,
@@ -991,6 +1018,8 @@ hipError_t launch_gemv_mixer_down(const MixerRow& m, const T* wo, int ld_wo, con
 #define INSTANTIATE(T)                                                                                                            \
     template hipError_t launch_gemv_step<T>(const RowStep&, const T*, int, int, float*, hipStream_t);                              \
     template hipError_t launch_gemv_plain<T>(const float*, int, const T*, int, int, float*, hipStream_t);                          \
+    template WeightsAhead::Part gemv_rows_ahead<T>(const T*, int, int, size_t);                                                    \
+    template WeightsAhead::Part gemv_gate_up_ahead<T>(const T*, int, int, int, size_t, size_t);                                    \
     template hipError_t launch_gemv_query<T>(const LatentRows&, const LatentShape&, const T*, int, float*, T*, const DepthAverage&, \
                                              int, float*, hipStream_t);                                                           \
     template hipError_t launch_gemv_absorb<T>(const float*, const LatentRows&, const LatentShape&, const T*, int, T*, hipStream_t); \

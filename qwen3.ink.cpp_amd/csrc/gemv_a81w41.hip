@@ -41,6 +41,7 @@
 // and never touches the min / scaled-sum fields (that variant's writers leave them unset).
 #include "gemv_common.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 
@@ -355,6 +356,22 @@ int gemv_waves_per_group_log2(int nb_n, int nb_k, bool paired_output) {
     if (paired_output)
         while ((t.waves >> wpg_log2) > 8) wpg_log2++;
     return wpg_log2;
+}
+
+WeightsAhead::Part gemv_weights_ahead(const void* B, int N, int K, bool paired_output, size_t budget) {
+    const int nb_n = N / 8, nb_k = K / 64;
+    // groups of a workgroup's first round; of a pair the four gate groups of a workgroup, which lie together, and the four of up
+    const int groups = paired_output ? 4 : pick_tune(nb_n, nb_k).waves >> gemv_waves_per_group_log2(nb_n, nb_k, false);
+    WeightsAhead::Part part;
+    part.base = static_cast<const uint8_t*>(B);
+    part.step = (unsigned)groups * nb_k * kWBlock16;
+    part.block_step = part.step;
+    part.count = (paired_output ? nb_n / 2 : nb_n) / groups;
+    if (!part.count) return part;
+    // up too where there is room for more than all of gate
+    if (paired_output && budget > (size_t)part.count * part.step) part.also = (size_t)part.count * part.step;
+    part.bytes = (unsigned)std::min<size_t>(part.step, budget / part.count / (part.also ? 2 : 1) & ~(size_t)1023);
+    return part;
 }
 
 namespace {

@@ -1,5 +1,5 @@
 // Attention of one token in latent space over a short context, and the product with W_uv behind it, in one launch: 32 rows of a head's
-// W_uv a workgroup, each of which repeats the head's attention for itself.
+// W_uv a workgroup, each of which repeats the head's attention for itself.  Further workgroups read weights ahead (weights_ahead.h).
 //
 // What bounds it: a chain of dependent steps (query, scores, weights, merge, product) and what one CU draws at a time.  As two
 // launches (attention with two workgroups for all heads, then the product that merges their shares) the chain has another launch, two
@@ -51,7 +51,11 @@ __device__ __forceinline__ float sum8(float v) {
 __global__ __launch_bounds__(kThreads, 4) void latent_token_kernel(const bf16* __restrict__ q_lat, const bf16* __restrict__ cache, int ld,
                                                                   const int* __restrict__ pos_dev, int max_seq, int rank, int rot, int vdim,
                                                                   float scale, const bf16* __restrict__ uv, int ld_uv,
-                                                                  const float* __restrict__ gates, float* __restrict__ attn) {
+                                                                  const float* __restrict__ gates, float* __restrict__ attn, const WeightsAhead ahead) {
+    if ((int)blockIdx.y * kRows >= vdim) {
+        const int linear = blockIdx.y * gridDim.x + blockIdx.x;
+        return read_ahead<kThreads>(ahead, linear - (vdim + kRows - 1) / kRows * gridDim.x, linear);
+    }
     __shared__ __attribute__((aligned(16))) float shares[kWaves * kRank];
     __shared__ __attribute__((aligned(16))) float merged[kRank];
     __shared__ float2 stats[kWaves];
@@ -159,9 +163,10 @@ __global__ __launch_bounds__(kThreads, 4) void latent_token_kernel(const bf16* _
 bool latent_token_fits(const LatentShape& sh) { return sh.rank % 8 == 0 && sh.rank <= kRank && sh.rot > 0 && sh.rot <= kRot; }
 
 hipError_t launch_latent_token(const bf16* q_lat, const LatentRows& in, const LatentShape& sh, const bf16* cache, const bf16* uv, int ld_uv,
-                               const float* gates, float* attn, hipStream_t s) {
-    hipLaunchKernelGGL(latent_token_kernel, dim3(sh.heads, (sh.vdim + kRows - 1) / kRows), dim3(kThreads), 0, s, q_lat, cache, sh.ld_cache,
-                       in.pos_dev, in.max_seq, sh.rank, sh.rot, sh.vdim, sh.scale, uv, ld_uv, gates, attn);
+                               const float* gates, float* attn, const WeightsAhead& ahead, hipStream_t s) {
+    const int more = (ahead.workgroups() + sh.heads - 1) / sh.heads;
+    hipLaunchKernelGGL(latent_token_kernel, dim3(sh.heads, (sh.vdim + kRows - 1) / kRows + more), dim3(kThreads), 0, s, q_lat, cache, sh.ld_cache,
+                       in.pos_dev, in.max_seq, sh.rank, sh.rot, sh.vdim, sh.scale, uv, ld_uv, gates, attn, ahead);
     return hipGetLastError();
 }
 

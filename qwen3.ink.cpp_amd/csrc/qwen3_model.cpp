@@ -209,13 +209,16 @@ namespace {
 int attention_step(a81w41_qwen3* m, LayerWeights& L, float* out, void* q_out, int splits, float scale, hipStream_t s,
                    const a81w41::ChainLink* link) {
     const a81w41_qwen3_config& c = m->cfg;
+    a81w41::WeightsAhead ahead;  // what the launches behind this one read first
+    ahead.add(a81w41::gemv_weights_ahead(a81w41_linear_weight_fp16_dev(L.lin[1]), c.hidden, c.n_q_heads * kHeadDim, false, ahead.room));
+    ahead.add(a81w41::gemv_weights_ahead(a81w41_linear_weight_fp16_dev(L.lin[2]), 2 * c.intermediate, c.hidden, !m->opt_no_pair, ahead.room));
     if (splits <= 1)
         Q_HIP(a81w41::launch_attention_one_token(m->qkv, c.n_q_heads, c.n_kv_heads, L.norm[2], L.norm[3], m->cos_t, m->sin_t,
-                                                 m->pos, L.k_cache, L.v_cache, out, q_out, c.max_seq, c.rms_eps, scale, s, link));
+                                                 m->pos, L.k_cache, L.v_cache, out, q_out, c.max_seq, c.rms_eps, scale, s, link, &ahead));
     else
         Q_HIP(a81w41::launch_attention_one_token_split(m->qkv, c.n_q_heads, c.n_kv_heads, L.norm[2], L.norm[3], m->cos_t,
                                                        m->sin_t, m->pos, L.k_cache, L.v_cache, out, q_out, m->attn_part,
-                                                       m->attn_arrive, splits, c.max_seq, c.rms_eps, scale, s, link));
+                                                       m->attn_arrive, splits, c.max_seq, c.rms_eps, scale, s, link, &ahead));
     return 0;
 }
 

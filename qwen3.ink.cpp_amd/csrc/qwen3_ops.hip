@@ -485,8 +485,10 @@ __global__ __launch_bounds__(1024) void attention_one_token_kernel(const float* 
                                                                  const int* __restrict__ pos_dev, __half* __restrict__ k_cache,
                                                                  __half* __restrict__ v_cache, float* __restrict__ out,
                                                                  uint8_t* __restrict__ q_out, int max_seq, float eps,
-                                                                 float scale, const ChainLink link) {
+                                                                 float scale, const ChainLink link,
+                                                                 const WeightsAhead ahead) {
     constexpr int kWaves = 16;
+    if (!CHAIN && (int)blockIdx.x >= n_q) return read_ahead<1024>(ahead, blockIdx.x - n_q, blockIdx.x);
     extern __shared__ float sm[];  // [0, kWaves*128): the waves' weighted values; 3*128: q, new key, new value
     __shared__ float wm[kWaves], wl[kWaves];
     float* part = sm;
@@ -601,8 +603,10 @@ __global__ __launch_bounds__(1024) void attention_one_token_split_kernel(
     const float* __restrict__ qkv, int n_q, int n_kv, const float* __restrict__ q_w, const float* __restrict__ k_w,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, const int* __restrict__ pos_dev,
     __half* __restrict__ k_cache, __half* __restrict__ v_cache, float* __restrict__ out, uint8_t* __restrict__ q_out,
-    float* __restrict__ partials, unsigned* __restrict__ arrivals, int max_seq, float eps, float scale, const ChainLink link) {
+    float* __restrict__ partials, unsigned* __restrict__ arrivals, int S, int max_seq, float eps, float scale, const ChainLink link,
+    const WeightsAhead ahead) {
     constexpr int kWaves = 16;
+    if (!CHAIN && (int)blockIdx.x >= n_q * S) return read_ahead<1024>(ahead, blockIdx.x - n_q * S, blockIdx.x);
     extern __shared__ float sm[];  // [0, kWaves*128): the waves' weighted values; 3*128: q, new key, new value
     __shared__ float wm[kWaves], wl[kWaves];
     __shared__ unsigned s_arrived;
@@ -610,7 +614,7 @@ __global__ __launch_bounds__(1024) void attention_one_token_split_kernel(
     float* q_s = sm + kWaves * kHeadDim;
     float* k_new = q_s + kHeadDim;
     float* v_new = k_new + kHeadDim;
-    const int head = blockIdx.x, split = blockIdx.y, S = gridDim.y, t = threadIdx.x;
+    const int split = blockIdx.x / n_q, head = blockIdx.x - split * n_q, t = threadIdx.x;
     const int wave = t >> 6, lane = t & 63, sub = lane & 15, grp = lane >> 4;
     const int pos = min(pos_dev[0], max_seq - 1);  // rows 0..pos-1 are cached, row pos is the new token
     const int chunk = (pos + S - 1) / S;
@@ -706,7 +710,7 @@ __global__ __launch_bounds__(1024) void attention_one_token_split_kernel(
     if (t == 0) s_arrived = atomicAdd(&arrivals[head], 1u);
     __syncthreads();
     if (s_arrived != (unsigned)(S - 1)) {
-        if (CHAIN) chain_signal(link, gridDim.x * gridDim.y);
+        if (CHAIN) chain_signal(link, gridDim.x);
         return;
     }
     if (t < kHeadDim) {
@@ -729,7 +733,7 @@ __global__ __launch_bounds__(1024) void attention_one_token_split_kernel(
             out[(size_t)head * kHeadDim + t] = val;
     }
     if (t == 0) __hip_atomic_store(&arrivals[head], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-    if (CHAIN) chain_signal(link, gridDim.x * gridDim.y);
+    if (CHAIN) chain_signal(link, gridDim.x);
 }
 
 // out[m][j] = silu(gate_up[m][j]) * gate_up[m][inter + j]
@@ -837,16 +841,17 @@ hipError_t launch_attention(const float* q, int q_row_stride, const void* k_cach
 hipError_t launch_attention_one_token(const float* qkv, int n_q, int n_kv, const float* q_w, const float* k_w,
                                       const float* cos_t, const float* sin_t, const int* pos_dev, void* k_cache, void* v_cache,
                                       float* out, void* q_out, int max_seq, float eps, float scale, hipStream_t s,
-                                      const ChainLink* link) {
+                                      const ChainLink* link, const WeightsAhead* ahead) {
+    const WeightsAhead more = ahead && !link ? *ahead : WeightsAhead{};
     const size_t lds = (size_t)(16 * kHeadDim + 3 * kHeadDim) * sizeof(float);
     if (link)
         hipLaunchKernelGGL(attention_one_token_kernel<true>, dim3(n_q), dim3(1024), lds, s, qkv, n_q, n_kv, q_w, k_w, cos_t, sin_t,
                            pos_dev, static_cast<__half*>(k_cache), static_cast<__half*>(v_cache), out,
-                           static_cast<uint8_t*>(q_out), max_seq, eps, scale, *link);
+                           static_cast<uint8_t*>(q_out), max_seq, eps, scale, *link, more);
     else
-        hipLaunchKernelGGL(attention_one_token_kernel<false>, dim3(n_q), dim3(1024), lds, s, qkv, n_q, n_kv, q_w, k_w, cos_t, sin_t,
+        hipLaunchKernelGGL(attention_one_token_kernel<false>, dim3(n_q + more.workgroups()), dim3(1024), lds, s, qkv, n_q, n_kv, q_w, k_w, cos_t, sin_t,
                            pos_dev, static_cast<__half*>(k_cache), static_cast<__half*>(v_cache), out,
-                           static_cast<uint8_t*>(q_out), max_seq, eps, scale, ChainLink{});
+                           static_cast<uint8_t*>(q_out), max_seq, eps, scale, ChainLink{}, more);
     return hipGetLastError();
 }
 
@@ -854,16 +859,17 @@ hipError_t launch_attention_one_token_split(const float* qkv, int n_q, int n_kv,
                                             const float* cos_t, const float* sin_t, const int* pos_dev, void* k_cache,
                                             void* v_cache, float* out, void* q_out, float* partials, unsigned* arrivals,
                                             int splits, int max_seq, float eps, float scale, hipStream_t s,
-                                            const ChainLink* link) {
+                                            const ChainLink* link, const WeightsAhead* ahead) {
+    const WeightsAhead more = ahead && !link ? *ahead : WeightsAhead{};
     const size_t lds = (size_t)(16 * kHeadDim + 3 * kHeadDim) * sizeof(float);
     if (link)
-        hipLaunchKernelGGL(attention_one_token_split_kernel<true>, dim3(n_q, splits), dim3(1024), lds, s, qkv, n_q, n_kv, q_w, k_w,
+        hipLaunchKernelGGL(attention_one_token_split_kernel<true>, dim3(n_q * splits + more.workgroups()), dim3(1024), lds, s, qkv, n_q, n_kv, q_w, k_w,
                            cos_t, sin_t, pos_dev, static_cast<__half*>(k_cache), static_cast<__half*>(v_cache), out,
-                           static_cast<uint8_t*>(q_out), partials, arrivals, max_seq, eps, scale, *link);
+                           static_cast<uint8_t*>(q_out), partials, arrivals, splits, max_seq, eps, scale, *link, more);
     else
-        hipLaunchKernelGGL(attention_one_token_split_kernel<false>, dim3(n_q, splits), dim3(1024), lds, s, qkv, n_q, n_kv, q_w, k_w,
+        hipLaunchKernelGGL(attention_one_token_split_kernel<false>, dim3(n_q * splits + more.workgroups()), dim3(1024), lds, s, qkv, n_q, n_kv, q_w, k_w,
                            cos_t, sin_t, pos_dev, static_cast<__half*>(k_cache), static_cast<__half*>(v_cache), out,
-                           static_cast<uint8_t*>(q_out), partials, arrivals, max_seq, eps, scale, ChainLink{});
+                           static_cast<uint8_t*>(q_out), partials, arrivals, splits, max_seq, eps, scale, ChainLink{}, more);
     return hipGetLastError();
 }
 

@@ -170,7 +170,8 @@ class TakosunModel final : public DenseModel<T> {
     int attend_formed(const Layer& L, const LatentShape& sh, int M, const float* gates, hipStream_t s);
     AttendArgs<T> shared_attend(const Layer& L, const LatentShape& sh, int M) const;
     int enqueue_one_token(int n_want, hipStream_t s);
-    int attend_one_token(const Layer& L, const LatentShape& sh, const LatentRows& in, const float* gates, hipStream_t s);
+    WeightsAhead weights_behind(const Layer& L, const LayerConfig& lc) const;
+    int attend_one_token(const Layer& L, const LayerConfig& lc, const LatentRows& in, const float* gates, hipStream_t s);
     int feed_forward_one_token(const Layer& L, const LayerConfig& lc, const RowStep& step, hipStream_t s);
     LatentRows latent_rows(const Layer& L) const;
     int feed_forward(const Layer& L, const LayerConfig& lc, int M, hipStream_t s, SublayerOut* out);
@@ -513,13 +514,31 @@ int TakosunModel<T>::feed_forward_one_token(const Layer& L, const LayerConfig& l
     return 0;
 }
 
+// What the launches behind a token's attention read first.
+template <typename T>
+WeightsAhead TakosunModel<T>::weights_behind(const Layer& L, const LayerConfig& lc) const {
+    const FeedForwardConfig& f = lc.mlp;
+    WeightsAhead w;
+    w.add(gemv_rows_ahead<T>(L.o.data, L.o.ld, cfg_.width, w.room));
+    if (!f.present) return w;
+    if (!f.experts_by_table) {
+        w.add(gemv_gate_up_ahead<T>(L.ff.gate_up.data, L.ff.gate_up.ld, f.ff, 0, 0, w.room));
+        return w;
+    }
+    w.ids = ids, w.table = L.table, w.vocab = cfg_.vocab, w.top = f.top, w.experts = f.experts;
+    if (f.shared_ff) w.add(gemv_gate_up_ahead<T>(L.shared.gate_up.data, L.shared.gate_up.ld, f.shared_ff, 0, 0, w.room / (f.top + 1)));
+    w.add(gemv_gate_up_ahead<T>(L.ff.gate_up.data, L.ff.gate_up.ld, f.ff, f.top, (size_t)pair_columns(f.ff) * L.ff.gate_up.ld, w.room));
+    return w;
+}
+
 // One token's attention: its queries are in q_, its gated values go to attn_row_.
 template <typename T>
-int TakosunModel<T>::attend_one_token(const Layer& L, const LatentShape& sh, const LatentRows& in, const float* gates, hipStream_t s) {
+int TakosunModel<T>::attend_one_token(const Layer& L, const LayerConfig& lc, const LatentRows& in, const float* gates, hipStream_t s) {
+    const LatentShape& sh = lc.mix;
     A81W41_HIP_TRY(launch_gemv_absorb<T>(q_, in, sh, L.uk_t.data, L.uk_t.ld, q_lat_, s));
     if constexpr (kMatrixAttention) {
         if (!opt_attention_ && !opt_split_ && plan_ctx <= kLatentTokenKeys && latent_token_fits(sh)) {
-            A81W41_HIP_TRY(launch_latent_token(q_lat_, in, sh, L.cache, L.uv.data, L.uv.ld, gates, attn_row_, s));
+            A81W41_HIP_TRY(launch_latent_token(q_lat_, in, sh, L.cache, L.uv.data, L.uv.ld, gates, attn_row_, weights_behind(L, lc), s));
             return 0;
         }
     }
@@ -562,7 +581,7 @@ int TakosunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
         depth.states = states_, depth.state_step = state_step(), depth.coef = L.dwa, depth.n = i + 1;
         const LatentRows in = latent_rows(L);
         A81W41_HIP_TRY(launch_gemv_query<T>(in, sh, L.uq.data, L.uq.ld, q_, own ? L.cache : nullptr, depth, W, before_, s));
-        A81W41_TRY(attend_one_token(L, sh, in, down_ + sh.q_rank + (own ? sh.rank + sh.rot : 0), s));
+        A81W41_TRY(attend_one_token(L, lc, in, down_ + sh.q_rank + (own ? sh.rank + sh.rot : 0), s));
         A81W41_HIP_TRY(launch_gemv_plain<T>(attn_row_, sh.heads * sh.vdim, L.o.data, L.o.ld, W, y_, s));
         step = RowStep{};
         step.width = W, step.x = x, step.y = y_, step.norm_y = norm(L.norm1b);

@@ -159,3 +159,27 @@ def test_block_scaled_gemm_plan_covers_every_unit_once(pkg):
                 shared += got > 0
     assert shared > 50
     assert L.a81w41_gemm_fp6_plan_selfcheck(0, 64, 64, 512) < 0
+
+
+@pytest.mark.parametrize("room", [0, 5000, 1 << 20, 20 << 20, 1 << 40])
+def test_weights_read_ahead_stay_in_the_matrix(pkg, room):
+    """A one-token pass reads weights of later launches beside its attention: inside the matrix and within the room given, and all of
+    what a launch reads first where there is room for it."""
+    L = pkg.capi.lib()
+    end = C.c_longlong()
+    for K, N in [(4096, 4096), (4096, 24576), (64, 64), (64, 8), (512, 256), (12288, 4096), (1024, 40), (4096, 1088), (1536, 192), (192, 151936)]:
+        for gate_up in (0, 1):
+            got = L.a81w41_gemv_ahead_selfcheck(N, K, gate_up, room, C.byref(end))
+            assert 0 <= got <= room and got <= end.value <= N // 8 * (K // 64) * 320, (K, N, gate_up)
+            if room == 1 << 40 and N % 64 == 0:
+                assert got == N // 8 * (K // 64) * 320, (K, N, gate_up)
+    D = pkg.capi.dense()
+    for ld, rows in [(2048, 2048), (64, 1), (64, 300), (768, 3072), (1024, 17), (6144, 2048), (2048, 40), (576, 255)]:
+        for bf16 in (0, 1):
+            for gate_up in (0, 1):
+                got = D.a81w41_dense_ahead_selfcheck(rows, ld, gate_up, room, bf16, C.byref(end))
+                whole = (32 * ((rows + 15) // 16) if gate_up else rows) * ld * (2 if bf16 else 4)
+                assert 0 <= got <= room and got <= end.value and end.value <= whole, (ld, rows, bf16, gate_up)
+                if room == 1 << 40 and rows % 512 == 0:
+                    assert got == whole
+    assert L.a81w41_gemv_ahead_selfcheck(7, 64, 0, 0, C.byref(end)) < 0
