@@ -353,6 +353,14 @@ hipError_t launch_gemv_gate_up(const RowStep& p, const float* h, const ExpertRow
 // The same of what it reads of one feed-forward of `ff` units, or of `slots` experts `slot_step` elements apart.
 template <typename T>
 WeightsAhead::Part gemv_gate_up_ahead(const T* w, int ld, int ff, int slots, size_t slot_step, size_t room);
+// A token's routed experts behind h [width] and, in the same launch, its mixer: launch_memory_steps of one token, or launch_attend_rows.
+bool memory_beside_fits(const MemoryArgs& a);
+template <typename T>
+hipError_t launch_gemv_experts_and_memory(const RowStep& p, const float* h, const ExpertRows& e, const T* experts, int ld, float* act, const MemoryArgs& a,
+                                          float* o, hipStream_t s);
+bool attend_beside_fits(const AttendArgs<bf16>& a);
+hipError_t launch_gemv_experts_and_attend(const RowStep& p, const float* h, const ExpertRows& e, const bf16* experts, int ld, float* act,
+                                          const AttendArgs<bf16>& a, int kv_heads, hipStream_t s);
 template <typename T>
 hipError_t launch_gemv_ff_down(const ExpertRows& e, const float* act, const T* experts, int ld, const T* dense, int ld_dense, int N,
                                float* y, hipStream_t s);

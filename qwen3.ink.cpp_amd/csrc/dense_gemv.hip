@@ -3,7 +3,8 @@
 // then stream weight rows in pairs, 16 bytes per lane and load, the next eight loads in flight while eight are used; the
 // first ones are requested before the prologue.  A row's sum is formed
 // in an order that depends on the row's length only.
-#include "dense_common.h"
+#include "attend_rows.h"
+#include "memory_steps.h"
 
 namespace a81w41 {
 namespace {
@@ -548,8 +549,8 @@ __device__ __forceinline__ int expert_of(const ExpertRows& e, int slot) {
     return min(max(e.table[(size_t)id * e.top + slot], 0), e.experts - 1);
 }
 
-// The router's choice for one token, formed by a whole workgroup from its logits (z, best: LDS): ids[0 .. top).
-__device__ __forceinline__ void choose_experts(const ExpertRows& e, float* z, int* ids, float* best) {
+// The router's choice for one token, formed by a whole workgroup from its logits (z, best: LDS): ids[0 .. top).  The first one writes it out.
+__device__ __forceinline__ void choose_experts(const ExpertRows& e, float* z, int* ids, float* best, bool first) {
     for (int i = threadIdx.x; i < e.experts; i += kThreads) z[i] = e.logits[i] + e.bias[i];
     __syncthreads();
     for (int i = threadIdx.x; i < e.experts; i += kThreads) {
@@ -560,7 +561,7 @@ __device__ __forceinline__ void choose_experts(const ExpertRows& e, float* z, in
         }
     }
     __syncthreads();
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 64) {
+    if (first && threadIdx.x < 64) {
         const int k = threadIdx.x;
         const float w = k < e.top ? expf(best[k] - best[0]) : 0.f, sum = dense_wave_sum(w);
         if (k < e.top) {
@@ -570,18 +571,17 @@ __device__ __forceinline__ void choose_experts(const ExpertRows& e, float* z, in
     }
 }
 
-// act = unit(gate, up) for the token's experts (blockIdx.y < top) and the dense or shared feed-forward (the last).
+// act = unit(gate, up) for the token's experts (slot < top) and the dense or shared feed-forward (the last).
 template <typename T, int PARTS>
 __device__ __forceinline__ void gate_up(const RowStep& p, const float* __restrict__ h, const ExpertRows& e, const T* __restrict__ experts,
-                                        const T* __restrict__ dense, int ld, float* __restrict__ act) {
+                                        const T* __restrict__ dense, int ld, float* __restrict__ act, int slot) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     __shared__ int ids[kMaxTop];
     __shared__ float best[kMaxTop];
     float *xs = smem, *red = xs + ld, *inv = red + kThreads / 64;
-    const int slot = blockIdx.y;
     StepRow<PARTS> row(p);
     if (!h) row.load();
-    if (e.logits) choose_experts(e, red, ids, best);  // the places of red and inv are free until the row is formed
+    if (e.logits) choose_experts(e, red, ids, best, blockIdx.x == 0 && slot == 0);  // the places of red and inv are free until the row is formed
     const T* w = slot < e.top ? experts + (size_t)(e.logits ? ids[slot] : expert_of(e, slot)) * e.pair_rows * ld : dense;
     const int ff = slot < e.top ? e.ff : e.dense_ff;
     const int chunks = ld * (int)sizeof(T) / 16;
@@ -611,14 +611,56 @@ __global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(const float* __r
                                                                float* __restrict__ act) {
     with_leading(p, x, norm_h, y, norm_y, width, groups);
     e.top = top;
-    gate_up<T, PARTS>(p, nullptr, e, experts, dense, ld, act);
+    gate_up<T, PARTS>(p, nullptr, e, experts, dense, ld, act, blockIdx.y);
 }
-template <typename T>
+// What else is done beside a token's experts: its mixer where both look at the same row.  The launch's first rows of workgroups do it.
+struct NothingBeside {
+    int workgroups() const { return 0; }
+    size_t lds() const { return 0; }
+    __device__ __forceinline__ void operator()(int, float*) const {}
+};
+struct MemoryBeside {  // a matrix memory's step
+    MemoryArgs a;
+    float* o;
+    __host__ __device__ int slices() const { return (a.sh.vdim + memory::kSlice - 1) / memory::kSlice; }
+    int workgroups() const { return slices() * a.sh.heads; }
+    size_t lds() const { return memory::step_floats(a.sh.dim, 4) * sizeof(float); }
+    __device__ __forceinline__ void operator()(int n, float* smem) const {
+        const int h = n / slices();
+        if (h < a.sh.heads) memory::memory_steps<4>(a, o, n - h * slices(), h, smem);
+    }
+};
+template <int D>
+struct AttendBeside {  // attention of a few rows of a key head, key and value columns D at most each
+    static constexpr int kTile = 64;
+    AttendArgs<bf16> a;
+    int heads;
+    __host__ __device__ int groups() const { return (a.rows + 15) / 16; }
+    int workgroups() const { return groups() * heads * a.splits; }
+    size_t lds() const { return attend::attend_lds(2 * D, kTile, 1) + attend::attend_scores(1, kTile) * sizeof(float); }
+    __device__ __forceinline__ void operator()(int n, float* smem) const {
+        const int share = n / (groups() * heads), m = n - share * groups() * heads, z = m / groups();
+        uint8_t* tile = reinterpret_cast<uint8_t*>(smem);
+        if (share < a.splits)
+            attend::attend_workgroup<2 * D, D, D, 4, 1, kTile, 1, true>(a, dim3(groups(), heads, a.splits), dim3(m - z * groups(), z, share), tile,
+                                                                        reinterpret_cast<float*>(tile + attend::attend_lds(2 * D, kTile, 1)));
+    }
+};
+
+// A row that is normed already.  What bounds it behind a router: the choice, then the experts' rows from memory at a rate that the trip to them
+// limits; the token's mixer, a few workgroups of trips one behind the other, costs next to nothing beside it.  Dimesun, width 2048, behind 33 to
+// 64 tokens: attention 5.0 us and experts 12.2 in two launches, 11.8 in one; a memory's step 6.4 and 12.2, 12.4 in one.  32 tokens 7180 -> 6430 us,
+// width 1536 6200 -> 5400, 1024 4900 -> 4400, behind 1500 tokens 0.91 of the time.  Attention has one tile of keys in LDS here, where its own launch
+// has two, so that three workgroups still fit a CU; with up to eight shares of a chunk it walks few tiles.
+template <typename T, typename Beside>
 __global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(const float* __restrict__ logits, const float* __restrict__ bias, const float* __restrict__ h,
                                                                const T* __restrict__ experts, int routed, int top, int ld, int width, RowStep p,
-                                                               ExpertRows e, const T* __restrict__ dense, float* __restrict__ act) {
+                                                               ExpertRows e, const T* __restrict__ dense, float* __restrict__ act, int rows_beside,
+                                                               Beside beside) {
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    if ((int)blockIdx.y < rows_beside) return beside(blockIdx.y * gridDim.x + blockIdx.x, smem);
     e.logits = logits, e.bias = bias, e.experts = routed, e.top = top, p.width = width;
-    gate_up<T, 4>(p, h, e, experts, dense, ld, act);
+    gate_up<T, 4>(p, h, e, experts, dense, ld, act, blockIdx.y - rows_beside);
 }
 
 // y[n] = mean over the token's experts of W_e[n] . act_e, plus the dense or shared feed-forward's.
@@ -975,26 +1017,55 @@ hipError_t launch_gemv_values(const float* o_lat, int ld_o, const LatentShares& 
                        (ld + teams * shares.ld) * sizeof(float), s, o_lat, ld_o, shares, sh, uv, ld, gates, attn);
     return hipGetLastError();
 }
-template <typename T>
-hipError_t launch_gemv_gate_up(const RowStep& p, const float* h, const ExpertRows& e, const T* experts, const T* dense, int ld, float* act,
-                               hipStream_t s) {
+namespace {
+template <typename T, typename Beside>
+hipError_t launch_gate_up(const RowStep& p, const float* h, const ExpertRows& e, const T* experts, const T* dense, int ld, float* act,
+                          const Beside& beside, hipStream_t s) {
     const int most = e.top && e.ff > e.dense_ff ? e.ff : e.dense_ff;
     const int slots = e.top + (e.dense_ff ? 1 : 0);
     const size_t router = e.logits ? (ld + e.experts) * sizeof(float) : 0, lds = step_lds(ld, p);
     // behind a router a workgroup first has to learn its expert: two rounds of rows for each of the 512 that fit the chip at once
     const int limit = e.logits && slots < 16 ? 512 / slots : e.logits ? 32 : kMaxGrid;
-    const dim3 grid(workgroups<T>(2 * most, ld, limit), slots), threads(kThreads);
-    const size_t bytes = lds > router ? lds : router;
+    const int columns = workgroups<T>(2 * most, ld, limit), rows_beside = (beside.workgroups() + columns - 1) / columns;
+    const dim3 grid(columns, slots + rows_beside), threads(kThreads);
+    const size_t bytes = std::max({lds, router, beside.lds()});
     // A row that is already normed is held in no parts: the workgroups that stream behind a router are two a CU, and the larger form
     // has the registers they want.  Dimesun, a token: rows of 4096 416 us with the smaller form and 413 with the larger, 2048 both 197,
     // 1536 167.0 and 166.3, 1024 133.5 and 133.1.
     if (h)
-        hipLaunchKernelGGL(gemv_gate_up_kernel<T>, grid, threads, bytes, s, e.logits, e.bias, h, experts, e.experts, e.top, ld, p.width, p, e, dense, act);
+        hipLaunchKernelGGL((gemv_gate_up_kernel<T, Beside>), grid, threads, bytes, s, e.logits, e.bias, h, experts, e.experts, e.top, ld, p.width, p, e, dense,
+                           act, rows_beside, beside);
+    else if (rows_beside)
+        return hipErrorInvalidValue;
     else if (fits_two_parts(p))
         hipLaunchKernelGGL((gemv_gate_up_kernel<T, 2>), grid, threads, bytes, s, LEADING_OF(p), dense, p.width, p.norm_h.groups, ld, e.top, p, e, experts, act);
     else
         hipLaunchKernelGGL((gemv_gate_up_kernel<T, 4>), grid, threads, bytes, s, LEADING_OF(p), dense, p.width, p.norm_h.groups, ld, e.top, p, e, experts, act);
     return hipGetLastError();
+}
+int widest_of(const AttendArgs<bf16>& a) { return std::max(a.k_own_width, a.v_width); }
+}  // namespace
+template <typename T>
+hipError_t launch_gemv_gate_up(const RowStep& p, const float* h, const ExpertRows& e, const T* experts, const T* dense, int ld, float* act,
+                               hipStream_t s) {
+    return launch_gate_up(p, h, e, experts, dense, ld, act, NothingBeside{}, s);
+}
+bool memory_beside_fits(const MemoryArgs& a) {
+    return a.M == 1 && a.sh.vdim % 4 == 0 && memory::step_floats(a.sh.dim, 4) * sizeof(float) <= 32 * 1024;
+}
+template <typename T>
+hipError_t launch_gemv_experts_and_memory(const RowStep& p, const float* h, const ExpertRows& e, const T* experts, int ld, float* act, const MemoryArgs& a,
+                                          float* o, hipStream_t s) {
+    if (!h || !memory_beside_fits(a)) return hipErrorInvalidValue;
+    return launch_gate_up<T>(p, h, e, experts, nullptr, ld, act, MemoryBeside{a, o}, s);
+}
+bool attend_beside_fits(const AttendArgs<bf16>& a) { return a.rows <= kAttendFewRows && attend_rows_fits(a.k_own_width, a.v_width) && widest_of(a) <= 128; }
+hipError_t launch_gemv_experts_and_attend(const RowStep& p, const float* h, const ExpertRows& e, const bf16* experts, int ld, float* act,
+                                          const AttendArgs<bf16>& a, int kv_heads, hipStream_t s) {
+    if (!h || !attend_beside_fits(a)) return hipErrorInvalidValue;
+    const bf16* none = nullptr;
+    if (widest_of(a) <= 64) return launch_gate_up(p, h, e, experts, none, ld, act, AttendBeside<64>{a, kv_heads}, s);
+    return launch_gate_up(p, h, e, experts, none, ld, act, AttendBeside<128>{a, kv_heads}, s);
 }
 template <typename T>
 hipError_t launch_gemv_ff_down(const ExpertRows& e, const float* act, const T* experts, int ld, const T* dense, int ld_dense, int N,
@@ -1027,6 +1098,8 @@ hipError_t launch_gemv_mixer_down(const MixerRow& m, const T* wo, int ld_wo, con
                                               const float*, float*, hipStream_t);                                                                       \
     template hipError_t launch_gemv_gate_up<T>(const RowStep&, const float*, const ExpertRows&, const T*, const T*, int, float*,    \
                                                hipStream_t);                                                                       \
+    template hipError_t launch_gemv_experts_and_memory<T>(const RowStep&, const float*, const ExpertRows&, const T*, int, float*,             \
+                                                          const MemoryArgs&, float*, hipStream_t);                                 \
     template hipError_t launch_gemv_step_heads<T>(const RowStep&, const T*, int, int, const HeadRows<T>&, hipStream_t);             \
     template hipError_t launch_gemv_mixer_down<T>(const MixerRow&, const T*, int, const ExpertRows&, const float*, const T*, int,   \
                                                   int, float*, hipStream_t);                                                       \

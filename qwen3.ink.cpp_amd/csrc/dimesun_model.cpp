@@ -227,7 +227,8 @@ class DimesunModel final : public DenseModel<T> {
     int attention(const Layer& L, const LayerConfig& lc, const RunCache& kept, int M, hipStream_t s);
     int memory(const Layer& L, const LayerConfig& lc, const RunCache& kept, int M, hipStream_t s);
     int routed_experts(const Layer& L, const LayerConfig& lc, int M, hipStream_t s, SublayerOut* out);
-    int mixer_one_token(const Layer& L, const LayerConfig& lc, const RunCache& kept, const RowStep& step, MixerRow* out, hipStream_t s);
+    int mixer_and_experts_one_token(const Layer& L, const LayerConfig& lc, const RunCache& kept, const RowStep& step, const ExpertRows& e,
+                                    MixerRow* out, hipStream_t s);
     int enqueue_one_token(int n_want, hipStream_t s);
 
     Config cfg_;
@@ -496,18 +497,29 @@ int DimesunModel<T>::routed_experts(const Layer& L, const LayerConfig& lc, int M
     return 0;
 }
 
-// A mixer for one token behind the residual step `step`; the router's logits go to in_.
+// A mixer and the routed experts (e.top of them) for one token behind the residual step `step`; the router's logits go to in_.  The experts look at the
+// same row as the mixer does, so that a mixer of a few workgroups runs in their launch: a Dimesun token has a launch a layer less.
 template <typename T>
-int DimesunModel<T>::mixer_one_token(const Layer& L, const LayerConfig& lc, const RunCache& kept, const RowStep& step, MixerRow* out,
-                                     hipStream_t s) {
+int DimesunModel<T>::mixer_and_experts_one_token(const Layer& L, const LayerConfig& lc, const RunCache& kept, const RowStep& step, const ExpertRows& e,
+                                                 MixerRow* out, hipStream_t s) {
+    const GatedWeights<T>& W = L.experts;
+    auto experts_alone = [&]() -> int {
+        if (e.top) A81W41_HIP_TRY(launch_gemv_gate_up<T>(step, h_row_, e, W.gate_up.data, nullptr, W.gate_up.ld, act_row_, s));
+        return 0;
+    };
     out->width = lc.mixer_width();
     out->row = mixer_row_;
     if (lc.memory) {
         const MemoryShape& sh = lc.mem;
         A81W41_HIP_TRY(launch_gemv_step<T>(step, L.in.data, L.in.ld, L.in.rows, in_, s));
-        A81W41_HIP_TRY(launch_memory_steps(memory_args(L, sh, kept, lc.row_stride(), 1), mixer_row_, s));
         out->heads = sh.heads, out->vdim = sh.vdim, out->norm = L.memory_norm, out->gates = in_ + sh.at_g, out->eps = sh.eps;
-        return 0;
+        const MemoryArgs a = memory_args(L, sh, kept, lc.row_stride(), 1);
+        if (e.top && memory_beside_fits(a)) {
+            A81W41_HIP_TRY(launch_gemv_experts_and_memory<T>(step, h_row_, e, W.gate_up.data, W.gate_up.ld, act_row_, a, mixer_row_, s));
+            return 0;
+        }
+        A81W41_HIP_TRY(launch_memory_steps(a, mixer_row_, s));
+        return experts_alone();
     }
     const AttentionConfig& c = lc.att;
     A81W41_HIP_TRY(launch_gemv_step_heads<T>(step, L.in.data, L.in.ld, L.in.rows, head_rows(L, c, kept, in_, lc.row_stride()), s));
@@ -516,13 +528,17 @@ int DimesunModel<T>::mixer_one_token(const Layer& L, const LayerConfig& lc, cons
     if constexpr (kMatrixAttention) {
         if (opt_attention_ != 1 && attend_rows_fits(c.key_width(), c.value_width())) {
             a.splits = std::max(2, std::min(a.splits, kMixerShares));  // shares stay fp32; the output product merges them
-            A81W41_HIP_TRY(launch_attend_rows(a, c.kv_heads, s));
             out->shares = LatentShares{a.part, a.part_stats, a.splits, a.ld_part};
-            return 0;
+            if (e.top && attend_beside_fits(a)) {
+                A81W41_HIP_TRY(launch_gemv_experts_and_attend(step, h_row_, e, W.gate_up.data, W.gate_up.ld, act_row_, a, c.kv_heads, s));
+                return 0;
+            }
+            A81W41_HIP_TRY(launch_attend_rows(a, c.kv_heads, s));
+            return experts_alone();
         }
     }
     A81W41_HIP_TRY((launch_attend_vector<T, float>(a, c.kv_heads, mixer_row_, s)));
-    return 0;
+    return experts_alone();
 }
 
 // The pass for one token, four launches a run: [residual step, norm, product of all that reads the norm], the mixer, [choice
@@ -538,14 +554,13 @@ int DimesunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
         const LayerConfig& lc = cfg_.layers[cfg_.runs[i].layer];
         step.before = step_of(i), step.x_out = row_x_[i & 1], step.h_out = h_row_;
         MixerRow mixed;
-        A81W41_TRY(mixer_one_token(L, lc, kept_[i], step, &mixed, s));
         ExpertRows e;
         if (lc.routed) {
             e.top = lc.moe.top, e.experts = lc.moe.experts, e.ff = lc.moe.ff, e.pair_rows = pair_columns(lc.moe.ff), e.ld_act = ld_act_row_;
             e.unit = GatedUnit{lc.moe.limit, 1.702f, 1.f};
             e.logits = lc.memory ? in_ + lc.mixer_columns() : in_, e.bias = L.router_bias, e.chosen = chosen_, e.weights = expert_weights_;
-            A81W41_HIP_TRY(launch_gemv_gate_up<T>(step, h_row_, e, L.experts.gate_up.data, nullptr, L.experts.gate_up.ld, act_row_, s));
         }
+        A81W41_TRY(mixer_and_experts_one_token(L, lc, kept_[i], step, e, &mixed, s));
         A81W41_HIP_TRY(launch_gemv_mixer_down<T>(mixed, L.o.data, L.o.ld, e, act_row_, L.experts.down.data, L.experts.down.ld, W, y_, s));
         step = RowStep{};
         step.width = W, step.x = row_x_[i & 1], step.y = y_, step.norm_y = residual(), step.norm_h = norm(next_norm(i));

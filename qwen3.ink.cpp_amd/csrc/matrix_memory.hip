@@ -8,26 +8,14 @@
 //   S_t^T q_t = e^(m_0 - M_t) S_0^T q_t + sum_{s <= t} e^(a_s - M_t) (q_t . k_s) v_s
 // so that a chunk needs S only at its start.  Three launches: every chunk's own sum over s for t = its last token (outer
 // products, all chunks at once); the chain over chunks, element by element; the outputs of all chunks.
-#include "dense_common.h"
+#include "memory_steps.h"
 
 namespace a81w41 {
 namespace {
 
-constexpr int kThreads = 256, C = kMemoryChunk;
+using namespace memory;
+constexpr int C = kMemoryChunk;
 static_assert(C == 64, "the lanes of a wave hold a chunk's gates");
-
-__device__ __forceinline__ float soft_cap(float z, float cap) { return cap * tanhf(z / cap); }
-__device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
-struct Gates {
-    float log_in, log_keep;
-};
-__device__ __forceinline__ Gates gates_of(const MemoryArgs& a, int m, int h) {
-    const float* row = a.in + (size_t)m * a.ld_in;
-    Gates g;
-    g.log_in = soft_cap(row[a.sh.at_i + h] + a.bias_i[h], a.sh.cap);
-    g.log_keep = log_sigmoid(soft_cap(row[a.sh.at_f + h] + a.bias_f[h], a.sh.cap));
-    return g;
-}
 
 __device__ __forceinline__ double shfl_up(double v, int by) {
     const long long u = __double_as_longlong(v);
@@ -56,85 +44,11 @@ __device__ __forceinline__ ChunkGates chunk_gates(const MemoryArgs& p, int m0, i
     return c;
 }
 
-__device__ __forceinline__ float* state_nm(const MemoryArgs& a, int parity) {
-    return a.state + a.sh.s_size() + (size_t)(parity & 1) * a.sh.heads * (a.sh.dim + 1);
-}
-
-// Token by token.  A workgroup has kSlice columns of one head's S; W columns and every (kThreads W / kSlice)-th row of them
-// are a thread's, in registers only while a token uses them.  n and m are formed by every workgroup of the head; the first
-// writes them to the copy that nobody reads.
-constexpr int kSlice = 32;
+// Token by token (memory_steps.h).
 template <int W>
 __global__ __launch_bounds__(kThreads) void memory_steps_kernel(MemoryArgs a, float* __restrict__ o) {
-    constexpr int kPer = kSlice / W, kRows = kThreads / kPer;  // threads of a row of the slice, rows worked on at a time
     extern __shared__ float smem[];
-    const MemoryShape sh = a.sh;
-    float *n = smem, *q = n + sh.dim, *k = q + sh.dim, *sums = k + sh.dim, *red = sums + kRows * kSlice;
-    const int t = threadIdx.x, h = blockIdx.y, pos = max(a.pos_dev[0], 0);
-    const int c = blockIdx.x * kSlice + (t % kPer) * W, r0 = t / kPer;
-    const bool mine = c < sh.vdim;  // W > 1: vdim is a multiple of W
-    float* S = a.state + (size_t)h * sh.dim * sh.vdim;
-    const float* nm = state_nm(a, pos) + (size_t)h * (sh.dim + 1);
-    for (int d = t; d < sh.dim; d += kThreads) n[d] = nm[d];
-    float m = nm[sh.dim];
-    for (int token = 0; token < a.M; token++) {
-        const float* row = a.in + (size_t)token * a.ld_in;
-        const Gates g = gates_of(a, token, h);
-        const float next = fmaxf(g.log_keep + m, g.log_in), keep = expf(g.log_keep + m - next), add = expf(g.log_in - next);
-        m = next;
-        float nq = 0.f;
-        for (int d = t; d < sh.dim; d += kThreads) {
-            q[d] = row[sh.at_q + h * sh.dim + d] * sh.q_scale;
-            k[d] = add * row[sh.at_k + h * sh.dim + d];
-            n[d] = fmaf(keep, n[d], k[d]);
-            nq = fmaf(n[d], q[d], nq);
-        }
-        nq = dense_wave_sum(nq);
-        if ((t & 63) == 0) red[t >> 6] = nq;
-        __syncthreads();
-        float acc[W], v[W];
-#pragma unroll
-        for (int w = 0; w < W; w++) {
-            acc[w] = 0.f;
-            v[w] = mine ? row[sh.at_v + h * sh.vdim + c + w] : 0.f;
-        }
-        if (mine) {
-#pragma unroll 8
-            for (int d = r0; d < sh.dim; d += kRows) {
-                float* at = S + (size_t)d * sh.vdim + c;
-                float s[W];
-                if constexpr (W == 4)
-                    *reinterpret_cast<float4*>(s) = load4(at);
-                else
-                    s[0] = at[0];
-#pragma unroll
-                for (int w = 0; w < W; w++) {
-                    s[w] = fmaf(keep, s[w], k[d] * v[w]);
-                    acc[w] = fmaf(s[w], q[d], acc[w]);
-                }
-                if constexpr (W == 4)
-                    store4(at, *reinterpret_cast<const float4*>(s));
-                else
-                    at[0] = s[0];
-            }
-        }
-#pragma unroll
-        for (int w = 0; w < W; w++) sums[r0 * kSlice + (t % kPer) * W + w] = acc[w];
-        __syncthreads();
-        const int col = blockIdx.x * kSlice + t;
-        if (t < kSlice && col < sh.vdim) {
-            float s = 0.f, den = 0.f;
-            for (int r = 0; r < kRows; r++) s += sums[r * kSlice + t];
-            for (int w = 0; w < kThreads / 64; w++) den += red[w];
-            o[((size_t)token * sh.heads + h) * sh.vdim + col] = s / (fmaxf(fabsf(den), expf(-m)) + kMemoryFloor);
-        }
-        __syncthreads();
-    }
-    if (blockIdx.x == 0) {
-        float* out = state_nm(a, pos + a.M) + (size_t)h * (sh.dim + 1);
-        for (int d = t; d < sh.dim; d += kThreads) out[d] = n[d];
-        if (t == 0) out[sh.dim] = m;
-    }
+    memory_steps<W>(a, o, blockIdx.x, blockIdx.y, smem);
 }
 
 // One workgroup per token.
@@ -587,7 +501,7 @@ hipError_t launch_chunks(const MemoryArgs& a, T* out, int ld_out, hipStream_t s)
 
 hipError_t launch_memory_steps(const MemoryArgs& a, float* o, hipStream_t s) {
     const dim3 grid((a.sh.vdim + kSlice - 1) / kSlice, a.sh.heads);
-    auto lds = [&](int w) { return (3 * (size_t)a.sh.dim + kThreads * w + kThreads / 64) * sizeof(float); };
+    auto lds = [&](int w) { return step_floats(a.sh.dim, w) * sizeof(float); };
     if (a.sh.vdim % 4 == 0)
         hipLaunchKernelGGL(memory_steps_kernel<4>, grid, dim3(kThreads), lds(4), s, a, o);
     else

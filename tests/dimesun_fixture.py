@@ -76,6 +76,15 @@ LARGE = config(64, 128, [
 # heads and memories past the matrix-core kernels' sizes
 HUGE = config(64, 64, [attention(2, 1, 264, 16, 30, 0.06, mlp=moe(2, 1, 24)), mlstm(1, 16, 520, mlp=moe(3, 2, 8)),
                        attention(2, 2, 8, 264, 13, 0.3, mlp=None)], (2, 3, 2))
+# mixers that run beside their experts for one token, by key and value columns up to 64 and 128, with two groups of query rows, over
+# two and three tiles of keys and more, and mixers that do not fit there
+BESIDE = config(67, 64, [
+    attention(17, 1, 24, 36, 130, 0.2, rot_dims=8, mlp=moe(5, 5, 40)),
+    attention(4, 2, 128, 72, 210, 0.1, mlp=moe(3, 3, 24)),
+    mlstm(2, 24, 36, mlp=moe(4, 4, 24)),
+    attention(2, 1, 136, 16, 64, 0.1, mlp=moe(2, 2, 16)),
+    mlstm(1, 12, 30, mlp=moe(3, 2, 8)),
+], (0, 1, 1))
 # rows that the row kernels do not hold in registers, and too long for the one-token pass
 LONG_ROWS = config(43, 4200, [attention(1, 1, 8, 8, 6, 0.4, mlp=moe(2, 1, 16)), mlstm(1, 8, 8, mlp=moe(2, 2, 16))], (0, 1, 2))
 MANY_VALUES = config(43, 64, [mlstm(40, 8, 400, mlp=moe(2, 1, 16)), attention(3, 1, 8, 8, 6, 0.4, mlp=None)], (1, 2, 2), eps=0.1)

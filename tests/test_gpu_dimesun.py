@@ -10,12 +10,12 @@ import numpy as np
 import pytest
 
 from oracle import dimesun_forward as df
-from tests.dimesun_fixture import (HUGE, LARGE, LONG_ROWS, MANY_VALUES, ODD, SMALL, TOL, WIDE, Truth, attention, config, mlstm, moe,
-                                   row_errors, write_model)
+from tests.dimesun_fixture import (BESIDE, HUGE, LARGE, LONG_ROWS, MANY_VALUES, ODD, SMALL, TOL, WIDE, Truth, attention, config, mlstm,
+                                   moe, row_errors, write_model)
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-CONFIGS = {"small": SMALL, "odd": ODD, "wide": WIDE, "large": LARGE, "huge": HUGE, "long_rows": LONG_ROWS, "many_values": MANY_VALUES}
+CONFIGS = {"small": SMALL, "odd": ODD, "wide": WIDE, "large": LARGE, "huge": HUGE, "long_rows": LONG_ROWS, "many_values": MANY_VALUES, "beside": BESIDE}
 OPTIONS = ("unfused", "attention", "attention_split", "memory", "keep_states")
 
 
@@ -285,6 +285,16 @@ def last_portion(n, sizes):
         last = min(sizes[min(k, len(sizes) - 1)], n)
         n, k = n - last, k + 1
     return last
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("split", [0, 1, 2, 7])
+def test_mixers_beside_experts(built, dtype, split):
+    """One token at a time over the edges of key tiles and chunks, the mixer in the experts' launch where it fits there."""
+    model, oracle, _ = built("beside", dtype)
+    t = truth("beside", oracle, 215)
+    model.set_option("attention_split", split)
+    close(feed(model, t.ids, [62, 1, 1, 1, 1, 60, 1, 1, 1, 1, 1, 1, 1, 1, 57, 1]), t.logits, t.limits[dtype])
 
 
 @pytest.mark.parametrize("name", ["wide", "large"])
