@@ -306,7 +306,7 @@ struct RowStep {
     int width = 0;
 };
 template <typename T>
-hipError_t launch_gemv_step(const RowStep& p, const T* w, int ld, int N, float* C, hipStream_t s);
+hipError_t launch_gemv_step(const RowStep& p, const T* w, int ld, int N, float* C, hipStream_t s, const WeightsAhead& ahead = {});
 // The product's columns are stored as HeadRows says.
 template <typename T>
 hipError_t launch_gemv_step_heads(const RowStep& p, const T* w, int ld, int N, const HeadRows<T>& heads, hipStream_t s);

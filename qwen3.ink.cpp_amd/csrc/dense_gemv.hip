@@ -290,8 +290,12 @@ __device__ __forceinline__ void with_leading(RowStep& p, const float* x, const f
 template <typename T, int PARTS, typename Emit>
 __global__ __launch_bounds__(kThreads) void gemv_step_kernel(const float* __restrict__ x, const float* __restrict__ norm_h, const float* __restrict__ y,
                                                             const float* __restrict__ norm_y, const T* __restrict__ w, int width, int groups, int ld,
-                                                            int N, RowStep p, Emit emit) {
+                                                            int N, RowStep p, Emit emit, WeightsAhead later) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    if (blockIdx.y) {  // behind the launch's own workgroups
+        const int n = (blockIdx.y - 1) * gridDim.x + blockIdx.x;
+        return read_ahead<kThreads>(later, (gridDim.y - 1) * gridDim.x, n, gridDim.x + n);
+    }
     with_leading(p, x, norm_h, y, norm_y, width, groups);
     float *xs = smem, *red = xs + ld, *inv = red + kThreads / 64;
     StepRow<PARTS> row(p);
@@ -947,25 +951,28 @@ size_t step_lds(int ld, const RowStep& p) {
 // 9.5 us.  Forcing the larger form into registers for four spills and is slower (gate and up 14.4 -> 19.6 us).
 bool fits_two_parts(const RowStep& p) { return RowParts<kThreads, 2>(p.width, p.norm_h.groups, 0).fits(); }
 
+constexpr int kReadAhead = 400;  // workgroups that read ahead beside a small product; multiples of its own
+
 template <typename T, typename Emit>
-hipError_t launch_step(const RowStep& p, const T* w, int ld, int N, const Emit& emit, hipStream_t s) {
-    const dim3 grid(workgroups<T>(N, ld, kMaxGrid)), threads(kThreads);
+hipError_t launch_step(const RowStep& p, const T* w, int ld, int N, const Emit& emit, const WeightsAhead& ahead, hipStream_t s) {
+    const int own = workgroups<T>(N, ld, kMaxGrid);
+    const dim3 grid(own, 1 + (ahead.parts ? (kReadAhead + own - 1) / own : 0)), threads(kThreads);
     if (fits_two_parts(p))
-        hipLaunchKernelGGL((gemv_step_kernel<T, 2, Emit>), grid, threads, step_lds(ld, p), s, LEADING_OF(p), w, p.width, p.norm_h.groups, ld, N, p, emit);
+        hipLaunchKernelGGL((gemv_step_kernel<T, 2, Emit>), grid, threads, step_lds(ld, p), s, LEADING_OF(p), w, p.width, p.norm_h.groups, ld, N, p, emit, ahead);
     else
-        hipLaunchKernelGGL((gemv_step_kernel<T, 4, Emit>), grid, threads, step_lds(ld, p), s, LEADING_OF(p), w, p.width, p.norm_h.groups, ld, N, p, emit);
+        hipLaunchKernelGGL((gemv_step_kernel<T, 4, Emit>), grid, threads, step_lds(ld, p), s, LEADING_OF(p), w, p.width, p.norm_h.groups, ld, N, p, emit, ahead);
     return hipGetLastError();
 }
 
 }  // namespace
 
 template <typename T>
-hipError_t launch_gemv_step(const RowStep& p, const T* w, int ld, int N, float* C, hipStream_t s) {
-    return launch_step(p, w, ld, N, PlainEmit{C, N, 1.f}, s);
+hipError_t launch_gemv_step(const RowStep& p, const T* w, int ld, int N, float* C, hipStream_t s, const WeightsAhead& ahead) {
+    return launch_step(p, w, ld, N, PlainEmit{C, N, 1.f}, ahead, s);
 }
 template <typename T>
 hipError_t launch_gemv_step_heads(const RowStep& p, const T* w, int ld, int N, const HeadRows<T>& heads, hipStream_t s) {
-    return launch_step(p, w, ld, N, HeadsEmit<T>{heads, N}, s);
+    return launch_step(p, w, ld, N, HeadsEmit<T>{heads, N}, WeightsAhead{}, s);
 }
 template <typename T>
 hipError_t launch_gemv_plain(const float* x, int K, const T* w, int ld, int N, float* C, hipStream_t s) {
@@ -1087,7 +1094,7 @@ hipError_t launch_gemv_mixer_down(const MixerRow& m, const T* wo, int ld_wo, con
 }
 
 #define INSTANTIATE(T)                                                                                                            \
-    template hipError_t launch_gemv_step<T>(const RowStep&, const T*, int, int, float*, hipStream_t);                              \
+    template hipError_t launch_gemv_step<T>(const RowStep&, const T*, int, int, float*, hipStream_t, const WeightsAhead&);         \
     template hipError_t launch_gemv_plain<T>(const float*, int, const T*, int, int, float*, hipStream_t);                          \
     template WeightsAhead::Part gemv_rows_ahead<T>(const T*, int, int, size_t);                                                    \
     template WeightsAhead::Part gemv_gate_up_ahead<T>(const T*, int, int, int, size_t, size_t);                                    \

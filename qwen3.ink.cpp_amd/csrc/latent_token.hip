@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kThreads, 4) void latent_token_kernel(const bf16* _
                                                                   const float* __restrict__ gates, float* __restrict__ attn, const WeightsAhead ahead) {
     if ((int)blockIdx.y * kRows >= vdim) {
         const int linear = blockIdx.y * gridDim.x + blockIdx.x;
-        return read_ahead<kThreads>(ahead, linear - (vdim + kRows - 1) / kRows * gridDim.x, linear);
+        return read_ahead<kThreads>(ahead, WeightsAhead::kWorkgroups, linear - (vdim + kRows - 1) / kRows * gridDim.x, linear);
     }
     __shared__ __attribute__((aligned(16))) float shares[kWaves * kRank];
     __shared__ __attribute__((aligned(16))) float merged[kRank];

@@ -488,7 +488,7 @@ __global__ __launch_bounds__(1024) void attention_one_token_kernel(const float* 
                                                                  float scale, const ChainLink link,
                                                                  const WeightsAhead ahead) {
     constexpr int kWaves = 16;
-    if (!CHAIN && (int)blockIdx.x >= n_q) return read_ahead<1024>(ahead, blockIdx.x - n_q, blockIdx.x);
+    if (!CHAIN && (int)blockIdx.x >= n_q) return read_ahead<1024>(ahead, WeightsAhead::kWorkgroups, blockIdx.x - n_q, blockIdx.x);
     extern __shared__ float sm[];  // [0, kWaves*128): the waves' weighted values; 3*128: q, new key, new value
     __shared__ float wm[kWaves], wl[kWaves];
     float* part = sm;
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(1024) void attention_one_token_split_kernel(
     float* __restrict__ partials, unsigned* __restrict__ arrivals, int S, int max_seq, float eps, float scale, const ChainLink link,
     const WeightsAhead ahead) {
     constexpr int kWaves = 16;
-    if (!CHAIN && (int)blockIdx.x >= n_q * S) return read_ahead<1024>(ahead, blockIdx.x - n_q * S, blockIdx.x);
+    if (!CHAIN && (int)blockIdx.x >= n_q * S) return read_ahead<1024>(ahead, WeightsAhead::kWorkgroups, blockIdx.x - n_q * S, blockIdx.x);
     extern __shared__ float sm[];  // [0, kWaves*128): the waves' weighted values; 3*128: q, new key, new value
     __shared__ float wm[kWaves], wl[kWaves];
     __shared__ unsigned s_arrived;

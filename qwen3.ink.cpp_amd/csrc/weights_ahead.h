@@ -49,13 +49,12 @@ struct WeightsAhead {
 };
 
 #if defined(__HIPCC__)
-// Workgroup `index` of the additional ones, workgroup `linear` of the launch, of THREADS threads.  A wave takes 4 KB of a unit at a time.
+// Workgroup `index` of `workgroups` additional ones, workgroup `linear` of the launch, of THREADS threads.  A wave takes 4 KB of a unit at a time.
 template <int THREADS>
-__device__ __forceinline__ void read_ahead(const WeightsAhead& w, int index, int linear) {
+__device__ __forceinline__ void read_ahead(const WeightsAhead& w, int workgroups, int index, int linear) {
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     constexpr int kLoads = 4, kWaves = THREADS / 64;
-    constexpr int turns = WeightsAhead::kWorkgroups / 8;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int turns = workgroups >> 3, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (index >> 3 >= turns) return;
     int n = (index >> 3) * kWaves + wave;
     for (int p = 0; p < w.parts; p++) {
