@@ -209,7 +209,10 @@ namespace {
 int attention_step(a81w41_qwen3* m, LayerWeights& L, float* out, void* q_out, int splits, float scale, hipStream_t s,
                    const a81w41::ChainLink* link) {
     const a81w41_qwen3_config& c = m->cfg;
-    a81w41::WeightsAhead ahead;  // what the launches behind this one read first
+    // What the launches behind this one read first.  Not beside four shares and more, which use the memory themselves: 64 tokens behind
+    // 700 (three shares) 17530 us without, 17220 with; behind 2000 (four) 21660 and 21770, width 2048 behind 1500 11550 and 11700.
+    a81w41::WeightsAhead ahead;
+    if (splits > 3) ahead.room = 0;
     ahead.add(a81w41::gemv_weights_ahead(a81w41_linear_weight_fp16_dev(L.lin[1]), c.hidden, c.n_q_heads * kHeadDim, false, ahead.room));
     ahead.add(a81w41::gemv_weights_ahead(a81w41_linear_weight_fp16_dev(L.lin[2]), 2 * c.intermediate, c.hidden, !m->opt_no_pair, ahead.room));
     if (splits <= 1)
