@@ -56,6 +56,9 @@ int a81w41_matrix_memory(const float *in, int ld_in, int M, int heads, int dim, 
 /* chosen [M][top]: the largest of logits [M][ld] (first `experts` columns) + bias, largest first; weights [M][top]: the softmax
  * over them. */
 int a81w41_router(const float *logits, int ld, const float *bias, int experts, int top, int M, int *chosen, float *weights, void *stream);
+/* Test hook, host only: the kernel that a81w41_dense_gemm or _gated takes: tiles of 0: 256 x 256, 1: 128 x 256, 2: 128 x 128, 3: 64 x 128, 64 x 64 with
+ * 4: four stages of K, 5: two, 6: 64 x 32; 7: 128 x 128 for strides past 32-bit offsets. */
+int a81w41_dense_form_selfcheck(int M, int N, int K, int lda, int ldw, int bf16);
 /* Test hook, host only: what a one-token pass reads ahead of a matrix [rows][ld] within `room` bytes (gate_up: of `rows` units, sixteen
  * rows of gate and sixteen of up in turn).  Returns the bytes, *extent: how far into the matrix they reach. */
 long long a81w41_dense_ahead_selfcheck(int rows, int ld, int gate_up, long long room, int bf16, long long *extent);

@@ -114,6 +114,7 @@ DENSE_SIGNATURES = {
     "a81w41_matrix_memory_state": (_sz, [_i, _i, _i]),
     "a81w41_matrix_memory_scratch": (_sz, [_i, _i, _i, _i]),
     "a81w41_matrix_memory": (_i, [_vp, _i, _i, _i, _i, _i, C.c_float, C.c_float, _vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp]),
+    "a81w41_dense_form_selfcheck": (_i, [_i, _i, _i, _i, _i, _i]),
     "a81w41_dense_ahead_selfcheck": (C.c_longlong, [_i, _i, _i, C.c_longlong, _i, C.POINTER(C.c_longlong)]),
     "a81w41_router": (_i, [_vp, _i, _vp, _i, _i, _i, _vp, _vp, _vp]),
 }

@@ -85,6 +85,10 @@ struct GroupTile {
 // width 1024, units of 512, 256 rows 40.6 / 27.4 and 45.8 / 27.6.
 constexpr int kGroupTileRows = 64, kGroupTileManyRows = 128;
 inline int group_tile_rows(long long rows, int experts) { return rows >= 128LL * experts ? kGroupTileManyRows : kGroupTileRows; }
+constexpr int kPassRows = 4096;  // tokens of one pass; longer portions are cut
+// The kernels of a product without a list of tiles: rows and columns of a tile; k64x64 with four stages of K in LDS and with two; kFew: 64 x 32;
+// kWide: 128 x 128 and 64-bit offsets, for any stride.
+enum class GemmForm { k256x256, k128x256, k128x128, k64x128, k64x64FourStages, k64x64TwoStages, kFew, kWide };
 struct GemmArgs {
     const void* A = nullptr;  // [M][lda], or gathered: row r of the product is row a_rows[r] of A
     const void* W = nullptr;  // [N][ldw]
@@ -106,6 +110,7 @@ struct GemmArgs {
         tiles = list, n_tiles = n, tile_rows = group_tile_rows(M, experts), max_tiles = M / tile_rows + (experts < M ? experts : M);
     }
 };
+GemmForm dense_gemm_form(const GemmArgs& g, bool is_bf16);  // that a launch takes
 template <typename T>
 hipError_t launch_dense_gemm(const GemmArgs& g, Epilogue epi, hipStream_t s);
 template <typename T>

@@ -83,6 +83,14 @@ int a81w41_latent_attention(const void* q, const void* cache, int ld, int rank, 
     return 0;
 }
 
+int a81w41_dense_form_selfcheck(int M, int N, int K, int lda, int ldw, int is_bf16) {
+    const int step = is_bf16 ? 64 : 32;
+    if (M < 1 || N < 1 || K < 1 || lda % step || ldw % step || lda < K || ldw < K) return -100 * failf(A81W41_ERR_INVALID_ARG, "bad product");
+    GemmArgs g;
+    g.M = M, g.N = N, g.K = is_bf16 ? pad_k<bf16>(K) : pad_k<float>(K), g.lda = lda, g.ldw = ldw;
+    return (int)dense_gemm_form(g, is_bf16 != 0);
+}
+
 long long a81w41_dense_ahead_selfcheck(int rows, int ld, int gate_up, long long room, int is_bf16, long long* extent) {
     if (rows < 1 || ld < 64 || ld % 64 || room < 0 || !extent) return -100 * failf(A81W41_ERR_INVALID_ARG, "bad arguments");
     auto part_of = [&](auto type) {

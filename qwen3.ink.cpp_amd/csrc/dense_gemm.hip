@@ -12,6 +12,7 @@
 // the CU's way to its caches for 1000 clocks; with branches around copies and 64-bit addresses 2530.  16 x 16 pieces take 3 to 5 % less than 32 x 32 at equal clocks.  Then
 // the weights' first trip: tiles whose LDS has room take W a stage further ahead than A.  us, so / as bursts: 4095 x 12288 x 2048 in bfloat16
 // 159 / 194, gated 168 / 203, 4095 x 2048 x 6144 82 / 105, x 2048 33 / 40, 2048^3 20.4 / 24.4, 8192^3 750 / 940 (1.47 PFLOP/s; the library 145, -, 83, 34, 21, 670).
+#include <algorithm>
 #include <type_traits>
 
 #include "dense_common.h"
@@ -228,7 +229,8 @@ constexpr int kBandRows = 2048;
 // Reads and copies go one by one between the matrix ops, kFirst of a stage's copies in that second phase and the rest in the next step's
 // first; requested in a row they kept every wave of the CU waiting for its turn at the caches while the matrix cores idled.  That holds where
 // a CU has several workgroups as well: 64 x 64 tiles with a step's copies in a row took 1.2 to 1.3 times as long.
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, Epilogue EPI, typename X>
+// WIDE: rows by 64-bit offsets, for strides with which a tile's rows reach past 4 GB.
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, Epilogue EPI, typename X, bool WIDE>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(GemmArgs g, X heads) {
     constexpr int kThreads = 64 * WAVES_M * WAVES_N;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, FM = WM / 16, FN = WN / 16;
@@ -263,26 +265,33 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N, 2) void dense_gemm_kernel(G
         rows = g.M - m0;
     }
     const int n0 = nt * BN;
-    // A tile's rows by 32-bit offsets from the first; gathered rows from the start of A, which models keep under 4 GB
+    // A tile's rows by offsets from the first, in 32 bits where tile_offsets_fit; gathered rows from the start of A
+    using Offset = std::conditional_t<WIDE, size_t, unsigned>;
     const T* const A = static_cast<const T*>(g.A) + (g.tiles ? 0 : batch * g.a_step) + (g.a_rows ? 0 : (size_t)m0 * g.lda);
     const T* const W = static_cast<const T*>(g.W) + batch * g.w_step + (size_t)n0 * g.ldw;
     const CopySource from_a = copy_source(A), from_w = copy_source(W);
-    unsigned a_at[LA], w_at[LB];
+    Offset a_at[LA], w_at[LB];
 #pragma unroll
     for (int i = 0; i < LA; i++) {
         const int c = i * kThreads + tid, r = c >> 3, row = min(r, rows - 1);
-        a_at[i] = (unsigned)(g.a_rows ? g.a_rows[m0 + row] : row) * (g.lda * (unsigned)sizeof(T)) + (((c & 7) ^ place_of_row(r)) << 4);
+        a_at[i] = (Offset)(g.a_rows ? g.a_rows[m0 + row] : row) * (g.lda * (Offset)sizeof(T)) + (((c & 7) ^ place_of_row(r)) << 4);
     }
 #pragma unroll
     for (int i = 0; i < LB; i++) {
         const int c = i * kThreads + tid, r = c >> 3;
-        w_at[i] = (unsigned)min(r, g.N - 1 - n0) * (g.ldw * (unsigned)sizeof(T)) + (((c & 7) ^ place_of_row(r)) << 4);
+        w_at[i] = (Offset)min(r, g.N - 1 - n0) * (g.ldw * (Offset)sizeof(T)) + (((c & 7) ^ place_of_row(r)) << 4);
     }
+    auto copy = [&](const T* base, CopySource from, uint8_t* to, Offset at, int step) {
+        if constexpr (WIDE)
+            copy16_to_lds(reinterpret_cast<const uint8_t*>(base) + at + (size_t)step * 128, to);
+        else
+            copy16_to_lds(from, to, at, step * 128);
+    };
     auto copy_a = [&](int i, int step, int stage) {
-        copy16_to_lds(from_a, lds + stage * kStageA + wave * 1024 + i * kThreads * 16, a_at[i], step * 128);
+        copy(A, from_a, lds + stage * kStageA + wave * 1024 + i * kThreads * 16, a_at[i], step);
     };
     auto copy_w = [&](int i, int step, int stage) {
-        copy16_to_lds(from_w, lds_w + stage * kStageW + wave * 1024 + i * kThreads * 16, w_at[i], step * 128);
+        copy(W, from_w, lds_w + stage * kStageW + wave * 1024 + i * kThreads * 16, w_at[i], step);
     };
     f32x4 acc[FM][FN];
 #pragma unroll
@@ -472,8 +481,14 @@ __global__ __launch_bounds__(384, 1) void dense_gemm_few_kernel(GemmArgs g, X he
     store_tile<T, EPI, 2, 2>(g, heads, acc, m0, rows, wave * 32, n0, batch);
 }
 
+// Whether the rows of any tile, 256 x 256 at most, lie within the 32 bits of its copies' offsets.  Rows that a_rows gathers are among a pass's.
+bool tile_offsets_fit(const GemmArgs& g, size_t element) {
+    const size_t rows_a = g.a_rows ? kPassRows : std::min(g.M, 256), rows_w = std::min(g.N, 256);
+    return std::max(rows_a * g.lda, rows_w * g.ldw) * element < (size_t)1 << 32;
+}
+
 // The kernels of a product without a list of tiles.  One is chosen by an estimate of its time, fitted to what each of them took.
-enum class Form { k256x256, k128x256, k128x128, k64x128, k64x64FourStages, k64x64TwoStages, kFew };
+using Form = GemmForm;
 struct FormTime {
     Form form;
     int rows, cols, per_cu;  // the tile, and how many of them fit a CU
@@ -512,10 +527,10 @@ Form fastest_form(const FormTime (&times)[N], const GemmArgs& g, int steps) {
     return best;
 }
 
-template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, Epilogue EPI, typename X>
+template <typename T, int BM, int BN, int WAVES_M, int WAVES_N, int SA, int SW, Epilogue EPI, bool WIDE = false, typename X>
 hipError_t launch_kernel(const GemmArgs& g, const X& heads, hipStream_t s) {
     const int n_mt = g.tiles ? g.max_tiles : (g.M + BM - 1) / BM, n_nt = (g.N + BN - 1) / BN;
-    hipLaunchKernelGGL((dense_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, SA, SW, EPI, X>), dim3(n_mt * n_nt, g.batches),
+    hipLaunchKernelGGL((dense_gemm_kernel<T, BM, BN, WAVES_M, WAVES_N, SA, SW, EPI, X, WIDE>), dim3(n_mt * n_nt, g.batches),
                        dim3(64 * WAVES_M * WAVES_N), 0, s, g, heads);
     return hipGetLastError();
 }
@@ -553,16 +568,23 @@ hipError_t launch_grouped(const GemmArgs& g, const X& heads, hipStream_t s) {
     return launch_kernel<T, kGroupTileRows, 64, 2, 2, 4, 4, EPI>(g, heads, s);
 }
 
+template <typename T>
+Form form_of(const GemmArgs& g) {
+    const int steps = g.K * (int)sizeof(T) / 128;
+    if (!tile_offsets_fit(g, sizeof(T))) return Form::kWide;
+    if constexpr (sizeof(T) == 2) return fastest_form(kTimesBf16, g, steps);
+    else return fastest_form(kTimesFloat, g, steps);
+}
+
 template <typename T, Epilogue EPI, typename X>
 hipError_t launch_by_size(const GemmArgs& g, const X& heads, hipStream_t s) {
+    // strides of 16 MB and more; a list's tiles of 64 rows fit those of 128
+    if (!tile_offsets_fit(g, sizeof(T))) return launch_kernel<T, 128, 128, 2, 2, 2, 2, EPI, true>(g, heads, s);
     if (g.tiles) {
         if constexpr (EPI == Epilogue::kGatedPair || EPI == Epilogue::kFloat) return launch_grouped<T, EPI>(g, heads, s);
         return hipErrorInvalidValue;
     }
-    const int steps = g.K * (int)sizeof(T) / 128;
-    Form form;
-    if constexpr (sizeof(T) == 2) form = fastest_form(kTimesBf16, g, steps);
-    else form = fastest_form(kTimesFloat, g, steps);
+    const Form form = form_of<T>(g);
     if constexpr (sizeof(T) == 2) {
         if (form == Form::k256x256) return launch_kernel<T, 256, 256, 2, 4, 2, 3, EPI>(g, heads, s);
         if (form == Form::k128x256) return launch_kernel<T, 128, 256, 2, 4, 3, 3, EPI>(g, heads, s);
@@ -602,5 +624,7 @@ hipError_t launch_dense_gemm_queries(const GemmArgs& g, const LatentQueries<T>& 
     template hipError_t launch_dense_gemm_queries<T>(const GemmArgs&, const LatentQueries<T>&, hipStream_t);
 INSTANTIATE(bf16)
 INSTANTIATE(float)
+
+GemmForm dense_gemm_form(const GemmArgs& g, bool is_bf16) { return is_bf16 ? form_of<bf16>(g) : form_of<float>(g); }
 
 }  // namespace a81w41

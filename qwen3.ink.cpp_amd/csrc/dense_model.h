@@ -15,7 +15,6 @@
 
 namespace a81w41 {
 
-constexpr int kPassRows = 4096;  // tokens of one pass; longer portions are cut
 
 inline void require(bool ok, const std::string& what) {
     if (!ok) throw std::runtime_error(what);

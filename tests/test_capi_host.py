@@ -183,3 +183,17 @@ def test_weights_read_ahead_stay_in_the_matrix(pkg, room):
                 if room == 1 << 40 and rows % 512 == 0:
                     assert got == whole
     assert L.a81w41_gemv_ahead_selfcheck(7, 64, 0, 0, C.byref(end)) < 0
+
+
+def test_strides_past_32_bit_offsets_have_a_kernel(pkg):
+    """Tiles up to 256 rows copy by 32-bit offsets; strides with which a tile's rows reach 4 GB go to the kernel with 64-bit ones."""
+    form = pkg.capi.dense().a81w41_dense_form_selfcheck
+    for bf16, step, size in ((0, 32, 4), (1, 64, 2)):
+        for rows in (1, 65, 256, 4000):
+            last = ((1 << 32) // size // min(rows, 256) - 1) // step * step   # the widest stride whose rows end before 4 GB
+            last = min(last, (1 << 31) - step)                              # strides are ints
+            for more, far in ((0, False), (step, min(rows, 256) * (last + step) * size >= 1 << 32)):
+                if last + more < 1 << 31:
+                    assert (form(rows, 8, step, last + more, step, bf16) == 7) == far, (bf16, rows, more)
+                    assert (form(8, rows, step, step, last + more, bf16) == 7) == far, (bf16, rows, more)
+    assert form(1, 1, 64, 100, 64, 1) < 0

@@ -299,6 +299,26 @@ def test_each_form_of_tile(pkg, M, N, steps, dtype):
     assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
 
 
+# Rows so far apart that a tile's reach past 4 GB: of A, of W, of W with gated units.
+@pytest.mark.parametrize("dtype,M,N,lda,ldw", [("float32", 65, 6136, 17_100_000, 64), ("bfloat16", 130, 300, 128, 8_400_000),
+                                               ("bfloat16", 257, 288, 8_388_608, 64)])
+def test_rows_far_apart(pkg, dtype, M, N, lda, ldw):
+    import torch
+    bf16 = dtype == "bfloat16"
+    K, g = 64, torch.Generator(device="cuda").manual_seed(M)
+    assert pkg.capi.dense().a81w41_dense_form_selfcheck(M, N, K, lda, ldw, bf16) == 7
+    near = [torch.randn(n, K, device="cuda", generator=g).to(getattr(torch, dtype)) for n in (M, N)]
+    a, w = far = [torch.empty(n, ld, device="cuda", dtype=near[0].dtype) for n, ld in ((M, lda), (N, ldw))]
+    for x, y in zip(far, near):
+        x[:, :K] = y
+    got = pkg.ops.dense_gemm(a, w, K)
+    # K products (exact in bfloat16) and K sums, rounded to 24 bits
+    assert (got.double() - near[0].double() @ near[1].double().t()).abs().max().item() <= 2 * K * 2.0 ** -24 * 4 * K ** 0.5
+    assert torch.equal(pkg.ops.dense_gemm(near[0], near[1], K), got)
+    if N % 32 == 0:
+        assert torch.equal(pkg.ops.dense_gated(near[0], near[1], K), pkg.ops.dense_gated(a, w, K))
+
+
 # The steps of K from which one round of 128 x 256 and of 64 x 128 tiles is taken, and those before: the same bits for a row in a call of
 # 33 rows, which goes through another kernel on either side.
 @pytest.mark.parametrize("M,N,dtype,steps", [(2045, 3100, "bfloat16", (10, 11, 12, 13)), (2045, 3100, "float32", (5, 6, 7)),
