@@ -277,6 +277,7 @@ struct MemoryArgs {
     MemoryShape sh;
     const float* in = nullptr;  // [M][ld_in]
     int ld_in = 0, M = 0;
+    int ahead = 0;  // step by step: tokens behind pos_dev's that are in the state already
     const float *bias_i = nullptr, *bias_f = nullptr;  // [heads]
     const float* norm = nullptr;                       // [heads vdim]
     float* state = nullptr;

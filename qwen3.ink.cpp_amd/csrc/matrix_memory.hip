@@ -499,8 +499,16 @@ hipError_t launch_chunks(const MemoryArgs& a, T* out, int ld_out, hipStream_t s)
 
 }  // namespace
 
-hipError_t launch_memory_steps(const MemoryArgs& a, float* o, hipStream_t s) {
+hipError_t launch_memory_steps(const MemoryArgs& all, float* o, hipStream_t s) {
+    MemoryArgs a = all;
     const dim3 grid((a.sh.vdim + kSlice - 1) / kSlice, a.sh.heads);
+    // Workgroups that start late may not find n and m overwritten (memory_steps.h): of an even number of tokens the last has a launch
+    // of its own.
+    if (grid.x > 1 && a.M % 2 == 0) {
+        a.M--;
+        if (hipError_t e = launch_memory_steps(a, o, s)) return e;
+        a.ahead += a.M, a.in += (size_t)a.M * a.ld_in, o += (size_t)a.M * a.sh.heads * a.sh.vdim, a.M = 1;
+    }
     auto lds = [&](int w) { return step_floats(a.sh.dim, w) * sizeof(float); };
     if (a.sh.vdim % 4 == 0)
         hipLaunchKernelGGL(memory_steps_kernel<4>, grid, dim3(kThreads), lds(4), s, a, o);

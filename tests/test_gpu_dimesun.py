@@ -203,6 +203,24 @@ def test_matrix_memory_halves_of_a_chunk(pkg, heads, dim, vdim, T):
     close(got, want, 5e-5, (T, heads, dim, vdim))   # as test_matrix_memory: sums of 32-bit products of up to 97 tokens
 
 
+@pytest.mark.parametrize("sizes", [[2], [4, 2], [1, 6], [3, 2, 1]])
+@pytest.mark.parametrize("heads,dim,vdim", [(64, 8, 1100), (96, 5, 1025)])
+def test_matrix_memory_steps_in_even_portions(pkg, heads, dim, vdim, sizes):
+    """More workgroups than run at a time, so that some start when others of their head are done: each has to start from the n and m before
+    the portion."""
+    import torch
+    cap, eps, T = 15.0, 0.3, sum(sizes)
+    assert heads * -(-vdim // 32) > 256 * 8   # eight workgroups of 256 threads fill a CU
+    rows, bi, bf, norm = _memory_rows(T, heads, dim, vdim, dim + T, *GATES["mixed"])
+    want = _memory_reference(rows, heads, dim, vdim, cap, eps, bi, bf, norm)
+    dev = [torch.from_numpy(x).cuda() for x in (bi, bf, norm)]
+    state, out, at = pkg.ops.matrix_memory_state(heads, dim, vdim), [], 0
+    for n in sizes:
+        out.append(pkg.ops.matrix_memory(torch.from_numpy(rows[at:at + n]).cuda(), heads, dim, vdim, cap, eps, *dev, state, at, 0).cpu().numpy())
+        at += n
+    close(np.concatenate(out), want, 5e-5, sizes)   # as test_matrix_memory
+
+
 def test_matrix_memory_finds_a_far_token(pkg):
     """One key among hundreds is asked for again, across chunks and portions: a lost or decayed state would not have it."""
     import torch
