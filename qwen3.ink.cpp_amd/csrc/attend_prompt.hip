@@ -326,14 +326,20 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
     if (a.head_gate) inv *= sigmoid(gate);
     bf16* dst = a.out + z * a.out_head + (size_t)my_token * a.out_token + (my_row - my_token * a.rows_per_token) * a.ld_out;
     const bool real = wave_row0 + l31 < a.rows;
-    // Eight neighbouring columns a lane: of two fours the halves of a row trade one.
-    const bool whole = ((a.dv | a.ld_out | a.out_token) & 7) == 0 && (a.out_head & 7) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
+    // Eight neighbouring columns a lane, of two fours the halves of a row trade one; or fours, or single columns, as widths and the target
+    // allow.  us of a call, fours / single columns: 16 heads of 192 + 124, 4095 rows 127 / 138; 16 heads on 4 of 128 + 124, 2048 rows 45 / 51.
+    const auto starts = [&](int together) {
+        return ((a.dv | a.ld_out | a.out_token) & (together - 1)) == 0 && (a.out_head & (together - 1)) == 0 &&
+               (reinterpret_cast<uintptr_t>(a.out) & (together * sizeof(bf16) - 1)) == 0;
+    };
+    const bool eights = starts(8), fours = starts(4);
     typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 #pragma unroll
     for (int f = 0; f < VF; f++)
 #pragma unroll
         for (int v = 0; v < 16; v += 8) {
-            if (whole) {
+            if (eights) {
                 unsigned first[2], second[2];
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
@@ -344,6 +350,13 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
                 }
                 const int d = 32 * f + 2 * v + 8 * half;
                 if (real && d < a.dv) *reinterpret_cast<lds16*>(dst + d) = lds16{first[0], first[1], second[0], second[1]};
+            } else if (fours) {
+#pragma unroll
+                for (int i = 0; i < 8; i += 4) {
+                    const int d = 32 * f + 2 * (v + i) + 4 * half;
+                    const bf16x4 x = {(bf16)(acc[f][v + i] * inv), (bf16)(acc[f][v + i + 1] * inv), (bf16)(acc[f][v + i + 2] * inv), (bf16)(acc[f][v + i + 3] * inv)};
+                    if (real && d < a.dv) *reinterpret_cast<bf16x4*>(dst + d) = x;
+                }
             } else {
 #pragma unroll
                 for (int i = 0; i < 8; i++) {

@@ -105,7 +105,8 @@ def _grouped_reference(q, k, v, pos, scale, chunk, sink):
 @pytest.mark.parametrize("M,heads,kv_heads,dim,vdim,pos,chunk", [
     (1, 4, 2, 24, 40, 0, 7), (1, 6, 1, 64, 64, 255, 64), (1, 16, 2, 128, 128, 256, 64), (1, 8, 1, 128, 96, 300, 128), (1, 40, 2, 96, 96, 190, 0),
     (2, 3, 3, 8, 16, 62, 63), (3, 20, 5, 136, 256, 200, 100), (5, 12, 4, 64, 8, 130, 1), (40, 6, 1, 56, 120, 0, 11), (65, 2, 2, 128, 64, 33, 32),
-    (130, 8, 2, 64, 64, 127, 65), (200, 5, 1, 200, 136, 0, 0), (90, 4, 4, 264, 272, 10, 40), (150, 6, 2, 72, 128, 64, 128)])
+    (130, 8, 2, 64, 64, 127, 65), (200, 5, 1, 200, 136, 0, 0), (90, 4, 4, 264, 272, 10, 40), (150, 6, 2, 72, 128, 64, 128),
+    (70, 6, 2, 64, 60, 3, 0), (90, 4, 1, 128, 124, 0, 64), (40, 4, 2, 200, 252, 5, 0)])
 @pytest.mark.parametrize("sink", [True, False])
 def test_grouped_attention(pkg, M, heads, kv_heads, dim, vdim, pos, chunk, sink):
     import torch

@@ -132,7 +132,8 @@ def test_latent_attention(pkg, M, heads, rank, rot, pos):
 
 @pytest.mark.parametrize("M,heads,dim,rot,vdim,pos", [
     (1, 2, 16, 8, 24, 0), (64, 3, 64, 16, 64, 0), (65, 2, 128, 64, 128, 63), (130, 1, 40, 24, 33, 200), (200, 2, 192, 64, 256, 1),
-    (129, 2, 56, 8, 128, 64), (17, 5, 24, 8, 7, 300)])
+    (129, 2, 56, 8, 128, 64), (17, 5, 24, 8, 7, 300),
+    (33, 3, 24, 8, 12, 0), (70, 2, 128, 64, 124, 10), (129, 1, 192, 64, 252, 5)])   # values that are stored four columns at a time
 def test_formed_attention(pkg, M, heads, dim, rot, vdim, pos):
     import torch
     rng = np.random.default_rng(5)
