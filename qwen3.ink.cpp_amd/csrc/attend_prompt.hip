@@ -322,10 +322,16 @@ __global__ __launch_bounds__(64 * KG * QW, KG * QW / 4) void attend_prompt_kerne
             }
         return;
     }
+    // The lane's row, formed again: a register that holds any of it over the loop costs the widest expanded form its second set of value
+    // operands, and a wait goes by with every product.  us of a call, so / held: 8 heads of 256 + 256 columns, 330 rows 50.6 / 52.0, 2000 rows
+    // 173.6 / 180; 16 heads of 320 + 256, 4000 rows 354 / 367; the other forms are level.
+    int out_lane = l31;
+    asm volatile("" : "+v"(out_lane));
+    const int out_row = min(wave_row0 + out_lane, a.rows - 1), out_token = out_row / a.rows_per_token;
     float inv = 1.0f / sum;
     if (a.head_gate) inv *= sigmoid(gate);
-    bf16* dst = a.out + z * a.out_head + (size_t)my_token * a.out_token + (my_row - my_token * a.rows_per_token) * a.ld_out;
-    const bool real = wave_row0 + l31 < a.rows;
+    bf16* dst = a.out + z * a.out_head + (size_t)out_token * a.out_token + (out_row - out_token * a.rows_per_token) * a.ld_out;
+    const bool real = wave_row0 + out_lane < a.rows;
     // Eight neighbouring columns a lane, of two fours the halves of a row trade one; or fours, or single columns, as widths and the target
     // allow.  us of a call, fours / single columns: 16 heads of 192 + 124, 4095 rows 127 / 138; 16 heads on 4 of 128 + 124, 2048 rows 45 / 51.
     const auto starts = [&](int together) {
@@ -387,7 +393,7 @@ hipError_t launch_attend_rows_prompt(const AttendArgs<bf16>& a, int heads, hipSt
     return launch_kernel<512, 256, 256, 1, kQW, 64, false>(a, heads, s);
 }
 
-// The widest form takes all 512 registers and spills 50 of them, addresses of copies, whose reloads wait for the copies before.  It is
+// The widest form takes all 512 registers and spills 45 of them, addresses of copies, whose reloads wait for the copies before.  It is
 // the faster one all the same (us, against 16 x 16): 8 heads, 192 + 64 and 256 columns, 330 rows 36 / 51, 2000 rows 159 / 212.
 hipError_t launch_attend_expanded(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
     const int dk = a.k_own_width + a.k_shared_width;
