@@ -504,34 +504,42 @@ struct FormTime {
     int rows, cols, per_cu;  // the tile, and how many of them fit a CU
     // us: of a launch; of each tile of the CU that has most of them, and of each of the tile's steps of K; of each round of per_cu tiles a CU
     float launch, tile, step, round, round_step;
+    // more of a step's time where one row of tiles streams weights whose rows are whole multiples of 4 KB apart and meet in the same channels of the
+    // caches: 1 row, 32768 x 4096 61 us with 64 x 128 tiles, 53 with 64 x 64; 30241 x 6336 72 and 71
+    float aligned;
 };
-// Fitted to 1418 products of 65 to 4074 rows, 256 to 12224 columns and 128 to 6144 of K in bfloat16, 536 of 65 to 4079, 256 to 12224 and 64
-// to 3072 in float, drawn evenly in the logarithm of each, every form timed on every product; 30 % of them were held back and come out
-// alike.  The form chosen takes 1.024 (bfloat16) and 1.014 (float) of the time of the best one for the product on average, where the
-// rules by counts of tiles that stood here before took 1.09 and 1.08; of 1014 and 491 products of 5.5 us or more, 13 and 12 take more
-// than 1.05 of the time that those rules gave them, the most 1.17 and 1.11.  On 200 and 80 more they gave 1.05 and 1.05 of what the estimate
-// gives.  One row to 64: 1.12 and 1.03.
-constexpr FormTime kTimesBf16[] = {{Form::k256x256, 256, 256, 1, 0.458f, 11.19f, 1.222f, 0, 0},
-                                   {Form::k128x256, 128, 256, 1, 0.637f, 6.33f, 0.649f, 0, 0},
-                                   {Form::k128x128, 128, 128, 1, 1.003f, 4.283f, 0.482f, 0, 0},
-                                   {Form::k64x128, 64, 128, 2, 2.251f, 1.026f, 0.245f, 0.513f, 0.051f},
-                                   {Form::kFew, 64, 32, 1, 1.338f, 1.852f, 0.199f, 0, 0},
-                                   {Form::k64x64FourStages, 64, 64, 2, 1.078f, 0.319f, 0.183f, 1.76f, 0.072f},
-                                   {Form::k64x64TwoStages, 64, 64, 5, 3.306f, 0.2f, 0.16f, 0.378f, 0.107f}};
+// Fitted to what every form took on 3402 products of 1 to 4096 rows, 64 to 65536 columns and 64 to 12288 of K in bfloat16 and 2101 of 1 to 4096,
+// 64 to 16384 and 32 to 8192 in float, the weights from memory as a pass finds them; about half of them drawn evenly in the logarithm of each size, the
+// rest with the whole multiples of 256 and 512 that models have.  The form chosen takes 1.003 (bfloat16) and 1.001 (float) of the time of the best one
+// for the product on average, 61 and 5 of them more than 1.05 of it; a fit to two thirds does as well on the other third.
+constexpr FormTime kTimesBf16[] = {{Form::k256x256, 256, 256, 1, 0.372f, 9.751f, 0.889f, 0, 0, 0.7f},
+                                   {Form::k128x256, 128, 256, 1, 0.116f, 5.816f, 0.599f, 0, 0, 1.04f},
+                                   {Form::k128x128, 128, 128, 1, 0.729f, 4.659f, 0.397f, 0, 0, 0.64f},
+                                   {Form::k64x128, 64, 128, 2, 2.947f, 1.193f, 0.261f, 0.064f, 0.076f, 1.1f},
+                                   {Form::kFew, 64, 32, 1, 1.397f, 1.887f, 0.163f, 0, 0, 0.05f},
+                                   {Form::k64x64FourStages, 64, 64, 2, 1.556f, 0.263f, 0.153f, 1.98f, 0.06f, 0.47f},
+                                   {Form::k64x64TwoStages, 64, 64, 5, 3.121f, 0.194f, 0.155f, 0.352f, 0.122f, 1.03f}};
 // The matrix ops of a step are 16 times as long in float and hide everything else: larger tiles gain nothing and round worse.
-constexpr FormTime kTimesFloat[] = {{Form::kFew, 64, 32, 1, 2.344f, 2.212f, 0.306f, 0, 0},
-                                    {Form::k64x64FourStages, 64, 64, 2, 2.612f, 0.92f, 0.44f, 0.51f, 0.073f},
-                                    {Form::k64x64TwoStages, 64, 64, 5, 3.133f, 0.784f, 0.427f, 0.017f, 0.103f}};
+constexpr FormTime kTimesFloat[] = {{Form::kFew, 64, 32, 1, 0.322f, 2.436f, 0.504f, 0, 0, 0},
+                                    {Form::k64x64FourStages, 64, 64, 2, 2.612f, 0.922f, 0.44f, 0.486f, 0.073f, 0},
+                                    {Form::k64x64TwoStages, 64, 64, 5, 3.134f, 0.774f, 0.427f, 0.029f, 0.103f, 0}};
 
 template <size_t N>
-Form fastest_form(const FormTime (&times)[N], const GemmArgs& g, int steps) {
+Form fastest_form(const FormTime (&times)[N], const GemmArgs& g, size_t element) {
     constexpr long long kCus = 256;
+    const int steps = g.K * (int)element / 128;
+    const bool aligned = g.M <= 64 && g.ldw * element % 4096 == 0;
     Form best{};
     float least = INFINITY;
     for (const FormTime& f : times) {
         const long long tiles = (long long)((g.M + f.rows - 1) / f.rows) * ((g.N + f.cols - 1) / f.cols) * g.batches;
+        // What no term of it says: over long K five to sixteen rows of 64 x 128 tiles that leave three eighths of the CUs without one are slower than
+        // 64 x 64.  13 such products, 64 x 64 / 64 x 128: 0.90 on average, from 0.78 to 1.06; 500 rows, 2112 x 4096 24.7 / 31.1 us, 800 rows, 1536 x 4608
+        // 27.6 / 34.9.
+        if (f.form == Form::k64x128 && tiles <= 160 && steps >= 32 && g.M > 256 && g.M <= 1024) continue;
         const float most = (tiles + kCus - 1) / kCus, rounds = (tiles + kCus * f.per_cu - 1) / (kCus * f.per_cu);
-        const float time = f.launch + most * (f.tile + f.step * steps) + rounds * (f.round + f.round_step * steps);
+        const float of_steps = steps * (aligned ? 1 + f.aligned : 1);
+        const float time = f.launch + most * (f.tile + f.step * of_steps) + rounds * (f.round + f.round_step * of_steps);
         if (time < least) least = time, best = f.form;
     }
     return best;
@@ -572,18 +580,17 @@ hipError_t launch_grouped(const GemmArgs& g, const X& heads, hipStream_t s) {
         if (g.max_tiles * panels(128) <= 1200) return launch_kernel<T, kGroupTileRows, 128, 2, 4, 3, 3, EPI>(g, heads, s);
         return launch_kernel<T, kGroupTileRows, 128, 2, 2, 2, 2, EPI>(g, heads, s);
     }
-    // Four stages fit a CU twice, two stages five times: past 512 tiles the first go in rounds.  kTimesBf16 has 7.0 / 7.5 us for 512 tiles
-    // of 8 steps, 11.1 / 9.0 for 513.
+    // Four stages fit a CU twice, two stages five times: past 512 tiles the first go in rounds.  kTimesBf16 has 7.0 / 7.3 us for 512 tiles
+    // of 8 steps, 10.9 / 8.8 for 513.
     if (g.max_tiles * panels(64) > 512) return launch_kernel<T, kGroupTileRows, 64, 2, 2, 2, 2, EPI>(g, heads, s);
     return launch_kernel<T, kGroupTileRows, 64, 2, 2, 4, 4, EPI>(g, heads, s);
 }
 
 template <typename T>
 Form form_of(const GemmArgs& g) {
-    const int steps = g.K * (int)sizeof(T) / 128;
     if (!tile_offsets_fit(g, sizeof(T))) return Form::kWide;
-    if constexpr (sizeof(T) == 2) return fastest_form(kTimesBf16, g, steps);
-    else return fastest_form(kTimesFloat, g, steps);
+    if constexpr (sizeof(T) == 2) return fastest_form(kTimesBf16, g, sizeof(T));
+    else return fastest_form(kTimesFloat, g, sizeof(T));
 }
 
 template <typename T, Epilogue EPI, typename X>
