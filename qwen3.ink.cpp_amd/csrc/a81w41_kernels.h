@@ -71,7 +71,8 @@ bool gemv_pair_fits(int N, int K);
 hipError_t launch_gemv_add_norm_silu_pair(const float* x, const GemvPrologue& pro, const void* B_gate_up, int N, int K,
                                           hipStream_t s);
 int gemv_waves_per_group_log2(int nb_n, int nb_k, bool paired_output);
-// At most `budget` bytes of what such a launch reads first: the same share of the first weights of each of its workgroups.
+// At most `budget` bytes of what a launch for one row reads first: the same share of the first weights of each of its workgroups.
+// paired_output: the launch above where gemv_pair_fits.
 WeightsAhead::Part gemv_weights_ahead(const void* B, int N, int K, bool paired_output, size_t budget);
 
 // ---- chains of overlapping launches, host side (chain.hip; the device side is in chain.h) ----------------------

@@ -360,6 +360,7 @@ int gemv_waves_per_group_log2(int nb_n, int nb_k, bool paired_output) {
 
 WeightsAhead::Part gemv_weights_ahead(const void* B, int N, int K, bool paired_output, size_t budget) {
     const int nb_n = N / 8, nb_k = K / 64;
+    paired_output = paired_output && gemv_pair_fits(N, K);
     // groups of a workgroup's first round; of a pair the four gate groups of a workgroup, which lie together, and the four of up
     const int groups = paired_output ? 4 : pick_tune(nb_n, nb_k).waves >> gemv_waves_per_group_log2(nb_n, nb_k, false);
     WeightsAhead::Part part;

@@ -183,6 +183,10 @@ def test_weights_read_ahead_stay_in_the_matrix(pkg, room):
                 if room == 1 << 40 and rows % 512 == 0:
                     assert got == whole
     assert L.a81w41_gemv_ahead_selfcheck(7, 64, 0, 0, C.byref(end)) < 0
+    # gate and up whose output is no product in one launch (sizes that are no multiple of 64, rows too long for its prologue): the plain launch's
+    for N, K in [(80, 64), (2 * 3112, 1024), (2 * 1000, 4096), (8192, 65536)]:
+        plain, paired = ((L.a81w41_gemv_ahead_selfcheck(N, K, gate_up, room, C.byref(end)), end.value) for gate_up in (0, 1))
+        assert plain == paired, (N, K)
 
 
 def test_strides_past_32_bit_offsets_have_a_kernel(pkg):
