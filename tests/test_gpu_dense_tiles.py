@@ -8,8 +8,17 @@ from tests import takosun_fixture as tx
 pytestmark = pytest.mark.gpu
 
 
-# 256 x 256 tiles; 128 x 128 two per CU; 128 x 128 alone on a CU with four stages, from fewer steps than stages on; 64 x 64, more of
-# them than fit two on every CU
+FORMS = ["256 x 256", "128 x 256", "128 x 128", "64 x 128", "64 x 64, four stages", "64 x 64, two stages", "64 x 32", "64-bit offsets"]
+
+
+def form_of(pkg, M, N, K, dtype="bfloat16"):
+    """The kernel of a product whose rows are as long as K, padded."""
+    step = 64 if dtype == "bfloat16" else 32
+    ld = -(-K // step) * step
+    return FORMS[pkg.capi.dense().a81w41_dense_form_selfcheck(M, N, K, ld, ld, dtype == "bfloat16")]
+
+
+# Ragged rows and columns, by 64 x 64 tiles with two stages but for 256 x 256 (1793 rows) and 128 x 128 (1921), against few rows of them
 @pytest.mark.parametrize("M,N,K", [(2047, 6136, 64), (1793, 6400, 192), (2300, 2050, 128), (2045, 2000, 64), (2045, 1990, 192),
                                    (1921, 2048, 320), (1025, 1990, 64), (1030, 2048, 192), (700, 3070, 320)])
 def test_rows_of_a_product(pkg, M, N, K):
@@ -21,11 +30,12 @@ def test_rows_of_a_product(pkg, M, N, K):
     want = a.double() @ w.double().t()
     # K exact products of size about 1, K sums rounded to 24 bits
     assert (got.double() - want).abs().max().item() <= K * 2.0 ** -24 * 4 * K ** 0.5
+    assert form_of(pkg, M, N, K) == {1793: FORMS[0], 1921: FORMS[2]}.get(M, FORMS[5])
     for m in (1, 32, 33, 64, 65, 100):   # the kernel for few rows and, where the product is wide, 64 x 64 tiles
         assert torch.equal(pkg.ops.dense_gemm(a[M - m:], w, K), got[M - m:]), m
 
 
-# The float forms of 128 x 128, two per CU, one per CU and 64 x 64.
+# In float: 64 x 64 tiles with two stages, against few rows of them.
 @pytest.mark.parametrize("M,N,K", [(2300, 2050, 32), (2047, 4100, 96), (2045, 1990, 160), (1025, 1990, 64)])
 def test_rows_of_a_float_product(pkg, M, N, K):
     import torch
@@ -39,7 +49,7 @@ def test_rows_of_a_float_product(pkg, M, N, K):
 
 
 # Steps of 128 bytes of K around the ring lengths of the kernel for few rows, 10 stages of rows and 20 of weights, and past them; one and
-# two row tiles, ragged columns.  The same rows among many more go through 64 x 64 and 128 x 128 tiles.
+# two row tiles, ragged columns.  The same rows among many more go through 64 x 128 and 128 x 128 tiles, in float 64 x 64.
 @pytest.mark.parametrize("steps", [9, 10, 11, 19, 20, 21, 22, 97])
 @pytest.mark.parametrize("M,N", [(33, 784), (65, 1990)])
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
@@ -51,6 +61,7 @@ def test_few_rows_around_the_ring(pkg, steps, M, N, dtype):
     a = torch.randn(2047, K, device="cuda", generator=g).to(getattr(torch, dtype))
     w = torch.randn(N, K, device="cuda", generator=g).to(getattr(torch, dtype))
     got = pkg.ops.dense_gemm(a[:M], w, K)
+    assert form_of(pkg, M, N, K, dtype) == FORMS[6] and form_of(pkg, 2047, N, K, dtype) in FORMS[2:6]
     # K products (exact in bfloat16) and K sums, rounded to 24 bits
     bound = (1 if bf16 else 2) * K * 2.0 ** -24 * 4 * K ** 0.5
     assert (got.double() - a[:M].double() @ w.double().t()).abs().max().item() <= bound
@@ -73,8 +84,11 @@ def _same_in_portions(pkg, cfg, n, cuts):
     assert np.isfinite(whole).all() and np.array_equal(whole, np.concatenate(parts))
 
 
-def test_gated_pairs_on_large_tiles(pkg):
-    cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.dense(6100))])
+# one step of K, which goes by 64 x 64 tiles, and four and eleven, by 256 x 256
+@pytest.mark.parametrize("width", [64, 256, 704])
+def test_gated_pairs_on_large_tiles(pkg, width):
+    assert form_of(pkg, 2100, 12224, width) == FORMS[5 if width == 64 else 0]
+    cfg = tx.config(64, width, 1, [tx.layer(tx.mixer(2, 8, 8, 8, 16, 24, 0.3), tx.dense(6100))])
     _same_in_portions(pkg, cfg, 2100, 100)
 
 
@@ -83,8 +97,12 @@ def test_experts_on_many_small_tiles(pkg):
     _same_in_portions(pkg, cfg, 2100, 100)
 
 
-def test_head_columns_on_large_tiles(pkg):
-    cfg = dx.config(64, 64, [dx.attention(32, 8, 128, 128, 70, 0.09, rot_dims=64, mlp=None)], (0, 1, 1))
+# one step of K, which goes by 64 x 64 tiles, and three and four, by 256 x 256; columns behind the heads, five of them, are no whole fours
+@pytest.mark.parametrize("width,experts", [(64, 0), (192, 0), (256, 5)])
+def test_head_columns_on_large_tiles(pkg, width, experts):
+    assert form_of(pkg, 2100, 6144 + experts, width) == FORMS[5 if width == 64 else 0]
+    mlp = dx.moe(experts, 2, 16) if experts else None
+    cfg = dx.config(64, width, [dx.attention(32, 8, 128, 128, 70, 0.09, rot_dims=64, mlp=mlp)], (0, 1, 1))
     _same_in_portions(pkg, cfg, 2100, 100)
 
 
@@ -245,8 +263,8 @@ def test_one_token_rows(pkg, width):
         assert np.linalg.norm(got[i] - want) <= 3e-5 * np.linalg.norm(want), i
 
 
-# Sizes of one round of 128 x 256 tiles, of 64 x 256 and of 64 x 128, three stages each, ragged rows and columns: fewer steps than stages, as many
-# and more for 64 x 256; the others are taken from some steps on, below, and these K lie on both sides of the line
+# Ragged rows and columns over K on both sides of the lines between 64 x 64 and larger tiles: 128 x 256 from two steps on (2045 rows); 64 x 64 with
+# two stages, four and 64 x 128 (1000); 64 x 64 with two stages for all of them (300, and all in float)
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 448])
 @pytest.mark.parametrize("M,N", [(2045, 3100), (300, 12280), (1000, 2000)])
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
@@ -264,13 +282,14 @@ def test_one_round_of_tiles(pkg, M, N, K, dtype):
     assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
 
 
-# 256 x 256 tiles, whose rings of A and W have two and three stages: fewer steps than stages, as many, more; rows of C that take four columns
-# at a time and rows that do not.
+# 256 x 256 tiles, whose rings of A and W have two and three stages: fewer steps than stages of W, as many, more (one step goes by 64 x 64 tiles);
+# rows of C that take four columns at a time and rows that do not.
 @pytest.mark.parametrize("N", [4096, 4094, 4093])
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 9])
 def test_rings_of_two_lengths(pkg, N, steps):
     import torch
     g, K, M = torch.Generator(device="cuda").manual_seed(steps), 64 * steps, 4090
+    assert form_of(pkg, M, N, K) == FORMS[0 if steps > 1 else 5]
     a = torch.randn(M, K, device="cuda", generator=g).bfloat16()
     w = torch.randn(N, K, device="cuda", generator=g).bfloat16()
     got = pkg.ops.dense_gemm(a, w, K)
@@ -279,16 +298,19 @@ def test_rings_of_two_lengths(pkg, N, steps):
     assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:])
 
 
-# The tile that the estimate of times takes, in each of its forms: as few steps as lead to it and one more, ragged rows and columns: 256 x 256;
-# 128 x 256; 128 x 128; 64 x 128; 64 x 64 with four stages and with two; the last two in float
-@pytest.mark.parametrize("M,N,steps", [(4090, 4093, 3), (4090, 4093, 4), (1921, 4093, 2), (2045, 4093, 3), (1000, 3100, 8), (1025, 3100, 9),
-                                       (300, 12280, 2), (129, 6136, 3), (3000, 6136, 8), (65, 6136, 1), (65, 6136, 3), (65, 6136, 4),
-                                       (500, 4093, 5), (129, 12280, 1), (1025, 1990, 2), (2045, 8000, 3)])
+# The tile that the estimate of times takes, in each of its forms, the one in bfloat16 beside the sizes: as few steps as lead to it and one more, ragged
+# rows and columns; of 128 x 128 tiles as many steps as they have stages.  In float 64 x 64 with two stages, and with four.
+@pytest.mark.parametrize("M,N,steps,form", [
+    (4090, 4093, 2, 0), (4090, 4093, 3, 0), (4090, 4093, 4, 0), (2045, 8000, 3, 0), (1921, 4093, 1, 1), (1921, 4093, 2, 1), (2045, 4093, 3, 1), (3000, 6136, 8, 1),
+    (1000, 3100, 4, 2), (1000, 3100, 5, 2), (1000, 3100, 8, 2), (1025, 3100, 9, 2), (500, 4093, 5, 3), (500, 4093, 6, 3), (65, 12280, 5, 3), (65, 6136, 3, 4),
+    (65, 6136, 4, 4), (500, 4093, 4, 4), (300, 12280, 2, 5), (129, 6136, 3, 5), (65, 6136, 1, 5), (129, 12280, 1, 5), (1025, 1990, 2, 5), (65, 6136, 8, 4),
+    (65, 6136, 12, 4)])
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
-def test_each_form_of_tile(pkg, M, N, steps, dtype):
+def test_each_form_of_tile(pkg, M, N, steps, form, dtype):
     import torch
     bf16 = dtype == "bfloat16"
     K = steps * (64 if bf16 else 32)
+    assert form_of(pkg, M, N, K, dtype) == FORMS[form if bf16 else 4 if steps >= 8 and M == 65 else 5]
     g = torch.Generator(device="cuda").manual_seed(M + steps)
     a = torch.randn(M, K, device="cuda", generator=g).to(getattr(torch, dtype))
     w = torch.randn(N, K, device="cuda", generator=g).to(getattr(torch, dtype))
@@ -319,8 +341,8 @@ def test_rows_far_apart(pkg, dtype, M, N, lda, ldw):
         assert torch.equal(pkg.ops.dense_gated(near[0], near[1], K), pkg.ops.dense_gated(a, w, K))
 
 
-# The steps of K from which one round of 128 x 256 and of 64 x 128 tiles is taken, and those before: the same bits for a row in a call of
-# 33 rows, which goes through another kernel on either side.
+# Step by step of K: the same bits for a row in a call of 33 rows, which goes through another kernel.  128 x 256 tiles and 64 x 64 with two stages and
+# four; in float 64 x 64 with two.
 @pytest.mark.parametrize("M,N,dtype,steps", [(2045, 3100, "bfloat16", (10, 11, 12, 13)), (2045, 3100, "float32", (5, 6, 7)),
                                              (1000, 2000, "bfloat16", (2, 3, 4)), (1000, 2000, "float32", (2, 3))])
 def test_one_round_from_some_steps_on(pkg, M, N, dtype, steps):
@@ -337,9 +359,10 @@ def test_one_round_from_some_steps_on(pkg, M, N, dtype, steps):
         assert torch.equal(pkg.ops.dense_gemm(a[M - 33:], w, K), got[M - 33:]), n
 
 
-# One round of 128 x 256 tiles over enough steps for it, with the epilogues of a prompt: queries turned and stored, gated units, columns of
+# 128 x 256 tiles over eleven steps, with the epilogues of a prompt: queries turned and stored, gated units, columns of
 # heads with what is no head's behind them; the same rows in portions go through small tiles.
 def test_epilogues_on_one_round_of_tiles(pkg):
+    assert form_of(pkg, 2045, 3072, 704) == form_of(pkg, 2045, 3104, 704) == FORMS[1]
     _same_in_portions(pkg, tx.config(64, 704, 1, [tx.layer(tx.mixer(16, 128, 64, 8, 704, 24, 0.1), tx.dense(1552))]), 2045, 100)
     _same_in_portions(pkg, dx.config(64, 704, [dx.attention(16, 4, 128, 128, 70, 0.09, rot_dims=64, mlp=None)], (0, 1, 1)), 2045, 100)
 
@@ -367,10 +390,12 @@ def test_gated_units_of_large_gates(pkg, tmp_path):
         assert err.max() <= tol, (dtype, err.max())
 
 
-# queries turned and stored by the product: heads of an odd and of an even width, on 256 x 256 and 128 x 128 tiles and on small ones
-@pytest.mark.parametrize("heads,dim,rot", [(41, 95, 62), (40, 96, 64), (9, 33, 2)])
-def test_query_columns_on_large_tiles(pkg, heads, dim, rot):
-    cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(heads, dim, rot, 8, 70, 24, 0.1), None)])
+# queries turned and stored by the product: heads of an odd and of an even width, on 256 x 256 tiles and on small ones
+@pytest.mark.parametrize("heads,dim,rot,rank,form", [(41, 95, 62, 70, 0), (40, 96, 64, 70, 5), (9, 33, 2, 70, 5), (41, 95, 62, 200, 0), (40, 96, 64, 200, 0),
+                                                     (9, 33, 2, 200, 4)])
+def test_query_columns_on_large_tiles(pkg, heads, dim, rot, rank, form):
+    assert form_of(pkg, 2100, heads * (dim + rot), rank) == FORMS[form]
+    cfg = tx.config(64, 64, 1, [tx.layer(tx.mixer(heads, dim, rot, 8, rank, 24, 0.1), None)])
     _same_in_portions(pkg, cfg, 2100, 100)
 
 
