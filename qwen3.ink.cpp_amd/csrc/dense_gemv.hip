@@ -655,7 +655,9 @@ struct AttendBeside {  // attention of a few rows of a key head, key and value c
 // limits; the token's mixer, a few workgroups of trips one behind the other, costs next to nothing beside it.  Dimesun, width 2048, behind 33 to
 // 64 tokens: attention 5.0 us and experts 12.2 in two launches, 11.8 in one; a memory's step 6.4 and 12.2, 12.4 in one.  32 tokens 7180 -> 6430 us,
 // width 1536 6200 -> 5400, 1024 4900 -> 4400, behind 1500 tokens 0.91 of the time.  Attention has one tile of keys in LDS here, where its own launch
-// has two, so that three workgroups still fit a CU; with up to eight shares of a chunk it walks few tiles.
+// has two, so that three workgroups still fit a CU.  A share then waits for each of its tiles, and is still done earlier than behind a launch of its own, also where
+// a chunk is long: chunks of 65536, two launches / one, us a token behind 1000, 4000 and 16000 tokens: 16 heads on 4 of 128 columns 167 / 135, 222 /
+// 184, 442 / 402; 32 on 8 of 64 161 / 133, 204 / 170, 385 / 350; width 512, 8 heads of 64, one expert of 8 103 / 88, 150 / 135, 303 / 290.
 template <typename T, typename Beside>
 __global__ __launch_bounds__(kThreads) void gemv_gate_up_kernel(const float* __restrict__ logits, const float* __restrict__ bias, const float* __restrict__ h,
                                                                const T* __restrict__ experts, int routed, int top, int ld, int width, RowStep p,

@@ -541,8 +541,9 @@ int DimesunModel<T>::mixer_and_experts_one_token(const Layer& L, const LayerConf
     return experts_alone();
 }
 
-// The pass for one token, four launches a run: [residual step, norm, product of all that reads the norm], the mixer, [choice
-// of the experts, gate and up], [the mixer's norm and gate or the merge of its shares, output and down products].
+// The pass for one token, three launches a run: [residual step, norm, product of all that reads the norm], [the mixer beside choice
+// of the experts, gate and up], [the mixer's norm and gate or the merge of its shares, output and down products].  A mixer that does not
+// fit beside the experts, or whose layer has none, has a launch of its own.
 template <typename T>
 int DimesunModel<T>::enqueue_one_token(int n_want, hipStream_t s) {
     const int W = cfg_.width;
