@@ -397,10 +397,14 @@ hipError_t launch_attend_rows_prompt(const AttendArgs<bf16>& a, int heads, hipSt
 // the faster one all the same (us, against 16 x 16): 8 heads, 192 + 64 and 256 columns, 330 rows 36 / 51, 2000 rows 159 / 212.
 hipError_t launch_attend_expanded(const AttendArgs<bf16>& a, int heads, hipStream_t s) {
     const int dk = a.k_own_width + a.k_shared_width;
-    // Workgroups of 64 rows where there are no more than two for a CU, their keys in four groups of 32: a long prompt's last rows then have
-    // half as many turns.  us, so / with 128 rows in two groups of 64: 8 heads, 500 rows 16.5 / 20, 900 rows 22 / 28, 2048 rows 37 / 49; 16 heads, 2048
-    // rows 50 / 52; 12 heads, 180 rows 13 / 14.  More of them copy more: every workgroup has its keys to itself.
-    const bool few = (long long)heads * ((a.rows + 63) / 64) <= 512;
+    // Workgroups of 64 rows where there is no more than one for a CU, their keys in four groups of 32: a long prompt's last rows then have
+    // half as many turns.  us, so / with 128 rows in two groups of 64: 8 heads, 500 rows 16.5 / 20, 900 rows 22 / 28; 12 heads, 180 rows 13 / 14.
+    // More of them copy more, every workgroup having its keys to itself, and begin a second round: over 420 drawn calls, so / with 128 rows, up to 256 of them
+    // 0.70 to 1.0 but for 64 rows and fewer without a context before them (up to 1.09); 257 to 512 of them up to 1024 rows 1.08 to 1.44, past 1024 rows
+    // 0.72 to 0.87 up to 384 of them, 0.94 to 1.06 past that, and past 2048 rows 0.91: the last rows' turns count there.  8 heads, 2048 rows 37 / 49; 16
+    // heads 50 / 52.
+    const int most = a.rows <= 1024 ? 256 : a.rows < 2048 ? 384 : 512;
+    const bool few = (long long)heads * ((a.rows + 63) / 64) <= most;
     if (dk <= 128 && a.dv <= 64)
         return few ? launch_kernel<128, 64, 0, 4, 2, 32, true>(a, heads, s) : launch_kernel<128, 64, 0, 2, kQW, 64, true>(a, heads, s);
     if (dk <= 192 && a.dv <= 128)

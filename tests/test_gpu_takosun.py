@@ -167,8 +167,11 @@ def test_formed_attention(pkg, M, heads, dim, rot, vdim, pos):
 
 
 @pytest.mark.parametrize("M,heads,dim,rot,vdim,pos", [
-    (64, 512, 24, 8, 40, 5),                                             # the most heads whose 64 rows have a workgroup of their own
-    (129, 171, 40, 24, 33, 3), (257, 103, 128, 64, 128, 30), (65, 257, 16, 16, 8, 0)])   # and more: 128 rows a workgroup
+    (64, 512, 24, 8, 40, 5),
+    (129, 171, 40, 24, 33, 3), (257, 103, 128, 64, 128, 30), (65, 257, 16, 16, 8, 0),   # and more: 128 rows a workgroup
+    # the most workgroups of 64 rows up to 1024 rows, past them and from 2048 on, and more
+    (64, 256, 24, 8, 40, 5), (65, 128, 16, 16, 8, 0), (65, 129, 16, 16, 8, 0), (1025, 22, 24, 8, 12, 3), (1025, 23, 24, 8, 12, 3), (2048, 16, 16, 8, 8, 0),
+    (2047, 16, 16, 8, 8, 0)])
 def test_formed_attention_rows_of_a_workgroup(pkg, M, heads, dim, rot, vdim, pos):
     test_formed_attention(pkg, M, heads, dim, rot, vdim, pos)
 
