@@ -392,11 +392,12 @@ hipError_t launch_attention_prefill(const float* q, int q_row_stride, const void
     // its output).  One head and four splits where every workgroup gets a CU; two heads, whose tiles two waves share, while the longest
     // workgroup counts; the whole group where there are many rounds.  us with 1 / 2 / 4 heads: 180 tokens, 16 heads on 4, 9.0 / 10.0 / 12.4;
     // 322 tokens, 8 on 2 10.8 / 11.9 / 16.6, 32 on 8 (352, 176, 88 workgroups) 18.5 / 13.2 / 17.4; 900 tokens, 12 on 3 31.9 / 24.5 / 35.8;
-    // 2048 tokens, 8 on 2 76 / 45 / 72, 32 on 8 252 / 157 / 152; 3000 tokens - / 244 / 234.
+    // 2048 tokens, 8 on 2 76 / 45 / 72, 32 on 8 252 / 157 / 152; 3000 tokens - / 244 / 234.  With 64 heads and more, whose prompts have that many
+    // workgroups sooner, no two heads past one workgroup a CU: 64 on 8, 295 tokens - / 20.2 / 17.9, 509 30.6 / 26.0, 990 82 / 72.5; 64 on 16, 339 22.4 / 19.8.
     // A81W41_ATTENTION_HEADS=<G> fixes the heads per workgroup (measurement aid, tuning builds only).
     static const int env_g = tuning_env_int("A81W41_ATTENTION_HEADS");
     int g = 1;
-    while (g < group && (long long)tiles * n_kv * (group / g) > (g == 1 ? 256 : 1024)) g <<= 1;
+    while (g < group && (long long)tiles * n_kv * (group / g) > (g == 1 || (g == 2 && n_q >= 64) ? 256 : 1024)) g <<= 1;
     if (env_g > 0 && env_g <= group && group % env_g == 0) g = env_g;
     if (heads_per_workgroup > 0) {
         if (heads_per_workgroup > group || group % heads_per_workgroup) return hipErrorInvalidValue;

@@ -102,6 +102,18 @@ def test_edges_of_tiles_and_rounds(pkg, synth, torch, n_q, n_kv, M, pos):
         assert row_err(got, want) < TOL, variant
 
 
+@pytest.mark.parametrize("M", [128, 129, 256, 257])
+def test_heads_a_workgroup_of_many_heads(pkg, synth, torch, M):
+    """64 heads on 16: what the number of workgroups chooses, one head, two and all four of a group, to the last row that each takes."""
+    scale = 1.0 / np.sqrt(128.0)
+    q, k, v = make(synth, M, 3, 64, 16, M + 3, 940 + M)
+    want = reference(q, k.astype(np.float32), v.astype(np.float32), 3, 64, 16, scale)
+    got = run(pkg, torch, q, k, v, 3, 64, 16, scale, 2)
+    heads = {128: 1, 129: 2, 256: 2, 257: 4}[M]   # 256 workgroups of one head at 128 tokens, 256 of two at 256
+    assert row_err(got, want) < TOL
+    assert np.array_equal(got, run(pkg, torch, q, k, v, 3, 64, 16, scale, {1: 3, 2: 4, 4: 5}[heads]))
+
+
 def test_sharp_and_flat_rows(pkg, synth, torch):
     """Scores far apart (one key dominates) and all equal (uniform weights): the running-maximum
     bookkeeping across tiles and the masked entries of partial tiles."""
