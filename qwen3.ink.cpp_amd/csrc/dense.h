@@ -277,7 +277,6 @@ struct MemoryArgs {
     MemoryShape sh;
     const float* in = nullptr;  // [M][ld_in]
     int ld_in = 0, M = 0;
-    int ahead = 0;  // step by step: tokens behind pos_dev's that are in the state already
     const float *bias_i = nullptr, *bias_f = nullptr;  // [heads]
     const float* norm = nullptr;                       // [heads vdim]
     float* state = nullptr;
@@ -285,10 +284,11 @@ struct MemoryArgs {
     // prompt kernels: [chunks][heads][chunk_size], [chunks + 1][heads], [chunks][heads][2], and the gates of a chunk's tokens [chunks][heads][3][kMemoryChunk]
     float *chunk_states = nullptr, *chunk_m = nullptr, *chunk_stats = nullptr;
     double* chunk_gates = nullptr;
+    float* held = nullptr;  // token by token, [heads][dim + 1]: n and m between the two launches of an even number of tokens
 };
-// Token by token, any sizes: o [M][heads vdim] as it is.
+// Token by token, any sizes: o [M][heads vdim] as it is.  Behind an even number of tokens the state is whole after launch_memory_norm only.
 hipError_t launch_memory_steps(const MemoryArgs& a, float* o, hipStream_t s);
-// A row of o, per head divided by its root mean square, times norm, times sigmoid(g), as T.
+// A row of o, per head divided by its root mean square, times norm, times sigmoid(g), as T; also what launch_memory_steps held back.
 template <typename T>
 hipError_t launch_memory_norm(const MemoryArgs& a, const float* o, T* out, int ld_out, hipStream_t s);
 // A prompt in chunks on the matrix cores (32-bit products), the row's norm and gate included.

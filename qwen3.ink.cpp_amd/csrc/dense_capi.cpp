@@ -189,7 +189,7 @@ static size_t memory_chunk_floats(const MemoryShape& sh, size_t chunks) {
 size_t a81w41_matrix_memory_scratch(int heads, int dim, int vdim, int M) {
     const MemoryShape sh = memory_shape(heads, dim, vdim);
     const size_t chunks = (M + kMemoryChunk - 1) / kMemoryChunk, H = heads;
-    return std::max(memory_chunk_floats(sh, chunks) + 2 * chunks * H * 3 * kMemoryChunk, (size_t)M * H * vdim);
+    return std::max(memory_chunk_floats(sh, chunks) + 2 * chunks * H * 3 * kMemoryChunk, (size_t)M * H * vdim + H * (dim + 1));
 }
 
 int a81w41_matrix_memory(const float* in, int ld_in, int M, int heads, int dim, int vdim, float cap, float eps, const float* bias_i,
@@ -205,6 +205,7 @@ int a81w41_matrix_memory(const float* in, int ld_in, int M, int heads, int dim, 
     a.in = in, a.ld_in = ld_in, a.M = M, a.bias_i = bias_i, a.bias_f = bias_f, a.norm = norm, a.state = state, a.pos_dev = pos_dev;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (variant == 0) {
+        a.held = scratch + (size_t)M * heads * vdim;
         A81W41_HIP_TRY(launch_memory_steps(a, scratch, s));
         A81W41_HIP_TRY(launch_memory_norm<float>(a, scratch, out, heads * vdim, s));
         return 0;

@@ -244,6 +244,7 @@ class DimesunModel final : public DenseModel<T> {
     size_t part_rows_ = 0;
     float *chunk_states_ = nullptr, *chunk_m_ = nullptr, *chunk_stats_ = nullptr;
     double* chunk_gates_ = nullptr;
+    float* memory_held_ = nullptr;
     int *chosen_ = nullptr, *src_rows_ = nullptr, *slot_rows_ = nullptr, *n_tiles_ = nullptr;
     float* expert_weights_ = nullptr;
     GroupTile* tiles_ = nullptr;
@@ -344,7 +345,7 @@ int DimesunModel<T>::allocate(int max_seq) {
     A81W41_TRY(init_session(max_seq, cfg_.vocab, rows_));
     ld_h_ = pad_k<T>(cfg_.width);
     const size_t R = rows_, W = cfg_.width, chunks = (R + kMemoryChunk - 1) / kMemoryChunk;
-    size_t q = 0, act = 0, o_memory = 0, chunk_states = 0, tiles = 0;
+    size_t q = 0, act = 0, o_memory = 0, held = 0, chunk_states = 0, tiles = 0;
     int top = 0, heads = 0, memory_heads = 0, vdim = 0;
     one_token_fits_ = ld_h_ + 1 <= kGemvMaxRow;
     for (const LayerConfig& lc : cfg_.layers) {
@@ -353,6 +354,7 @@ int DimesunModel<T>::allocate(int max_seq) {
         int row = pad_k<T>(lc.mixer_width());
         if (lc.memory) {
             o_memory = std::max(o_memory, (size_t)lc.mixer_width());
+            held = std::max(held, (size_t)lc.mem.heads * (lc.mem.dim + 1));
             chunk_states = std::max(chunk_states, lc.mem.heads * lc.mem.chunk_size());
             memory_heads = std::max(memory_heads, lc.mem.heads);
             row += lc.mem.heads;
@@ -385,6 +387,7 @@ int DimesunModel<T>::allocate(int max_seq) {
     }
     if (memory_heads) {
         A81W41_TRY(allocate_array(R * o_memory, &o_memory_));
+        A81W41_TRY(allocate_array(held, &memory_held_));
         A81W41_TRY(allocate_array(chunks * chunk_states, &chunk_states_));
         A81W41_TRY(allocate_array((chunks + 1) * memory_heads, &chunk_m_));
         A81W41_TRY(allocate_array(chunks * memory_heads * 2, &chunk_stats_));
@@ -441,6 +444,7 @@ MemoryArgs DimesunModel<T>::memory_args(const Layer& L, const MemoryShape& sh, c
     a.sh = sh, a.in = in_, a.ld_in = ld_in, a.M = M, a.bias_i = L.bias_i, a.bias_f = L.bias_f, a.norm = L.memory_norm;
     a.state = kept.state, a.pos_dev = pos;
     a.chunk_states = chunk_states_, a.chunk_m = chunk_m_, a.chunk_stats = chunk_stats_, a.chunk_gates = chunk_gates_;
+    a.held = memory_held_;
     return a;
 }
 

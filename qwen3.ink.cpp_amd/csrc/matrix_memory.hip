@@ -58,6 +58,10 @@ __global__ __launch_bounds__(kThreads) void memory_norm_kernel(MemoryArgs a, con
     const int width = a.sh.heads * a.sh.vdim;
     float *inv = smem, *red = inv + a.sh.heads;
     const float *row = o + (size_t)blockIdx.x * width, *gate = a.in + (size_t)blockIdx.x * a.ld_in + a.sh.at_g;
+    if (steps_held_back(a)) {
+        float* to = state_nm(a, max(a.pos_dev[0], 0) + a.M);
+        for (int i = blockIdx.x * kThreads + threadIdx.x; i < a.sh.heads * (a.sh.dim + 1); i += gridDim.x * kThreads) to[i] = a.held[i];
+    }
     group_inverse_rms<kThreads>([&](int i) { return row[i]; }, width, a.sh.heads, a.sh.eps, inv, red);
     T* dst = out + (size_t)blockIdx.x * ld_out;
     for (int i = threadIdx.x; i < width; i += kThreads) dst[i] = (T)(row[i] * inv[i / a.sh.vdim] * a.norm[i] * sigmoid(gate[i]));
@@ -499,16 +503,9 @@ hipError_t launch_chunks(const MemoryArgs& a, T* out, int ld_out, hipStream_t s)
 
 }  // namespace
 
-hipError_t launch_memory_steps(const MemoryArgs& all, float* o, hipStream_t s) {
-    MemoryArgs a = all;
+hipError_t launch_memory_steps(const MemoryArgs& a, float* o, hipStream_t s) {
+    if (steps_held_back(a) && !a.held) return hipErrorInvalidValue;
     const dim3 grid((a.sh.vdim + kSlice - 1) / kSlice, a.sh.heads);
-    // Workgroups that start late may not find n and m overwritten (memory_steps.h): of an even number of tokens the last has a launch
-    // of its own.
-    if (grid.x > 1 && a.M % 2 == 0) {
-        a.M--;
-        if (hipError_t e = launch_memory_steps(a, o, s)) return e;
-        a.ahead += a.M, a.in += (size_t)a.M * a.ld_in, o += (size_t)a.M * a.sh.heads * a.sh.vdim, a.M = 1;
-    }
     auto lds = [&](int w) { return step_floats(a.sh.dim, w) * sizeof(float); };
     if (a.sh.vdim % 4 == 0)
         hipLaunchKernelGGL(memory_steps_kernel<4>, grid, dim3(kThreads), lds(4), s, a, o);

@@ -28,16 +28,17 @@ __device__ __forceinline__ float* state_nm(const MemoryArgs& a, int parity) {
 // Token by token.  A workgroup has kSlice columns of one head's S; W columns and every (kThreads W / kSlice)-th row of them
 // are a thread's, in registers only while a token uses them.  n and m are formed by every workgroup of the head; the first
 // writes them to the copy of the parity behind the tokens, which nobody reads if their number is odd.  With an even number it is the copy
-// that all of them start from, and a head must have one workgroup.
+// that all of them start from, also those that start when the first has ended: n and m are then held back for the launch behind (memory_norm_kernel).
 constexpr int kSlice = 32;
 // smem: step_floats(dim, W)
 __host__ __device__ inline int step_floats(int dim, int w) { return 3 * dim + kThreads * w + kThreads / 64; }
+__host__ __device__ inline bool steps_held_back(const MemoryArgs& a) { return a.M % 2 == 0 && a.sh.vdim > kSlice; }
 template <int W>
 __device__ __forceinline__ void memory_steps(const MemoryArgs& a, float* __restrict__ o, int slice, int h, float* smem) {
     constexpr int kPer = kSlice / W, kRows = kThreads / kPer;  // threads of a row of the slice, rows worked on at a time
     const MemoryShape sh = a.sh;
     float *n = smem, *q = n + sh.dim, *k = q + sh.dim, *sums = k + sh.dim, *red = sums + kRows * kSlice;
-    const int t = threadIdx.x, pos = max(a.pos_dev[0], 0) + a.ahead;
+    const int t = threadIdx.x, pos = max(a.pos_dev[0], 0);
     const int c = slice * kSlice + (t % kPer) * W, r0 = t / kPer;
     const bool mine = c < sh.vdim;  // W > 1: vdim is a multiple of W
     float* S = a.state + (size_t)h * sh.dim * sh.vdim;
@@ -98,7 +99,7 @@ __device__ __forceinline__ void memory_steps(const MemoryArgs& a, float* __restr
         __syncthreads();
     }
     if (slice == 0) {
-        float* out = state_nm(a, pos + a.M) + (size_t)h * (sh.dim + 1);
+        float* out = (steps_held_back(a) ? a.held : state_nm(a, pos + a.M)) + (size_t)h * (sh.dim + 1);
         for (int d = t; d < sh.dim; d += kThreads) out[d] = n[d];
         if (t == 0) out[sh.dim] = m;
     }
